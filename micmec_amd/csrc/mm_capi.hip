@@ -89,7 +89,7 @@ int build_param_table(int model, int32_t nrows, int32_t max_states, const int32_
       } else {
         voigt_average(c0 + ts * 81, e + kCvOffset);
       }
-      for (int q = 0; q < 36; ++q) e[kCvwOffset + q] = e[9] * e[kCvOffset + q];
+      metric_entry(h0 + ts * 9, e, e[9], e + kCvOffset, e + kMetricOffset, e + kRestOffset);
     }
   }
   return MM_OK;

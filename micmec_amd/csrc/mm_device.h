@@ -7,7 +7,7 @@
 //   B_a = h0^-1 M_a, eps_a = (B_a B_a^T - I)/2 (Green-Lagrange), u_a = eps_a : C0 : eps_a / 2.
 // The gradient is the adjoint of that chain: dE/dB = S B with S the symmetric stress built from
 // the Voigt vector C e, and dE/dM = h0^-T dE/dB; it equals the derivative-table route of
-// nanocell.py:98-132.
+// nanocell.py:98-132. The force kernels evaluate both in the metric of the edges (state_stress).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -21,10 +21,13 @@ namespace mm {
 //   [10]     free energy of the state
 //   [11]     unused
 //   [12..47] Voigt matrix Cv[6][6] (row-major), averaged over index orderings
-//   [48..83] w * Cv, the weighted matrix of the force kernels
-constexpr int kTabStride = 84;
+//   [48..83] K = T^T (w Cv) T, the weighted matrix of the force kernels (metric_entry)
+//   [84..89] rest metric R = h0 h0^T: R00/2, R11/2, R22/2, R12, R02, R01
+//   [90..91] unused
+constexpr int kTabStride = 92;
 constexpr int kCvOffset = 12;
-constexpr int kCvwOffset = 48;
+constexpr int kMetricOffset = 48;
+constexpr int kRestOffset = 84;
 
 // 3x3 inverse (row-major) by cofactors; returns the determinant. Shared by the host and the
 // device table builders, without contraction, so both round the same way.
@@ -46,6 +49,45 @@ __host__ __device__ inline double inverse3_cof(const double* h, double* inv) {
   return det;
 }
 
+// K and R of one table entry from h0, P = h0^-1, w and Cv. T maps the Gram entries e6 to the
+// engineering strain: eps_ij = sum_ab P_ia P_jb e_ab, i.e. with (i,j) and (a,b) the pairs of
+// rows I and columns J, T_IJ = P_ia P_ja (a = b) or (P_ia P_jb + P_ib P_ja) / 2 (a != b, where
+// e6 holds 2 e_ab), doubled for the shear rows I >= 3. Shared by the host and the device table
+// builders, without contraction, so both round the same way.
+__host__ __device__ inline void metric_entry(const double* h0, const double* P, double w,
+                                             const double* Cv, double* K, double* R) {
+#pragma clang fp contract(off)
+  const int pi[6] = {0, 1, 2, 1, 0, 0}, pj[6] = {0, 1, 2, 2, 2, 1};
+  double T[36], CT[36];
+  for (int I = 0; I < 6; ++I) {
+    const double* a = P + 3 * pi[I];
+    const double* b = P + 3 * pj[I];
+    for (int J = 0; J < 6; ++J) {
+      const double cross = a[pi[J]] * b[pj[J]] + a[pj[J]] * b[pi[J]];
+      T[6 * I + J] = (I < 3) == (J < 3) ? (I < 3 ? a[pi[J]] * b[pi[J]] : cross)
+                                        : (I < 3 ? 0.5 * cross : cross);
+    }
+  }
+  for (int I = 0; I < 6; ++I)
+    for (int J = 0; J < 6; ++J) {
+      double t = 0.0;
+      for (int L = 0; L < 6; ++L) t += (w * Cv[6 * I + L]) * T[6 * L + J];
+      CT[6 * I + J] = t;
+    }
+  for (int I = 0; I < 6; ++I)
+    for (int J = 0; J < 6; ++J) {
+      double t = 0.0;
+      for (int L = 0; L < 6; ++L) t += T[6 * L + I] * CT[6 * L + J];
+      K[6 * I + J] = t;
+    }
+  for (int I = 0; I < 6; ++I) {
+    const double* a = h0 + 3 * pi[I];
+    const double* b = h0 + 3 * pj[I];
+    const double r = (a[0] * b[0] + a[1] * b[1]) + a[2] * b[2];
+    R[I] = I < 3 ? 0.5 * r : r;
+  }
+}
+
 // Edge endpoints: corner a, axis d -> lower / upper corner of the edge along d through a.
 __device__ constexpr int kLo[8][3] = {
     {0, 0, 0}, {0, 1, 1}, {2, 0, 2}, {3, 3, 0}, {2, 1, 4}, {3, 5, 1}, {6, 3, 2}, {6, 5, 4}};
@@ -61,145 +103,253 @@ __device__ constexpr int kEdgeHi[12] = {1, 4, 5, 7, 2, 4, 6, 7, 3, 5, 6, 7};
 __device__ constexpr int kEdge[8][3] = {{0, 4, 8},  {0, 5, 9},  {1, 4, 10}, {2, 6, 8},
                                         {1, 5, 11}, {2, 7, 9},  {3, 6, 10}, {3, 7, 11}};
 
-// Strain energy density of one corner (or of the averaged matrix) and, if kGrad, the
-// derivative with respect to the corner matrix M, both for one (type, state) entry `tab`.
-// M is given row-major (rows = edges). Returns u = e.Cv.e / 2; writes G = dU/dM (unscaled).
-// kVir: also adds the corner's virial G^T M = (S B)^T B = B^T S B (P M = B; symmetric) to
-// V[6] = (00, 11, 22, 12, 02, 01) — the sum over its edges of dU/d(edge) (x) edge, which is what
-// the vertex gradients give as sum_v g_v (x) r_v — without forming G when kGrad is false.
-template <bool kGrad, bool kVir = false>
-__device__ __forceinline__ double corner_energy(const double* __restrict__ tab, const double M[9],
-                                                double G[9], int cv_offset = kCvOffset,
-                                                double* V = nullptr) {
-  const double* P = tab;
-  double B[9];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      B[3 * i + j] = P[3 * i + 0] * M[0 + j] + P[3 * i + 1] * M[3 + j] + P[3 * i + 2] * M[6 + j];
-    }
+// A cell's energy in the metric of its edges. With M_a the corner matrix (rows = edges) and
+// G = M M^T its Gram matrix, the Green-Lagrange strain of the corner is
+//   eps = (P M M^T P^T - I)/2 = P e P^T,  e = (G - h0 h0^T)/2,
+// linear in G, so the energy w u = e6 . K e6 / 2 and the stress S6 = K e6 need only the Gram
+// entries e6 = (e00, e11, e22, 2 e12, 2 e02, 2 e01) and one matrix K = T^T (w Cv) T per (type,
+// state), T the map of e6 to the engineering strain (metric_entry); and dU/dM = S M with S the
+// symmetric matrix of S6. No B = P M and no products with P remain per corner, an edge's
+// length is shared by its two corners, and several states share the whole geometry: about 830
+// FP64 instructions a cell instead of 1500 for one state.
+//
+// kModel 0 (corner8, nanocell.py) has 8 corners and 12 edges, kModel 1 (original,
+// nanocell_original.py) one averaged corner with 3 edges H_d (the mean of the four edges along d).
+template <int kModel>
+struct Frame {
+  static constexpr int NC = kModel == 0 ? 8 : 1;
+  static constexpr int NE = kModel == 0 ? 12 : 3;
+  // the i-th corner: neighbours on the cube follow each other, so that an edge's two corners
+  // come close together and few edges are open at a time
+  __device__ static constexpr int corner(int i) {
+    constexpr int kOrder[8] = {0, 1, 4, 2, 3, 5, 7, 6};
+    return kModel == 0 ? kOrder[i] : 0;
   }
-  // Q = B B^T; engineering strain e = (eps00, eps11, eps22, 2eps12, 2eps02, 2eps01)
-  double e[6];
-  e[0] = 0.5 * (B[0] * B[0] + B[1] * B[1] + B[2] * B[2] - 1.0);
-  e[1] = 0.5 * (B[3] * B[3] + B[4] * B[4] + B[5] * B[5] - 1.0);
-  e[2] = 0.5 * (B[6] * B[6] + B[7] * B[7] + B[8] * B[8] - 1.0);
-  e[3] = B[3] * B[6] + B[4] * B[7] + B[5] * B[8];
-  e[4] = B[0] * B[6] + B[1] * B[7] + B[2] * B[8];
-  e[5] = B[0] * B[3] + B[1] * B[4] + B[2] * B[5];
-  const double* Cv = tab + cv_offset;
-  double s[6];
+  __device__ static constexpr int rank(int a) {
+    constexpr int kRank[8] = {0, 1, 3, 4, 2, 5, 7, 6};
+    return kRank[a];
+  }
+  __device__ static constexpr int edge(int a, int d) { return kModel == 0 ? kEdge[a][d] : d; }
+  // the two axes of off-diagonal entry q: 12, 02, 01
+  __device__ static constexpr int axis0(int q) { return q == 0 ? 1 : 0; }
+  __device__ static constexpr int axis1(int q) { return q == 2 ? 1 : 2; }
+  // axis along which edge e runs, and the ranks of its first and last corner
+  __device__ static constexpr int along(int e) { return kModel == 0 ? e / 4 : e; }
+  __device__ static constexpr int first(int e) {
+    return kModel != 0 ? 0 : rank(kEdgeLo[e]) < rank(kEdgeHi[e]) ? rank(kEdgeLo[e]) : rank(kEdgeHi[e]);
+  }
+  __device__ static constexpr int last(int e) {
+    return kModel != 0 ? 0 : rank(kEdgeLo[e]) > rank(kEdgeHi[e]) ? rank(kEdgeLo[e]) : rank(kEdgeHi[e]);
+  }
+};
+
+// Stress of the i-th corner from its strain x: the diagonal entries are added to their edges' D,
+// the off-diagonal ones go to O, and their energy terms to u.
+template <int kModel>
+__device__ __forceinline__ void corner_stress(const double* __restrict__ K, int i,
+                                              const double (&x)[6],
+                                              double (&D)[Frame<kModel>::NE], double (&O)[3],
+                                              double& u) {
+#pragma clang fp contract(off)
+  using F = Frame<kModel>;
 #pragma unroll
   for (int I = 0; I < 6; ++I) {
-    s[I] = Cv[6 * I + 0] * e[0] + Cv[6 * I + 1] * e[1] + Cv[6 * I + 2] * e[2] +
-           Cv[6 * I + 3] * e[3] + Cv[6 * I + 4] * e[4] + Cv[6 * I + 5] * e[5];
+    const int e = I < 3 ? F::edge(F::corner(i), I) : 0;
+    double t = I < 3 && F::first(e) < i ? __builtin_fma(K[6 * I], x[0], D[e]) : K[6 * I] * x[0];
+#pragma unroll
+    for (int J = 1; J < 6; ++J) t = __builtin_fma(K[6 * I + J], x[J], t);
+    if (I < 3) D[e] = t;
+    else O[I < 3 ? 0 : I - 3] = t;
   }
-  const double u = 0.5 * (e[0] * s[0] + e[1] * s[1] + e[2] * s[2] + e[3] * s[3] + e[4] * s[4] +
-                          e[5] * s[5]);
-  if (kGrad || kVir) {
-    // S (symmetric): S00=s0 S11=s1 S22=s2 S12=s3 S02=s4 S01=s5 ; T = S B ; G = P^T T
-    const double S[9] = {s[0], s[5], s[4], s[5], s[1], s[3], s[4], s[3], s[2]};
-    double T[9];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        T[3 * i + j] = S[3 * i + 0] * B[0 + j] + S[3 * i + 1] * B[3 + j] + S[3 * i + 2] * B[6 + j];
-      }
-    }
-    if (kGrad) {
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          G[3 * i + j] = P[0 + i] * T[0 + j] + P[3 + i] * T[3 + j] + P[6 + i] * T[6 + j];
-        }
-      }
-    }
-    if (kVir) {
-      // (T^T B)_kl = sum_i T_ik B_il
-      constexpr int kK[6] = {0, 1, 2, 1, 0, 0}, kL[6] = {0, 1, 2, 2, 2, 1};
-#pragma unroll
-      for (int q = 0; q < 6; ++q)
-        V[q] += T[0 + kK[q]] * B[0 + kL[q]] + T[3 + kK[q]] * B[3 + kL[q]] + T[6 + kK[q]] * B[6 + kL[q]];
-    }
-  }
-  return u;
+  for (int o = 0; o < 3; ++o) u = __builtin_fma(x[3 + o], O[o], u);
 }
 
-// Energy of one metastable state of a cell (without the free-energy offset) and, if kGrad,
-// the gradient with respect to the eight vertices, accumulated (scaled by gscale) into g[8][3].
-// The weight w enters through the weighted Voigt matrix w Cv, so the corner terms come out
-// already multiplied by w. kUnit: gscale is 1 (single-state cells) and is not applied.
-// kModel: 0 = corner8 (nanocell.py), 1 = original (nanocell_original.py).
-// kVir: also adds the state's virial sum_v g_v (x) r_v, as the sum of its corners' B^T S B
-// (see corner_energy; for the averaged matrix H the vertex rows are +-1/4 of dU/dH and
-// sum_v +-r_v along d is 4 H_d, so the same form), to V[6] — unscaled by gscale.
-template <int kModel, bool kGrad, bool kUnit = false, bool kVir = false>
-__device__ __forceinline__ double state_energy(const double* __restrict__ tab, const double r[8][3],
-                                               double g[8][3], double gscale = 1.0,
-                                               double* V = nullptr) {
-  if (kModel == 0) {
-    // the twelve edges once (each is a row of two corner matrices)
-    double E[12][3];
+// Off-diagonal strain o of the corner with edges E: their dot product less the rest metric's.
+__device__ __forceinline__ double edge_dot(const double (&A)[3], const double (&B)[3], double g0) {
+#pragma clang fp contract(off)
+  return __builtin_fma(A[2], B[2], __builtin_fma(A[1], B[1], __builtin_fma(A[0], B[0], -g0)));
+}
+__device__ __forceinline__ double edge_square(const double (&A)[3]) {
+#pragma clang fp contract(off)
+  return __builtin_fma(A[2], A[2], __builtin_fma(A[1], A[1], A[0] * A[0]));
+}
+
+// Energy (weighted, without the free-energy offset) and stress of one (type, state) at all
+// corners, from the edges E and their squared lengths s: D[e] = the diagonal stress along edge
+// e summed over its corners, O[a][q] the off-diagonal stresses of corner a. The sums are fused
+// multiply-adds in a fixed order, so every kernel that evaluates a state gets the same bits.
+template <int kModel>
+__device__ __forceinline__ double state_stress(const double* __restrict__ tab,
+                                               const double (&E)[Frame<kModel>::NE][3],
+                                               const double (&s)[Frame<kModel>::NE],
+                                               double (&D)[Frame<kModel>::NE],
+                                               double (&O)[Frame<kModel>::NC][3]) {
+#pragma clang fp contract(off)
+  using F = Frame<kModel>;
+  const double* g0 = tab + kRestOffset;
+  double u = 0.0;
 #pragma unroll
-    for (int e = 0; e < 12; ++e)
+  for (int i = 0; i < F::NC; ++i) {
+    const int a = F::corner(i);
+    double x[6];
 #pragma unroll
-      for (int j = 0; j < 3; ++j) E[e][j] = r[kEdgeHi[e]][j] - r[kEdgeLo[e]][j];
-    double usum = -0.0;
+    for (int d = 0; d < 3; ++d) x[d] = __builtin_fma(0.5, s[F::edge(a, d)], -g0[d]);
 #pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      double M[9], G[9];
+    for (int o = 0; o < 3; ++o)
+      x[3 + o] = edge_dot(E[F::edge(a, F::axis0(o))], E[F::edge(a, F::axis1(o))], g0[3 + o]);
+    corner_stress<kModel>(tab + kMetricOffset, i, x, D, O[a], u);
 #pragma unroll
-      for (int d = 0; d < 3; ++d) {
+    for (int d = 0; d < 3; ++d)
+      if (F::last(F::edge(a, d)) == i) u = __builtin_fma(x[d], D[F::edge(a, d)], u);
+    asm("" : "+v"(u));
+  }
+  return 0.5 * u;
+}
+
+// The virial sum_e gE_e (x) E_e (= sum_a M^T S M, symmetric) as (00, 11, 22, 12, 02, 01).
+__device__ __forceinline__ void edge_virial(const double (&gE)[3], const double (&E)[3],
+                                            double (&vir)[6]) {
+#pragma clang fp contract(off)
+  constexpr int kK[6] = {0, 1, 2, 1, 0, 0}, kL[6] = {0, 1, 2, 2, 2, 1};
 #pragma unroll
-        for (int j = 0; j < 3; ++j) M[3 * d + j] = E[kEdge[a][d]][j];
-      }
-      usum += corner_energy<kGrad, kVir>(tab, M, G, kCvwOffset, V);
-      if (kGrad) {
+  for (int v = 0; v < 6; ++v) vir[v] = __builtin_fma(gE[kK[v]], E[kL[v]], vir[v]);
+}
+
+// An edge pulls at its upper corner and pushes at its lower one (averaged model: a quarter of
+// H_d's derivative at every corner). g starts at -0.0, the identity of addition.
+template <int kModel>
+__device__ __forceinline__ void edge_to_vertices(int e, const double (&gE)[3],
+                                                 double (&g)[8][3]) {
+#pragma clang fp contract(off)
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
+  for (int j = 0; j < 3; ++j) {
+    if (kModel == 0) {
+      g[kEdgeHi[e]][j] += gE[j];
+      g[kEdgeLo[e]][j] -= gE[j];
+    } else {
+      const double t = 0.25 * gE[j];
 #pragma unroll
-          for (int j = 0; j < 3; ++j) {
-            const double v = kUnit ? G[3 * d + j] : gscale * G[3 * d + j];
-            g[kHi[a][d]][j] += v;
-            g[kLo[a][d]][j] -= v;
-          }
-        }
-      }
+      for (int v = 0; v < 8; ++v) g[v][j] += kOff[v][e] ? t : -t;
     }
-    return usum;
-  } else {
-    // H = (1/8) sum_a M_a: row d is a quarter of the sum of the four edges along d.
-    double H[9], G[9];
+  }
+}
+
+// dU/d(edge) of every edge from the stresses, gE_e = D_e E_e + the rows of S M off the diagonal,
+// its share of the virial, and with kGrad of the vertex gradient g.
+template <int kModel, bool kGrad>
+__device__ __forceinline__ void edge_gradient(const double (&E)[Frame<kModel>::NE][3],
+                                              const double (&D)[Frame<kModel>::NE],
+                                              const double (&O)[Frame<kModel>::NC][3],
+                                              double (&vir)[6], double (&g)[8][3]) {
+#pragma clang fp contract(off)
+  using F = Frame<kModel>;
+  double gE[F::NE][3];
+#pragma unroll
+  for (int i = 0; i < F::NC; ++i) {
+    const int a = F::corner(i);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
+      const int e = F::edge(a, d);
+      if (F::first(e) == i) {
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        double acc = 0.0;
-#pragma unroll
-        for (int a = 0; a < 8; ++a) acc += r[kHi[a][d]][j] - r[kLo[a][d]][j];
-        H[3 * d + j] = 0.125 * acc;
+        for (int j = 0; j < 3; ++j) gE[e][j] = D[e] * E[e][j];
       }
     }
-    const double u = corner_energy<kGrad, kVir>(tab, H, G, kCvwOffset, V);
-    if (kGrad) {
-      const double q = kUnit ? 0.25 : 0.25 * gscale;
 #pragma unroll
-      for (int v = 0; v < 8; ++v) {
+    for (int o = 0; o < 3; ++o) {
+      const int e0 = F::edge(a, F::axis0(o)), e1 = F::edge(a, F::axis1(o));
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
+      for (int j = 0; j < 3; ++j) {
+        gE[e0][j] = __builtin_fma(O[a][o], E[e1][j], gE[e0][j]);
+        gE[e1][j] = __builtin_fma(O[a][o], E[e0][j], gE[e1][j]);
+      }
+    }
 #pragma unroll
-          for (int j = 0; j < 3; ++j) {
-            const double t = q * G[3 * d + j];
-            g[v][j] += kOff[v][d] ? t : -t;
-          }
+    for (int d = 0; d < 3; ++d) {
+      const int e = F::edge(a, d);
+      if (F::last(e) == i) {
+        edge_virial(gE[e], E[e], vir);
+        if (kGrad) edge_to_vertices<kModel>(e, gE[e], g);
+      }
+    }
+  }
+}
+
+// Edge e of a cell: the difference of its corners' positions plus f * rv, the domain vector of
+// its axis when the cell wraps along it (f = 0 or 1).
+__device__ __forceinline__ void form_edge(const double (&p)[8][3], int e, double f,
+                                          const double* rv, double (&E)[3]) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+    E[j] = __builtin_fma(f, rv[j], p[kEdgeHi[e]][j] - p[kEdgeLo[e]][j]);
+}
+
+// One state of an eight-corner cell in one sweep over its corners: an edge is formed at its
+// first corner and gives its energy, virial and vertex terms at its second, so that at most five
+// of the twelve edges are held at a time (kOut as the cell pass's: 0 energy, 1 and virial, 2 and
+// vertex gradient). f, rv: wrap factors and domain vectors.
+template <int kOut>
+__device__ __forceinline__ double sweep_cell(const double* __restrict__ tab,
+                                             const double (&p)[8][3], const double (&f)[3],
+                                             const double (&rv)[9], double (&vir)[6],
+                                             double (&g)[8][3]) {
+#pragma clang fp contract(off)
+  using F = Frame<0>;
+  const double* g0 = tab + kRestOffset;
+  double E[12][3], q[12], D[12], gE[12][3];
+  double u = 0.0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int a = F::corner(i);
+    double x[6], O[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const int e = F::edge(a, d);
+      if (F::first(e) == i) {
+        form_edge(p, e, f[d], &rv[3 * d], E[e]);
+        q[e] = __builtin_fma(0.5, edge_square(E[e]), -g0[d]);
+      }
+      x[d] = q[e];
+    }
+#pragma unroll
+    for (int o = 0; o < 3; ++o)
+      x[3 + o] = edge_dot(E[F::edge(a, F::axis0(o))], E[F::edge(a, F::axis1(o))], g0[3 + o]);
+    corner_stress<0>(tab + kMetricOffset, i, x, D, O, u);
+    if (kOut != 0) {
+      bool open[3];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) open[d] = F::first(F::edge(a, d)) < i;
+#pragma unroll
+      for (int o = 0; o < 3; ++o) {
+        const int d0 = F::axis0(o), d1 = F::axis1(o);
+        const int e0 = F::edge(a, d0), e1 = F::edge(a, d1);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          gE[e0][j] = open[d0] ? __builtin_fma(O[o], E[e1][j], gE[e0][j]) : O[o] * E[e1][j];
+          gE[e1][j] = open[d1] ? __builtin_fma(O[o], E[e0][j], gE[e1][j]) : O[o] * E[e0][j];
+        }
+        open[d0] = open[d1] = true;
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const int e = F::edge(a, d);
+      if (F::last(e) == i) {
+        u = __builtin_fma(q[e], D[e], u);
+        if (kOut != 0) {
+#pragma unroll
+          for (int j = 0; j < 3; ++j) gE[e][j] = __builtin_fma(D[e], E[e][j], gE[e][j]);
+          edge_virial(gE[e], E[e], vir);
+          if (kOut == 2) edge_to_vertices<0>(e, gE[e], g);
         }
       }
     }
-    return u;
+    // keeps the corners apart: moved into each other they would need 200 registers
+    asm("" : "+v"(u));
   }
+  return 0.5 * u;
 }
 
 template <int NV>

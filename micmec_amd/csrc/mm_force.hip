@@ -20,9 +20,9 @@
 // Cells are grouped by type into 256-slot segments, so the type, its number of states and its
 // parameter row are uniform per block and the parameters are read with scalar loads.
 //
-// One lane per cell: the lane gathers the cell's eight nodes, evaluates the corner matrices of
-// every state and accumulates the eight vertex gradients in registers (for multistate cells
-// each state's; their weighted sum over the states is kept in LDS).
+// One lane per cell: the lane gathers the cell's eight nodes, evaluates strains and stresses of
+// every corner in the metric of the edges (mm_device.h) and forms the eight vertex gradients in
+// registers (for multistate cells the stresses' weighted sum over the states is kept in LDS).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -31,50 +31,43 @@
 
 namespace mm {
 
-// Deterministic block reduction (the reduce-scatter butterfly per wave, 17 exchanges for up to
-// 16 values, then the waves in order); the block's totals are written SoA to out[q * stride].
-template <int NV, int BS>
-__device__ __forceinline__ void block_reduce_store(double (&v)[NV], double* smem, double* out,
-                                                   int64_t stride) {
+// Block totals of the energy and the six virial entries (00, 11, 22, 12, 02, 01): the
+// reduce-scatter butterfly per wave, then the waves in order; the energy and the full 3x3 virial
+// are written SoA to out[q * stride], q < 10.
+__device__ __forceinline__ void cell_totals_store(double (&v)[7], double* smem, double* out,
+                                                  int64_t stride) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   {
-    const double t = wave_reduce_scatter<NV>(v, lane);
+    const double t = wave_reduce_scatter<7>(v, lane);
     const int q = scatter_index(lane);
-    if ((lane & 3) == 0 && q < NV) smem[wave * NV + q] = t;
+    if ((lane & 3) == 0 && q < 7) smem[wave * 7 + q] = t;
   }
   __syncthreads();
-  if (threadIdx.x < NV) {
-    double s = smem[threadIdx.x];
+  if (threadIdx.x < 10) {
+    constexpr int kEntry[10] = {0, 1, 6, 5, 6, 2, 4, 5, 4, 3};
+    const int q = kEntry[threadIdx.x];
+    double s = smem[q];
 #pragma unroll
-    for (int w = 1; w < BS / 64; ++w) s += smem[w * NV + threadIdx.x];
+    for (int w = 1; w < kCellBlock / 64; ++w) s += smem[w * 7 + q];
     out[threadIdx.x * stride] = s;
   }
 }
 
-// Gather the eight vertices of a cell relative to corner 0: r_0 = 0, r_k = (pos[n_k] -
-// pos[n_0]) + sum_d shift_kd rvecs[d] with shift_kd = 1 when the cell is in the last layer
-// along a periodic axis d and corner k lies at +d (mmff.py:347-371 with get_mic 258-286). The
-// reference adds pos[n_0] back before taking edge differences; the energy depends on the edges
-// only and the virial on r_v - r_0, and leaving the origin out avoids rounding the vertices at
-// the magnitude of the absolute coordinates.
-// All 24 loads are issued before any arithmetic, and the shifts are formed with factors 0 or 1
-// (exact products) rather than data-dependent selects, so that no load ends up behind a branch
-// and a full wait; the sums are those of the selects, in the same order.
-// With kXmat every position is first taken through the pending transforms: xm2 (when not
-// null), then xm (vecmat, the products the scaling pass stores, in its order).
-template <bool kXmat = false>
-__device__ __forceinline__ void gather_vertices(const double* __restrict__ pos,
-                                                const double* __restrict__ rv, const int n[8],
-                                                int wrap, double r[8][3],
-                                                const double* __restrict__ xm = nullptr,
-                                                const double* __restrict__ xm2 = nullptr) {
-  double p[8][3];
+// The node positions of a cell's eight corners. All 24 loads are issued before any arithmetic.
+// With xm every position is taken through the pending transforms: xm2 (when not null), then xm
+// (vecmat, the products the scaling pass stores, in its order).
+__device__ __forceinline__ void load_corners(const double* __restrict__ pos, const int n[8],
+                                             double (&p)[8][3], const double* __restrict__ xm,
+                                             const double* __restrict__ xm2) {
 #pragma unroll
-  for (int k = 0; k < 8; ++k)
+  for (int k = 0; k < 8; ++k) {
+    // 3 n < 2^32 (n < 2^30): a 32-bit product
+    const double* t = pos + (uint64_t)(3u * (uint32_t)n[k]);
 #pragma unroll
-    for (int j = 0; j < 3; ++j) p[k][j] = pos[3 * (int64_t)n[k] + j];
-  if (kXmat && xm2) {
+    for (int j = 0; j < 3; ++j) p[k][j] = t[j];
+  }
+  if (xm2) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       double t[3];
@@ -83,7 +76,7 @@ __device__ __forceinline__ void gather_vertices(const double* __restrict__ pos,
       for (int j = 0; j < 3; ++j) p[k][j] = t[j];
     }
   }
-  if (kXmat) {
+  if (xm) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       double t[3];
@@ -92,26 +85,29 @@ __device__ __forceinline__ void gather_vertices(const double* __restrict__ pos,
       for (int j = 0; j < 3; ++j) p[k][j] = t[j];
     }
   }
-  const double fx = (double)(wrap & 1), fy = (double)((wrap >> 1) & 1),
-               fz = (double)((wrap >> 2) & 1);
-  double sx[3], sy[3], sz[3];
+}
+
+// The edges of a cell (or the averaged matrix): pos[n_hi] - pos[n_lo] of the edge's corners, plus
+// rvecs[d] for the edges along d when the cell is in the last layer along the periodic axis d
+// (mmff.py:347-371 with get_mic 258-286). The reference forms vertices relative to corner 0
+// and then edge differences; taking the differences of the positions directly avoids the
+// vertices' rounding. The shifts use factors f of 0 or 1 (exact products) rather than
+// data-dependent selects.
+template <int kModel>
+__device__ __forceinline__ void form_edges(const double (&p)[8][3], const double (&f)[3],
+                                           const double (&rv)[9],
+                                           double (&E)[Frame<kModel>::NE][3]) {
+#pragma clang fp contract(off)
+  double t[12][3];
 #pragma unroll
-  for (int j = 0; j < 3; ++j) {
-    sx[j] = fx * rv[0 + j];
-    sy[j] = fy * rv[3 + j];
-    sz[j] = fz * rv[6 + j];
-  }
+  for (int e = 0; e < 12; ++e) form_edge(p, e, f[e / 4], &rv[3 * (e / 4)], t[e]);
 #pragma unroll
-  for (int j = 0; j < 3; ++j) r[0][j] = 0.0;
+  for (int e = 0; e < Frame<kModel>::NE; ++e)
 #pragma unroll
-  for (int k = 1; k < 8; ++k) {
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const double sh = ((kOff[k][0] ? sx[j] : 0.0) + (kOff[k][1] ? sy[j] : 0.0)) +
-                        (kOff[k][2] ? sz[j] : 0.0);
-      r[k][j] = (p[k][j] - p[0][j]) + sh;
-    }
-  }
+    for (int j = 0; j < 3; ++j)
+      E[e][j] = kModel == 0 ? t[e][j]
+                            : 0.25 * ((t[4 * e % 12][j] + t[(4 * e + 1) % 12][j]) +
+                                      (t[(4 * e + 2) % 12][j] + t[(4 * e + 3) % 12][j]));
 }
 
 // Corners of the lower (z = 0) and upper (z = 1) face of a cell, in face-class order: upper
@@ -119,18 +115,31 @@ __device__ __forceinline__ void gather_vertices(const double* __restrict__ pos,
 __device__ constexpr int kLowerCorner[4] = {0, 1, 2, 4};
 __device__ constexpr int kUpperCorner[4] = {3, 5, 6, 7};
 
+// Entry i of a gradient plane (S < 2^29, so that the byte offset fits 32 bits beside the plane's
+// uniform base).
+__device__ __forceinline__ void store_record(double* plane, uint32_t i, double v) {
+  __builtin_nontemporal_store(
+      v, reinterpret_cast<double*>(reinterpret_cast<char*>(plane) + (size_t)(i * 8u)));
+}
+
 // One lane per cell. Energies of all states of the block's cell type, combined by the
 // log-sum-exp of mmff.py:386-398; the vertex gradient of the combined energy goes to gcell and
-// the cell's energy and virial sum_v g_v (x) (r_v - r_0) enter the block partials. A block holds
+// the cell's energy and virial (symmetric, from the edges) enter the block partials. A block holds
 // one cell type; single-state and multistate blocks run in separate instances (kMulti), each
 // launched over its own range of blocks (blk0 + blockIdx.x) when the work order allows, so that
 // the single-state instance does not carry the registers of the state combination.
-// kVir: the virial as the sum of the corners' B^T S B (state_energy), which the vertex
-// gradients give as sum_v g_v (x) r_v; with kGrad false the pass then forms no gradient at all
-// (energy and virial only). The passes with gradients and the vertex virial, and those with the
-// corner virial and no gradients, take the node positions through the pending transforms xmat
-// (and xmat2 first, when its flag is set) when they are given: a barostat call whose position
-// scaling is stored by a later node pass.
+// kOut: kOutEnergy, kOutVirial (energy and virial, no vertex gradient) or kOutGradient (the vertex
+// gradient too); the energies and virials of all three are the same bits. The latter two take the
+// node positions through the pending transforms xmat (and xmat2 first, when its flag is set) when
+// they are given: a barostat call whose position scaling is stored by a later node pass.
+// The single-state instance sweeps the corners (sweep_cell) in 166 VGPRs, three waves a SIMD (146
+// without the gradient); the multistate one keeps the stresses of all corners for the state sum
+// (219 VGPRs and 72 KB of LDS a block, two waves). The compiler's default scheduler is the one that
+// keeps both free of spills. HBM bounds the gradient pass: about 450 MB at 128^3 (20% two-state,
+// 5% empty) in 100 us, with 1000 / 1800 VALU instructions a wave (60 us of issue); the form
+// with B = P M per corner took 1735 / 4000 and 150 us, and 120 us for the pass without
+// gradient that now takes 84 us.
+constexpr int kOutEnergy = 0, kOutVirial = 1, kOutGradient = 2;
 #define MM_CELL_PARAMS                                                                        \
   const double *__restrict__ pos, const double *__restrict__ rvecs, int64_t rvecs_stride,     \
       const int32_t *__restrict__ blk_sys, const int32_t *__restrict__ cnode,                 \
@@ -145,12 +154,14 @@ __device__ constexpr int kUpperCorner[4] = {3, 5, 6, 7};
       max_states, W, cbase, S, gcell, partials, blk0, nblocks, xmat, xmat2, xmat2_on
 
 // The work of cell block bid (see cell_kernel).
-template <int kModel, bool kGrad, bool kMulti, bool kVir>
+template <int kModel, int kOut, bool kMulti>
 __device__ __forceinline__ void cell_body(int bid, MM_CELL_PARAMS) {
-  __shared__ double red[10 * (kCellBlock / 64)];
-  __shared__ double es_sh[(kMulti && !kGrad && !kVir) ? kMaxStates * kCellBlock : 1];
-  // running weighted gradient sum of the one-pass multistate gradient: [24][kCellBlock]
-  __shared__ double gs_sh[(kMulti && kGrad) ? 24 * kCellBlock : 1];
+  using F = Frame<kModel>;
+  constexpr bool kGrad = kOut == kOutGradient, kVir = kOut != kOutEnergy;
+  constexpr int NS = F::NE + 3 * F::NC;  // stresses of a cell
+  __shared__ double red[7 * (kCellBlock / 64)];
+  // running weighted sum of the states' stresses, one column a lane: [NS][kCellBlock]
+  __shared__ double st_sh[(kMulti && kVir) ? NS * kCellBlock : 1];
   const int trow = blk_row[bid];
   // a block of the other kind (full-range launches only) leaves its partials to the other
   // instance
@@ -158,131 +169,95 @@ __device__ __forceinline__ void cell_body(int bid, MM_CELL_PARAMS) {
   const int ns = nstates_g[trow];
   const double kt = kt_g[trow];
   const double* tab = tab_g + (int64_t)trow * max_states * kTabStride;
-  const double* rvb = rvecs + (blk_sys ? (int64_t)blk_sys[bid] * rvecs_stride : 0);
+  const int64_t soff = blk_sys ? (int64_t)blk_sys[bid] * rvecs_stride : 0;
+  const double* rvb = rvecs + soff;
   double rv[9];
 #pragma unroll
   for (int q = 0; q < 9; ++q) rv[q] = rvb[q];
-  constexpr bool kCanX = kVir != kGrad;
-  const int64_t soff = blk_sys ? (int64_t)blk_sys[bid] * rvecs_stride : 0;
-  const double* xm = (kCanX && xmat) ? xmat + soff : nullptr;
-  const double* xm2 =
-      (kCanX && xmat2 && xmat2_on[soff] != 0.0) ? xmat2 + soff : nullptr;
+  const double* xm = (kVir && xmat) ? xmat + soff : nullptr;
+  const double* xm2 = (kVir && xmat2 && xmat2_on[soff] != 0.0) ? xmat2 + soff : nullptr;
 
   const int64_t w = (int64_t)bid * kCellBlock + threadIdx.x;
   int n[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) n[k] = cnode[w * 8 + k];
-  // sums start at -0.0, the identity of addition ((-0.0) + x == x for every x), so that the
-  // first term of each needs no add
-  double acc[10];
-#pragma unroll
-  for (int q = 0; q < 10; ++q) acc[q] = -0.0;
+  double ecell = 0.0;
+  double vir[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   double gacc[8][3];
 #pragma unroll
   for (int v = 0; v < 8; ++v)
 #pragma unroll
     for (int j = 0; j < 3; ++j) gacc[v][j] = -0.0;
-  double vir[6];
-#pragma unroll
-  for (int q = 0; q < 6; ++q) vir[q] = -0.0;
   const bool valid = n[0] >= 0;
   const int wrap = valid ? cwrap[w] : 0;
   if (valid) {
-    double r[8][3];
-    if (kCanX && xm)
-      gather_vertices<true>(pos, rv, n, wrap, r, xm, xm2);
-    else
-      gather_vertices(pos, rv, n, wrap, r);
-    double ecell;
-    if (!kMulti) {
-      ecell = tab[10] + state_energy<kModel, kGrad, true, kVir>(tab, r, gacc, 1.0, vir);
-    } else if (!kGrad && !kVir) {
-      // energies of all states, E = E_min - kT ln sum exp(-(E_s - E_min)/kT) (mmff.py:386-395);
-      // the state energies are kept in LDS
-      double emin = 0.0;
-      for (int s = 0; s < ns; ++s) {
-        const double* ts = tab + s * kTabStride;
-        const double es = ts[10] + state_energy<kModel, false>(ts, r, gacc);
-        es_sh[s * kCellBlock + threadIdx.x] = es;
-        emin = (s == 0 || es < emin) ? es : emin;
-      }
-      double zsum = 0.0;
-      for (int s = 0; s < ns; ++s) zsum += exp(-(es_sh[s * kCellBlock + threadIdx.x] - emin) / kt);
-      ecell = emin - kt * log(zsum);
+    double p[8][3], f[3];
+    load_corners(pos, n, p, xm, xm2);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) f[d] = (double)((wrap >> d) & 1);
+    if constexpr (kModel == 0 && !kMulti) {
+      ecell = tab[10] + sweep_cell<kOut>(tab, p, f, rv, vir, gacc);
     } else {
-      // one pass over the states: energy and gradient of each, and the gradient
-      // sum_s p_s dE_s/dr with p_s = exp(-(E_s - E_min)/kT) / Z (mmff.py:386-398) accumulated
-      // in LDS with weights relative to the lowest energy so far, rescaled when it moves
-      // (kVir: the state virials combine the same way, in registers)
-      double* gsum = gs_sh + threadIdx.x;
-      double emin = 0.0, zsum = 0.0, vsum[6];
-      for (int s = 0; s < ns; ++s) {
-        const double* ts = tab + s * kTabStride;
-        double gs[8][3], vs[6];
+      double E[F::NE][3], s2[F::NE], D[F::NE], O[F::NC][3];
+      form_edges<kModel>(p, f, rv, E);
 #pragma unroll
-        for (int v = 0; v < 8; ++v)
-#pragma unroll
-          for (int j = 0; j < 3; ++j) gs[v][j] = -0.0;
-#pragma unroll
-        for (int q = 0; q < 6; ++q) vs[q] = -0.0;
-        const double es = ts[10] + state_energy<kModel, kGrad, true, kVir>(ts, r, gs, 1.0, vs);
-        if (s == 0) {
-          emin = es;
-          zsum = 1.0;
-          if (kGrad) {
-#pragma unroll
-            for (int q = 0; q < 24; ++q) gsum[q * kCellBlock] = gs[q / 3][q % 3];
+      for (int e = 0; e < F::NE; ++e) s2[e] = edge_square(E[e]);
+      if (!kMulti) {
+        ecell = tab[10] + state_stress<kModel>(tab, E, s2, D, O);
+      } else {
+        // one pass over the states (mmff.py:386-398): E = E_min - kT ln Z with Z = sum_s c_s,
+        // c_s = exp(-(E_s - E_min)/kT), and the stresses sum_s c_s S_s accumulated in LDS, both
+        // relative to the lowest energy so far and rescaled when it moves
+        double* acc = st_sh + threadIdx.x;
+        double emin = 0.0, zsum = 0.0;
+        for (int s = 0; s < ns; ++s) {
+          const double* ts = tab + s * kTabStride;
+          const double es = ts[10] + state_stress<kModel>(ts, E, s2, D, O);
+          double keep = 0.0, c = 1.0;  // factors of the sums so far and of this state
+          if (s == 0) {
+            emin = es;
+            zsum = 1.0;
+          } else if (es < emin) {
+            keep = exp(-(emin - es) / kt);
+            zsum = zsum * keep + 1.0;
+            emin = es;
+          } else {
+            keep = 1.0;
+            c = exp(-(es - emin) / kt);
+            zsum += c;
           }
+          if (kVir) {
+            if (s == 0) {
 #pragma unroll
-          for (int q = 0; q < 6; ++q) vsum[q] = vs[q];
-        } else if (es < emin) {
-          const double c = exp(-(emin - es) / kt);
-          zsum = zsum * c + 1.0;
-          if (kGrad) {
+              for (int e = 0; e < F::NE; ++e) acc[e * kCellBlock] = D[e];
 #pragma unroll
-            for (int q = 0; q < 24; ++q)
-              gsum[q * kCellBlock] = gsum[q * kCellBlock] * c + gs[q / 3][q % 3];
+              for (int q = 0; q < 3 * F::NC; ++q) acc[(F::NE + q) * kCellBlock] = O[q / 3][q % 3];
+            } else {
+#pragma unroll
+              for (int e = 0; e < F::NE; ++e) {
+                if (e % 6 == 0) __builtin_amdgcn_sched_barrier(0);
+                acc[e * kCellBlock] = __builtin_fma(c, D[e], keep * acc[e * kCellBlock]);
+              }
+#pragma unroll
+              for (int q = 0; q < 3 * F::NC; ++q) {
+                // six columns in flight at a time: all of them would not fit the registers
+                if (q % 6 == 0) __builtin_amdgcn_sched_barrier(0);
+                double* t = acc + (F::NE + q) * kCellBlock;
+                *t = __builtin_fma(c, O[q / 3][q % 3], keep * *t);
+              }
+            }
           }
+        }
+        ecell = emin - kt * log(zsum);
+        if (kVir) {
+          const double inv = 1.0 / zsum;
 #pragma unroll
-          for (int q = 0; q < 6; ++q) vsum[q] = vsum[q] * c + vs[q];
-          emin = es;
-        } else {
-          const double c = exp(-(es - emin) / kt);
-          zsum += c;
-          if (kGrad) {
+          for (int e = 0; e < F::NE; ++e) D[e] = acc[e * kCellBlock] * inv;
 #pragma unroll
-            for (int q = 0; q < 24; ++q) gsum[q * kCellBlock] += c * gs[q / 3][q % 3];
-          }
-#pragma unroll
-          for (int q = 0; q < 6; ++q) vsum[q] += c * vs[q];
+          for (int q = 0; q < 3 * F::NC; ++q) O[q / 3][q % 3] = acc[(F::NE + q) * kCellBlock] * inv;
         }
       }
-      ecell = emin - kt * log(zsum);
-      const double inv = 1.0 / zsum;
-      if (kGrad) {
-#pragma unroll
-        for (int q = 0; q < 24; ++q) gacc[q / 3][q % 3] = gsum[q * kCellBlock] * inv;
-      }
-      if (kVir) {
-#pragma unroll
-        for (int q = 0; q < 6; ++q) vir[q] = vsum[q] * inv;
-      }
-    }
-    acc[0] = ecell;
-    if (kVir) {
-      // vtens[k][l] from the symmetric corner sums (00, 11, 22, 12, 02, 01)
-      constexpr int kSym[9] = {0, 5, 4, 5, 1, 3, 4, 3, 2};
-#pragma unroll
-      for (int q = 0; q < 9; ++q) acc[1 + q] = vir[kSym[q]];
-    } else if (kGrad) {
-      // virial: vtens[k][l] = sum_v g_v[k] (r_v - r_0)[l]
-#pragma unroll
-      for (int v = 1; v < 8; ++v) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-#pragma unroll
-          for (int l = 0; l < 3; ++l) acc[1 + 3 * k + l] += gacc[v][k] * r[v][l];
-      }
+      if (kVir) edge_gradient<kModel, kGrad>(E, D, O, vir, gacc);
     }
   }
   if (kGrad) {
@@ -307,40 +282,41 @@ __device__ __forceinline__ void cell_body(int bid, MM_CELL_PARAMS) {
       for (int q = 0; q < 4; ++q)
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-          __builtin_nontemporal_store(gacc[kLowerCorner[q]][j], &gcell[(int64_t)(3 * q + j) * S + w]);
+          store_record(gcell + (int64_t)(3 * q + j) * S, (uint32_t)w, gacc[kLowerCorner[q]][j]);
     }
     const bool open_top = valid && !(wrap & 16);
     const uint64_t tops = __ballot(open_top);
     if (open_top) {
       const int lane = threadIdx.x & 63;
-      const int64_t ci = W + cbase[w >> 6] + __popcll(tops & ((1ull << lane) - 1ull));
+      const uint32_t ci =
+          (uint32_t)W + (uint32_t)cbase[w >> 6] + __popcll(tops & ((1ull << lane) - 1ull));
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-          __builtin_nontemporal_store(gacc[kUpperCorner[q]][j], &gcell[(int64_t)(3 * q + j) * S + ci]);
+          store_record(gcell + (int64_t)(3 * q + j) * S, ci, gacc[kUpperCorner[q]][j]);
     }
   }
-  block_reduce_store<10, kCellBlock>(acc, red, partials + bid, nblocks);
+  double acc[7] = {ecell, vir[0], vir[1], vir[2], vir[3], vir[4], vir[5]};
+  cell_totals_store(acc, red, partials + bid, nblocks);
 }
 
-template <int kModel, bool kGrad, bool kMulti, bool kVir>
-__global__ void __launch_bounds__(kCellBlock, (kVir && !kGrad && !kMulti) ? 3 : 2)
-cell_kernel(MM_CELL_PARAMS) {
-  cell_body<kModel, kGrad, kMulti, kVir>(blk0 + xcd_block((int)blockIdx.x, (int)gridDim.x),
-                                         MM_CELL_ARGS);
+template <int kModel, int kOut, bool kMulti>
+__global__ void __launch_bounds__(kCellBlock, kMulti ? 2 : 3) cell_kernel(MM_CELL_PARAMS) {
+  cell_body<kModel, kOut, kMulti>(blk0 + xcd_block((int)blockIdx.x, (int)gridDim.x),
+                                  MM_CELL_ARGS);
 }
 
 // Both kinds of block in one launch, each block running the body of its own kind: for a pass
 // that the device holds at once, where the two instances would otherwise run one after the
 // other, each taking about one block's time.
-template <int kModel, bool kGrad, bool kVir>
+template <int kModel, int kOut>
 __global__ void __launch_bounds__(kCellBlock, 2) cell_kernel_both(MM_CELL_PARAMS) {
   const int bid = blk0 + xcd_block((int)blockIdx.x, (int)gridDim.x);
   if (nstates_g[blk_row[bid]] > 1)
-    cell_body<kModel, kGrad, true, kVir>(bid, MM_CELL_ARGS);
+    cell_body<kModel, kOut, true>(bid, MM_CELL_ARGS);
   else
-    cell_body<kModel, kGrad, false, kVir>(bid, MM_CELL_ARGS);
+    cell_body<kModel, kOut, false>(bid, MM_CELL_ARGS);
 }
 #undef MM_CELL_ARGS
 #undef MM_CELL_PARAMS
@@ -478,7 +454,9 @@ reduce_items_kernel(ReduceList list, int* __restrict__ nanflag) {
 
 hipError_t launch_cells(const ForceArgs& a, hipStream_t stream) {
   const int nb = (int)(a.W / kCellBlock);
-  const bool grad = a.gpos != nullptr || a.vtens != nullptr || a.force_grad;
+  const int out = (a.gpos != nullptr || a.force_grad) && a.store_records ? kOutGradient
+                  : a.vtens != nullptr || a.force_grad                     ? kOutVirial
+                                                                           : kOutEnergy;
   if (nb == 0) return hipSuccess;
   // Multistate blocks [0, split), single-state blocks [split, nb) when the work order is so
   // partitioned (split >= 0); otherwise both instances cover every block.
@@ -503,56 +481,43 @@ hipError_t launch_cells(const ForceArgs& a, hipStream_t stream) {
     if (e == hipSuccess) e = hipStreamWaitEvent(a.side, a.ev_fork, 0);
     if (e != hipSuccess) return e;
   }
-#define MM_LAUNCH_CELL(MODEL, GRAD, MULTI, S, B0, NBL)                                       \
-  hipLaunchKernelGGL((cell_kernel<MODEL, GRAD, MULTI, VIR>), dim3(NBL), dim3(kCellBlock), 0, S, \
+#define MM_LAUNCH_CELL(MODEL, OUT, MULTI, S, B0, NBL)                                        \
+  hipLaunchKernelGGL((cell_kernel<MODEL, OUT, MULTI>), dim3(NBL), dim3(kCellBlock), 0, S,       \
                      a.pos, a.rvecs, a.rvecs_stride, a.blk_sys, a.cnode, a.cwrap, a.blk_row, \
                      a.tab, a.kt, a.nstates, a.max_states, a.W, a.cbase, a.rstride, a.gcell,  \
                      a.partials, B0, nb, a.xmat, a.xmat2, a.xmat2_on)
-  // corner_virial: the virial from the corners; without records the pass then forms no
-  // gradient at all
-  const bool vir = a.corner_virial != 0;
-  const bool kgrad = grad && !(vir && !a.store_records);
-  // pending position transforms: the gradient pass with the vertex virial or the corner-virial
-  // pass without gradients, xmat with every use, xmat2 with its flag
+  // pending position transforms: xmat with every use, xmat2 with its flag, and not for the
+  // energy alone
   if ((a.xmat2 != nullptr) != (a.xmat2_on != nullptr)) return hipErrorInvalidValue;
   if (a.xmat2 != nullptr && a.xmat == nullptr) return hipErrorInvalidValue;
-  if (a.xmat != nullptr && kgrad == vir) return hipErrorInvalidValue;
-  // The instance that takes longer is launched first, on the caller's stream: it then starts
-  // right behind the preceding kernel instead of after the side stream's. That is the one
-  // with more state evaluations (a multistate block counted as two), and the multistate one
-  // without gradients and with the corner virial, where the single-state instance runs three
-  // waves a SIMD and the multistate one two.
-  const bool multi_lead = (vir && !kgrad) || 2 * (int64_t)mn > (int64_t)sn;
+  if (a.xmat != nullptr && out == kOutEnergy) return hipErrorInvalidValue;
+  // The multistate instance is launched first, on the caller's stream: its blocks hold twice the
+  // time and 74 KB of LDS each, and started behind the single-state instance they find their
+  // place only as that drains (npt 128^3 step 0.580 -> 0.576 ms; equal at 72x80x96 with seven
+  // of ten cells two-state).
   // a pass that the device holds at once, with blocks of both kinds: one launch
   const bool both = mn > 0 && sn > 0 && nb <= kForkMinBlocks;
-#define MM_LAUNCH_BOTH(MODEL, GRAD)                                                          \
-  hipLaunchKernelGGL((cell_kernel_both<MODEL, GRAD, VIR>), dim3(nb), dim3(kCellBlock), 0,      \
-                     stream, a.pos, a.rvecs, a.rvecs_stride, a.blk_sys, a.cnode, a.cwrap,      \
+#define MM_LAUNCH_BOTH(MODEL, OUT)                                                           \
+  hipLaunchKernelGGL((cell_kernel_both<MODEL, OUT>), dim3(nb), dim3(kCellBlock), 0, stream,     \
+                     a.pos, a.rvecs, a.rvecs_stride, a.blk_sys, a.cnode, a.cwrap,              \
                      a.blk_row, a.tab, a.kt, a.nstates, a.max_states, a.W, a.cbase, a.rstride, \
                      a.gcell, a.partials, 0, nb, a.xmat, a.xmat2, a.xmat2_on)
-#define MM_LAUNCH_PAIR(MODEL, GRAD)                                                          \
+#define MM_LAUNCH_PAIR(MODEL, OUT)                                                           \
   do {                                                                                       \
     if (both) {                                                                              \
-      MM_LAUNCH_BOTH(MODEL, GRAD);                                                           \
-    } else if (multi_lead) {                                                                 \
-      if (mn > 0) MM_LAUNCH_CELL(MODEL, GRAD, true, stream, m0, mn);                        \
-      if (sn > 0) MM_LAUNCH_CELL(MODEL, GRAD, false, ms, s0, sn);                           \
+      MM_LAUNCH_BOTH(MODEL, OUT);                                                            \
     } else {                                                                                 \
-      if (sn > 0) MM_LAUNCH_CELL(MODEL, GRAD, false, stream, s0, sn);                       \
-      if (mn > 0) MM_LAUNCH_CELL(MODEL, GRAD, true, ms, m0, mn);                            \
+      if (mn > 0) MM_LAUNCH_CELL(MODEL, OUT, true, stream, m0, mn);                         \
+      if (sn > 0) MM_LAUNCH_CELL(MODEL, OUT, false, ms, s0, sn);                            \
     }                                                                                        \
   } while (0)
 #define MM_LAUNCH_MODEL(MODEL)                                                                \
   do {                                                                                        \
-    if (kgrad) MM_LAUNCH_PAIR(MODEL, true); else MM_LAUNCH_PAIR(MODEL, false);               \
+    if (out == kOutGradient) MM_LAUNCH_PAIR(MODEL, kOutGradient);                            \
+    else if (out == kOutVirial) MM_LAUNCH_PAIR(MODEL, kOutVirial);                           \
+    else MM_LAUNCH_PAIR(MODEL, kOutEnergy);                                                  \
   } while (0)
-  if (vir) {
-    constexpr bool VIR = true;
-    if (a.model == 0) MM_LAUNCH_MODEL(0); else MM_LAUNCH_MODEL(1);
-  } else {
-    constexpr bool VIR = false;
-    if (a.model == 0) MM_LAUNCH_MODEL(0); else MM_LAUNCH_MODEL(1);
-  }
+  if (a.model == 0) MM_LAUNCH_MODEL(0); else MM_LAUNCH_MODEL(1);
 #undef MM_LAUNCH_MODEL
 #undef MM_LAUNCH_PAIR
 #undef MM_LAUNCH_BOTH
@@ -732,11 +697,11 @@ build_table_kernel(int corner8, int nrows, int max_states, const int32_t* __rest
   e[10] = free_energy[ts];
   e[11] = 0.0;
 #pragma unroll
-  for (int q = 0; q < 36; ++q) {
-    const double c = cv[(int64_t)ts * 36 + q];
-    e[kCvOffset + q] = c;
-    e[kCvwOffset + q] = w * c;
-  }
+  for (int q = 0; q < 36; ++q) e[kCvOffset + q] = cv[(int64_t)ts * 36 + q];
+  metric_entry(h0 + (int64_t)ts * 9, inv, w, cv + (int64_t)ts * 36, e + kMetricOffset,
+               e + kRestOffset);
+  e[kRestOffset + 6] = 0.0;
+  e[kRestOffset + 7] = 0.0;
 }
 
 hipError_t launch_build_table(int corner8, int nrows, int max_states, const int32_t* nstates,

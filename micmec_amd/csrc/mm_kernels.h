@@ -47,14 +47,11 @@ struct ForceArgs {
   int model;               // 0 corner8, 1 original
   int* nanflag;
   int force_grad = 0;       // compute gradients even when gpos and vtens are null
-  int corner_virial = 0;    // 1: the virial as the corners' sum of B^T S B (no vertex gradient
-                            //    needed for it)
-  int store_records = 1;    // with corner_virial: 0 forms no gradient and stores no records
+  int store_records = 1;    // 0: energy and virial only, no vertex gradient and no records
   // pending position transforms [3][3] (row vectors, system s at xmat + s * rvecs_stride) that
   // the pass applies to every node position it reads, xmat2 first when the flag at
   // xmat2_on + s * rvecs_stride is set (both null: none): the position scaling of a barostat
-  // call that its own pass does not store. Only for the passes with gradients and the vertex
-  // virial, or with the corner virial and no gradients.
+  // call that its own pass does not store. Not for passes that form the energy alone.
   const double* xmat = nullptr;
   const double* xmat2 = nullptr;
   const double* xmat2_on = nullptr;

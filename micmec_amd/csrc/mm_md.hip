@@ -1326,10 +1326,8 @@ hipError_t scalar(mm_md* md, int phase, int with_vtens, hipStream_t s) {
 // (gather_kick_kernel): kGatherNone leaves out the records altogether, so the cell pass skips
 // them too, and without scale_v there is then no node pass at all (energy and virial only).
 hipError_t force(mm_md* md, bool kick, bool lt, hipStream_t s, bool scale_v = false,
-                 int gmode = kGatherStore, bool corner_virial = false,
-                 const double* xmat = nullptr) {
+                 int gmode = kGatherStore, const double* xmat = nullptr) {
   ForceArgs a = force_args(md);
-  a.corner_virial = corner_virial;
   a.xmat = xmat;
   if (gmode == kGatherNone) {
     if (kick) return hipErrorInvalidValue;
@@ -1404,8 +1402,8 @@ hipError_t gather_drift(mm_md* md, bool lt, hipStream_t s) {
 // (scale_v) or stays pending; with defer_x (a post call without records) its position scaling
 // also waits (the cell pass applies it on the fly, the next gather_drift stores it).
 hipError_t baro_call(mm_md* md, int end_phase, hipStream_t s, bool scale_v,
-                     int gmode = kGatherStore, bool corner_virial = false,
-                     bool pre_call = false, bool defer_x = false) {
+                     int gmode = kGatherStore, bool pre_call = false,
+                     bool defer_x = false) {
   if (!defer_x && !pre_call) MM_TRY(node(md, kScalePos, s));
   if (pre_call) {
     // the pre call's scaling (after a pending post-call one) is applied by its cell pass as it
@@ -1416,8 +1414,7 @@ hipError_t baro_call(mm_md* md, int end_phase, hipStream_t s, bool scale_v,
     a.xmat2_on = md->S + MM_S_XMAT2_ON;
     MM_TRY(launch_cells(a, s));
   } else {
-    MM_TRY(force(md, false, false, s, scale_v, gmode, corner_virial,
-                 defer_x ? md->S + MM_S_XMAT : nullptr));
+    MM_TRY(force(md, false, false, s, scale_v, gmode, defer_x ? md->S + MM_S_XMAT : nullptr));
   }
   MM_TRY(scalar(md, end_phase, 1, s));
   return hipSuccess;
@@ -1441,18 +1438,17 @@ hipError_t enqueue_step(mm_md* md, hipStream_t s, bool lean = false, bool pre = 
   if (md->baro) {
     if (pre) MM_TRY(scalar(md, kPhBaroPre, 1, s));
     // the pre call's gradient drives only the first half kick: its gather is the kick-drift
-    MM_TRY(baro_call(md, kPhBaroEndPre, s, false, kGatherKeep, false, true));
+    MM_TRY(baro_call(md, kPhBaroEndPre, s, false, kGatherKeep, true));
     MM_TRY(gather_drift(md, lt, s));
     MM_TRY(force(md, true, lt, s, false, lean ? kGatherKeep : kGatherStore));
     MM_TRY(scalar(md, kPhMainEndNpt, 1, s));
     // the post call's velocity transform stays pending in a lean step (its node sums follow
     // from the ones before it), and so does its position scaling (the cell pass applies it
     // as it reads the positions, the next step's scaling pass stores it), so its force
-    // evaluation has no node pass at all; its virial comes from the corners (B^T S B, no
-    // vertex gradient needed), in the last step too, so that lean and full steps agree to
-    // the bit
+    // evaluation has no node pass at all and forms no vertex gradient (the virial comes from
+    // the edges, the same bits either way)
     MM_TRY(baro_call(md, lean ? kPhBaroEndPostPre : kPhBaroEndPost, s, !lean,
-                     lean ? kGatherNone : kGatherStore, true, false, lean));
+                     lean ? kGatherNone : kGatherStore, false, lean));
   } else if (md->thermo == MM_THERMO_NHC) {
     if (pre) MM_TRY(scalar(md, kPhNvtPre, 1, s));
     MM_TRY(node(md, kKickDrift, s));
