@@ -29,6 +29,11 @@ constexpr int kCvOffset = 12;
 constexpr int kMetricOffset = 48;
 constexpr int kRestOffset = 84;
 
+// Tables that no kernel of a launch writes: read with scalar loads wherever the index is uniform,
+// also where other memory changes during the launch.
+typedef const __attribute__((address_space(4))) double* const_f64;
+typedef const __attribute__((address_space(4))) int32_t* const_i32;
+
 // 3x3 inverse (row-major) by cofactors; returns the determinant. Shared by the host and the
 // device table builders, without contraction, so both round the same way.
 __host__ __device__ inline double inverse3_cof(const double* h, double* inv) {
@@ -146,7 +151,7 @@ struct Frame {
 // Stress of the i-th corner from its strain x: the diagonal entries are added to their edges' D,
 // the off-diagonal ones go to O, and their energy terms to u.
 template <int kModel>
-__device__ __forceinline__ void corner_stress(const double* __restrict__ K, int i,
+__device__ __forceinline__ void corner_stress(const_f64 K, int i,
                                               const double (&x)[6],
                                               double (&D)[Frame<kModel>::NE], double (&O)[3],
                                               double& u) {
@@ -180,14 +185,14 @@ __device__ __forceinline__ double edge_square(const double (&A)[3]) {
 // e summed over its corners, O[a][q] the off-diagonal stresses of corner a. The sums are fused
 // multiply-adds in a fixed order, so every kernel that evaluates a state gets the same bits.
 template <int kModel>
-__device__ __forceinline__ double state_stress(const double* __restrict__ tab,
+__device__ __forceinline__ double state_stress(const_f64 tab,
                                                const double (&E)[Frame<kModel>::NE][3],
                                                const double (&s)[Frame<kModel>::NE],
                                                double (&D)[Frame<kModel>::NE],
                                                double (&O)[Frame<kModel>::NC][3]) {
 #pragma clang fp contract(off)
   using F = Frame<kModel>;
-  const double* g0 = tab + kRestOffset;
+  const const_f64 g0 = tab + kRestOffset;
   double u = 0.0;
 #pragma unroll
   for (int i = 0; i < F::NC; ++i) {
@@ -291,13 +296,13 @@ __device__ __forceinline__ void form_edge(const double (&p)[8][3], int e, double
 // of the twelve edges are held at a time (kOut as the cell pass's: 0 energy, 1 and virial, 2 and
 // vertex gradient). f, rv: wrap factors and domain vectors.
 template <int kOut>
-__device__ __forceinline__ double sweep_cell(const double* __restrict__ tab,
+__device__ __forceinline__ double sweep_cell(const_f64 tab,
                                              const double (&p)[8][3], const double (&f)[3],
                                              const double (&rv)[9], double (&vir)[6],
                                              double (&g)[8][3]) {
 #pragma clang fp contract(off)
   using F = Frame<0>;
-  const double* g0 = tab + kRestOffset;
+  const const_f64 g0 = tab + kRestOffset;
   double E[12][3], q[12], D[12], gE[12][3];
   double u = 0.0;
 #pragma unroll
@@ -378,30 +383,31 @@ __device__ __forceinline__ void vecmat(const double v[3], const double* M, doubl
 // more VGPRs; the same bits as skipping the nones. Without it each record is loaded behind
 // the test of its index, which keeps the registers few: the form for passes with enough
 // waves to hide the latency.
-template <bool kAllLoads>
+// kStream: the loads carry the non-temporal hint.
+template <bool kAllLoads, bool kStream = true>
 __device__ __forceinline__ void sum_node_records(const int32_t* __restrict__ ncell,
-                                                 const double* __restrict__ gcell, int64_t N,
-                                                 int64_t RS, int rshift, int64_t n,
-                                                 double g[3]) {
+                                                 const double* gcell, int64_t N, int64_t RS,
+                                                 int rshift, int64_t n, double g[3]) {
+  auto load = [](const auto* p) { return kStream ? __builtin_nontemporal_load(p) : *p; };
 #pragma unroll
   for (int j = 0; j < 3; ++j) g[j] = 0.0;
   if (!kAllLoads) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const int32_t e = __builtin_nontemporal_load(&ncell[k * N + n]);
+      const int32_t e = load(&ncell[k * N + n]);
       if (e >= 0) {
         const int64_t w = e >> rshift;
         const int p = e & ((1 << rshift) - 1);
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-          g[j] += __builtin_nontemporal_load(&gcell[(int64_t)(3 * p + j) * RS + w]);
+          g[j] += load(&gcell[(int64_t)(3 * p + j) * RS + w]);
       }
     }
     return;
   }
   int32_t e[8];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) e[k] = __builtin_nontemporal_load(&ncell[k * N + n]);
+  for (int k = 0; k < 8; ++k) e[k] = load(&ncell[k * N + n]);
   double r[8][3];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
@@ -410,7 +416,7 @@ __device__ __forceinline__ void sum_node_records(const int32_t* __restrict__ nce
     const int p = c & ((1 << rshift) - 1);
 #pragma unroll
     for (int j = 0; j < 3; ++j)
-      r[k][j] = __builtin_nontemporal_load(&gcell[(int64_t)(3 * p + j) * RS + w]);
+      r[k][j] = load(&gcell[(int64_t)(3 * p + j) * RS + w]);
   }
 #pragma unroll
   for (int k = 0; k < 8; ++k)

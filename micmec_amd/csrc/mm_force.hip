@@ -26,101 +26,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "mm_cell.h"
 #include "mm_device.h"
 #include "mm_kernels.h"
 
 namespace mm {
-
-// Block totals of the energy and the six virial entries (00, 11, 22, 12, 02, 01): the
-// reduce-scatter butterfly per wave, then the waves in order; the energy and the full 3x3 virial
-// are written SoA to out[q * stride], q < 10.
-__device__ __forceinline__ void cell_totals_store(double (&v)[7], double* smem, double* out,
-                                                  int64_t stride) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  {
-    const double t = wave_reduce_scatter<7>(v, lane);
-    const int q = scatter_index(lane);
-    if ((lane & 3) == 0 && q < 7) smem[wave * 7 + q] = t;
-  }
-  __syncthreads();
-  if (threadIdx.x < 10) {
-    constexpr int kEntry[10] = {0, 1, 6, 5, 6, 2, 4, 5, 4, 3};
-    const int q = kEntry[threadIdx.x];
-    double s = smem[q];
-#pragma unroll
-    for (int w = 1; w < kCellBlock / 64; ++w) s += smem[w * 7 + q];
-    out[threadIdx.x * stride] = s;
-  }
-}
-
-// The node positions of a cell's eight corners. All 24 loads are issued before any arithmetic.
-// With xm every position is taken through the pending transforms: xm2 (when not null), then xm
-// (vecmat, the products the scaling pass stores, in its order).
-__device__ __forceinline__ void load_corners(const double* __restrict__ pos, const int n[8],
-                                             double (&p)[8][3], const double* __restrict__ xm,
-                                             const double* __restrict__ xm2) {
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    // 3 n < 2^32 (n < 2^30): a 32-bit product
-    const double* t = pos + (uint64_t)(3u * (uint32_t)n[k]);
-#pragma unroll
-    for (int j = 0; j < 3; ++j) p[k][j] = t[j];
-  }
-  if (xm2) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      double t[3];
-      vecmat(p[k], xm2, t);
-#pragma unroll
-      for (int j = 0; j < 3; ++j) p[k][j] = t[j];
-    }
-  }
-  if (xm) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      double t[3];
-      vecmat(p[k], xm, t);
-#pragma unroll
-      for (int j = 0; j < 3; ++j) p[k][j] = t[j];
-    }
-  }
-}
-
-// The edges of a cell (or the averaged matrix): pos[n_hi] - pos[n_lo] of the edge's corners, plus
-// rvecs[d] for the edges along d when the cell is in the last layer along the periodic axis d
-// (mmff.py:347-371 with get_mic 258-286). The reference forms vertices relative to corner 0
-// and then edge differences; taking the differences of the positions directly avoids the
-// vertices' rounding. The shifts use factors f of 0 or 1 (exact products) rather than
-// data-dependent selects.
-template <int kModel>
-__device__ __forceinline__ void form_edges(const double (&p)[8][3], const double (&f)[3],
-                                           const double (&rv)[9],
-                                           double (&E)[Frame<kModel>::NE][3]) {
-#pragma clang fp contract(off)
-  double t[12][3];
-#pragma unroll
-  for (int e = 0; e < 12; ++e) form_edge(p, e, f[e / 4], &rv[3 * (e / 4)], t[e]);
-#pragma unroll
-  for (int e = 0; e < Frame<kModel>::NE; ++e)
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-      E[e][j] = kModel == 0 ? t[e][j]
-                            : 0.25 * ((t[4 * e % 12][j] + t[(4 * e + 1) % 12][j]) +
-                                      (t[(4 * e + 2) % 12][j] + t[(4 * e + 3) % 12][j]));
-}
-
-// Corners of the lower (z = 0) and upper (z = 1) face of a cell, in face-class order: upper
-// corner kUpperCorner[q] of a cell is lower corner kLowerCorner[q] of its +z neighbour.
-__device__ constexpr int kLowerCorner[4] = {0, 1, 2, 4};
-__device__ constexpr int kUpperCorner[4] = {3, 5, 6, 7};
-
-// Entry i of a gradient plane (S < 2^29, so that the byte offset fits 32 bits beside the plane's
-// uniform base).
-__device__ __forceinline__ void store_record(double* plane, uint32_t i, double v) {
-  __builtin_nontemporal_store(
-      v, reinterpret_cast<double*>(reinterpret_cast<char*>(plane) + (size_t)(i * 8u)));
-}
 
 // One lane per cell. Energies of all states of the block's cell type, combined by the
 // log-sum-exp of mmff.py:386-398; the vertex gradient of the combined energy goes to gcell and
@@ -139,7 +49,6 @@ __device__ __forceinline__ void store_record(double* plane, uint32_t i, double v
 // 5% empty) in 100 us, with 1000 / 1800 VALU instructions a wave (60 us of issue); the form
 // with B = P M per corner took 1735 / 4000 and 150 us, and 120 us for the pass without
 // gradient that now takes 84 us.
-constexpr int kOutEnergy = 0, kOutVirial = 1, kOutGradient = 2;
 #define MM_CELL_PARAMS                                                                        \
   const double *__restrict__ pos, const double *__restrict__ rvecs, int64_t rvecs_stride,     \
       const int32_t *__restrict__ blk_sys, const int32_t *__restrict__ cnode,                 \
@@ -157,7 +66,7 @@ constexpr int kOutEnergy = 0, kOutVirial = 1, kOutGradient = 2;
 template <int kModel, int kOut, bool kMulti>
 __device__ __forceinline__ void cell_body(int bid, MM_CELL_PARAMS) {
   using F = Frame<kModel>;
-  constexpr bool kGrad = kOut == kOutGradient, kVir = kOut != kOutEnergy;
+  constexpr bool kVir = kOut != kOutEnergy;
   constexpr int NS = F::NE + 3 * F::NC;  // stresses of a cell
   __shared__ double red[7 * (kCellBlock / 64)];
   // running weighted sum of the states' stresses, one column a lane: [NS][kCellBlock]
@@ -168,137 +77,28 @@ __device__ __forceinline__ void cell_body(int bid, MM_CELL_PARAMS) {
   if (kMulti != (nstates_g[trow] > 1)) return;
   const int ns = nstates_g[trow];
   const double kt = kt_g[trow];
-  const double* tab = tab_g + (int64_t)trow * max_states * kTabStride;
+  const const_f64 tab = (const_f64)tab_g + (int64_t)trow * max_states * kTabStride;
   const int64_t soff = blk_sys ? (int64_t)blk_sys[bid] * rvecs_stride : 0;
   const double* rvb = rvecs + soff;
   double rv[9];
 #pragma unroll
   for (int q = 0; q < 9; ++q) rv[q] = rvb[q];
-  const double* xm = (kVir && xmat) ? xmat + soff : nullptr;
-  const double* xm2 = (kVir && xmat2 && xmat2_on[soff] != 0.0) ? xmat2 + soff : nullptr;
+  const bool on = kVir && xmat, on2 = on && xmat2 && xmat2_on[soff] != 0.0;
 
   const int64_t w = (int64_t)bid * kCellBlock + threadIdx.x;
   int n[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) n[k] = cnode[w * 8 + k];
-  double ecell = 0.0;
-  double vir[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  double gacc[8][3];
-#pragma unroll
-  for (int v = 0; v < 8; ++v)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) gacc[v][j] = -0.0;
   const bool valid = n[0] >= 0;
   const int wrap = valid ? cwrap[w] : 0;
-  if (valid) {
-    double p[8][3], f[3];
-    load_corners(pos, n, p, xm, xm2);
-#pragma unroll
-    for (int d = 0; d < 3; ++d) f[d] = (double)((wrap >> d) & 1);
-    if constexpr (kModel == 0 && !kMulti) {
-      ecell = tab[10] + sweep_cell<kOut>(tab, p, f, rv, vir, gacc);
-    } else {
-      double E[F::NE][3], s2[F::NE], D[F::NE], O[F::NC][3];
-      form_edges<kModel>(p, f, rv, E);
-#pragma unroll
-      for (int e = 0; e < F::NE; ++e) s2[e] = edge_square(E[e]);
-      if (!kMulti) {
-        ecell = tab[10] + state_stress<kModel>(tab, E, s2, D, O);
-      } else {
-        // one pass over the states (mmff.py:386-398): E = E_min - kT ln Z with Z = sum_s c_s,
-        // c_s = exp(-(E_s - E_min)/kT), and the stresses sum_s c_s S_s accumulated in LDS, both
-        // relative to the lowest energy so far and rescaled when it moves
-        double* acc = st_sh + threadIdx.x;
-        double emin = 0.0, zsum = 0.0;
-        for (int s = 0; s < ns; ++s) {
-          const double* ts = tab + s * kTabStride;
-          const double es = ts[10] + state_stress<kModel>(ts, E, s2, D, O);
-          double keep = 0.0, c = 1.0;  // factors of the sums so far and of this state
-          if (s == 0) {
-            emin = es;
-            zsum = 1.0;
-          } else if (es < emin) {
-            keep = exp(-(emin - es) / kt);
-            zsum = zsum * keep + 1.0;
-            emin = es;
-          } else {
-            keep = 1.0;
-            c = exp(-(es - emin) / kt);
-            zsum += c;
-          }
-          if (kVir) {
-            if (s == 0) {
-#pragma unroll
-              for (int e = 0; e < F::NE; ++e) acc[e * kCellBlock] = D[e];
-#pragma unroll
-              for (int q = 0; q < 3 * F::NC; ++q) acc[(F::NE + q) * kCellBlock] = O[q / 3][q % 3];
-            } else {
-#pragma unroll
-              for (int e = 0; e < F::NE; ++e) {
-                if (e % 6 == 0) __builtin_amdgcn_sched_barrier(0);
-                acc[e * kCellBlock] = __builtin_fma(c, D[e], keep * acc[e * kCellBlock]);
-              }
-#pragma unroll
-              for (int q = 0; q < 3 * F::NC; ++q) {
-                // six columns in flight at a time: all of them would not fit the registers
-                if (q % 6 == 0) __builtin_amdgcn_sched_barrier(0);
-                double* t = acc + (F::NE + q) * kCellBlock;
-                *t = __builtin_fma(c, O[q / 3][q % 3], keep * *t);
-              }
-            }
-          }
-        }
-        ecell = emin - kt * log(zsum);
-        if (kVir) {
-          const double inv = 1.0 / zsum;
-#pragma unroll
-          for (int e = 0; e < F::NE; ++e) D[e] = acc[e * kCellBlock] * inv;
-#pragma unroll
-          for (int q = 0; q < 3 * F::NC; ++q) O[q / 3][q % 3] = acc[(F::NE + q) * kCellBlock] * inv;
-        }
-      }
-      if (kVir) edge_gradient<kModel, kGrad>(E, D, O, vir, gacc);
-    }
-  }
-  if (kGrad) {
-    // The upper face (corners 3, 5, 6, 7) of the slot below is added to this slot's lower face
-    // (corners 0, 1, 2, 4) when that slot holds the -z neighbour (wrap bit 3); the lower faces
-    // go to their class planes, the upper faces that were not folded (wrap bit 4 clear) to the
-    // wave's compact slots, in lane order. The move from lane - 1 is a DPP wave shift (lane 0,
-    // which never folds, keeps its own value).
-    const bool fold = (wrap & 8) != 0;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const double up = gacc[kUpperCorner[q]][j];
-        const double t = dpp_f64<0x138, 0xF>(up, up);  // wave_shr:1
-        const double lo = gacc[kLowerCorner[q]][j];
-        gacc[kLowerCorner[q]][j] = fold ? lo + t : lo;
-      }
-    }
-    if (valid) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-          store_record(gcell + (int64_t)(3 * q + j) * S, (uint32_t)w, gacc[kLowerCorner[q]][j]);
-    }
-    const bool open_top = valid && !(wrap & 16);
-    const uint64_t tops = __ballot(open_top);
-    if (open_top) {
-      const int lane = threadIdx.x & 63;
-      const uint32_t ci =
-          (uint32_t)W + (uint32_t)cbase[w >> 6] + __popcll(tops & ((1ull << lane) - 1ull));
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-          store_record(gcell + (int64_t)(3 * q + j) * S, ci, gacc[kUpperCorner[q]][j]);
-    }
-  }
-  double acc[7] = {ecell, vir[0], vir[1], vir[2], vir[3], vir[4], vir[5]};
-  cell_totals_store(acc, red, partials + bid, nblocks);
+  double ecell, vir[6], gacc[8][3];
+  cell_eval<kModel, kOut, kMulti>(tab, ns, kt, pos, n, wrap, rv, on, xmat + soff, on2,
+                                  xmat2 + soff, st_sh + threadIdx.x, ecell, vir, gacc);
+  if (kOut == kOutGradient) store_cell<true>(w, wrap, valid, cbase, W, S, gcell, gacc);
+  cell_wave_totals(ecell, vir, red + 7 * (threadIdx.x >> 6));
+  __syncthreads();
+  if (threadIdx.x < 10)
+    partials[(int64_t)threadIdx.x * nblocks + bid] = cell_block_total(red, threadIdx.x);
 }
 
 template <int kModel, int kOut, bool kMulti>

@@ -44,12 +44,10 @@ constexpr int kScalarSlices = 32;  // most blocks a scalar phase spreads its red
 constexpr int kSliceQ = 10 + kNodeSums;  // force and node sums per slice
 
 enum NodeMode {
-  kKickDrift = 0,
   kScalePos = 1,
   kVV = 3,
   kApplyV = 4,
   kRmsd = 5,
-  kKickDriftLT = 6,  // kick-drift preceded by the Langevin thermostat's pre update
 };
 
 enum Phase {
@@ -182,31 +180,95 @@ __device__ __forceinline__ void apply_vtransform(const double* __restrict__ S, d
                    S[MM_S_VSCALE_B_ON] != 0.0 ? S + MM_S_VSCALE_B : nullptr, v);
 }
 
-// The transforms read from the scalar block once, for a pass over several nodes a lane.
-struct VTransform {
-  bool a_on, m_on, m2_on, b_on;
-  double fa, fb, m[9], m2[9];
-};
+// What a step does to one node, on values that the caller has loaded; S is the system's scalar
+// block (in HBM or LDS).
 
-__device__ __forceinline__ VTransform load_vtransform(const double* __restrict__ S) {
-  VTransform T;
-  T.a_on = S[MM_S_VSCALE_A_ON] != 0.0;
-  T.m_on = S[MM_S_VMAT_ON] != 0.0;
-  T.m2_on = S[MM_S_VMAT2_ON] != 0.0;
-  T.b_on = S[MM_S_VSCALE_B_ON] != 0.0;
-  T.fa = T.a_on ? S[MM_S_VSCALE_A] : 1.0;
-  T.fb = T.b_on ? S[MM_S_VSCALE_B] : 1.0;
-#pragma unroll
-  for (int q = 0; q < 9; ++q) {
-    T.m[q] = T.m_on ? S[MM_S_VMAT + q] : 0.0;
-    T.m2[q] = T.m2_on ? S[MM_S_VMAT2 + q] : 0.0;
+// First half kick and drift (verlet.py:141-146): the pending velocity transforms, with kLT the
+// Langevin thermostat's pre update (its kinetic energy after it added to lt), then
+// v += a dt / 2 and x += dt v.
+template <bool kLT>
+__device__ __forceinline__ void kick_drift_node(const double* S, int64_t n, double mass,
+                                                const double g[3], double v[3], double x[3],
+                                                double& lt) {
+#pragma clang fp contract(off)
+  const double dt = S[MM_S_TIMESTEP];
+  apply_vtransform(S, v);
+  if (kLT) {
+    langevin_thermo(S, n, 0, mass, v);
+    lt += node_ekin(v, mass);
   }
-  return T;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const double a = -g[j] / mass;
+    v[j] = v[j] + (0.5 * a) * dt;
+    x[j] = x[j] + dt * v[j];
+  }
 }
 
-__device__ __forceinline__ void apply_vtransform(const VTransform& T, double v[3]) {
-  apply_vtransform(T.a_on ? &T.fa : nullptr, T.m_on ? T.m : nullptr, T.m2_on ? T.m2 : nullptr,
-                   T.b_on ? &T.fb : nullptr, v);
+// The pending position transforms: an earlier call's when it still waits (the previous post
+// call's, of steps in a row), then the last one's.
+__device__ __forceinline__ void scale_position(const double* S, double x[3]) {
+  double t[3];
+  if (S[MM_S_XMAT2_ON] != 0.0) {
+    vecmat(x, S + MM_S_XMAT2, t);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) x[j] = t[j];
+  }
+  vecmat(x, S + MM_S_XMAT, t);
+#pragma unroll
+  for (int j = 0; j < 3; ++j) x[j] = t[j];
+}
+
+// Second half kick (verlet.py:152-153) and the node sums acc[0..9] of the new velocities; with
+// kLT the Langevin thermostat's post update in between (the kinetic energy before it in lt).
+template <bool kLT, int NA>
+__device__ __forceinline__ void kick_node(const double* S, int64_t n, double mass,
+                                          const double g[3], double v[3], double (&acc)[NA],
+                                          double& lt) {
+#pragma clang fp contract(off)
+  const double dt = S[MM_S_TIMESTEP];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const double a = -g[j] / mass;
+    v[j] = v[j] + (0.5 * a) * dt;
+  }
+  if (kLT) {
+    lt += node_ekin(v, mass);
+    langevin_thermo(S, n, 1, mass, v);
+  }
+  node_vv(v, mass, acc);
+}
+
+// Half kick and drift from a stored gradient, one node a thread: latency bounds it on a small
+// system, above all with the Langevin noise (some 300 dependent instructions a node), so the
+// nodes are spread over as many waves as there are. 40x36x47 Langevin step 52 -> 46 us against
+// four nodes a lane; without noise and on large systems the two are equal (128^3 and the batch of
+// 192 replicas within 0.5%).
+template <bool kLT>
+__global__ void __launch_bounds__(kNodeBlock)
+kick_drift_kernel(double* __restrict__ x, double* __restrict__ v, const double* __restrict__ g,
+                  const double* __restrict__ m, const double* __restrict__ S0,
+                  const int32_t* __restrict__ blk_sys, int64_t N, double* __restrict__ partials) {
+  const double* S = S0 + (blk_sys ? (int64_t)blk_sys[blockIdx.x] * MM_S_COUNT : 0);
+  const int64_t n = (int64_t)blockIdx.x * kNodeBlock + threadIdx.x;
+  double lt[1] = {0.0};
+  if (n < N) {
+    const double mass = m[n];
+    double vv[3], gg[3], xx[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      vv[j] = v[3 * n + j];
+      gg[j] = g[3 * n + j];
+      xx[j] = x[3 * n + j];
+    }
+    kick_drift_node<kLT>(S, n, mass, gg, vv, xx, lt[0]);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      v[3 * n + j] = vv[j];
+      x[3 * n + j] = xx[j];
+    }
+  }
+  if (kLT) block_sum_store_wide<1>(lt, partials + (int64_t)14 * gridDim.x, blockIdx.x);
 }
 
 template <int kMode>
@@ -220,69 +282,19 @@ node_kernel(double* __restrict__ x, double* __restrict__ v, const double* __rest
   double acc[13];
 #pragma unroll
   for (int q = 0; q < 13; ++q) acc[q] = 0.0;
-  double lt[1] = {0.0};
   constexpr int kIt = kNodeBlock / kNodeThreads;
   const int64_t n0 = (int64_t)blockIdx.x * kNodeBlock + threadIdx.x;
-  if (kMode == kKickDrift || kMode == kKickDriftLT) {
-    // every load of the lane's nodes first, then the arithmetic and the stores, so that the
-    // loads are in flight together (a pass over a small system is then one memory round trip
-    // instead of two a node)
-    const double dt = S[MM_S_TIMESTEP];
-    const VTransform T = load_vtransform(S);
-    double mass[kIt], vv[kIt][3], gg[kIt][3], xx[kIt][3];
-#pragma unroll
-    for (int it = 0; it < kIt; ++it) {
-      const int64_t n = n0 + it * kNodeThreads;
-      mass[it] = 1.0;
-#pragma unroll
-      for (int j = 0; j < 3; ++j) vv[it][j] = gg[it][j] = xx[it][j] = 0.0;
-      if (n < N) {
-        mass[it] = m[n];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          vv[it][j] = v[3 * n + j];
-          gg[it][j] = g[3 * n + j];
-          xx[it][j] = x[3 * n + j];
-        }
-      }
-    }
-#pragma unroll
-    for (int it = 0; it < kIt; ++it) {
-      const int64_t n = n0 + it * kNodeThreads;
-      if (n >= N) break;
-      apply_vtransform(T, vv[it]);
-      if (kMode == kKickDriftLT) {
-        langevin_thermo(S, n, 0, mass[it], vv[it]);
-        lt[0] += node_ekin(vv[it], mass[it]);
-      }
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const double a = -gg[it][j] / mass[it];
-        vv[it][j] = vv[it][j] + (0.5 * a) * dt;
-        v[3 * n + j] = vv[it][j];
-        x[3 * n + j] = xx[it][j] + dt * vv[it][j];
-      }
-    }
-  }
 #pragma unroll
   for (int it = 0; it < kIt; ++it) {
     const int64_t n = n0 + it * kNodeThreads;
     if (n >= N) break;
-    if (kMode == kKickDrift || kMode == kKickDriftLT) {
-      // done above
-    } else if (kMode == kScalePos) {
-      double p[3], t[3];
+    if (kMode == kScalePos) {
+      double p[3];
 #pragma unroll
       for (int j = 0; j < 3; ++j) p[j] = x[3 * n + j];
-      // a pending earlier transform first (the previous post call's, of steps in a row)
-      if (S[MM_S_XMAT2_ON] != 0.0) {
-        vecmat(p, S + MM_S_XMAT2, t);
+      scale_position(S, p);
 #pragma unroll
-        for (int j = 0; j < 3; ++j) p[j] = t[j];
-      }
-      vecmat(p, S + MM_S_XMAT, t);
-#pragma unroll
-      for (int j = 0; j < 3; ++j) x[3 * n + j] = t[j];
+      for (int j = 0; j < 3; ++j) x[3 * n + j] = p[j];
     } else if (kMode == kVV || kMode == kApplyV) {
       double vv[3];
 #pragma unroll
@@ -306,7 +318,6 @@ node_kernel(double* __restrict__ x, double* __restrict__ v, const double* __rest
   if (kMode == kVV || kMode == kRmsd) {
     block_sum_store<13>(acc, partials);
   }
-  if (kMode == kKickDriftLT) block_sum_store<1>(lt, partials + (int64_t)14 * gridDim.x);
 }
 
 // gpos[n] = sum of the node's face-class records (mmff.py:303-318; the cell pass has already
@@ -371,57 +382,25 @@ gather_kick_kernel(const int32_t* __restrict__ ncell, const double* __restrict__
     }
     if (!kAllLoads) load_node();
     if (kKick) {
-#pragma clang fp contract(off)
-      const double dt = S[MM_S_TIMESTEP];
-      double vv[3];
+      double lt = 0.0;
+      kick_node<kLT>(S, n, mass, g, v0, acc, lt);
+      if (kLT) acc[NA - 1] += lt;
 #pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const double a = -g[j] / mass;
-        vv[j] = v0[j] + (0.5 * a) * dt;
-      }
-      if (kLT) {
-        acc[NA - 1] += node_ekin(vv, mass);
-        langevin_thermo(S, n, 1, mass, vv);
-      }
-#pragma unroll
-      for (int j = 0; j < 3; ++j) v[3 * n + j] = vv[j];
-      node_vv(vv, mass, acc);
+      for (int j = 0; j < 3; ++j) v[3 * n + j] = v0[j];
     }
     if (kScaleV) {
-      double vv[3];
+      apply_vtransform(S, v0);
 #pragma unroll
-      for (int j = 0; j < 3; ++j) vv[j] = v0[j];
-      apply_vtransform(S, vv);
-#pragma unroll
-      for (int j = 0; j < 3; ++j) v[3 * n + j] = vv[j];
+      for (int j = 0; j < 3; ++j) v[3 * n + j] = v0[j];
     }
     if (kDrift) {
-#pragma clang fp contract(off)
-      const double dt = S[MM_S_TIMESTEP];
-      double vv[3];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) vv[j] = v0[j];
-      apply_vtransform(S, vv);
-      if (kLT) {
-        langevin_thermo(S, n, 0, mass, vv);
-        acc[0] += node_ekin(vv, mass);
-      }
       // the positions as the cell pass read them: the pending scaling(s) of the barostat call
-      double p[3], t[3];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) p[j] = x0[j];
-      if (S[MM_S_XMAT2_ON] != 0.0) {
-        vecmat(p, S + MM_S_XMAT2, t);
-#pragma unroll
-        for (int j = 0; j < 3; ++j) p[j] = t[j];
-      }
-      vecmat(p, S + MM_S_XMAT, t);
+      scale_position(S, x0);
+      kick_drift_node<kLT>(S, n, mass, g, v0, x0, acc[0]);
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        const double a = -g[j] / mass;
-        vv[j] = vv[j] + (0.5 * a) * dt;
-        v[3 * n + j] = vv[j];
-        x[3 * n + j] = t[j] + dt * vv[j];
+        v[3 * n + j] = v0[j];
+        x[3 * n + j] = x0[j];
       }
     }
     }
@@ -472,6 +451,7 @@ __device__ constexpr double kInvK[15] = {0.0,       1.0,        1.0 / 2,  1.0 / 
 // barostat velocity times dt / 2 is of order 1e-5, where m = 3), and the result is squared s
 // times. Multiply-adds only: no square roots or divisions on the serial path.
 __device__ void expm_sym_half(const double* A, double sign, double dt, double* R) {
+#pragma clang fp contract(off)
   const double h = (sign * dt) / 2.0;
   double X[9];
   double nrm = 0.0;
@@ -511,9 +491,11 @@ __device__ void expm_sym_half(const double* A, double sign, double dt, double* R
     for (int i = 0; i < 3; ++i)
 #pragma unroll
       for (int j = 0; j < 3; ++j)
-        T[3 * i + j] = X[3 * i + 0] * P[0 + j] + X[3 * i + 1] * P[3 + j] + X[3 * i + 2] * P[6 + j];
+        T[3 * i + j] = __builtin_fma(
+            X[3 * i + 2], P[6 + j],
+            __builtin_fma(X[3 * i + 1], P[3 + j], X[3 * i + 0] * P[0 + j]));
 #pragma unroll
-    for (int q = 0; q < 9; ++q) P[q] = T[q] * inv + ((q % 4 == 0) ? 1.0 : 0.0);
+    for (int q = 0; q < 9; ++q) P[q] = __builtin_fma(T[q], inv, (q % 4 == 0) ? 1.0 : 0.0);
   }
   for (int i = 0; i < s; ++i) matmul3(P, P, P);
 #pragma unroll
@@ -908,25 +890,26 @@ __device__ void take_nodes_after_vmat(double* S, const double (&nd)[kNodeSums]) 
 // The force partials fpart[q * nbf + b] over the blocks b = fidx[ff + i] (or ff + i), i < fc,
 // and the node partials npart[q * nbn + nf + i], i < nc, summed in a fixed order: each thread
 // over its strided share in index order, then the wave by the reduce-scatter butterfly, then
-// the waves in order. The loads of both kinds are issued before any sum, and every thread of
-// the block receives the totals.
-__device__ void reduce_force_nodes(const double* __restrict__ fpart, int nbf,
-                                   const int32_t* __restrict__ fidx, int ff, int fc,
-                                   const double* __restrict__ npart, int nbn, int nf, int nc,
-                                   double (&f)[10], double (&nd)[kNodeSums]) {
+// the waves in order, into tot[kSliceQ] in LDS. The loads of both kinds are issued before any
+// sum. Called by a whole block of at least kScalarThreads threads, of which the first
+// kScalarThreads sum.
+__device__ __forceinline__ void reduce_force_nodes(const double* fpart, int nbf,
+                                                   const int32_t* __restrict__ fidx, int ff,
+                                                   int fc, const double* npart, int nbn, int nf,
+                                                   int nc, double* tot) {
   constexpr int kWaves = kScalarThreads / 64;
-  constexpr int NV = 10 + kNodeSums;
+  constexpr int NV = kSliceQ;
   __shared__ double red[NV * kWaves];
-  __shared__ double tot[NV];
   double acc[NV];
 #pragma unroll
   for (int q = 0; q < NV; ++q) acc[q] = 0.0;
-  for (int i = threadIdx.x; i < fc; i += kScalarThreads) {
+  const bool on = threadIdx.x < kScalarThreads;
+  for (int i = threadIdx.x; on && i < fc; i += kScalarThreads) {
     const int b = fidx ? fidx[ff + i] : ff + i;
 #pragma unroll
     for (int q = 0; q < 10; ++q) acc[q] += fpart[(int64_t)q * nbf + b];
   }
-  for (int i = threadIdx.x; i < nc; i += kScalarThreads) {
+  for (int i = threadIdx.x; on && i < nc; i += kScalarThreads) {
 #pragma unroll
     for (int q = 0; q < kNodeSums; ++q) acc[10 + q] += npart[(int64_t)q * nbn + nf + i];
   }
@@ -940,7 +923,7 @@ __device__ void reduce_force_nodes(const double* __restrict__ fpart, int nbf,
     const double tl = wave_reduce_scatter<16>(lo, lane);
     const double th = wave_reduce_scatter<NV - 16>(hi, lane);
     const int q = scatter_index(lane);
-    if ((lane & 3) == 0) {
+    if (on && (lane & 3) == 0) {
       red[wave * NV + q] = tl;
       if (q < NV - 16) red[wave * NV + 16 + q] = th;
     }
@@ -951,11 +934,6 @@ __device__ void reduce_force_nodes(const double* __restrict__ fpart, int nbf,
     for (int w = 1; w < kWaves; ++w) t += red[w * NV + threadIdx.x];
     tot[threadIdx.x] = t;
   }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < 10; ++q) f[q] = tot[q];
-#pragma unroll
-  for (int q = 0; q < kNodeSums; ++q) nd[q] = tot[10 + q];
   __syncthreads();
 }
 
@@ -1128,6 +1106,22 @@ __device__ void run_phase(int phase, double* S, const double (&f)[10],
   }
 }
 
+// One phase, or the end of one step and the start of the next on the same copy of the block; tot
+// holds the force and node sums.
+__device__ __forceinline__ void run_phases(int phase, double* S, const double* tot,
+                                           int with_vtens, int sys) {
+  const double(&f)[10] = *reinterpret_cast<const double(*)[10]>(tot);
+  const double(&nd)[kNodeSums] = *reinterpret_cast<const double(*)[kNodeSums]>(tot + 10);
+  const bool chained = phase == kPhBaroEndPostPre;
+  const int next = chained ? kPhBaroPre : phase == kPhNvtEndPre ? kPhNvtPre : -1;
+  int now = chained ? kPhBaroEndPost : phase == kPhNvtEndPre ? kPhNvtEnd : phase;
+  for (;;) {
+    run_phase(now, S, f, nd, with_vtens, sys, chained);
+    if (now == next || next < 0) break;
+    now = next;
+  }
+}
+
 // Grid (slices, systems). Block (g, sys) reduces slice g of that system's force and node
 // partials; the last block of the system to finish (counted with an atomic counter, which it
 // resets) sums the slices in slice order and runs the phase on a copy of the system's scalar
@@ -1146,7 +1140,6 @@ scalar_kernel(int phase, double* __restrict__ S0, const double* __restrict__ fpa
   double* Sg = S0 + (int64_t)sys * MM_S_COUNT;
   // the scalar block is loaded up front, so that its latency hides behind the reduction
   const double s_own = threadIdx.x < MM_S_COUNT ? Sg[threadIdx.x] : 0.0;
-  double f[10], nd[kNodeSums];
   {
     int ff = 0, fc = 0, nf = 0, nc = 0;
     if (phase_uses_force(phase)) {
@@ -1159,13 +1152,12 @@ scalar_kernel(int phase, double* __restrict__ S0, const double* __restrict__ fpa
       nf = b0 + (int)((int64_t)cnt * gi / G);
       nc = b0 + (int)((int64_t)cnt * (gi + 1) / G) - nf;
     }
-    reduce_force_nodes(fpart, nbf, fsys_idx, ff, fc, npart, nbn, nf, nc, f, nd);
+    reduce_force_nodes(fpart, nbf, fsys_idx, ff, fc, npart, nbn, nf, nc, tot);
   }
   if (G > 1) {
     if (threadIdx.x == 0) {
       double* sl = slices + ((int64_t)sys * G + gi) * kSliceQ;
-      for (int q = 0; q < 10; ++q) sl[q] = f[q];
-      for (int q = 0; q < kNodeSums; ++q) sl[10 + q] = nd[q];
+      for (int q = 0; q < kSliceQ; ++q) sl[q] = tot[q];
       __threadfence();
       const unsigned int prev = atomicAdd(&counters[sys], 1u);
       is_last = prev == (unsigned int)(G - 1);
@@ -1184,25 +1176,11 @@ scalar_kernel(int phase, double* __restrict__ S0, const double* __restrict__ fpa
       tot[threadIdx.x] = t;
     }
     if (threadIdx.x == 0) counters[sys] = 0u;
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 10; ++q) f[q] = tot[q];
-#pragma unroll
-    for (int q = 0; q < kNodeSums; ++q) nd[q] = tot[10 + q];
   }
   if (threadIdx.x < MM_S_COUNT) Sl[threadIdx.x] = s_own;
   __syncthreads();
   if (threadIdx.x == 0) {
-    // the end of one step and the start of the next, on the same copy of the block
-    if (phase == kPhBaroEndPostPre) {
-      run_phase(kPhBaroEndPost, Sl, f, nd, with_vtens, sys, true);
-      run_phase(kPhBaroPre, Sl, f, nd, with_vtens, sys);
-    } else if (phase == kPhNvtEndPre) {
-      run_phase(kPhNvtEnd, Sl, f, nd, with_vtens, sys);
-      run_phase(kPhNvtPre, Sl, f, nd, with_vtens, sys);
-    } else {
-      run_phase(phase, Sl, f, nd, with_vtens, sys);
-    }
+    run_phases(phase, Sl, tot, with_vtens, sys);
   }
   __syncthreads();
   for (int q = threadIdx.x; q < MM_S_COUNT; q += kScalarThreads) Sg[q] = Sl[q];
@@ -1292,14 +1270,24 @@ hipError_t node(mm_md* md, int mode, hipStream_t s) {
   hipLaunchKernelGGL((node_kernel<M>), grid, block, 0, s, md->pos, md->vel, md->gpos,        \
                      md->masses, md->posold, md->S, md->node_blk_sys, md->N, md->npart)
   switch (mode) {
-    case kKickDrift: MM_NODE(kKickDrift); break;
     case kScalePos: MM_NODE(kScalePos); break;
     case kVV: MM_NODE(kVV); break;
     case kApplyV: MM_NODE(kApplyV); break;
     case kRmsd: MM_NODE(kRmsd); break;
-    case kKickDriftLT: MM_NODE(kKickDriftLT); break;
   }
 #undef MM_NODE
+  return hipGetLastError();
+}
+
+hipError_t kick_drift(mm_md* md, bool lt, hipStream_t s) {
+#define MM_KD(T)                                                                            \
+  hipLaunchKernelGGL((kick_drift_kernel<T>), dim3(md->nbn), dim3(kNodeBlock), 0, s, md->pos,  \
+                     md->vel, md->gpos, md->masses, md->S, md->node_blk_sys, md->N, md->npart)
+  if (lt)
+    MM_KD(true);
+  else
+    MM_KD(false);
+#undef MM_KD
   return hipGetLastError();
 }
 
@@ -1451,15 +1439,15 @@ hipError_t enqueue_step(mm_md* md, hipStream_t s, bool lean = false, bool pre = 
                      lean ? kGatherNone : kGatherStore, false, lean));
   } else if (md->thermo == MM_THERMO_NHC) {
     if (pre) MM_TRY(scalar(md, kPhNvtPre, 1, s));
-    MM_TRY(node(md, kKickDrift, s));
+    MM_TRY(kick_drift(md, false, s));
     MM_TRY(force(md, true, false, s));
     MM_TRY(scalar(md, lean ? kPhNvtEndPre : kPhNvtEnd, 1, s));
   } else if (lt) {
-    MM_TRY(node(md, kKickDriftLT, s));
+    MM_TRY(kick_drift(md, true, s));
     MM_TRY(force(md, true, true, s));
     MM_TRY(scalar(md, kPhNvtEnd, 1, s));
   } else {
-    MM_TRY(node(md, kKickDrift, s));
+    MM_TRY(kick_drift(md, false, s));
     MM_TRY(force(md, true, false, s));
     MM_TRY(scalar(md, kPhNveEnd, 1, s));
   }
