@@ -427,30 +427,72 @@ gather_kick_kernel(const int32_t* __restrict__ ncell, const double* __restrict__
 }
 
 // ----------------------------------------------------------------------------- scalar math
+//
+// The scalar phases are one long dependence chain on a few dozen numbers, and every kernel of the
+// step waits for them. They run on the 64 lanes of one wave: what is one number is computed by
+// all lanes alike, the nine entries of a 3x3 matrix by nine lanes at once (entry_of), the beads of
+// a chain by a lane each, the two exponentials of a barostat call by the two halves of the wave,
+// and the divisions of the properties together, so that the chain holds few divisions and few
+// waits for LDS; the scalar block is in LDS, where a wave's accesses keep their order. A wave
+// alone on its SIMD issues an instruction every four to eight cycles, so the length of this code is
+// its time: all phases of a step took 5.4 us (NVT-NHC) and 23 us (NPT) on one lane, now 3.4 and
+// 10.7 us; 32^3 NVT step 37.7 -> 34.8 us, 24x19x27 NPT 82 -> 72 us, 128^3 NPT 579 -> 572 us.
 
-__device__ void matmul3(const double* A, const double* B, double* C) {
-#pragma clang fp contract(off)
-  double T[9];
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j)
-      T[3 * i + j] = (A[3 * i + 0] * B[0 + j] + A[3 * i + 1] * B[3 + j]) + A[3 * i + 2] * B[6 + j];
-  for (int i = 0; i < 9; ++i) C[i] = T[i];
+// The scalar block of a phase, in LDS; six more doubles behind it are scratch.
+typedef __attribute__((address_space(3))) double lds_f64;
+constexpr int kScratch = MM_S_COUNT;
+
+// Lane l's copy of v.
+__device__ __forceinline__ double lane_value(double v, int l) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, l);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// 1 / k for the Horner steps of expm_sym_half (correctly rounded, as the division gives).
-__device__ constexpr double kInvK[15] = {0.0,       1.0,        1.0 / 2,  1.0 / 3,  1.0 / 4,
-                                         1.0 / 5,   1.0 / 6,    1.0 / 7,  1.0 / 8,  1.0 / 9,
-                                         1.0 / 10,  1.0 / 11,   1.0 / 12, 1.0 / 13, 1.0 / 14};
+// The matrix entry of a lane: lanes 0..8 own one each, the others repeat the last.
+__device__ __forceinline__ int entry_of(int lane) { return lane < 9 ? lane : 8; }
+__device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
+
+// exp(x): for |x| <= 1/16, where the chains' and barostats' arguments lie, the Taylor polynomial of
+// degree 11 (first omitted term below 2e-22) as 1 + (x + x^2 q), a dozen instructions in six
+// dependent steps; the general function otherwise.
+__device__ __attribute__((noinline)) double exp_far(double x) { return exp(x); }
+__device__ __forceinline__ double exp_near0(double x) {
+  if (__any(!(fabs(x) <= 0.0625))) return exp_far(x);
+  const double x2 = x * x, x4 = x2 * x2;
+  const double a0 = __builtin_fma(x, 1.0 / 6, 1.0 / 2), a1 = __builtin_fma(x, 1.0 / 120, 1.0 / 24),
+               a2 = __builtin_fma(x, 1.0 / 5040, 1.0 / 720),
+               a3 = __builtin_fma(x, 1.0 / 362880, 1.0 / 40320),
+               a4 = __builtin_fma(x, 1.0 / 39916800, 1.0 / 3628800);
+  const double b0 = __builtin_fma(x2, a1, a0), b1 = __builtin_fma(x2, a3, a2);
+  const double q = __builtin_fma(x4, __builtin_fma(x4, a4, b1), b0);
+  return 1.0 + __builtin_fma(x2, q, x);
+}
+
+// D = C + A B (D may be C).
+__device__ __forceinline__ void fma_matmul(const double (&A)[9], const double (&B)[9],
+                                           const double (&C)[9], double (&D)[9]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+      D[3 * i + j] = __builtin_fma(
+          A[3 * i + 2], B[6 + j],
+          __builtin_fma(A[3 * i + 1], B[3 + j],
+                        __builtin_fma(A[3 * i + 0], B[0 + j], C[3 * i + j])));
+}
 
 // R = exp(sign * A * dt / 2) for symmetric A: the matrix the reference forms from
 // eigh(A) = (w, Q) as Q diag(exp(sign w dt / 2)) Q^T (npt.py:686-690, 709-726), here by scaling
-// and squaring. X = sign * A * dt / 2 is halved s times until r = ||X||_inf <= 1/2, exp(X) is
-// the Taylor polynomial in Horner form to the smallest degree m <= 14 whose first omitted term
-// bound r^(m+1) / (m+1)! is below 1e-17 (the remainder is at most that times e^r against
-// ||exp(X)|| >= e^-r: below 3e-17 relative, the bound of the full degree 14 at r = 1/2; a
-// barostat velocity times dt / 2 is of order 1e-5, where m = 3), and the result is squared s
-// times. Multiply-adds only: no square roots or divisions on the serial path.
-__device__ void expm_sym_half(const double* A, double sign, double dt, double* R) {
+// and squaring, one matrix a lane. X = sign * A * dt / 2 is halved s times until
+// r = ||X||_inf <= 1/2, exp(X) is the Taylor polynomial of degree 6 where r <= 1/80 on every lane
+// (its first omitted term r^7 / 7! is then below 1e-17; a barostat velocity times dt / 2 is of
+// order 1e-5 to 1e-3), as I + X + X^2 / 2 + X^3 (I / 6 + X / 24 + X^2 / 120 + X^3 / 720), and of
+// degree 14 otherwise (the remainder is at most e^r times the first omitted term against
+// ||exp(X)|| >= e^-r: below 3e-17 relative at r = 1/2); the result is squared s times.
+__device__ __forceinline__ void expm_sym_half(const double (&A)[9], double sign, double dt,
+                                              double (&P)[9]) {
 #pragma clang fp contract(off)
   const double h = (sign * dt) / 2.0;
   double X[9];
@@ -465,6 +507,22 @@ __device__ void expm_sym_half(const double* A, double sign, double dt, double* R
     }
     nrm = fmax(nrm, r);
   }
+  if (__all(nrm <= 0.0125)) {
+    double X2[9], X3[9], B[9];
+    const double zero[9] = {};
+    fma_matmul(X, X, zero, X2);
+    fma_matmul(X2, X, zero, X3);
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+      const double one = (q % 4 == 0) ? 1.0 : 0.0;
+      P[q] = __builtin_fma(X2[q], 0.5, one + X[q]);
+      B[q] = __builtin_fma(X3[q], 1.0 / 720,
+                           __builtin_fma(X2[q], 1.0 / 120,
+                                         __builtin_fma(X[q], 1.0 / 24, one * (1.0 / 6))));
+    }
+    fma_matmul(X3, B, P, P);
+    return;
+  }
   int s = 0;
   double scale = 1.0;
   while (nrm * scale > 0.5 && s < 64) {
@@ -473,37 +531,32 @@ __device__ void expm_sym_half(const double* A, double sign, double dt, double* R
   }
 #pragma unroll
   for (int q = 0; q < 9; ++q) X[q] *= scale;
-  const double r = nrm * scale;
-  int m = 1;
-  double bound = (r * r) / 2.0;
-  while (m < 14 && bound > 1e-17) {
-    ++m;
-    bound *= r / (double)(m + 1);
-  }
-  double P[9];
 #pragma unroll
   for (int q = 0; q < 9; ++q) P[q] = (q % 4 == 0) ? 1.0 : 0.0;
-  for (int k = m; k >= 1; --k) {
+#pragma unroll 1
+  for (int k = 14; k >= 1; --k) {
     // P <- I + X P / k
-    const double inv = kInvK[k];
+    double T[9];
+    const double zero[9] = {};
+    fma_matmul(X, P, zero, T);
+#pragma unroll
+    for (int q = 0; q < 9; ++q) P[q] = __builtin_fma(T[q], 1.0 / k, (q % 4 == 0) ? 1.0 : 0.0);
+  }
+  for (int t = 0; t < s; ++t) {
     double T[9];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
       for (int j = 0; j < 3; ++j)
-        T[3 * i + j] = __builtin_fma(
-            X[3 * i + 2], P[6 + j],
-            __builtin_fma(X[3 * i + 1], P[3 + j], X[3 * i + 0] * P[0 + j]));
+        T[3 * i + j] =
+            (P[3 * i + 0] * P[0 + j] + P[3 * i + 1] * P[3 + j]) + P[3 * i + 2] * P[6 + j];
 #pragma unroll
-    for (int q = 0; q < 9; ++q) P[q] = __builtin_fma(T[q], inv, (q % 4 == 0) ? 1.0 : 0.0);
+    for (int q = 0; q < 9; ++q) P[q] = T[q];
   }
-  for (int i = 0; i < s; ++i) matmul3(P, P, P);
-#pragma unroll
-  for (int q = 0; q < 9; ++q) R[q] = P[q];
 }
 
 // |det| of the domain vectors, as micmec/pes/domain.c:42-48.
-__device__ double volume3(const double* r) {
+__device__ double volume3(const lds_f64* r) {
 #pragma clang fp contract(off)
   return fabs(r[0] * (r[4] * r[8] - r[5] * r[7]) + r[1] * (r[5] * r[6] - r[3] * r[8]) +
               r[2] * (r[3] * r[7] - r[4] * r[6]));
@@ -519,76 +572,100 @@ constexpr ChainSlots kThermoChain{MM_S_CHAIN_LEN, MM_S_THERMO_TEMP, MM_S_CHAIN_N
 constexpr ChainSlots kBaroChain{MM_S_BCHAIN_LEN, MM_S_BCHAIN_TEMP, MM_S_BCHAIN_NDOF,
                                 MM_S_BCHAIN_MASS, MM_S_BCHAIN_POS, MM_S_BCHAIN_VEL};
 
-// NHChain.__call__ (nvt.py:410-451): returns the velocity factor; updates ekin in place.
-__device__ double nhc_chain(double* S, double* ekin_io, bool has_g1, double g1,
-                            const ChainSlots& c = kThermoChain) {
+// The value of the next / previous lane (a DPP wave shift; the end lane keeps its own).
+__device__ __forceinline__ double next_lane(double v) { return dpp_f64<0x130, 0xF>(v, v); }
+__device__ __forceinline__ double previous_lane(double v) { return dpp_f64<0x138, 0xF>(v, v); }
+
+// NHChain.__call__ (nvt.py:410-451): the velocity factor and the new kinetic energy. Lane k holds
+// bead k. The sweep from the last bead to the first takes each bead's force from the old velocity
+// of the bead before it, so all forces are formed at once and only the factors (from the new
+// velocity of the bead behind) follow each other; the sweep back the other way round. The forces
+// are divided by the masses through their reciprocals with one correction step, which rounds
+// as the division does; (g dt) / 4 and (v dt) / 8 round as g (dt / 4) and v (dt / 8).
+struct ChainStep {
+  double factor, ekin;
+};
+__device__ __forceinline__ ChainStep nhc_chain(lds_f64* S, double ekin, bool has_g1, double g1,
+                                               const ChainSlots& c) {
 #pragma clang fp contract(off)
-  const int L = (int)S[c.len];
-  const double dt = S[MM_S_TIMESTEP];
-  const double temp = S[c.temp];
-  const double kb = S[MM_S_BOLTZMANN];
-  const double ndof = S[c.ndof];
-  double* mass = S + c.mass;
-  double* pos = S + c.pos;
-  double* vel = S + c.vel;
-  auto bead = [&](int k, double ekin) {
-    double g;
-    if (k == 0) {
-      g = 2.0 * ekin - (ndof * temp) * kb;
-      if (has_g1) g += g1;
-    } else {
-      g = mass[k - 1] * (vel[k - 1] * vel[k - 1]) - temp * kb;
-    }
-    g /= mass[k];
-    if (k == L - 1) {
-      vel[k] += (g * dt) / 4.0;
-    } else {
-      // the same factor before and after the force term (vel[k + 1] does not change between)
-      const double e = exp(((-vel[k + 1]) * dt) / 8.0);
-      vel[k] *= e;
-      vel[k] += (g * dt) / 4.0;
-      vel[k] *= e;
-    }
+  const int lane = lane_id(), own = lane & 7;
+  const int L = __builtin_amdgcn_readfirstlane((int)S[c.len]);
+  const double dt = S[MM_S_TIMESTEP], dt4 = dt / 4.0, dt8 = dt / 8.0;
+  const double kt = S[c.temp] * S[MM_S_BOLTZMANN];
+  const double nkt = (S[c.ndof] * S[c.temp]) * S[MM_S_BOLTZMANN];
+  const double mass = S[c.mass + own];
+  double vel = S[c.vel + own];
+  const double pos = S[c.pos + own];
+  const double inv = 1.0 / mass, mass_before = previous_lane(mass);
+  auto kick = [&](double v_before, double ek) {
+    double first = 2.0 * ek - nkt;
+    if (has_g1) first += g1;
+    const double g = lane == 0 ? first : mass_before * (v_before * v_before) - kt;
+    const double q = g * inv;
+    return __builtin_fma(__builtin_fma(-q, mass, g), inv, q) * dt4;
   };
-  double ekin = *ekin_io;
-  for (int k = L - 1; k >= 0; --k) bead(k, ekin);
-  for (int k = 0; k < L; ++k) pos[k] += (vel[k] * dt) / 2.0;
-  const double factor = exp(((-vel[0]) * dt) / 2.0);
+  auto damping = [&](double v) {
+    const double e = exp_near0((-next_lane(v)) * dt8);
+    return lane == L - 1 ? 1.0 : e;
+  };
+  const double down = kick(previous_lane(vel), ekin);
+#pragma unroll 1
+  for (int k = L - 1; k >= 0; --k) {
+    const double e = damping(vel);
+    const double v = (vel * e + down) * e;
+    vel = lane == k ? v : vel;
+  }
+  if (lane < L) S[c.pos + own] = pos + (vel * dt) / 2.0;
+  const double factor = exp_near0(((-lane_value(vel, 0)) * dt) / 2.0);
   ekin *= factor * factor;
-  for (int k = 0; k < L; ++k) bead(k, ekin);
-  *ekin_io = ekin;
-  return factor;
+  const double e = damping(vel);
+#pragma unroll 1
+  for (int k = 0; k < L; ++k) {
+    const double v = (vel * e + kick(previous_lane(vel), ekin)) * e;
+    vel = lane == k ? v : vel;
+  }
+  if (lane < L) S[c.vel + own] = vel;
+  return {factor, ekin};
 }
 
 // NHChain.get_econs_correction (nvt.py:453-458)
-__device__ double nhc_econs(const double* S, const ChainSlots& c = kThermoChain) {
+__device__ __forceinline__ double nhc_econs(const lds_f64* S, const ChainSlots& c = kThermoChain) {
 #pragma clang fp contract(off)
-  const int L = (int)S[c.len];
+  const int L = __builtin_amdgcn_readfirstlane((int)S[c.len]);
+  const int own = lane_id() & 7;
   const double kt = S[MM_S_BOLTZMANN] * S[c.temp];
+  const double vel = S[c.vel + own], pos = S[c.pos + own];
+  const double twice = (vel * vel) * S[c.mass + own];
   double kin = 0.0, rest = 0.0;
-  for (int k = 0; k < L; ++k) kin += (S[c.vel + k] * S[c.vel + k]) * S[c.mass + k];
-  for (int k = 1; k < L; ++k) rest += S[c.pos + k];
-  return 0.5 * kin + kt * (S[c.ndof] * S[c.pos] + rest);
+#pragma unroll 1
+  for (int k = 0; k < L; ++k) {
+    kin += lane_value(twice, k);
+    if (k > 0) rest += lane_value(pos, k);
+  }
+  return 0.5 * kin + kt * (S[c.ndof] * lane_value(pos, 0) + rest);
 }
 
-__device__ __forceinline__ bool baro_chain_on(const double* S) {
+__device__ __forceinline__ bool baro_chain_on(const lds_f64* S) {
   return S[MM_S_BCHAIN_ON] != 0.0;
 }
 
 // MTKBarostat._compute_ekin_baro (npt.py:748-757): W tr(v_g^T v_g) / 2, or W v_g^2 / 2 in the
 // isotropic form.
-__device__ double baro_ekin(const double* S) {
+__device__ __forceinline__ double baro_ekin(const lds_f64* S) {
 #pragma clang fp contract(off)
   if (S[MM_S_BARO_ANISO] == 0.0)
     return (0.5 * S[MM_S_MASS_PRESS]) * (S[MM_S_VEL_PRESS] * S[MM_S_VEL_PRESS]);
-  double tr = 0.0;
-  for (int i = 0; i < 9; ++i) tr += S[MM_S_VEL_PRESS + i] * S[MM_S_VEL_PRESS + i];
+  double v[9], tr = 0.0;
+#pragma unroll
+  for (int i = 0; i < 9; ++i) v[i] = S[MM_S_VEL_PRESS + i];
+#pragma unroll
+  for (int i = 0; i < 9; ++i) tr += v[i] * v[i];
   return (0.5 * S[MM_S_MASS_PRESS]) * tr;
 }
 
 // MTKBarostat.add_press_cont (npt.py:738-746); with its own chain the barostat is decoupled
 // from the particle thermostat and contributes 0.
-__device__ double add_press_cont(const double* S) {
+__device__ double add_press_cont(const lds_f64* S) {
 #pragma clang fp contract(off)
   if (baro_chain_on(S)) return 0.0;
   return 2.0 * baro_ekin(S) - S[MM_S_BARO_NDOF] * (S[MM_S_BARO_TEMP] * S[MM_S_BOLTZMANN]);
@@ -597,27 +674,30 @@ __device__ double add_press_cont(const double* S) {
 // The barostat chain's half step on the barostat kinetic energy (npt.py:625-629, 634-638): the
 // chain advances, the velocity factor it returns is discarded (v_g is damped inside
 // update_baro_vel through chainvel0).
-__device__ void baro_chain_step(double* S) {
-  double ekin = baro_ekin(S);
-  (void)nhc_chain(S, &ekin, true, 0.0, kBaroChain);
+__device__ void baro_chain_step(lds_f64* S) {
+  (void)nhc_chain(S, baro_ekin(S), true, 0.0, kBaroChain);
 }
 
-__device__ __forceinline__ bool baro_langevin(const double* S) {
+__device__ __forceinline__ bool baro_langevin(const lds_f64* S) {
   return S[MM_S_BARO] == (double)MM_BARO_LANGEVIN;
 }
-__device__ __forceinline__ bool baro_aniso(const double* S) {
+__device__ __forceinline__ bool baro_aniso(const lds_f64* S) {
   return S[MM_S_BARO_ANISO] != 0.0;
 }
-__device__ __forceinline__ bool thermo_nhc(const double* S) {
+__device__ __forceinline__ bool thermo_nhc(const lds_f64* S) {
   return S[MM_S_THERMO] == (double)MM_THERMO_NHC;
 }
 
 // LangevinBarostat.getR (npt.py:489-505): a symmetric matrix whose lower triangle is a draw of
-// N(0, 1) x RSCALE, here the normals of system sys at hook call 2 counter + post, update sub.
-__device__ void langevin_random_force(const double* S, int sys, int post, int sub, double R[9]) {
+// N(0, 1) x RSCALE, here the normals of system sys at hook call 2 counter + post, update sub:
+// the triangle row by row (00, 10, 11, 20, 21, 22).
+__device__ __attribute__((noinline)) void langevin_random_force(const lds_f64* S, int sys,
+                                                                 int post, int sub,
+                                                                 lds_f64* R) {
 #pragma clang fp contract(off)
   const uint64_t call = 2ull * (uint64_t)S[MM_S_COUNTER] + (uint64_t)post;
-  const uint64_t key = seed_from(S + MM_S_LB_SEED);
+  const double seed[2] = {S[MM_S_LB_SEED], S[MM_S_LB_SEED + 1]};
+  const uint64_t key = seed_from(seed);
   double z[8];
 #pragma unroll
   for (int b = 0; b < 2; ++b) {
@@ -625,132 +705,119 @@ __device__ void langevin_random_force(const double* S, int sys, int post, int su
     normals4(ctr, key, kStreamBarostat, z + 4 * b);
   }
   const double sc = S[MM_S_LB_RSCALE];
-  int k = 0;
 #pragma unroll
-  for (int i = 0; i < 3; ++i) {
-#pragma unroll
-    for (int j = 0; j <= i; ++j) {
-      const double r = z[k++] * sc;
-      R[3 * i + j] = r;
-      R[3 * j + i] = r;
-    }
-  }
+  for (int k = 0; k < 6; ++k) R[k] = z[k] * sc;
 }
 
 // update_baro_vel of MTKBarostat.baro (npt.py:654-681) and of LangevinBarostat.baro
 // (npt.py:394-432: friction exp(-dt / 8 tau) on both sides, random force R, optional volume
 // constraint and isotropic form). sub is 0 for the first and 1 for the second update of a call.
-__device__ __forceinline__ void update_baro_vel(double* S, int sys, int post, int sub) {
+// One entry of v_g a lane (the isotropic form has one for all).
+__device__ __forceinline__ void update_baro_vel(lds_f64* S, int sys, int post, int sub) {
 #pragma clang fp contract(off)
-  const double dt = S[MM_S_TIMESTEP];
-  double* vp = S + MM_S_VEL_PRESS;
-  const bool lb = baro_langevin(S);
-  const bool aniso = baro_aniso(S);
-  const int nv = aniso ? 9 : 1;
+  const int q = entry_of(lane_id()), i = q / 3, j = q - 3 * i, qt = 3 * j + i;
+  const double dt = S[MM_S_TIMESTEP], W = S[MM_S_MASS_PRESS];
+  const bool lb = baro_langevin(S), aniso = baro_aniso(S), volcon = S[MM_S_BARO_VOLCON] != 0.0;
   const bool has = S[MM_S_HAS_CHAINVEL0] != 0.0;
-  const double cv0 = S[MM_S_CHAINVEL0];
-  const double fric = lb ? exp((-dt) / (8.0 * S[MM_S_LB_TIMECON])) : 1.0;
+  const double fric = lb ? exp_near0((-dt) / (8.0 * S[MM_S_LB_TIMECON])) : 1.0;
   // the chain's damping factor, applied before and after the force term
-  const double fchain = has ? exp(((-dt) * cv0) / 8.0) : 1.0;
-  if (lb)
-    for (int i = 0; i < nv; ++i) vp[i] *= fric;
-  if (has) {
-    for (int i = 0; i < nv; ++i) vp[i] *= fchain;
-  }
-  double P[9], G[9];
-  for (int i = 0; i < 9; ++i) P[i] = S[MM_S_SVV + i] - S[MM_S_VTENS + i];
+  const double fchain = has ? exp_near0(((-dt) * S[MM_S_CHAINVEL0]) / 8.0) : 1.0;
+  lds_f64* slot = S + MM_S_VEL_PRESS + (aniso ? q : 0);
+  double vp = *slot;
+  if (lb) vp *= fric;
+  if (has) vp *= fchain;
   const double diag = (2.0 * S[MM_S_EKIN]) / S[MM_S_NDOF] - S[MM_S_BARO_PRESS] * S[MM_S_VOLUME];
-  for (int i = 0; i < 3; ++i) {
-    for (int j = 0; j < 3; ++j) {
-      double p = 0.5 * (P[3 * j + i] + P[3 * i + j]);
-      if (i == j) p = p + diag;
-      G[3 * i + j] = p / S[MM_S_MASS_PRESS];
-    }
-  }
+  const double Pq = S[MM_S_SVV + q] - S[MM_S_VTENS + q];
+  const double Pt = S[MM_S_SVV + qt] - S[MM_S_VTENS + qt];
+  double p = 0.5 * (Pt + Pq);
+  if (i == j) p = p + diag;
+  double G = p / W;
+  const double trace = (lane_value(G, 0) + lane_value(G, 4)) + lane_value(G, 8);
   if (!lb) {
     // MTK (npt.py:671-676): the isotropic form takes the trace, the volume constraint removes
     // it (the two together are refused at construction, utils.py:498-500)
     if (!aniso) {
-      vp[0] += ((((G[0] + G[4]) + G[8])) * dt) / 4.0;
-    } else {
-      if (S[MM_S_BARO_VOLCON] != 0.0) {
-        const double tg = ((G[0] + G[4]) + G[8]) / S[MM_S_NVEC];
-        for (int i = 0; i < 9; i += 4) G[i] -= tg;
-      }
-      for (int i = 0; i < 9; ++i) vp[i] += (G[i] * dt) / 4.0;
+      G = trace;
+    } else if (volcon) {
+      const double tg = trace / S[MM_S_NVEC];
+      if (i == j) G -= tg;
     }
+    vp += (G * dt) / 4.0;
   } else {
-    const double W = S[MM_S_MASS_PRESS];
-    double R[9];
+    lds_f64* R = S + kScratch;
     langevin_random_force(S, sys, post, sub, R);
-    if (S[MM_S_BARO_VOLCON] != 0.0) {
+    double r = R[i >= j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i];
+    double r00 = R[0];
+    if (volcon) {
       const double dim = S[MM_S_NVEC];
-      const double tg = ((G[0] + G[4]) + G[8]) / dim;
-      const double tr = ((R[0] + R[4]) + R[8]) / dim;
-      for (int i = 0; i < 9; i += 4) {
-        G[i] -= tg;
-        R[i] -= tr;
+      const double tg = trace / dim, tr = ((R[0] + R[2]) + R[5]) / dim;
+      if (i == j) {
+        G -= tg;
+        r -= tr;
       }
+      r00 -= tr;
     }
     if (aniso) {
-      for (int i = 0; i < 9; ++i) vp[i] += ((G[i] - R[i] / W) * dt) / 4.0;
+      vp += ((G - r / W) * dt) / 4.0;
     } else {
-      const double g = (G[0] + G[4]) + G[8];
-      vp[0] += ((g - R[0] / W) * dt) / 4.0;
+      const double g = (lane_value(G, 0) + lane_value(G, 4)) + lane_value(G, 8);
+      vp += ((g - r00 / W) * dt) / 4.0;
     }
-    for (int i = 0; i < nv; ++i) vp[i] *= fric;
+    vp *= fric;
   }
-  if (has) {
-    for (int i = 0; i < nv; ++i) vp[i] *= fchain;
-  }
+  if (has) vp *= fchain;
+  *slot = vp;
 }
 
-// First half of the barostat call: v_g update, then positions and domain scaled by
-// exp(v_g dt / 2) (npt.py:683-702, 434-452). The position transform is left in XMAT.
-__device__ __forceinline__ void baro_part1(double* S, int sys, int post) {
+// First half of a barostat call: v_g update, then its two transforms. The positions and the domain
+// are scaled by exp(v_g dt / 2) (npt.py:683-702, 434-452); the position transform is left in XMAT.
+// The velocities are taken through exp(-(v_g + tr(v_g)/ndof) dt / 2) (npt.py:709-726; without
+// the trace term under a volume constraint, and exp(-(1 + 3/ndof) v_g dt / 2) in the isotropic
+// form, npt.py:466-484), which does not depend on the call's force: it stays pending after any
+// pending velocity factor and matrix (in the second matrix slot when the previous call's matrix
+// still waits). The lower half of the wave forms the first transform, the upper half the second.
+__device__ __forceinline__ void baro_transforms(lds_f64* S, int sys, int post) {
 #pragma clang fp contract(off)
   update_baro_vel(S, sys, post, 0);
+  const bool upper = lane_id() >= 32;
+  const double dt = S[MM_S_TIMESTEP];
+  const bool second = S[MM_S_VMAT_ON] != 0.0;
+  lds_f64* out = S + (upper ? (second ? MM_S_VMAT2 : MM_S_VMAT) : MM_S_XMAT);
   double R[9];
   if (baro_aniso(S)) {
-    expm_sym_half(S + MM_S_VEL_PRESS, 1.0, S[MM_S_TIMESTEP], R);
+    double A[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) A[k] = S[MM_S_VEL_PRESS + k];
+    if (S[MM_S_BARO_VOLCON] == 0.0) {
+      const double sh = ((A[0] + A[4]) + A[8]) / S[MM_S_NDOF];
+      if (upper) {
+        A[0] += sh;
+        A[4] += sh;
+        A[8] += sh;
+      }
+    }
+    expm_sym_half(A, upper ? -1.0 : 1.0, dt, R);
   } else {
-    const double c = exp((S[MM_S_VEL_PRESS] * S[MM_S_TIMESTEP]) / 2.0);
-    for (int i = 0; i < 9; ++i) R[i] = (i % 4 == 0) ? c : 0.0;
+    const double v0 = S[MM_S_VEL_PRESS];
+    const double x = upper ? -((1.0 + 3.0 / S[MM_S_NDOF]) * v0) : v0;
+    const double c = exp_near0((x * dt) / 2.0);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) R[k] = (k % 4 == 0) ? c : 0.0;
   }
-  for (int i = 0; i < 9; ++i) S[MM_S_XMAT + i] = R[i];
-  matmul3(S + MM_S_RVECS, R, S + MM_S_RVECS);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) out[k] = R[k];
+  S[second ? MM_S_VMAT2_ON : MM_S_VMAT_ON] = 1.0;
+  const int q = entry_of(lane_id()), i = q / 3, j = q - 3 * i;
+  const lds_f64* rv = S + MM_S_RVECS;
+  const lds_f64* X = S + MM_S_XMAT;
+  const double r =
+      (rv[3 * i + 0] * X[0 + j] + rv[3 * i + 1] * X[3 + j]) + rv[3 * i + 2] * X[6 + j];
+  S[MM_S_RVECS + q] = r;
   S[MM_S_VOLUME] = volume3(S + MM_S_RVECS);
 }
 
-// Velocity transform of the barostat call: exp(-(v_g + tr(v_g)/ndof) dt / 2) (npt.py:709-726;
-// without the trace term under a volume constraint, and exp(-(1 + 3/ndof) v_g dt / 2) in the
-// isotropic form, npt.py:466-484), pending after any pending velocity factor and matrix (into
-// the second matrix slot when the previous call's matrix still waits).
-__device__ __forceinline__ void baro_part2(double* S) {
-#pragma clang fp contract(off)
-  const double* vp = S + MM_S_VEL_PRESS;
-  const bool second = S[MM_S_VMAT_ON] != 0.0;
-  double* dst = S + (second ? MM_S_VMAT2 : MM_S_VMAT);
-  if (baro_aniso(S)) {
-    double A[9];
-    for (int i = 0; i < 9; ++i) A[i] = vp[i];
-    if (S[MM_S_BARO_VOLCON] == 0.0) {
-      const double tr = (vp[0] + vp[4]) + vp[8];
-      const double sh = tr / S[MM_S_NDOF];
-      A[0] += sh;
-      A[4] += sh;
-      A[8] += sh;
-    }
-    expm_sym_half(A, -1.0, S[MM_S_TIMESTEP], dst);
-  } else {
-    const double f = exp(((-((1.0 + 3.0 / S[MM_S_NDOF]) * vp[0])) * S[MM_S_TIMESTEP]) / 2.0);
-    for (int i = 0; i < 9; ++i) dst[i] = (i % 4 == 0) ? f : 0.0;
-  }
-  S[second ? MM_S_VMAT2_ON : MM_S_VMAT_ON] = 1.0;
-}
-
 // LangevinBarostat.pre/post bookkeeping (npt.py:374-392): energies at the start of the call.
-__device__ void baro_call_begin(double* S) {
+__device__ void baro_call_begin(lds_f64* S) {
   if (baro_langevin(S)) {
     S[MM_S_BARO_EPOT0] = S[MM_S_EPOT];
     S[MM_S_BARO_EKIN0] = S[MM_S_EKIN];
@@ -758,7 +825,7 @@ __device__ void baro_call_begin(double* S) {
 }
 
 // ... and the econs correction at its end: += epot0 - epot1 + ekin0 - ekin1.
-__device__ void baro_call_end(double* S) {
+__device__ void baro_call_end(lds_f64* S) {
 #pragma clang fp contract(off)
   if (baro_langevin(S))
     S[MM_S_ECONS_BARO] += ((S[MM_S_BARO_EPOT0] - S[MM_S_EPOT]) + S[MM_S_BARO_EKIN0]) - S[MM_S_EKIN];
@@ -766,29 +833,29 @@ __device__ void baro_call_end(double* S) {
 
 // LangevinThermostat.pre/post bookkeeping (nvt.py:197-209) for the two updates of a step made
 // in the node passes: econs += ekin0 - ekin1 for each.
-__device__ void langevin_thermo_econs(double* S, double ekin_before_pre, const double (&nd)[kNodeSums]) {
+__device__ void langevin_thermo_econs(lds_f64* S, double ekin_before_pre, const lds_f64* nd) {
 #pragma clang fp contract(off)
   S[MM_S_ECONS_THERMO] += ekin_before_pre - nd[14];
   S[MM_S_ECONS_THERMO] += nd[13] - S[MM_S_EKIN];
 }
 
-__device__ void clear_vtransforms(double* S) {
+__device__ void clear_vtransforms(lds_f64* S) {
   S[MM_S_VSCALE_A_ON] = 0.0;
   S[MM_S_VMAT_ON] = 0.0;
   S[MM_S_VSCALE_B_ON] = 0.0;
   // the second matrix slot is used only by steps in a row; clearing its entries as well keeps
   // the scalar block the same as after steps taken one per call
   S[MM_S_VMAT2_ON] = 0.0;
-  for (int i = 0; i < 9; ++i) S[MM_S_VMAT2 + i] = 0.0;
+  S[MM_S_VMAT2 + entry_of(lane_id())] = 0.0;
 }
 
-__device__ void set_vscale(double* S, int slot, double f) {
+__device__ void set_vscale(lds_f64* S, int slot, double f) {
   S[slot] = f;
   S[slot + 1] = 1.0;
 }
 
 // Hook econs corrections as summed by compute_properties (verlet.py:176-181, npt.py:135-148).
-__device__ double econs_correction(const double* S) {
+__device__ double econs_correction(const lds_f64* S) {
 #pragma clang fp contract(off)
   const bool th = S[MM_S_THERMO] != 0.0, ba = S[MM_S_BARO] != 0.0;
   if (th && ba) {
@@ -803,64 +870,80 @@ __device__ double econs_correction(const double* S) {
   return 0.0;
 }
 
-// VerletIntegrator.compute_properties (verlet.py:171-190) minus the rmsd terms.
-__device__ void properties(double* S, bool advance) {
+// VerletIntegrator.compute_properties (verlet.py:171-190) minus the rmsd terms. The divisions are
+// made together: lanes 0..8 the pressure tensor's, lanes 9..12 those of the temperature and of
+// the running means, then two lanes the pressure's and the error ratio's.
+__device__ __forceinline__ void properties(lds_f64* S, bool advance) {
 #pragma clang fp contract(off)
   if (advance) {
     S[MM_S_TIME] += S[MM_S_TIMESTEP];
     S[MM_S_COUNTER] += 1.0;
   }
+  const int lane = lane_id(), e = entry_of(lane);
   const double ekin = S[MM_S_EKIN];
-  S[MM_S_TEMP] = (ekin / S[MM_S_NDOF]) * (2.0 / S[MM_S_BOLTZMANN]);
-  S[MM_S_ETOT] = ekin + S[MM_S_EPOT];
-  S[MM_S_ECONS_CORR] = econs_correction(S);
-  const double econs = S[MM_S_ETOT] + S[MM_S_ECONS_CORR];
-  S[MM_S_ECONS] = econs;
-  double* ce = S + MM_S_CE;  // ConsErrTracker (verlet.py:275-307)
-  if (ce[0] == 0.0) {
-    ce[1] = ekin;
-    ce[3] = econs;
+  const double etot = ekin + S[MM_S_EPOT];
+  const double corr = econs_correction(S);
+  const double econs = etot + corr;
+  lds_f64* ce = S + MM_S_CE;  // ConsErrTracker (verlet.py:275-307)
+  const double count = ce[0];
+  double ekin_m = ce[1], ekin_s = ce[2], econs_m = ce[3], econs_s = ce[4];
+  const double t1 = ekin - ekin_m, t2 = econs - econs_m;
+  double num = S[MM_S_SVV + e] - S[MM_S_VTENS + e], den = S[MM_S_VOLUME];
+  if (lane == 9) num = ekin, den = S[MM_S_NDOF];
+  if (lane == 10) num = 2.0, den = S[MM_S_BOLTZMANN];
+  if (lane == 11) num = t1, den = count + 1.0;
+  if (lane == 12) num = t2, den = count + 1.0;
+  const double r = num / den;
+  if (count == 0.0) {
+    ekin_m = ekin;
+    econs_m = econs;
   } else {
-    const double t1 = ekin - ce[1];
-    ce[1] += t1 / (ce[0] + 1.0);
-    ce[2] += t1 * (ekin - ce[1]);
-    const double t2 = econs - ce[3];
-    ce[3] += t2 / (ce[0] + 1.0);
-    ce[4] += t2 * (econs - ce[3]);
+    ekin_m += lane_value(r, 11);
+    ekin_s += t1 * (ekin - ekin_m);
+    econs_m += lane_value(r, 12);
+    econs_s += t2 * (econs - econs_m);
   }
-  ce[0] += 1.0;
-  S[MM_S_CONS_ERR] = ce[0] > 1.0 ? sqrt(ce[4] / ce[2]) : 0.0;
+  const double trace = (lane_value(r, 0) + lane_value(r, 4)) + lane_value(r, 8);
+  const double r2 = lane == 0 ? trace / 3.0 : econs_s / ekin_s;
+  S[MM_S_TEMP] = lane_value(r, 9) * lane_value(r, 10);
+  S[MM_S_ETOT] = etot;
+  S[MM_S_ECONS_CORR] = corr;
+  S[MM_S_ECONS] = econs;
+  ce[0] = count + 1.0;
+  ce[1] = ekin_m;
+  ce[2] = ekin_s;
+  ce[3] = econs_m;
+  ce[4] = econs_s;
+  S[MM_S_CONS_ERR] = count + 1.0 > 1.0 ? sqrt(lane_value(r2, 1)) : 0.0;
   if (S[MM_S_NVEC] > 0.0) {
-    const double V = S[MM_S_VOLUME];
-    for (int i = 0; i < 9; ++i) S[MM_S_PTENS + i] = (S[MM_S_SVV + i] - S[MM_S_VTENS + i]) / V;
-    S[MM_S_PRESS] = ((S[MM_S_PTENS + 0] + S[MM_S_PTENS + 4]) + S[MM_S_PTENS + 8]) / 3.0;
+    if (lane < 9) S[MM_S_PTENS + lane] = r;
+    S[MM_S_PRESS] = lane_value(r2, 0);
   }
 }
 
-// Energy and virial from the force partials, plus the external-pressure part (P V, P V I).
-__device__ void take_force(double* S, const double (&f)[10], bool with_vtens) {
+// Energy and virial from the force sums f (in LDS), plus the external-pressure part (P V, P V I).
+__device__ __forceinline__ void take_force(lds_f64* S, const lds_f64* f, bool with_vtens) {
 #pragma clang fp contract(off)
-  S[MM_S_EPOT_MECH] = f[0];
+  const int q = entry_of(lane_id());
+  const double e = f[0];
+  S[MM_S_EPOT_MECH] = e;
   const double P = S[MM_S_EXT_PRESS];
   const double pv = P * S[MM_S_VOLUME];
-  S[MM_S_EPOT] = P != 0.0 ? f[0] + S[MM_S_VOLUME] * P : f[0];
+  S[MM_S_EPOT] = P != 0.0 ? e + S[MM_S_VOLUME] * P : e;
+  bool bad = e != e;
   if (with_vtens) {
-    for (int q = 0; q < 9; ++q) {
-      S[MM_S_VTENS + q] = f[1 + q];
-      if (f[1 + q] != f[1 + q]) S[MM_S_NAN] = 1.0;
-    }
-    if (P != 0.0) {
-      S[MM_S_VTENS + 0] += pv;
-      S[MM_S_VTENS + 4] += pv;
-      S[MM_S_VTENS + 8] += pv;
-    }
+    double v = f[1 + q];
+    bad = bad || v != v;
+    if (P != 0.0 && q % 4 == 0) v += pv;
+    S[MM_S_VTENS + q] = v;
   }
-  if (f[0] != f[0]) S[MM_S_NAN] = 1.0;
+  if (__any(bad)) S[MM_S_NAN] = 1.0;
 }
 
-__device__ void take_nodes(double* S, const double (&nd)[kNodeSums]) {
+__device__ __forceinline__ void take_nodes(lds_f64* S, const lds_f64* nd) {
+  const int q = entry_of(lane_id());
   S[MM_S_EKIN] = nd[0];
-  for (int q = 0; q < 9; ++q) S[MM_S_SVV + q] = nd[1 + q];
+  S[MM_S_SVV + q] = nd[1 + q];
   if (nd[12] != 0.0) S[MM_S_NAN] = 1.0;
 }
 
@@ -868,21 +951,20 @@ __device__ void take_nodes(double* S, const double (&nd)[kNodeSums]) {
 // call changes every velocity to v M (row vectors, npt.py:709-726), so sum m (v M) (x) (v M) =
 // M^T (sum m v (x) v) M and the kinetic energy is half its trace. Only the NaN flag comes from
 // the node pass (the gather of the same force), when there is one.
-__device__ void take_nodes_after_vmat(double* S, const double (&nd)[kNodeSums]) {
+__device__ __forceinline__ void take_nodes_after_vmat(lds_f64* S, const lds_f64* nd) {
 #pragma clang fp contract(off)
   const bool second = S[MM_S_VMAT2_ON] != 0.0;
   if (second || S[MM_S_VMAT_ON] != 0.0) {
-    const double* M = S + (second ? MM_S_VMAT2 : MM_S_VMAT);
-    const double* V = S + MM_S_SVV;
-    double T[9], R[9];
-    for (int i = 0; i < 3; ++i)
-      for (int j = 0; j < 3; ++j)
-        T[3 * i + j] = (V[3 * i + 0] * M[0 + j] + V[3 * i + 1] * M[3 + j]) + V[3 * i + 2] * M[6 + j];
-    for (int i = 0; i < 3; ++i)
-      for (int j = 0; j < 3; ++j)
-        R[3 * i + j] = (M[0 + i] * T[0 + j] + M[3 + i] * T[3 + j]) + M[6 + i] * T[6 + j];
-    for (int q = 0; q < 9; ++q) S[MM_S_SVV + q] = R[q];
-    S[MM_S_EKIN] = 0.5 * ((R[0] + R[4]) + R[8]);
+    const int q = entry_of(lane_id()), i = q / 3, j = q - 3 * i;
+    const lds_f64* M = S + (second ? MM_S_VMAT2 : MM_S_VMAT);
+    const lds_f64* V = S + MM_S_SVV;
+    double T[3];  // column j of V M
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      T[k] = (V[3 * k + 0] * M[0 + j] + V[3 * k + 1] * M[3 + j]) + V[3 * k + 2] * M[6 + j];
+    const double r = (M[0 + i] * T[0] + M[3 + i] * T[1]) + M[6 + i] * T[2];
+    S[MM_S_SVV + q] = r;
+    S[MM_S_EKIN] = 0.5 * ((lane_value(r, 0) + lane_value(r, 4)) + lane_value(r, 8));
   }
   if (nd[12] != 0.0) S[MM_S_NAN] = 1.0;
 }
@@ -951,8 +1033,8 @@ __device__ __forceinline__ bool phase_uses_nodes(int phase) {
 // The scalar update of one phase on the scalar block S of system sys. chained: the phase closes
 // a step that another step of the same call follows (kPhBaroEndPost: its velocity transforms
 // stay pending for the next kick-drift pass).
-__device__ void run_phase(int phase, double* S, const double (&f)[10],
-                          const double (&nd)[kNodeSums], int with_vtens, int sys,
+__device__ void run_phase(int phase, lds_f64* S, const lds_f64* f,
+                          const lds_f64* nd, int with_vtens, int sys,
                           bool chained = false) {
   const bool nhc = thermo_nhc(S);
   const bool lt = S[MM_S_THERMO] == (double)MM_THERMO_LANGEVIN;
@@ -973,9 +1055,9 @@ __device__ void run_phase(int phase, double* S, const double (&f)[10],
       properties(S, true);
       break;
     case kPhNvtPre: {
-      double ekin = S[MM_S_EKIN];
-      const double fac = nhc_chain(S, &ekin, false, 0.0);
-      S[MM_S_EKIN] = ekin;
+      const ChainStep step = nhc_chain(S, S[MM_S_EKIN], false, 0.0, kThermoChain);
+      const double fac = step.factor;
+      S[MM_S_EKIN] = step.ekin;
       set_vscale(S, MM_S_VSCALE_B, fac);
       break;
     }
@@ -990,11 +1072,11 @@ __device__ void run_phase(int phase, double* S, const double (&f)[10],
         break;
       }
       take_nodes(S, nd);
-      double ekin = S[MM_S_EKIN];
-      const double fac = nhc_chain(S, &ekin, false, 0.0);
+      const ChainStep step = nhc_chain(S, S[MM_S_EKIN], false, 0.0, kThermoChain);
+      const double fac = step.factor;
       set_vscale(S, MM_S_VSCALE_A, fac);
-      for (int q = 0; q < 9; ++q) S[MM_S_SVV + q] *= fac * fac;
-      S[MM_S_EKIN] = ekin;
+      S[MM_S_SVV + entry_of(lane_id())] *= fac * fac;
+      S[MM_S_EKIN] = step.ekin;
       S[MM_S_ECONS_THERMO] = nhc_econs(S);
       properties(S, true);
       break;
@@ -1011,10 +1093,9 @@ __device__ void run_phase(int phase, double* S, const double (&f)[10],
       // (a pending thermostat factor is already in m v (x) v: the phases that set one scale
       // the sums by its square)
       baro_call_begin(S);
-      baro_part1(S, sys, 0);
-      // the velocity transform of this call does not depend on its force; it stays pending
-      // for the kick-drift pass, which applies it before the chain's factor
-      baro_part2(S);
+      // the velocity transform stays pending for the kick-drift pass, which applies it before
+      // the chain's factor
+      baro_transforms(S, sys, 0);
       break;
     case kPhBaroEndPre: {
       // the barostat's velocity transform is still pending (see kPhBaroPre): the node sums
@@ -1028,9 +1109,9 @@ __device__ void run_phase(int phase, double* S, const double (&f)[10],
       // a Langevin thermostat's pre update follows in the kick-drift pass
       if (nhc) {
         const double g1 = g1_on ? add_press_cont(S) : 0.0;
-        double ekin = S[MM_S_EKIN];
-        const double fac = nhc_chain(S, &ekin, g1_on, g1);
-        S[MM_S_EKIN] = ekin;
+        const ChainStep step = nhc_chain(S, S[MM_S_EKIN], g1_on, g1, kThermoChain);
+        const double fac = step.factor;
+        S[MM_S_EKIN] = step.ekin;
         set_vscale(S, MM_S_VSCALE_B, fac);
       }
       break;
@@ -1039,18 +1120,18 @@ __device__ void run_phase(int phase, double* S, const double (&f)[10],
       // gather_drift has stored the positions through a pending earlier position transform; its
       // slot is cleared, entries included, as after steps taken one per call
       S[MM_S_XMAT2_ON] = 0.0;
-      for (int q = 0; q < 9; ++q) S[MM_S_XMAT2 + q] = 0.0;
+      S[MM_S_XMAT2 + entry_of(lane_id())] = 0.0;
       clear_vtransforms(S);
       take_force(S, f, true);
       const double ekin0 = S[MM_S_EKIN];
       take_nodes(S, nd);
       if (nhc) {
         const double g1 = g1_on ? add_press_cont(S) : 0.0;
-        double ekin = S[MM_S_EKIN];
-        const double fac = nhc_chain(S, &ekin, g1_on, g1);
-        S[MM_S_EKIN] = ekin;
+        const ChainStep step = nhc_chain(S, S[MM_S_EKIN], g1_on, g1, kThermoChain);
+        const double fac = step.factor;
+        S[MM_S_EKIN] = step.ekin;
         set_vscale(S, MM_S_VSCALE_A, fac);
-        for (int q = 0; q < 9; ++q) S[MM_S_SVV + q] *= fac * fac;
+        S[MM_S_SVV + entry_of(lane_id())] *= fac * fac;
         S[MM_S_ECONS_THERMO] = nhc_econs(S);
       } else if (lt) {
         langevin_thermo_econs(S, ekin0, nd);
@@ -1065,8 +1146,7 @@ __device__ void run_phase(int phase, double* S, const double (&f)[10],
         S[MM_S_CHAINVEL0] = S[MM_S_BCHAIN_VEL];
       }
       baro_call_begin(S);
-      baro_part1(S, sys, 1);
-      baro_part2(S);
+      baro_transforms(S, sys, 1);
       break;
     }
     case kPhBaroEndPost:
@@ -1079,7 +1159,8 @@ __device__ void run_phase(int phase, double* S, const double (&f)[10],
       // chained, the positions still wait for this call's transform (its force evaluation
       // applied it on the fly): it moves to the earlier slot, before the next call's
       if (chained) {
-        for (int q = 0; q < 9; ++q) S[MM_S_XMAT2 + q] = S[MM_S_XMAT + q];
+        const int q = entry_of(lane_id());
+        S[MM_S_XMAT2 + q] = S[MM_S_XMAT + q];
         S[MM_S_XMAT2_ON] = 1.0;
       }
       update_baro_vel(S, sys, 1, 1);
@@ -1108,10 +1189,9 @@ __device__ void run_phase(int phase, double* S, const double (&f)[10],
 
 // One phase, or the end of one step and the start of the next on the same copy of the block; tot
 // holds the force and node sums.
-__device__ __forceinline__ void run_phases(int phase, double* S, const double* tot,
+__device__ __forceinline__ void run_phases(int phase, lds_f64* S, const lds_f64* tot,
                                            int with_vtens, int sys) {
-  const double(&f)[10] = *reinterpret_cast<const double(*)[10]>(tot);
-  const double(&nd)[kNodeSums] = *reinterpret_cast<const double(*)[kNodeSums]>(tot + 10);
+  const lds_f64 *f = tot, *nd = tot + 10;
   const bool chained = phase == kPhBaroEndPostPre;
   const int next = chained ? kPhBaroPre : phase == kPhNvtEndPre ? kPhNvtPre : -1;
   int now = chained ? kPhBaroEndPost : phase == kPhNvtEndPre ? kPhNvtEnd : phase;
@@ -1132,7 +1212,7 @@ scalar_kernel(int phase, double* __restrict__ S0, const double* __restrict__ fpa
               const double* __restrict__ npart, int nbn, const int32_t* __restrict__ nsys_ptr,
               int with_vtens, double* __restrict__ slices, unsigned int* __restrict__ counters) {
   static_assert(MM_S_COUNT <= kScalarThreads, "one scalar-block entry per thread");
-  __shared__ double Sl[MM_S_COUNT];
+  __shared__ double Sl[MM_S_COUNT + 6];
   __shared__ double tot[kSliceQ];
   __shared__ int is_last;
   const int sys = blockIdx.y;
@@ -1179,8 +1259,8 @@ scalar_kernel(int phase, double* __restrict__ S0, const double* __restrict__ fpa
   }
   if (threadIdx.x < MM_S_COUNT) Sl[threadIdx.x] = s_own;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    run_phases(phase, Sl, tot, with_vtens, sys);
+  if (threadIdx.x < 64) {
+    run_phases(phase, (lds_f64*)Sl, (const lds_f64*)tot, with_vtens, sys);
   }
   __syncthreads();
   for (int q = threadIdx.x; q < MM_S_COUNT; q += kScalarThreads) Sg[q] = Sl[q];
