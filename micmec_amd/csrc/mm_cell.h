@@ -90,8 +90,8 @@ __device__ __forceinline__ void store_record(double* plane, uint32_t i, double v
 // (00, 11, 22, 12, 02, 01) and vertex gradient as kOut asks. tab: the table entries of the cell's
 // type, ns its states; n: its nodes (n[0] < 0: a padding slot, which gives zeros); on, xm, on2, xm2:
 // pending transforms of the positions (load_corners); acc: the lane's
-// column of an LDS array [NE + 3 NC][kCellBlock] (kMulti with a virial only).
-template <int kModel, int kOut, bool kMulti>
+// column of an LDS array [NE + 3 NC][kStride] (kMulti with a virial only).
+template <int kModel, int kOut, bool kMulti, int kStride = kCellBlock>
 __device__ __forceinline__ void cell_eval(const_f64 tab, int ns, double kt,
                                           const double* pos, const int n[8], int wrap,
                                           const double (&rv)[9], bool on, const double* xm,
@@ -146,20 +146,20 @@ __device__ __forceinline__ void cell_eval(const_f64 tab, int ns, double kt,
           if (kVir) {
             if (s == 0) {
 #pragma unroll
-              for (int e = 0; e < F::NE; ++e) acc[e * kCellBlock] = D[e];
+              for (int e = 0; e < F::NE; ++e) acc[e * kStride] = D[e];
 #pragma unroll
-              for (int q = 0; q < 3 * F::NC; ++q) acc[(F::NE + q) * kCellBlock] = O[q / 3][q % 3];
+              for (int q = 0; q < 3 * F::NC; ++q) acc[(F::NE + q) * kStride] = O[q / 3][q % 3];
             } else {
 #pragma unroll
               for (int e = 0; e < F::NE; ++e) {
                 if (e % 6 == 0) __builtin_amdgcn_sched_barrier(0);
-                acc[e * kCellBlock] = __builtin_fma(c, D[e], keep * acc[e * kCellBlock]);
+                acc[e * kStride] = __builtin_fma(c, D[e], keep * acc[e * kStride]);
               }
 #pragma unroll
               for (int q = 0; q < 3 * F::NC; ++q) {
                 // six columns in flight at a time: all of them would not fit the registers
                 if (q % 6 == 0) __builtin_amdgcn_sched_barrier(0);
-                double* t = acc + (F::NE + q) * kCellBlock;
+                double* t = acc + (F::NE + q) * kStride;
                 *t = __builtin_fma(c, O[q / 3][q % 3], keep * *t);
               }
             }
@@ -169,9 +169,9 @@ __device__ __forceinline__ void cell_eval(const_f64 tab, int ns, double kt,
         if (kVir) {
           const double inv = 1.0 / zsum;
 #pragma unroll
-          for (int e = 0; e < F::NE; ++e) D[e] = acc[e * kCellBlock] * inv;
+          for (int e = 0; e < F::NE; ++e) D[e] = acc[e * kStride] * inv;
 #pragma unroll
-          for (int q = 0; q < 3 * F::NC; ++q) O[q / 3][q % 3] = acc[(F::NE + q) * kCellBlock] * inv;
+          for (int q = 0; q < 3 * F::NC; ++q) O[q / 3][q % 3] = acc[(F::NE + q) * kStride] * inv;
         }
       }
       if (kVir) edge_gradient<kModel, kGrad>(E, D, O, vir, gacc);
@@ -179,17 +179,11 @@ __device__ __forceinline__ void cell_eval(const_f64 tab, int ns, double kt,
   }
 }
 
-// The vertex gradient of the cell in slot w as records (every lane of the wave calls this).
-template <bool kStream>
-__device__ __forceinline__ void store_cell(int64_t w, int wrap, bool valid,
-                                           const int32_t* __restrict__ cbase, int64_t W,
-                                           int64_t S, double* gcell, double (&gacc)[8][3]) {
+// The upper face (corners 3, 5, 6, 7) of the slot below is added to this slot's lower face (corners
+// 0, 1, 2, 4) when that slot holds the -z neighbour (wrap bit 3). The move from lane - 1 is a DPP
+// wave shift (lane 0, which never folds, keeps its own value). Every lane of the wave calls this.
+__device__ __forceinline__ void fold_cell(int wrap, double (&gacc)[8][3]) {
 #pragma clang fp contract(off)
-  // The upper face (corners 3, 5, 6, 7) of the slot below is added to this slot's lower face
-  // (corners 0, 1, 2, 4) when that slot holds the -z neighbour (wrap bit 3); the lower faces
-  // go to their class planes, the upper faces that were not folded (wrap bit 4 clear) to the
-  // wave's compact slots, in lane order. The move from lane - 1 is a DPP wave shift (lane 0,
-  // which never folds, keeps its own value).
   const bool fold = (wrap & 8) != 0;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -201,6 +195,16 @@ __device__ __forceinline__ void store_cell(int64_t w, int wrap, bool valid,
       gacc[kLowerCorner[q]][j] = fold ? lo + t : lo;
     }
   }
+}
+
+// The vertex gradient of the cell in slot w as records (every lane of the wave calls this).
+template <bool kStream>
+__device__ __forceinline__ void store_cell(int64_t w, int wrap, bool valid,
+                                           const int32_t* __restrict__ cbase, int64_t W,
+                                           int64_t S, double* gcell, double (&gacc)[8][3]) {
+  // the lower faces go to their class planes, the upper faces that were not folded (wrap bit 4
+  // clear) to the wave's compact slots, in lane order
+  fold_cell(wrap, gacc);
   if (valid) {
 #pragma unroll
     for (int q = 0; q < 4; ++q)
@@ -232,11 +236,15 @@ __device__ __forceinline__ void cell_wave_totals(double ecell, const double (&vi
   if ((lane & 3) == 0 && q < 7) red[q] = t;
 }
 
-// Entry q < 10 of a block's totals (energy, the full 3x3 virial) from its waves' red[4][7], in
-// wave order.
+// Where a wave's totals (cell_wave_totals) hold entry q < 10 of the energy and the full 3x3 virial:
+// {0, 1, 6, 5, 6, 2, 4, 5, 4, 3}, as nibbles (a table would be a load from memory).
+__device__ __forceinline__ int total_entry(int q) {
+  return (int)(0x3454265610ull >> (4 * q)) & 0xf;
+}
+
+// Entry q < 10 of a block's totals from its waves' red[4][7], in wave order.
 __device__ __forceinline__ double cell_block_total(const double* red, int q) {
-  constexpr int kEntry[10] = {0, 1, 6, 5, 6, 2, 4, 5, 4, 3};
-  const int e = kEntry[q];
+  const int e = total_entry(q);
   double s = red[e];
 #pragma unroll
   for (int w = 1; w < kCellBlock / 64; ++w) s += red[w * 7 + e];

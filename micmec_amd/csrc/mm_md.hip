@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "../../include/micmec_amd.h"
+#include "mm_cell.h"
 #include "mm_device.h"
 #include "mm_internal.h"
 #include "mm_kernels.h"
@@ -1266,6 +1267,289 @@ scalar_kernel(int phase, double* __restrict__ S0, const double* __restrict__ fpa
   for (int q = threadIdx.x; q < MM_S_COUNT; q += kScalarThreads) Sg[q] = Sl[q];
 }
 
+// ----------------------------------------------------------------------------- small systems
+
+// The steps of a call in one launch by one workgroup, for a system of at most kSmall work slots
+// and nodes. Such a system leaves the chip idle whatever the launches are: its step is bound by
+// the four to eight launches, the gaps between them (2.3 us each) and the trips to memory that
+// hand over the results. Thread t owns cell slot t and node t: the node's velocity, gradient and
+// mass stay in its registers, positions, vertex-gradient records, wave sums and the scalar block
+// in LDS (a slot's column holds its multistate sums, then its records: lower faces in rows 0..11,
+// upper in 12..23). Arithmetic, blocks and the order of all sums are those of the step's kernels:
+// the same bits. What is left is one wave's instruction stream a SIMD: cells 15k cycles (corner8
+// with a two-state type) or 7k (original), node passes 4k to 6k, scalar phases 2k (NVE) to 22k
+// (NPT). Per step, launches -> this kernel, corner8 / original model: 3^3 NVE 24.4 -> 10.0 /
+// 23.1 -> 5.8 us, 3^3 NVT 27.2 -> 12.0 / 23.6 -> 8.2 us, 3^3 NPT 54.6 -> 34.8 / 48.8 -> 23.6 us;
+// 7^3 (two types, at the limit) NVE 27.2 -> 10.6 / 24.7 -> 6.9 us, NPT 62.3 -> 35.7 / 53.2 -> 24.9
+// us. The limit is what LDS holds: 36 columns of 512 sums are 144 of its 160 KB.
+constexpr int kSmall = 512;
+
+struct SmallArgs {
+  const int32_t *cnode, *cwrap, *blk_row, *nstates, *nrec, *cbase;
+  const double *tab, *kt;
+  int32_t max_states;
+  int W, N;
+  double *pos, *vel, *gpos;
+  const double* masses;
+  double* S;
+  int thermo, baro, nsteps;
+};
+
+enum SmallGather { kSmallNone = 0, kSmallKick, kSmallDrift, kSmallScale };
+
+template <int kModel, bool kLT>
+__global__ void __launch_bounds__(kSmall, 2) small_kernel(SmallArgs a) {
+  using F = Frame<kModel>;
+  constexpr int NS = F::NE + 3 * F::NC;
+  constexpr int NR = NS > 24 ? NS : 24;
+  constexpr int NA = kLT ? 14 : 13;
+  constexpr int kWaves = kSmall / 64;
+  __shared__ double col[NR * kSmall];
+  __shared__ double xs[3 * kSmall];
+  __shared__ double Sl[MM_S_COUNT + 6];
+  // sums of every wave, zero where nothing writes: energy and virial, node sums, thermostat ekin
+  __shared__ double red[24 * kWaves];
+  __shared__ double tot[kSliceQ];
+  double *cred = red, *nred = red + 7 * kWaves, *lred = red + 23 * kWaves;
+  unsigned short* top_slot = reinterpret_cast<unsigned short*>(col);  // before the first step only
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  if (t < MM_S_COUNT) Sl[t] = a.S[t];
+  if (t < 24 * kWaves) red[t] = 0.0;
+  // the slot
+  const bool has_slot = 64 * wave < a.W;  // W is a multiple of the block size
+  uint32_t nodes[4];  // its nodes, two to a word
+  const bool valid = has_slot && a.cnode[8 * t] >= 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    nodes[k] = valid ? (uint32_t)a.cnode[8 * t + 2 * k] | (uint32_t)a.cnode[8 * t + 2 * k + 1] << 16
+                     : 0u;
+  const int wrap = valid ? a.cwrap[t] : 0;
+  const int trow = has_slot ? ((const_i32)a.blk_row)[wave >> 2] : 0;
+  const int ns = ((const_i32)a.nstates)[trow];
+  const double kt = ((const_f64)a.kt)[trow];
+  const_f64 tab = (const_f64)a.tab + (int64_t)trow * a.max_states * kTabStride;
+  {
+    const bool open_top = valid && !(wrap & 16);
+    const uint64_t tops = __ballot(open_top);
+    if (open_top)
+      top_slot[((const_i32)a.cbase)[wave] + __popcll(tops & ((1ull << lane) - 1ull))] = t;
+  }
+  __syncthreads();
+  // the node: its records as places in col, two to a word, 0xffff for none
+  const bool own = t < a.N;
+  uint32_t places[4] = {};
+  double mass = 1.0, v[3] = {0.0, 0.0, 0.0}, g[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int e = own ? a.nrec[k * a.N + t] : -1;
+    const int slot = e >> 2, row = 3 * (e & 3);
+    const int place = e < 0 ? 0xffff
+                      : slot < a.W ? row * kSmall + slot
+                                   : (12 + row) * kSmall + top_slot[slot - a.W];
+    places[k / 2] |= (uint32_t)place << (16 * (k & 1));
+  }
+  if (own) {
+    mass = a.masses[t];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      v[j] = a.vel[3 * t + j];
+      g[j] = a.gpos[3 * t + j];
+      xs[3 * t + j] = a.pos[3 * t + j];
+    }
+  }
+  __syncthreads();
+
+  const bool opens = a.baro != 0 || a.thermo == MM_THERMO_NHC;
+  int step = 0, seg = opens ? -1 : 0;
+  while (step < a.nsteps) {
+    const bool last = step + 1 == a.nsteps;
+    // the parts of this segment, in order: a node pass (half kick and drift, or the position
+    // scaling), a cell pass, a scalar phase, a gather, a scalar phase
+    bool cells = true, records = true, drift0 = false, scale0 = false, on = false, on2 = false;
+    int gather = kSmallKick, phase0 = -1, phase1 = -1;
+    if (seg < 0) {
+      cells = false;
+      gather = kSmallNone;
+      phase0 = a.baro ? kPhBaroPre : kPhNvtPre;
+    } else if (!a.baro) {
+      drift0 = true;
+      phase1 = a.thermo == MM_THERMO_NONE ? kPhNveEnd
+               : a.thermo == MM_THERMO_NHC && !last ? kPhNvtEndPre : kPhNvtEnd;
+    } else if (seg == 0) {
+      on = true;
+      on2 = Sl[MM_S_XMAT2_ON] != 0.0;
+      phase0 = kPhBaroEndPre;
+      gather = kSmallDrift;
+    } else if (seg == 1) {
+      phase1 = kPhMainEndNpt;
+    } else if (!last) {
+      on = true;
+      records = false;
+      gather = kSmallNone;
+      phase0 = kPhBaroEndPostPre;
+    } else {
+      scale0 = true;
+      gather = kSmallScale;
+      phase1 = kPhBaroEndPost;
+    }
+
+    if (drift0 || scale0) {
+      double lt[1] = {0.0};
+      if (own) {
+        double x[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) x[j] = xs[3 * t + j];
+        if (drift0)
+          kick_drift_node<kLT>(Sl, t, mass, g, v, x, lt[0]);
+        else
+          scale_position(Sl, x);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) xs[3 * t + j] = x[j];
+      }
+      if (kLT && drift0) {
+        const double s = wave_reduce_scatter<1>(lt, lane);
+        if (lane == 0) lred[wave] = s;
+      }
+      __syncthreads();
+    }
+
+    if (cells) {
+      if (has_slot) {
+        double rv[9];
+#pragma unroll
+        for (int q = 0; q < 9; ++q) rv[q] = lane_value(Sl[MM_S_RVECS + q], 0);
+        // the table and the packed words are taken anew in every step: hoisted out of the loop
+        // they would not fit the registers
+        asm volatile("" : "+s"(tab));
+        int n[8];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          asm volatile("" : "+v"(nodes[k]));
+          n[2 * k] = valid ? (int)(nodes[k] & 0xffffu) : -1;
+          n[2 * k + 1] = (int)(nodes[k] >> 16);
+        }
+        double* acc = col + t;
+        double ecell, vir[6], gacc[8][3];
+        if (ns > 1)
+          cell_eval<kModel, kOutGradient, true, kSmall>(tab, ns, kt, xs, n, wrap, rv, on,
+                                                        Sl + MM_S_XMAT, on2, Sl + MM_S_XMAT2, acc,
+                                                        ecell, vir, gacc);
+        else
+          cell_eval<kModel, kOutGradient, false, kSmall>(tab, ns, kt, xs, n, wrap, rv, on,
+                                                         Sl + MM_S_XMAT, on2, Sl + MM_S_XMAT2,
+                                                         acc, ecell, vir, gacc);
+        if (records) {
+          fold_cell(wrap, gacc);
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+              acc[(3 * q + j) * kSmall] = gacc[kLowerCorner[q]][j];
+              acc[(12 + 3 * q + j) * kSmall] = gacc[kUpperCorner[q]][j];
+            }
+        }
+        cell_wave_totals(ecell, vir, cred + 7 * wave);
+      }
+      __syncthreads();
+    }
+
+    for (int part = 0; part < 2; ++part) {
+      if (part == 1) {
+        if (gather == kSmallNone) break;
+        double acc[NA];
+#pragma unroll
+        for (int q = 0; q < NA; ++q) acc[q] = 0.0;
+        double lt = 0.0;
+        if (own) {
+#pragma unroll
+          for (int j = 0; j < 3; ++j) g[j] = 0.0;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) asm volatile("" : "+v"(places[k]));
+          double r[8][3];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            const int place = places[k / 2] >> (16 * (k & 1)) & 0xffffu;
+#pragma unroll
+            for (int j = 0; j < 3; ++j) r[k][j] = col[(place == 0xffff ? 0 : place) + j * kSmall];
+          }
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            const bool none = (places[k / 2] >> (16 * (k & 1)) & 0xffffu) == 0xffffu;
+#pragma unroll
+            for (int j = 0; j < 3; ++j) g[j] = none ? g[j] : g[j] + r[k][j];
+          }
+#pragma unroll
+          for (int j = 0; j < 3; ++j)
+            if (g[j] != g[j]) acc[12] = 1.0;
+          if (gather == kSmallKick) {
+            kick_node<kLT>(Sl, t, mass, g, v, acc, lt);
+            if (kLT) acc[NA - 1] = lt;
+          } else if (gather == kSmallDrift) {
+            double x[3];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) x[j] = xs[3 * t + j];
+            scale_position(Sl, x);
+            kick_drift_node<kLT>(Sl, t, mass, g, v, x, lt);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) xs[3 * t + j] = x[j];
+          } else {
+            apply_vtransform(Sl, v);
+          }
+        }
+        if (gather == kSmallDrift) {
+          if (kLT) {
+            const double one[1] = {lt};
+            const double s = wave_reduce_scatter<1>(one, lane);
+            if (lane == 0) lred[wave] = s;
+          }
+        } else {
+          const double s = wave_reduce_scatter<NA>(acc, lane);
+          const int q = scatter_index(lane);
+          if ((lane & 3) == 0 && q < NA)
+            nred[16 * wave + q] = gather == kSmallKick ? s : q == 12 && s != 0.0 ? 1.0 : 0.0;
+        }
+        __syncthreads();
+      }
+      const int ph = part ? phase1 : phase0;
+      if (ph < 0) continue;
+      if (wave == 0) {
+        // the blocks' sums (their waves in order), the two blocks in order
+        static_assert(kWaves == 8 && kCellBlock == 256 && kNodeBlock == 256, "two blocks of sums");
+        const bool force = lane < 10, ltq = lane == 24;
+        const int each = force ? 7 : ltq ? 1 : 16;
+        const double* w = force ? cred + total_entry(lane)
+                          : ltq ? lred : nred + (lane < 24 ? lane - 10 : 0);
+        double p[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) p[k] = w[k * each];
+        double s = 0.0 + (((p[0] + p[1]) + p[2]) + p[3]);
+        s += ((p[4] + p[5]) + p[6]) + p[7];
+        if (!(force ? phase_uses_force(ph) : phase_uses_nodes(ph))) s = 0.0;
+        if (lane < kSliceQ) tot[lane] = s;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        run_phases(ph, (lds_f64*)Sl, (const lds_f64*)tot, 1, 0);
+      }
+      __syncthreads();
+    }
+    if (seg >= 0 && (!a.baro || seg == 2)) {
+      ++step;
+      seg = 0;
+    } else {
+      ++seg;
+    }
+  }
+  if (own) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      a.pos[3 * t + j] = xs[3 * t + j];
+      a.vel[3 * t + j] = v[j];
+      a.gpos[3 * t + j] = g[j];
+    }
+  }
+  if (t < MM_S_COUNT) a.S[t] = Sl[t];
+}
+
 }  // namespace mm
 
 using namespace mm;
@@ -1534,6 +1818,33 @@ hipError_t enqueue_step(mm_md* md, hipStream_t s, bool lean = false, bool pre = 
   return hipSuccess;
 }
 
+// Whether the one-workgroup kernel steps this system.
+bool small_system(const mm_md* md) {
+  return md->nsys == 1 && md->N > 0 && md->N <= kSmall && md->field->W > 0 &&
+         md->field->W <= kSmall;
+}
+
+// nsteps steps (the last one full), at most kSmallSteps in a launch (some 20 to 80 ms: a call can be
+// any number of steps, a kernel should end within a reasonable time).
+constexpr int kSmallSteps = 2048;
+hipError_t run_small(mm_md* md, int nsteps, hipStream_t s) {
+  for (; nsteps > kSmallSteps; nsteps -= kSmallSteps) MM_TRY(run_small(md, kSmallSteps, s));
+  const mm_field* f = md->field;
+  const SmallArgs a{f->cnode, f->cwrap, f->blk_row, f->nstates, f->nrec, f->cbase, f->tab, f->kt,
+                    f->max_states, (int)f->W, (int)md->N, md->pos, md->vel, md->gpos,
+                    md->masses, md->S, md->thermo, md->baro, nsteps};
+  const dim3 block(std::max(f->W, md->N) > kSmall / 2 ? kSmall : kSmall / 2);
+  const bool lt = md->thermo == MM_THERMO_LANGEVIN;
+#define MM_SMALL(M, T) hipLaunchKernelGGL((small_kernel<M, T>), dim3(1), block, 0, s, a)
+  if (f->model == 0) {
+    if (lt) MM_SMALL(0, true); else MM_SMALL(0, false);
+  } else {
+    if (lt) MM_SMALL(1, true); else MM_SMALL(1, false);
+  }
+#undef MM_SMALL
+  return hipGetLastError();
+}
+
 int begin(mm_md* md, void* stream) {
   hipError_t e = hipEventRecord(md->ev_in, (hipStream_t)stream);
   if (e == hipSuccess) e = hipStreamWaitEvent(md->stream, md->ev_in, 0);
@@ -1691,7 +2002,9 @@ int mm_md_step(mm_md* md, int32_t nsteps, int use_graph, void* stream) {
   int rc = begin(md, stream);
   if (rc) return rc;
   hipError_t e = hipSuccess;
-  if (use_graph) {
+  if (use_graph && small_system(md)) {
+    e = run_small(md, nsteps, md->stream);
+  } else if (use_graph) {
     // the launch ranges of the cell pass follow the field's block split: a new split (new
     // state counts through mm_field_set_params) needs a new graph
     if (md->graph_split != md->field->split) drop_graph(md);
