@@ -39,7 +39,7 @@ constexpr int kNodeThreads = 64;  // one wave per block, kNodeBlock / kNodeThrea
 // node sums: [0] ekin [1..9] sum m v(x)v [10] sum g^2 [11] sum d^2 [12] nan
 // [13] ekin before the Langevin post update [14] ekin after the Langevin pre update
 constexpr int kNodePartial = 16;
-constexpr int kNodeSums = 15;
+constexpr int kNodeSums = 16;
 constexpr int kScalarThreads = 256;
 constexpr int kScalarSlices = 32;  // most blocks a scalar phase spreads its reduction over
 constexpr int kSliceQ = 10 + kNodeSums;  // force and node sums per slice
@@ -65,6 +65,11 @@ enum Phase {
   kPhApplied = 11,       // pending transforms were applied
   kPhBaroEndPostPre = 12,  // kPhBaroEndPost, then the next step's kPhBaroPre (steps in a row)
   kPhNvtEndPre = 13,       // kPhNvtEnd, then the next step's kPhNvtPre (steps in a row)
+  // kPhNvtEnd of a Langevin step in a row of steps: the thermostat's pre update is accounted for in
+  // the phase of the step whose gather made it (nd[14]), the first step's (nd[15]) in its own
+  kPhLtFirst = 14,
+  kPhLtNext = 15,
+  kPhLtLast = 16,
 };
 
 // ----------------------------------------------------------------------------- node kernels
@@ -119,11 +124,12 @@ __device__ __forceinline__ void node_vv(const double v[3], double m, double (&ac
 }
 
 // LangevinThermostat.thermo (nvt.py:211-218): v = c1 v + sqrt((1 - c1^2) T k_B / m) xi with
-// xi the standard normals of node n at hook call 2 counter + post.
-__device__ __forceinline__ void langevin_thermo(const double* S, int64_t n, int post, double m,
+// xi the standard normals of node n at hook call 2 counter + call (0: pre, 1: post, 2: the next
+// step's pre, before the counter moves).
+__device__ __forceinline__ void langevin_thermo(const double* S, int64_t n, int call, double m,
                                                 double v[3]) {
 #pragma clang fp contract(off)
-  const uint64_t ctr[4] = {(uint64_t)n, 2ull * (uint64_t)S[MM_S_COUNTER] + (uint64_t)post, 0ull,
+  const uint64_t ctr[4] = {(uint64_t)n, 2ull * (uint64_t)S[MM_S_COUNTER] + (uint64_t)call, 0ull,
                            0ull};
   double z[4];
   normals4(ctr, seed_from(S + MM_S_LT_SEED), kStreamThermostat, z);
@@ -184,18 +190,16 @@ __device__ __forceinline__ void apply_vtransform(const double* __restrict__ S, d
 // What a step does to one node, on values that the caller has loaded; S is the system's scalar
 // block (in HBM or LDS).
 
-// First half kick and drift (verlet.py:141-146): the pending velocity transforms, with kLT the
-// Langevin thermostat's pre update (its kinetic energy after it added to lt), then
-// v += a dt / 2 and x += dt v.
+// First half kick and drift (verlet.py:141-146): with kLT the Langevin thermostat's pre update (its
+// kinetic energy after it added to lt), then v += a dt / 2 and x += dt v.
 template <bool kLT>
-__device__ __forceinline__ void kick_drift_node(const double* S, int64_t n, double mass,
-                                                const double g[3], double v[3], double x[3],
-                                                double& lt) {
+__device__ __forceinline__ void half_step_node(const double* S, int64_t n, int call, double mass,
+                                               const double g[3], double v[3], double x[3],
+                                               double& lt) {
 #pragma clang fp contract(off)
   const double dt = S[MM_S_TIMESTEP];
-  apply_vtransform(S, v);
   if (kLT) {
-    langevin_thermo(S, n, 0, mass, v);
+    langevin_thermo(S, n, call, mass, v);
     lt += node_ekin(v, mass);
   }
 #pragma unroll
@@ -204,6 +208,15 @@ __device__ __forceinline__ void kick_drift_node(const double* S, int64_t n, doub
     v[j] = v[j] + (0.5 * a) * dt;
     x[j] = x[j] + dt * v[j];
   }
+}
+
+// The same after the pending velocity transforms.
+template <bool kLT>
+__device__ __forceinline__ void kick_drift_node(const double* S, int64_t n, double mass,
+                                                const double g[3], double v[3], double x[3],
+                                                double& lt) {
+  apply_vtransform(S, v);
+  half_step_node<kLT>(S, n, 0, mass, g, v, x, lt);
 }
 
 // The pending position transforms: an earlier call's when it still waits (the previous post
@@ -269,7 +282,7 @@ kick_drift_kernel(double* __restrict__ x, double* __restrict__ v, const double* 
       x[3 * n + j] = xx[j];
     }
   }
-  if (kLT) block_sum_store_wide<1>(lt, partials + (int64_t)14 * gridDim.x, blockIdx.x);
+  if (kLT) block_sum_store_wide<1>(lt, partials + (int64_t)15 * gridDim.x, blockIdx.x);
 }
 
 template <int kMode>
@@ -334,10 +347,16 @@ node_kernel(double* __restrict__ x, double* __restrict__ v, const double* __rest
 // records: the force evaluation fed only the energy and the virial.
 // With kDrift instead, the first half kick and the drift of the step (verlet.py:141-146) with
 // the barostat's pre-call gradient, which nothing else reads: the pending velocity transforms
-// (and the Langevin thermostat's pre update, its ekin after the update in partial row 14),
+// (and the Langevin thermostat's pre update, its ekin after the update in partial row 15),
 // then v += a dt / 2 and x += dt v, as the node pass kKickDrift does from a stored gpos, with
 // x first taken through the barostat call's pending position scaling (the previous post
 // call's when it still waits, then the pre call's), which its cell pass applied on the fly.
+// With kKick and kDrift, the second half kick of a step and the first half kick and drift of the next
+// (with kLT the thermostat's pre update too, its ekin in partial row 14), for a step in a row of
+// steps whose scalar phase moves neither: the node sums are those in between. The kick-drift pass
+// with its launch and its trip to memory for x, v and g falls away: NVE / Langevin step 28.5 / 30.8
+// -> 23.5 / 27.5 us at 10^3 cells, 42.8 / 48.3 -> 35.8 / 41.2 us at 48^3, 274 / 306 -> 237 / 289 us
+// at 128^3.
 // One node per thread (the gathers need every wave in flight that they can get); the node
 // blocks are dealt to the XCDs in contiguous ranges (xcd_block), and the partial sums are
 // stored per logical block.
@@ -350,7 +369,7 @@ gather_kick_kernel(const int32_t* __restrict__ ncell, const double* __restrict__
                    int gmode, double* __restrict__ x = nullptr) {
   const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
   const double* S = S0 + (blk_sys ? (int64_t)blk_sys[blk] * MM_S_COUNT : 0);
-  constexpr int NA = kLT ? 14 : 13;
+  constexpr int NA = kLT ? (kKick && kDrift ? 15 : 14) : 13;
   double acc[NA];
 #pragma unroll
   for (int q = 0; q < NA; ++q) acc[q] = 0.0;
@@ -385,7 +404,14 @@ gather_kick_kernel(const int32_t* __restrict__ ncell, const double* __restrict__
     if (kKick) {
       double lt = 0.0;
       kick_node<kLT>(S, n, mass, g, v0, acc, lt);
-      if (kLT) acc[NA - 1] += lt;
+      if (kLT) acc[13] += lt;
+      if (kDrift) {
+        lt = 0.0;
+        half_step_node<kLT>(S, n, 2, mass, g, v0, x0, lt);
+        if (kLT) acc[NA - 1] += lt;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) x[3 * n + j] = x0[j];
+      }
 #pragma unroll
       for (int j = 0; j < 3; ++j) v[3 * n + j] = v0[j];
     }
@@ -394,7 +420,7 @@ gather_kick_kernel(const int32_t* __restrict__ ncell, const double* __restrict__
 #pragma unroll
       for (int j = 0; j < 3; ++j) v[3 * n + j] = v0[j];
     }
-    if (kDrift) {
+    if (kDrift && !kKick) {
       // the positions as the cell pass read them: the pending scaling(s) of the barostat call
       scale_position(S, x0);
       kick_drift_node<kLT>(S, n, mass, g, v0, x0, acc[0]);
@@ -406,10 +432,10 @@ gather_kick_kernel(const int32_t* __restrict__ ncell, const double* __restrict__
     }
     }
   }
-  if (kDrift) {
+  if (kDrift && !kKick) {
     if (kLT) {
       double lt[1] = {acc[0]};
-      block_sum_store_wide<1>(lt, partials + (int64_t)14 * gridDim.x, blk);
+      block_sum_store_wide<1>(lt, partials + (int64_t)15 * gridDim.x, blk);
     }
   } else if (kKick) {
     block_sum_store_wide<NA>(acc, partials, blk);
@@ -836,7 +862,7 @@ __device__ void baro_call_end(lds_f64* S) {
 // in the node passes: econs += ekin0 - ekin1 for each.
 __device__ void langevin_thermo_econs(lds_f64* S, double ekin_before_pre, const lds_f64* nd) {
 #pragma clang fp contract(off)
-  S[MM_S_ECONS_THERMO] += ekin_before_pre - nd[14];
+  S[MM_S_ECONS_THERMO] += ekin_before_pre - nd[15];
   S[MM_S_ECONS_THERMO] += nd[13] - S[MM_S_EKIN];
 }
 
@@ -1023,11 +1049,11 @@ __device__ __forceinline__ void reduce_force_nodes(const double* fpart, int nbf,
 __device__ __forceinline__ bool phase_uses_force(int phase) {
   return phase == kPhInitForce || phase == kPhNveEnd || phase == kPhNvtEnd ||
          phase == kPhBaroEndPre || phase == kPhMainEndNpt || phase == kPhBaroEndPost ||
-         phase == kPhBaroEndPostPre || phase == kPhNvtEndPre;
+         phase == kPhBaroEndPostPre || phase >= kPhNvtEndPre;
 }
 __device__ __forceinline__ bool phase_uses_nodes(int phase) {
   return phase == kPhInitProps || phase == kPhNveEnd || phase == kPhNvtEnd ||
-         phase == kPhMainEndNpt || phase == kPhBaroEndPost || phase == kPhNvtEndPre ||
+         phase == kPhMainEndNpt || phase == kPhBaroEndPost || phase >= kPhNvtEndPre ||
          phase == kPhRmsd;
 }
 
@@ -1080,6 +1106,19 @@ __device__ void run_phase(int phase, lds_f64* S, const lds_f64* f,
       S[MM_S_EKIN] = step.ekin;
       S[MM_S_ECONS_THERMO] = nhc_econs(S);
       properties(S, true);
+      break;
+    }
+    case kPhLtFirst:
+    case kPhLtNext:
+    case kPhLtLast: {
+      clear_vtransforms(S);
+      take_force(S, f, true);
+      const double ekin0 = S[MM_S_EKIN];
+      take_nodes(S, nd);
+      if (phase == kPhLtFirst) S[MM_S_ECONS_THERMO] += ekin0 - nd[15];
+      S[MM_S_ECONS_THERMO] += nd[13] - S[MM_S_EKIN];
+      properties(S, true);
+      if (phase != kPhLtLast) S[MM_S_ECONS_THERMO] += S[MM_S_EKIN] - nd[14];
       break;
     }
     case kPhBaroPre:
@@ -1515,10 +1554,10 @@ __global__ void __launch_bounds__(kSmall, 2) small_kernel(SmallArgs a) {
       if (wave == 0) {
         // the blocks' sums (their waves in order), the two blocks in order
         static_assert(kWaves == 8 && kCellBlock == 256 && kNodeBlock == 256, "two blocks of sums");
-        const bool force = lane < 10, ltq = lane == 24;
+        const bool force = lane < 10, ltq = lane == 25;
         const int each = force ? 7 : ltq ? 1 : 16;
         const double* w = force ? cred + total_entry(lane)
-                          : ltq ? lred : nred + (lane < 24 ? lane - 10 : 0);
+                          : ltq ? lred : nred + (lane < 26 ? lane - 10 : 0);
         double p[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) p[k] = w[k * each];
@@ -1574,9 +1613,9 @@ struct mm_md {
   unsigned int* counters = nullptr;  // [nsys] last-block counters (kept at zero between calls)
   hipStream_t stream = nullptr;
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
-  // One step; runs whose step opens with a scalar phase replay, for several steps in a call,
-  // that phase, then the lean step without it (which opens the next step) and then the full
-  // step without it.
+  // One step alone; a call of several replays the lean step without its opening part (the scalar
+  // phase or the kick-drift pass that the step before has done) and ends with a full step
+  // without it.
   hipGraph_t graph = nullptr, graph_lean = nullptr, graph_last = nullptr;
   hipGraphExec_t exec = nullptr, exec_lean = nullptr, exec_last = nullptr;
   int graph_split = 0;                // the field's block split the graphs were captured with
@@ -1658,7 +1697,7 @@ hipError_t kick_drift(mm_md* md, bool lt, hipStream_t s) {
 bool reduces(int phase) {
   return phase == kPhInitForce || phase == kPhNveEnd || phase == kPhNvtEnd ||
          phase == kPhMainEndNpt || phase == kPhInitProps || phase == kPhBaroEndPre ||
-         phase == kPhBaroEndPost || phase == kPhBaroEndPostPre || phase == kPhNvtEndPre ||
+         phase == kPhBaroEndPost || phase == kPhBaroEndPostPre || phase >= kPhNvtEndPre ||
          phase == kPhRmsd;
 }
 
@@ -1674,11 +1713,12 @@ hipError_t scalar(mm_md* md, int phase, int with_vtens, hipStream_t s) {
 }
 
 // force evaluation: cells, then gather (+ second half kick when kick, + the Langevin
-// thermostat's post update when lt; + the pending velocity transforms when scale_v). gmode
+// thermostat's post update when lt; with next also the next step's kick and drift; + the pending
+// velocity transforms when scale_v). gmode
 // (gather_kick_kernel): kGatherNone leaves out the records altogether, so the cell pass skips
 // them too, and without scale_v there is then no node pass at all (energy and virial only).
 hipError_t force(mm_md* md, bool kick, bool lt, hipStream_t s, bool scale_v = false,
-                 int gmode = kGatherStore, const double* xmat = nullptr) {
+                 int gmode = kGatherStore, const double* xmat = nullptr, bool next = false) {
   ForceArgs a = force_args(md);
   a.xmat = xmat;
   if (gmode == kGatherNone) {
@@ -1690,25 +1730,29 @@ hipError_t force(mm_md* md, bool kick, bool lt, hipStream_t s, bool scale_v = fa
   // with no records, no transform to apply and no kick, the evaluation has no node pass
   if (md->N > 0 && !(gmode == kGatherNone && !scale_v && !kick)) {
     const bool all = md->nbn <= kGatherAllLoadsMaxBlocks;
-#define MM_GATHER1(K, T, V, A)                                                               \
-  hipLaunchKernelGGL((gather_kick_kernel<K, T, V, false, A>), dim3(md->nbn), dim3(kNodeBlock), \
-                     0, s, a.ncell, a.gcell, md->N, a.rstride, md->gpos, md->vel, md->masses,  \
-                     md->S, md->node_blk_sys, md->npart, gmode)
-#define MM_GATHER(K, T, V)          \
-  do {                              \
-    if (all)                        \
-      MM_GATHER1(K, T, V, true);    \
-    else                            \
-      MM_GATHER1(K, T, V, false);   \
+#define MM_GATHER1(K, T, V, D, A)                                                            \
+  hipLaunchKernelGGL((gather_kick_kernel<K, T, V, D, A>), dim3(md->nbn), dim3(kNodeBlock), 0, s, \
+                     a.ncell, a.gcell, md->N, a.rstride, md->gpos, md->vel, md->masses, md->S, \
+                     md->node_blk_sys, md->npart, gmode, md->pos)
+#define MM_GATHER(K, T, V, D)          \
+  do {                                 \
+    if (all)                           \
+      MM_GATHER1(K, T, V, D, true);    \
+    else                               \
+      MM_GATHER1(K, T, V, D, false);   \
   } while (0)
-    if (kick && lt)
-      MM_GATHER(true, true, false);
+    if (kick && next && lt)
+      MM_GATHER(true, true, false, true);
+    else if (kick && next)
+      MM_GATHER(true, false, false, true);
+    else if (kick && lt)
+      MM_GATHER(true, true, false, false);
     else if (kick)
-      MM_GATHER(true, false, false);
+      MM_GATHER(true, false, false, false);
     else if (scale_v)
-      MM_GATHER(false, false, true);
+      MM_GATHER(false, false, true, false);
     else
-      MM_GATHER(false, false, false);
+      MM_GATHER(false, false, false, false);
 #undef MM_GATHER
 #undef MM_GATHER1
     e = hipGetLastError();
@@ -1772,18 +1816,14 @@ hipError_t baro_call(mm_md* md, int end_phase, hipStream_t s, bool scale_v,
   return hipSuccess;
 }
 
-// Ensembles whose step opens with a scalar phase (the barostat's or the chain's pre update).
-bool opens_with_phase(const mm_md* md) {
-  return md->baro != 0 || md->thermo == MM_THERMO_NHC;
-}
-
 // One step. lean: a step that another step of the same call follows, so that nothing reads
 // the node gradients or the scalar block in between. With a barostat, the gradient of its main
 // force evaluation is then used only by the kick in the gather, and that of the barostat's post
 // call by nothing (the next step's pre call evaluates the force again before its kick,
 // verlet.py:141-143 with npt.py:616-620), so those evaluations keep their gradients out of
 // HBM; and a lean step ends with the next step's opening phase (kPhBaroEndPostPre,
-// kPhNvtEndPre), so that step is enqueued with pre = false. Positions, velocities, energies,
+// kPhNvtEndPre) or, where no phase opens a step, with its kick and drift, so that step is enqueued
+// with pre = false. Positions, velocities, energies,
 // virials and every scalar are those of full steps, bit for bit.
 hipError_t enqueue_step(mm_md* md, hipStream_t s, bool lean = false, bool pre = true) {
   const bool lt = md->thermo == MM_THERMO_LANGEVIN;
@@ -1806,14 +1846,14 @@ hipError_t enqueue_step(mm_md* md, hipStream_t s, bool lean = false, bool pre = 
     MM_TRY(kick_drift(md, false, s));
     MM_TRY(force(md, true, false, s));
     MM_TRY(scalar(md, lean ? kPhNvtEndPre : kPhNvtEnd, 1, s));
-  } else if (lt) {
-    MM_TRY(kick_drift(md, true, s));
-    MM_TRY(force(md, true, true, s));
-    MM_TRY(scalar(md, kPhNvtEnd, 1, s));
   } else {
-    MM_TRY(kick_drift(md, false, s));
-    MM_TRY(force(md, true, false, s));
-    MM_TRY(scalar(md, kPhNveEnd, 1, s));
+    // no scalar phase stands between the second kick of a step and the first of the next: the
+    // gather of a lean step does both, and the drift
+    if (pre) MM_TRY(kick_drift(md, lt, s));
+    MM_TRY(force(md, true, lt, s, false, lean ? kGatherKeep : kGatherStore, nullptr, lean));
+    const int end = !lt ? kPhNveEnd
+                    : pre ? (lean ? kPhLtFirst : kPhNvtEnd) : (lean ? kPhLtNext : kPhLtLast);
+    MM_TRY(scalar(md, end, 1, s));
   }
   return hipSuccess;
 }
@@ -2010,22 +2050,29 @@ int mm_md_step(mm_md* md, int32_t nsteps, int use_graph, void* stream) {
     if (md->graph_split != md->field->split) drop_graph(md);
     md->graph_split = md->field->split;
     // every step but the last is followed by another before the call returns
-    const bool lean = opens_with_phase(md) && nsteps > 1;
+    const bool lean = nsteps > 1;
     if (!lean && !md->exec) e = capture_step(md, false, true, &md->graph, &md->exec);
     if (lean && !md->exec_lean) e = capture_step(md, true, false, &md->graph_lean, &md->exec_lean);
     if (lean && e == hipSuccess && !md->exec_last)
       e = capture_step(md, false, false, &md->graph_last, &md->exec_last);
     if (e != hipSuccess) return hip_error(e, "capturing the MD step");
     if (lean) {
-      e = scalar(md, md->baro ? kPhBaroPre : kPhNvtPre, 1, md->stream);
-      for (int i = 0; i + 1 < nsteps && e == hipSuccess; ++i)
+      int i = 0;
+      if (md->baro || md->thermo == MM_THERMO_NHC) {
+        e = scalar(md, md->baro ? kPhBaroPre : kPhNvtPre, 1, md->stream);
+      } else {
+        // the first step is like no other
+        e = enqueue_step(md, md->stream, true, true);
+        ++i;
+      }
+      for (; i + 1 < nsteps && e == hipSuccess; ++i)
         e = hipGraphLaunch(md->exec_lean, md->stream);
       if (e == hipSuccess) e = hipGraphLaunch(md->exec_last, md->stream);
     } else {
-      for (int i = 0; i < nsteps && e == hipSuccess; ++i) e = hipGraphLaunch(md->exec, md->stream);
+      e = hipGraphLaunch(md->exec, md->stream);
     }
   } else {
-    const bool lean = opens_with_phase(md) && nsteps > 1;
+    const bool lean = nsteps > 1;
     for (int i = 0; i < nsteps && e == hipSuccess; ++i)
       e = enqueue_step(md, md->stream, lean && i + 1 < nsteps, !lean || i == 0);
   }

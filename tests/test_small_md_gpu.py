@@ -91,3 +91,19 @@ def test_new_state_counts_between_calls(shape):
             float(units.boltzmann), _native.stream_ptr())
         assert rc == 0
     assert_same_bits(a, b, (1, 7))
+
+
+@pytest.mark.parametrize("graph", [True, False])
+@pytest.mark.parametrize("ensemble", ["nve", "langevin"])
+@pytest.mark.parametrize("shape,pbc", [((3, 4, 2), True), ((9, 10, 8), False), ((20, 20, 20), True)])
+def test_rows_of_steps_match_single_steps(shape, pbc, ensemble, graph):
+    """Steps in one call do the second kick, the next first kick and the drift in one pass; steps
+    of one call each do not: the same bits."""
+    a, b = (integrator(shape, 0.3, 0.05, pbc, ensemble, "corner8", graph) for _ in range(2))
+    for n in (2, 3, 11):
+        a.run(n)
+        for _ in range(n):
+            b.propagate()
+        for name in ("pos", "vel", "gpos", "S"):
+            assert torch.equal(getattr(a._engine, name), getattr(b._engine, name)), (n, name)
+        assert a.econs == b.econs
