@@ -88,15 +88,13 @@ __device__ __forceinline__ void store_record(double* plane, uint32_t i, double v
 
 // Energies of all states of a cell, combined by the log-sum-exp of mmff.py:386-398, with virial
 // (00, 11, 22, 12, 02, 01) and vertex gradient as kOut asks. tab: the table entries of the cell's
-// type, ns its states; n: its nodes (n[0] < 0: a padding slot, which gives zeros); on, xm, on2, xm2:
-// pending transforms of the positions (load_corners); acc: the lane's
-// column of an LDS array [NE + 3 NC][kStride] (kMulti with a virial only).
-template <int kModel, int kOut, bool kMulti, int kStride = kCellBlock>
-__device__ __forceinline__ void cell_eval(const_f64 tab, int ns, double kt,
-                                          const double* pos, const int n[8], int wrap,
-                                          const double (&rv)[9], bool on, const double* xm,
-                                          bool on2, const double* xm2, double* acc,
-                                          double& ecell, double (&vir)[6],
+// type, ns its states; valid: false for a padding slot, which gives zeros; corners(p) puts the node
+// positions of the cell's corners into p; acc: the lane's column of an LDS array
+// [NE + 3 NC][kStride] (kMulti with a virial only).
+template <int kModel, int kOut, bool kMulti, int kStride, typename Corners>
+__device__ __forceinline__ void cell_eval(const_f64 tab, int ns, double kt, bool valid,
+                                          Corners corners, int wrap, const double (&rv)[9],
+                                          double* acc, double& ecell, double (&vir)[6],
                                           double (&gacc)[8][3]) {
 #pragma clang fp contract(off)
   using F = Frame<kModel>;
@@ -108,9 +106,9 @@ __device__ __forceinline__ void cell_eval(const_f64 tab, int ns, double kt,
   for (int v = 0; v < 8; ++v)
 #pragma unroll
     for (int j = 0; j < 3; ++j) gacc[v][j] = -0.0;
-  if (n[0] >= 0) {
+  if (valid) {
     double p[8][3], f[3];
-    load_corners(pos, n, p, on, xm, on2, xm2);
+    corners(p);
 #pragma unroll
     for (int d = 0; d < 3; ++d) f[d] = (double)((wrap >> d) & 1);
     if constexpr (kModel == 0 && !kMulti) {

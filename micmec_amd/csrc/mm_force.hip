@@ -92,8 +92,10 @@ __device__ __forceinline__ void cell_body(int bid, MM_CELL_PARAMS) {
   const bool valid = n[0] >= 0;
   const int wrap = valid ? cwrap[w] : 0;
   double ecell, vir[6], gacc[8][3];
-  cell_eval<kModel, kOut, kMulti>(tab, ns, kt, pos, n, wrap, rv, on, xmat + soff, on2,
-                                  xmat2 + soff, st_sh + threadIdx.x, ecell, vir, gacc);
+  cell_eval<kModel, kOut, kMulti, kCellBlock>(
+      tab, ns, kt, valid,
+      [&](double (&p)[8][3]) { load_corners(pos, n, p, on, xmat + soff, on2, xmat2 + soff); },
+      wrap, rv, st_sh + threadIdx.x, ecell, vir, gacc);
   if (kOut == kOutGradient) store_cell<true>(w, wrap, valid, cbase, W, S, gcell, gacc);
   cell_wave_totals(ecell, vir, red + 7 * (threadIdx.x >> 6));
   __syncthreads();

@@ -42,6 +42,9 @@ constexpr int kNodePartial = 16;
 constexpr int kNodeSums = 16;
 constexpr int kScalarThreads = 256;
 constexpr int kScalarSlices = 32;  // most blocks a scalar phase spreads its reduction over
+// Systems of at most this many cell and node blocks run the phases of a row of steps inside the
+// kernels after them (and sum a phase's partials in one block otherwise).
+constexpr int kMergeMaxBlocks = 512;
 constexpr int kSliceQ = 10 + kNodeSums;  // force and node sums per slice
 
 enum NodeMode {
@@ -253,38 +256,6 @@ __device__ __forceinline__ void kick_node(const double* S, int64_t n, double mas
   node_vv(v, mass, acc);
 }
 
-// Half kick and drift from a stored gradient, one node a thread: latency bounds it on a small
-// system, above all with the Langevin noise (some 300 dependent instructions a node), so the
-// nodes are spread over as many waves as there are. 40x36x47 Langevin step 52 -> 46 us against
-// four nodes a lane; without noise and on large systems the two are equal (128^3 and the batch of
-// 192 replicas within 0.5%).
-template <bool kLT>
-__global__ void __launch_bounds__(kNodeBlock)
-kick_drift_kernel(double* __restrict__ x, double* __restrict__ v, const double* __restrict__ g,
-                  const double* __restrict__ m, const double* __restrict__ S0,
-                  const int32_t* __restrict__ blk_sys, int64_t N, double* __restrict__ partials) {
-  const double* S = S0 + (blk_sys ? (int64_t)blk_sys[blockIdx.x] * MM_S_COUNT : 0);
-  const int64_t n = (int64_t)blockIdx.x * kNodeBlock + threadIdx.x;
-  double lt[1] = {0.0};
-  if (n < N) {
-    const double mass = m[n];
-    double vv[3], gg[3], xx[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      vv[j] = v[3 * n + j];
-      gg[j] = g[3 * n + j];
-      xx[j] = x[3 * n + j];
-    }
-    kick_drift_node<kLT>(S, n, mass, gg, vv, xx, lt[0]);
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      v[3 * n + j] = vv[j];
-      x[3 * n + j] = xx[j];
-    }
-  }
-  if (kLT) block_sum_store_wide<1>(lt, partials + (int64_t)15 * gridDim.x, blockIdx.x);
-}
-
 template <int kMode>
 __global__ void __launch_bounds__(kNodeThreads)
 node_kernel(double* __restrict__ x, double* __restrict__ v, const double* __restrict__ g,
@@ -331,125 +302,6 @@ node_kernel(double* __restrict__ x, double* __restrict__ v, const double* __rest
   }
   if (kMode == kVV || kMode == kRmsd) {
     block_sum_store<13>(acc, partials);
-  }
-}
-
-// gpos[n] = sum of the node's face-class records (mmff.py:303-318; the cell pass has already
-// added the faces shared along z), fused with the second half kick
-// v += a dt / 2 (verlet.py:152-153) and the node sums of the new velocities; with kLT also
-// the Langevin thermostat's post update (the node sums then hold the ekin before it in [13]).
-// With kScaleV instead (a barostat call, npt.py:704-735), the pending velocity transforms are
-// applied (the barostat's exp(-(v_g + tr(v_g)/ndof) dt / 2), known before its force) in the
-// same pass; the phase after it takes the kinetic sums from those before the matrix, so this
-// pass leaves only the NaN flag of the gradient.
-// gmode: kGatherStore sums the records and stores gpos; kGatherKeep sums them for the kick only
-// (the step overwrites gpos before anything reads it); kGatherNone (kScaleV only) reads no
-// records: the force evaluation fed only the energy and the virial.
-// With kDrift instead, the first half kick and the drift of the step (verlet.py:141-146) with
-// the barostat's pre-call gradient, which nothing else reads: the pending velocity transforms
-// (and the Langevin thermostat's pre update, its ekin after the update in partial row 15),
-// then v += a dt / 2 and x += dt v, as the node pass kKickDrift does from a stored gpos, with
-// x first taken through the barostat call's pending position scaling (the previous post
-// call's when it still waits, then the pre call's), which its cell pass applied on the fly.
-// With kKick and kDrift, the second half kick of a step and the first half kick and drift of the next
-// (with kLT the thermostat's pre update too, its ekin in partial row 14), for a step in a row of
-// steps whose scalar phase moves neither: the node sums are those in between. The kick-drift pass
-// with its launch and its trip to memory for x, v and g falls away: NVE / Langevin step 28.5 / 30.8
-// -> 23.5 / 27.5 us at 10^3 cells, 42.8 / 48.3 -> 35.8 / 41.2 us at 48^3, 274 / 306 -> 237 / 289 us
-// at 128^3.
-// One node per thread (the gathers need every wave in flight that they can get); the node
-// blocks are dealt to the XCDs in contiguous ranges (xcd_block), and the partial sums are
-// stored per logical block.
-template <bool kKick, bool kLT, bool kScaleV, bool kDrift, bool kAllLoads>
-__global__ void __launch_bounds__(kNodeBlock)
-gather_kick_kernel(const int32_t* __restrict__ ncell, const double* __restrict__ gcell,
-                   int64_t N, int64_t RS, double* __restrict__ gpos, double* __restrict__ v,
-                   const double* __restrict__ m, const double* __restrict__ S0,
-                   const int32_t* __restrict__ blk_sys, double* __restrict__ partials,
-                   int gmode, double* __restrict__ x = nullptr) {
-  const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
-  const double* S = S0 + (blk_sys ? (int64_t)blk_sys[blk] * MM_S_COUNT : 0);
-  constexpr int NA = kLT ? (kKick && kDrift ? 15 : 14) : 13;
-  double acc[NA];
-#pragma unroll
-  for (int q = 0; q < NA; ++q) acc[q] = 0.0;
-  {
-    const int64_t n = (int64_t)blk * kNodeBlock + threadIdx.x;
-    if (n < N) {
-    // the node's own values: with kAllLoads loaded before the records, so that they arrive
-    // with them
-    double mass = 1.0, v0[3] = {0.0, 0.0, 0.0}, x0[3] = {0.0, 0.0, 0.0};
-    auto load_node = [&]() {
-      if (kKick || kDrift) mass = m[n];
-      if (kKick || kDrift || kScaleV) {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) v0[j] = v[3 * n + j];
-      }
-      if (kDrift) {
-#pragma unroll
-        for (int j = 0; j < 3; ++j) x0[j] = x[3 * n + j];
-      }
-    };
-    if (kAllLoads) load_node();
-    double g[3] = {0.0, 0.0, 0.0};
-    if (gmode != kGatherNone) {
-      sum_node_records<kAllLoads>(ncell, gcell, N, RS, 2, n, g);
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        if (gmode == kGatherStore) gpos[3 * n + j] = g[j];
-        if (g[j] != g[j]) acc[12] = 1.0;
-      }
-    }
-    if (!kAllLoads) load_node();
-    if (kKick) {
-      double lt = 0.0;
-      kick_node<kLT>(S, n, mass, g, v0, acc, lt);
-      if (kLT) acc[13] += lt;
-      if (kDrift) {
-        lt = 0.0;
-        half_step_node<kLT>(S, n, 2, mass, g, v0, x0, lt);
-        if (kLT) acc[NA - 1] += lt;
-#pragma unroll
-        for (int j = 0; j < 3; ++j) x[3 * n + j] = x0[j];
-      }
-#pragma unroll
-      for (int j = 0; j < 3; ++j) v[3 * n + j] = v0[j];
-    }
-    if (kScaleV) {
-      apply_vtransform(S, v0);
-#pragma unroll
-      for (int j = 0; j < 3; ++j) v[3 * n + j] = v0[j];
-    }
-    if (kDrift && !kKick) {
-      // the positions as the cell pass read them: the pending scaling(s) of the barostat call
-      scale_position(S, x0);
-      kick_drift_node<kLT>(S, n, mass, g, v0, x0, acc[0]);
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        v[3 * n + j] = v0[j];
-        x[3 * n + j] = x0[j];
-      }
-    }
-    }
-  }
-  if (kDrift && !kKick) {
-    if (kLT) {
-      double lt[1] = {acc[0]};
-      block_sum_store_wide<1>(lt, partials + (int64_t)15 * gridDim.x, blk);
-    }
-  } else if (kKick) {
-    block_sum_store_wide<NA>(acc, partials, blk);
-  } else {
-    // only the NaN flag: any lane's flag, per block
-    const unsigned long long bad = __ballot(acc[12] != 0.0);
-    __shared__ int any_bad;
-    if (threadIdx.x == 0) any_bad = 0;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0 && bad) any_bad = 1;
-    __syncthreads();
-    if (threadIdx.x < 13)
-      partials[(int64_t)threadIdx.x * gridDim.x + blk] =
-          (threadIdx.x == 12 && any_bad) ? 1.0 : 0.0;
   }
 }
 
@@ -996,22 +848,15 @@ __device__ __forceinline__ void take_nodes_after_vmat(lds_f64* S, const lds_f64*
   if (nd[12] != 0.0) S[MM_S_NAN] = 1.0;
 }
 
-// The force partials fpart[q * nbf + b] over the blocks b = fidx[ff + i] (or ff + i), i < fc,
-// and the node partials npart[q * nbn + nf + i], i < nc, summed in a fixed order: each thread
-// over its strided share in index order, then the wave by the reduce-scatter butterfly, then
-// the waves in order, into tot[kSliceQ] in LDS. The loads of both kinds are issued before any
-// sum. Called by a whole block of at least kScalarThreads threads, of which the first
-// kScalarThreads sum.
-__device__ __forceinline__ void reduce_force_nodes(const double* fpart, int nbf,
-                                                   const int32_t* __restrict__ fidx, int ff,
-                                                   int fc, const double* npart, int nbn, int nf,
-                                                   int nc, double* tot) {
-  constexpr int kWaves = kScalarThreads / 64;
-  constexpr int NV = kSliceQ;
-  __shared__ double red[NV * kWaves];
-  double acc[NV];
+// This thread's share of a phase's sums, of at least kScalarThreads threads (the first of them sum):
+// the force partials fpart[q * nbf + b] over the blocks b = fidx[ff + i] (or ff + i), i < fc, and
+// the node partials npart[q * nbn + nf + i], i < nc, each in index order.
+__device__ __forceinline__ void load_partials(const double* fpart, int nbf,
+                                              const int32_t* __restrict__ fidx, int ff, int fc,
+                                              const double* npart, int nbn, int nf, int nc,
+                                              double (&acc)[kSliceQ]) {
 #pragma unroll
-  for (int q = 0; q < NV; ++q) acc[q] = 0.0;
+  for (int q = 0; q < kSliceQ; ++q) acc[q] = 0.0;
   const bool on = threadIdx.x < kScalarThreads;
   for (int i = threadIdx.x; on && i < fc; i += kScalarThreads) {
     const int b = fidx ? fidx[ff + i] : ff + i;
@@ -1022,36 +867,51 @@ __device__ __forceinline__ void reduce_force_nodes(const double* fpart, int nbf,
 #pragma unroll
     for (int q = 0; q < kNodeSums; ++q) acc[10 + q] += npart[(int64_t)q * nbn + nf + i];
   }
+}
+
+// The shares summed in a fixed order (the wave by the reduce-scatter butterfly, then the waves in
+// order) into tot[kSliceQ] in LDS; red: kSliceQ * kScalarThreads / 64 doubles of LDS. kNodes: with
+// the node sums (zero otherwise).
+template <bool kNodes>
+__device__ __forceinline__ void sum_partials(const double (&acc)[kSliceQ], double* red,
+                                             double* tot) {
+  constexpr int kWaves = kScalarThreads / 64;
+  constexpr int NV = kSliceQ, NL = kNodes ? 16 : 10;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const bool on = threadIdx.x < kScalarThreads;
+  const int q = scatter_index(lane);
   {
-    double lo[16], hi[NV - 16];
+    double lo[NL];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) lo[q] = acc[q];
+    for (int k = 0; k < NL; ++k) lo[k] = acc[k];
+    const double t = wave_reduce_scatter<NL>(lo, lane);
+    if (on && (lane & 3) == 0 && q < NL) red[wave * NV + q] = t;
+  }
+  if (kNodes) {
+    double hi[NV - 16];
 #pragma unroll
-    for (int q = 16; q < NV; ++q) hi[q - 16] = acc[q];
-    const double tl = wave_reduce_scatter<16>(lo, lane);
-    const double th = wave_reduce_scatter<NV - 16>(hi, lane);
-    const int q = scatter_index(lane);
-    if (on && (lane & 3) == 0) {
-      red[wave * NV + q] = tl;
-      if (q < NV - 16) red[wave * NV + 16 + q] = th;
-    }
+    for (int k = 16; k < NV; ++k) hi[k - 16] = acc[k];
+    const double t = wave_reduce_scatter<NV - 16>(hi, lane);
+    if (on && (lane & 3) == 0 && q < NV - 16) red[wave * NV + 16 + q] = t;
   }
   __syncthreads();
   if (threadIdx.x < NV) {
-    double t = red[threadIdx.x];
-    for (int w = 1; w < kWaves; ++w) t += red[w * NV + threadIdx.x];
+    double t = 0.0;
+    if (kNodes || threadIdx.x < 10) {
+      t = red[threadIdx.x];
+      for (int w = 1; w < kWaves; ++w) t += red[w * NV + threadIdx.x];
+    }
     tot[threadIdx.x] = t;
   }
   __syncthreads();
 }
 
-__device__ __forceinline__ bool phase_uses_force(int phase) {
+__device__ __forceinline__ constexpr bool phase_uses_force(int phase) {
   return phase == kPhInitForce || phase == kPhNveEnd || phase == kPhNvtEnd ||
          phase == kPhBaroEndPre || phase == kPhMainEndNpt || phase == kPhBaroEndPost ||
          phase == kPhBaroEndPostPre || phase >= kPhNvtEndPre;
 }
-__device__ __forceinline__ bool phase_uses_nodes(int phase) {
+__device__ __forceinline__ constexpr bool phase_uses_nodes(int phase) {
   return phase == kPhInitProps || phase == kPhNveEnd || phase == kPhNvtEnd ||
          phase == kPhMainEndNpt || phase == kPhBaroEndPost || phase >= kPhNvtEndPre ||
          phase == kPhRmsd;
@@ -1272,7 +1132,10 @@ scalar_kernel(int phase, double* __restrict__ S0, const double* __restrict__ fpa
       nf = b0 + (int)((int64_t)cnt * gi / G);
       nc = b0 + (int)((int64_t)cnt * (gi + 1) / G) - nf;
     }
-    reduce_force_nodes(fpart, nbf, fsys_idx, ff, fc, npart, nbn, nf, nc, tot);
+    __shared__ double red[kSliceQ * (kScalarThreads / 64)];
+    double acc[kSliceQ];
+    load_partials(fpart, nbf, fsys_idx, ff, fc, npart, nbn, nf, nc, acc);
+    sum_partials<true>(acc, red, tot);
   }
   if (G > 1) {
     if (threadIdx.x == 0) {
@@ -1304,6 +1167,328 @@ scalar_kernel(int phase, double* __restrict__ S0, const double* __restrict__ fpa
   }
   __syncthreads();
   for (int q = threadIdx.x; q < MM_S_COUNT; q += kScalarThreads) Sg[q] = Sl[q];
+}
+
+// ----------------------------------------------------------------------------- merged phases
+//
+// On a mid-sized system a step of three to eight kernels is bound by their number: each waits for
+// the one before it to drain, starts (2.3 us from kernel to kernel) and then for its first loads.
+// In a row of steps the scalar phases are therefore no kernels of their own. The kernel after a
+// phase begins with it: every block sums the partials and runs the phase on a copy of the scalar
+// block in LDS, all alike, so that nothing has to be handed from block to block, and block 0
+// stores the result to the other of two copies in memory (the rest of the grid still reads the
+// first); the block's own loads are under way meanwhile. Where a phase gates nothing (NVE, the
+// Langevin thermostat) one extra block of the next cell pass runs it beside the others. A cell
+// pass that reads the sums of the pass before stores its own to a second buffer; a gather copies
+// back what the next kernels expect in the first (Carry). The arithmetic and the order of all sums
+// are those of the separate kernels: the same bits. Kernels of a step: NVE and Langevin 3 -> 2,
+// NVT 4 -> 3, NPT 8 -> 5. Step at 10^3 / 32^3 / 48^3 cells: NVE 23.6 / 25.8 / 36.0 -> 19.0 / 21.0 /
+// 28.1 us, Langevin 27.5 / 29.6 / 41.7 -> 22.6 / 24.6 / 33.7, NVT 31.2 / 33.6 / 45.4 -> 25.9 / 29.0
+// / 42.3, NPT 64.1 / 68.5 / 90.4 -> 54.8 / 59.1 / 79.5. (A cell pass that moved the nodes as it
+// read them, for an NVT step of two kernels, took three loads a corner value instead of one: 26.6 /
+// 31.9 / 50.6 us.) With more than kMergeMaxBlocks blocks the cells run as two launches side by
+// side and a block's share of the repeated sums grows with the system; there a phase is a kernel.
+
+// What a gather copies for the kernels after it: the scalar block and the cell passes' sums.
+struct Carry {
+  double* s = nullptr;  // destination of the scalar block (null: stays)
+  const double* f_src = nullptr;
+  double* f_dst = nullptr;
+  int f_count = 0;
+};
+__device__ __forceinline__ void carry(const Carry& c, const double* S, int blk, int blocks) {
+  if (c.s && blk == 0 && threadIdx.x < MM_S_COUNT) c.s[threadIdx.x] = S[threadIdx.x];
+  for (int i = blk * kNodeBlock + threadIdx.x; i < c.f_count; i += blocks * kNodeBlock)
+    c.f_dst[i] = c.f_src[i];
+}
+
+// The partials and the copies of the scalar block of a merged phase.
+struct PhaseArgs {
+  const double* s_in = nullptr;
+  double* s_out = nullptr;
+  const double* fpart = nullptr;
+  const double* npart = nullptr;
+  int nbf = 0, nbn = 0;
+};
+
+// Phase kPhase on Sl (LDS, MM_S_COUNT + 6 doubles; s_own is the thread's entry of the block as it
+// came from memory), from the threads' shares acc of the partials. Every thread calls this.
+template <int kPhase>
+__device__ __forceinline__ void merged_phase(double s_own, const double (&acc)[kSliceQ],
+                                             double* Sl) {
+  __shared__ double red[kSliceQ * (kScalarThreads / 64)];
+  __shared__ double tot[kSliceQ];
+  if (threadIdx.x < MM_S_COUNT) Sl[threadIdx.x] = s_own;
+  sum_partials<phase_uses_nodes(kPhase)>(acc, red, tot);
+  if (threadIdx.x < 64) run_phases(kPhase, (lds_f64*)Sl, (const lds_f64*)tot, 1, 0);
+  __syncthreads();
+}
+template <int kPhase>
+__device__ __forceinline__ void load_merged(const PhaseArgs& a, double (&acc)[kSliceQ]) {
+  load_partials(a.fpart, a.nbf, nullptr, 0, phase_uses_force(kPhase) ? a.nbf : 0, a.npart, a.nbn, 0,
+                phase_uses_nodes(kPhase) ? a.nbn : 0, acc);
+}
+
+// Half kick and drift from a stored gradient, one node a thread: latency bounds it on a small
+// system, above all with the Langevin noise (some 300 dependent instructions a node), so the
+// nodes are spread over as many waves as there are. 40x36x47 Langevin step 52 -> 46 us against
+// four nodes a lane; without noise and on large systems the two are equal (128^3 and the batch of
+// 192 replicas within 0.5%).
+// kPhase >= 0: the kernel begins with that scalar phase (merged_phase), on the loads' time.
+template <bool kLT, int kPhase = -1>
+__global__ void __launch_bounds__(kNodeBlock, kPhase >= 0 ? 2 : 1)
+kick_drift_kernel(double* __restrict__ x, double* __restrict__ v, const double* __restrict__ g,
+                  const double* __restrict__ m, const double* __restrict__ S0,
+                  const int32_t* __restrict__ blk_sys, int64_t N, double* __restrict__ partials,
+                  PhaseArgs ph) {
+  __shared__ double Sl[kPhase >= 0 ? MM_S_COUNT + 6 : 1];
+  const double* S =
+      kPhase >= 0 ? Sl : S0 + (blk_sys ? (int64_t)blk_sys[blockIdx.x] * MM_S_COUNT : 0);
+  double s_own = 0.0, share[kSliceQ];
+  if constexpr (kPhase >= 0) {
+    if (threadIdx.x < MM_S_COUNT) s_own = ph.s_in[threadIdx.x];
+    load_merged<kPhase>(ph, share);
+  }
+  const int64_t n = (int64_t)blockIdx.x * kNodeBlock + threadIdx.x;
+  double lt[1] = {0.0};
+  double mass = 1.0, vv[3], gg[3], xx[3];
+  if (n < N) {
+    mass = m[n];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      vv[j] = v[3 * n + j];
+      gg[j] = g[3 * n + j];
+      xx[j] = x[3 * n + j];
+    }
+  }
+  if constexpr (kPhase >= 0) {
+    merged_phase<kPhase>(s_own, share, Sl);
+    if (blockIdx.x == 0 && threadIdx.x < MM_S_COUNT) ph.s_out[threadIdx.x] = Sl[threadIdx.x];
+  }
+  if (n < N) {
+    kick_drift_node<kLT>(S, n, mass, gg, vv, xx, lt[0]);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      v[3 * n + j] = vv[j];
+      x[3 * n + j] = xx[j];
+    }
+  }
+  if (kLT) block_sum_store_wide<1>(lt, partials + (int64_t)15 * gridDim.x, blockIdx.x);
+}
+
+// gpos[n] = sum of the node's face-class records (mmff.py:303-318; the cell pass has already
+// added the faces shared along z), fused with the second half kick
+// v += a dt / 2 (verlet.py:152-153) and the node sums of the new velocities; with kLT also
+// the Langevin thermostat's post update (the node sums then hold the ekin before it in [13]).
+// With kScaleV instead (a barostat call, npt.py:704-735), the pending velocity transforms are
+// applied (the barostat's exp(-(v_g + tr(v_g)/ndof) dt / 2), known before its force) in the
+// same pass; the phase after it takes the kinetic sums from those before the matrix, so this
+// pass leaves only the NaN flag of the gradient.
+// gmode: kGatherStore sums the records and stores gpos; kGatherKeep sums them for the kick only
+// (the step overwrites gpos before anything reads it); kGatherNone (kScaleV only) reads no
+// records: the force evaluation fed only the energy and the virial.
+// With kDrift instead, the first half kick and the drift of the step (verlet.py:141-146) with
+// the barostat's pre-call gradient, which nothing else reads: the pending velocity transforms
+// (and the Langevin thermostat's pre update, its ekin after the update in partial row 15),
+// then v += a dt / 2 and x += dt v, as the node pass kKickDrift does from a stored gpos, with
+// x first taken through the barostat call's pending position scaling (the previous post
+// call's when it still waits, then the pre call's), which its cell pass applied on the fly.
+// With kKick and kDrift, the second half kick of a step and the first half kick and drift of the next
+// (with kLT the thermostat's pre update too, its ekin in partial row 14), for a step in a row of
+// steps whose scalar phase moves neither: the node sums are those in between. The kick-drift pass
+// with its launch and its trip to memory for x, v and g falls away: NVE / Langevin step 28.5 / 30.8
+// -> 23.5 / 27.5 us at 10^3 cells, 42.8 / 48.3 -> 35.8 / 41.2 us at 48^3, 274 / 306 -> 237 / 289 us
+// at 128^3.
+// One node per thread (the gathers need every wave in flight that they can get); the node
+// blocks are dealt to the XCDs in contiguous ranges (xcd_block), and the partial sums are
+// stored per logical block.
+// kPhase >= 0: the kernel begins with that scalar phase (merged_phase), after the loads that do not
+// depend on it.
+template <bool kKick, bool kLT, bool kScaleV, bool kDrift, bool kAllLoads, int kPhase = -1>
+__global__ void __launch_bounds__(kNodeBlock, kPhase >= 0 ? 2 : 1)
+gather_kick_kernel(const int32_t* __restrict__ ncell, const double* __restrict__ gcell,
+                   int64_t N, int64_t RS, double* __restrict__ gpos, double* __restrict__ v,
+                   const double* __restrict__ m, const double* __restrict__ S0,
+                   const int32_t* __restrict__ blk_sys, double* __restrict__ partials,
+                   int gmode, double* __restrict__ x, Carry c, PhaseArgs ph) {
+  const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
+  __shared__ double Sl[kPhase >= 0 ? MM_S_COUNT + 6 : 1];
+  const double* S = kPhase >= 0 ? Sl : S0 + (blk_sys ? (int64_t)blk_sys[blk] * MM_S_COUNT : 0);
+  double s_own = 0.0, share[kSliceQ];
+  if constexpr (kPhase >= 0) {
+    if (threadIdx.x < MM_S_COUNT) s_own = ph.s_in[threadIdx.x];
+    load_merged<kPhase>(ph, share);
+  } else {
+    carry(c, S, blk, (int)gridDim.x);
+  }
+  constexpr int NA = kLT ? (kKick && kDrift ? 15 : 14) : 13;
+  double acc[NA];
+#pragma unroll
+  for (int q = 0; q < NA; ++q) acc[q] = 0.0;
+  const int64_t n = (int64_t)blk * kNodeBlock + threadIdx.x;
+  const bool own = n < N;
+  // the node's own values: with kAllLoads loaded before the records, so that they arrive with them
+  double mass = 1.0, v0[3] = {0.0, 0.0, 0.0}, x0[3] = {0.0, 0.0, 0.0}, g[3] = {0.0, 0.0, 0.0};
+  auto load_node = [&]() {
+    if (kKick || kDrift) mass = m[n];
+    if (kKick || kDrift || kScaleV) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) v0[j] = v[3 * n + j];
+    }
+    if (kDrift) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) x0[j] = x[3 * n + j];
+    }
+  };
+  if (own) {
+    if (kAllLoads) load_node();
+    if (gmode != kGatherNone) {
+      sum_node_records<kAllLoads>(ncell, gcell, N, RS, 2, n, g);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        if (gmode == kGatherStore) gpos[3 * n + j] = g[j];
+        if (g[j] != g[j]) acc[12] = 1.0;
+      }
+    }
+    if (!kAllLoads) load_node();
+  }
+  if constexpr (kPhase >= 0) {
+    merged_phase<kPhase>(s_own, share, Sl);
+    if (blk == 0 && threadIdx.x < MM_S_COUNT) ph.s_out[threadIdx.x] = Sl[threadIdx.x];
+  }
+  if (own) {
+    if (kKick) {
+      double lt = 0.0;
+      kick_node<kLT>(S, n, mass, g, v0, acc, lt);
+      if (kLT) acc[13] += lt;
+      if (kDrift) {
+        lt = 0.0;
+        half_step_node<kLT>(S, n, 2, mass, g, v0, x0, lt);
+        if (kLT) acc[NA - 1] += lt;
+#pragma unroll
+        for (int j = 0; j < 3; ++j) x[3 * n + j] = x0[j];
+      }
+#pragma unroll
+      for (int j = 0; j < 3; ++j) v[3 * n + j] = v0[j];
+    }
+    if (kScaleV) {
+      apply_vtransform(S, v0);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) v[3 * n + j] = v0[j];
+    }
+    if (kDrift && !kKick) {
+      // the positions as the cell pass read them: the pending scaling(s) of the barostat call
+      scale_position(S, x0);
+      kick_drift_node<kLT>(S, n, mass, g, v0, x0, acc[0]);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        v[3 * n + j] = v0[j];
+        x[3 * n + j] = x0[j];
+      }
+    }
+  }
+  if (kDrift && !kKick) {
+    if (kLT) {
+      double lt[1] = {acc[0]};
+      block_sum_store_wide<1>(lt, partials + (int64_t)15 * gridDim.x, blk);
+    }
+  } else if (kKick) {
+    block_sum_store_wide<NA>(acc, partials, blk);
+  } else {
+    // only the NaN flag: any lane's flag, per block
+    const unsigned long long bad = __ballot(acc[12] != 0.0);
+    __shared__ int any_bad;
+    if (threadIdx.x == 0) any_bad = 0;
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0 && bad) any_bad = 1;
+    __syncthreads();
+    if (threadIdx.x < 13)
+      partials[(int64_t)threadIdx.x * gridDim.x + blk] =
+          (threadIdx.x == 12 && any_bad) ? 1.0 : 0.0;
+  }
+}
+
+// The cells of one system as the step's own cell passes read them.
+struct CellPass {
+  const int32_t *cnode, *cwrap, *blk_row, *nstates, *cbase;
+  const double *tab, *kt;
+  int32_t max_states;
+  int64_t W, S;
+  double* gcell;
+};
+
+// The cell pass of a row of steps, both kinds of block in one launch (as cell_kernel_both), with
+// the scalar phase before it. kPhBaroEndPostPre and kPhMainEndNpt gate the pass and open every
+// block; the positions are then taken through the pending transforms. The other phases run in
+// block 0,
+// beside the cells of the blocks behind it, and store all of the scalar block but the domain
+// vectors, which they leave alone and the others read.
+constexpr bool phase_gates(int phase) {
+  return phase == kPhBaroEndPostPre || phase == kPhMainEndNpt;
+}
+template <int kModel, int kOut, int kPhase>
+__global__ void __launch_bounds__(kCellBlock, 2)
+md_cells_kernel(CellPass c, const double* __restrict__ x, PhaseArgs ph,
+                double* __restrict__ partials) {
+  using F = Frame<kModel>;
+  constexpr int NS = F::NE + 3 * F::NC;
+  constexpr bool kGates = phase_gates(kPhase), kPost = kPhase == kPhBaroEndPostPre;
+  __shared__ double st_sh[NS * kCellBlock];
+  __shared__ double cred[7 * (kCellBlock / 64)];
+  __shared__ double Sl[MM_S_COUNT + 6];
+  const int t = threadIdx.x;
+  double s_own = 0.0, share[kSliceQ];
+  if (kGates || blockIdx.x == 0) {
+    if (t < MM_S_COUNT) s_own = ph.s_in[t];
+    load_merged<kPhase>(ph, share);
+  }
+  if (!kGates && blockIdx.x == 0) {
+    merged_phase<kPhase>(s_own, share, Sl);
+    if (t < MM_S_COUNT && (t < MM_S_RVECS || t >= MM_S_RVECS + 9)) ph.s_out[t] = Sl[t];
+    return;
+  }
+  const int extra = kGates ? 0 : 1, nblocks = (int)gridDim.x - extra;
+  const int bid = xcd_block((int)blockIdx.x - extra, nblocks);
+  const int64_t w = (int64_t)bid * kCellBlock + t;
+  int n[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) n[k] = c.cnode[w * 8 + k];
+  const bool valid = n[0] >= 0;
+  const int wrap = valid ? c.cwrap[w] : 0;
+  if constexpr (kGates) {
+    // one word of every corner's position: the lines are in the cache by the time they are needed
+    uint32_t word[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      word[k] = reinterpret_cast<const uint32_t*>(x + 3 * (int64_t)(valid ? n[k] : 0))[0];
+    merged_phase<kPhase>(s_own, share, Sl);
+    if (bid == 0 && t < MM_S_COUNT) ph.s_out[t] = Sl[t];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) asm volatile("" ::"v"(word[k]));
+  }
+  const int trow = ((const_i32)c.blk_row)[bid];
+  const int ns = ((const_i32)c.nstates)[trow];
+  const double kt = ((const_f64)c.kt)[trow];
+  const const_f64 tab = (const_f64)c.tab + (int64_t)trow * c.max_states * kTabStride;
+  double rv[9];
+#pragma unroll
+  for (int q = 0; q < 9; ++q)
+    rv[q] = kGates ? lane_value(Sl[MM_S_RVECS + q], 0) : ((const_f64)ph.s_in)[MM_S_RVECS + q];
+  auto corners = [&](double (&p)[8][3]) {
+    load_corners(x, n, p, kGates, Sl + MM_S_XMAT, kPost && Sl[MM_S_XMAT2_ON] != 0.0,
+                 Sl + MM_S_XMAT2);
+  };
+  double ecell, vir[6], gacc[8][3];
+  if (ns > 1)
+    cell_eval<kModel, kOut, true, kCellBlock>(tab, ns, kt, valid, corners, wrap, rv, st_sh + t,
+                                              ecell, vir, gacc);
+  else
+    cell_eval<kModel, kOut, false, kCellBlock>(tab, ns, kt, valid, corners, wrap, rv, st_sh + t,
+                                               ecell, vir, gacc);
+  if (kOut == kOutGradient) store_cell<true>(w, wrap, valid, c.cbase, c.W, c.S, c.gcell, gacc);
+  cell_wave_totals(ecell, vir, cred + 7 * (t >> 6));
+  __syncthreads();
+  if (t < 10) partials[(int64_t)t * nblocks + bid] = cell_block_total(cred, t);
 }
 
 // ----------------------------------------------------------------------------- small systems
@@ -1469,13 +1654,14 @@ __global__ void __launch_bounds__(kSmall, 2) small_kernel(SmallArgs a) {
         }
         double* acc = col + t;
         double ecell, vir[6], gacc[8][3];
+        auto corners = [&](double (&p)[8][3]) {
+          load_corners(xs, n, p, on, Sl + MM_S_XMAT, on2, Sl + MM_S_XMAT2);
+        };
         if (ns > 1)
-          cell_eval<kModel, kOutGradient, true, kSmall>(tab, ns, kt, xs, n, wrap, rv, on,
-                                                        Sl + MM_S_XMAT, on2, Sl + MM_S_XMAT2, acc,
+          cell_eval<kModel, kOutGradient, true, kSmall>(tab, ns, kt, valid, corners, wrap, rv, acc,
                                                         ecell, vir, gacc);
         else
-          cell_eval<kModel, kOutGradient, false, kSmall>(tab, ns, kt, xs, n, wrap, rv, on,
-                                                         Sl + MM_S_XMAT, on2, Sl + MM_S_XMAT2,
+          cell_eval<kModel, kOutGradient, false, kSmall>(tab, ns, kt, valid, corners, wrap, rv,
                                                          acc, ecell, vir, gacc);
         if (records) {
           fold_cell(wrap, gacc);
@@ -1611,6 +1797,9 @@ struct mm_md {
   int slices = 1;                    // blocks per system of a reducing scalar phase
   double* slice_buf = nullptr;       // [nsys][slices][kSliceQ]
   unsigned int* counters = nullptr;  // [nsys] last-block counters (kept at zero between calls)
+  bool merge = false;                // phases of a row of steps merged into the kernels after them
+  double* S2 = nullptr;              // [MM_S_COUNT] the scalar block's other copy (merge)
+  double* fpart2 = nullptr;          // the second cell pass's sums (merge)
   hipStream_t stream = nullptr;
   hipEvent_t ev_in = nullptr, ev_out = nullptr;
   // One step alone; a call of several replays the lean step without its opening part (the scalar
@@ -1683,13 +1872,21 @@ hipError_t node(mm_md* md, int mode, hipStream_t s) {
 }
 
 hipError_t kick_drift(mm_md* md, bool lt, hipStream_t s) {
-#define MM_KD(T)                                                                            \
-  hipLaunchKernelGGL((kick_drift_kernel<T>), dim3(md->nbn), dim3(kNodeBlock), 0, s, md->pos,  \
-                     md->vel, md->gpos, md->masses, md->S, md->node_blk_sys, md->N, md->npart)
+#define MM_KD(T, P, A)                                                                      \
+  hipLaunchKernelGGL((kick_drift_kernel<T, P>), dim3(md->nbn), dim3(kNodeBlock), 0, s, md->pos, \
+                     md->vel, md->gpos, md->masses, md->S, md->node_blk_sys, md->N, md->npart, A)
   if (lt)
-    MM_KD(true);
+    MM_KD(true, -1, PhaseArgs{});
   else
-    MM_KD(false);
+    MM_KD(false, -1, PhaseArgs{});
+  return hipGetLastError();
+}
+
+// The same, begun with the phase kPhNvtEndPre on the sums of the step before.
+hipError_t kick_drift_merged(mm_md* md, hipStream_t s) {
+  const mm_field* f = md->field;
+  const PhaseArgs ph{md->S, md->S2, f->partials, md->npart, (int)(f->W / kCellBlock), md->nbn};
+  MM_KD(false, kPhNvtEndPre, ph);
 #undef MM_KD
   return hipGetLastError();
 }
@@ -1717,6 +1914,38 @@ hipError_t scalar(mm_md* md, int phase, int with_vtens, hipStream_t s) {
 // velocity transforms when scale_v). gmode
 // (gather_kick_kernel): kGatherNone leaves out the records altogether, so the cell pass skips
 // them too, and without scale_v there is then no node pass at all (energy and virial only).
+hipError_t gather_kick(mm_md* md, bool kick, bool lt, hipStream_t s, bool scale_v, int gmode,
+                       bool next, const double* S, const Carry& c) {
+  const mm_field* f = md->field;
+  const bool all = md->nbn <= kGatherAllLoadsMaxBlocks;
+#define MM_GATHER1(K, T, V, D, A)                                                            \
+  hipLaunchKernelGGL((gather_kick_kernel<K, T, V, D, A>), dim3(md->nbn), dim3(kNodeBlock), 0, s, \
+                     f->nrec, f->gcell, md->N, f->S, md->gpos, md->vel, md->masses, S,        \
+                     md->node_blk_sys, md->npart, gmode, md->pos, c, PhaseArgs{})
+#define MM_GATHER(K, T, V, D)          \
+  do {                                 \
+    if (all)                           \
+      MM_GATHER1(K, T, V, D, true);    \
+    else                               \
+      MM_GATHER1(K, T, V, D, false);   \
+  } while (0)
+  if (kick && next && lt)
+    MM_GATHER(true, true, false, true);
+  else if (kick && next)
+    MM_GATHER(true, false, false, true);
+  else if (kick && lt)
+    MM_GATHER(true, true, false, false);
+  else if (kick)
+    MM_GATHER(true, false, false, false);
+  else if (scale_v)
+    MM_GATHER(false, false, true, false);
+  else
+    MM_GATHER(false, false, false, false);
+#undef MM_GATHER
+#undef MM_GATHER1
+  return hipGetLastError();
+}
+
 hipError_t force(mm_md* md, bool kick, bool lt, hipStream_t s, bool scale_v = false,
                  int gmode = kGatherStore, const double* xmat = nullptr, bool next = false) {
   ForceArgs a = force_args(md);
@@ -1728,35 +1957,8 @@ hipError_t force(mm_md* md, bool kick, bool lt, hipStream_t s, bool scale_v = fa
   hipError_t e = launch_cells(a, s);
   if (e != hipSuccess) return e;
   // with no records, no transform to apply and no kick, the evaluation has no node pass
-  if (md->N > 0 && !(gmode == kGatherNone && !scale_v && !kick)) {
-    const bool all = md->nbn <= kGatherAllLoadsMaxBlocks;
-#define MM_GATHER1(K, T, V, D, A)                                                            \
-  hipLaunchKernelGGL((gather_kick_kernel<K, T, V, D, A>), dim3(md->nbn), dim3(kNodeBlock), 0, s, \
-                     a.ncell, a.gcell, md->N, a.rstride, md->gpos, md->vel, md->masses, md->S, \
-                     md->node_blk_sys, md->npart, gmode, md->pos)
-#define MM_GATHER(K, T, V, D)          \
-  do {                                 \
-    if (all)                           \
-      MM_GATHER1(K, T, V, D, true);    \
-    else                               \
-      MM_GATHER1(K, T, V, D, false);   \
-  } while (0)
-    if (kick && next && lt)
-      MM_GATHER(true, true, false, true);
-    else if (kick && next)
-      MM_GATHER(true, false, false, true);
-    else if (kick && lt)
-      MM_GATHER(true, true, false, false);
-    else if (kick)
-      MM_GATHER(true, false, false, false);
-    else if (scale_v)
-      MM_GATHER(false, false, true, false);
-    else
-      MM_GATHER(false, false, false, false);
-#undef MM_GATHER
-#undef MM_GATHER1
-    e = hipGetLastError();
-  }
+  if (md->N > 0 && !(gmode == kGatherNone && !scale_v && !kick))
+    e = gather_kick(md, kick, lt, s, scale_v, gmode, next, md->S, Carry{});
   return e;
 }
 
@@ -1773,19 +1975,30 @@ hipError_t gather_drift(mm_md* md, bool lt, hipStream_t s) {
   if (md->N == 0) return hipSuccess;
   mm_field* f = md->field;
   const bool all = md->nbn <= kGatherAllLoadsMaxBlocks;
-#define MM_DRIFT(T, A)                                                                       \
-  hipLaunchKernelGGL((gather_kick_kernel<false, T, false, true, A>), dim3(md->nbn),          \
+#define MM_DRIFT(T, A, P, C)                                                                 \
+  hipLaunchKernelGGL((gather_kick_kernel<false, T, false, true, A, P>), dim3(md->nbn),       \
                      dim3(kNodeBlock), 0, s, f->nrec, f->gcell, md->N, f->S, md->gpos,       \
                      md->vel, md->masses, md->S, md->node_blk_sys, md->npart, kGatherKeep,   \
-                     md->pos)
+                     md->pos, Carry{}, C)
   if (lt && all)
-    MM_DRIFT(true, true);
+    MM_DRIFT(true, true, -1, PhaseArgs{});
   else if (lt)
-    MM_DRIFT(true, false);
+    MM_DRIFT(true, false, -1, PhaseArgs{});
   else if (all)
-    MM_DRIFT(false, true);
+    MM_DRIFT(false, true, -1, PhaseArgs{});
   else
-    MM_DRIFT(false, false);
+    MM_DRIFT(false, false, -1, PhaseArgs{});
+  return hipGetLastError();
+}
+
+// The same, begun with the phase kPhBaroEndPre on the sums of the last cell pass.
+hipError_t gather_drift_merged(mm_md* md, bool lt, hipStream_t s) {
+  mm_field* f = md->field;
+  const PhaseArgs ph{md->S, md->S2, f->partials, md->npart, (int)(f->W / kCellBlock), md->nbn};
+  if (lt)
+    MM_DRIFT(true, true, kPhBaroEndPre, ph);
+  else
+    MM_DRIFT(false, true, kPhBaroEndPre, ph);
 #undef MM_DRIFT
   return hipGetLastError();
 }
@@ -1858,6 +2071,98 @@ hipError_t enqueue_step(mm_md* md, hipStream_t s, bool lean = false, bool pre = 
   return hipSuccess;
 }
 
+// A merged cell pass: phase on the sums fin (and the node sums) from s_in to s_out, its own to fout.
+hipError_t md_cells(mm_md* md, int phase, const double* s_in, double* s_out, const double* fin,
+                    double* fout, hipStream_t s) {
+  const mm_field* f = md->field;
+  const CellPass c{f->cnode, f->cwrap, f->blk_row, f->nstates, f->cbase, f->tab, f->kt,
+                   f->max_states, f->W, f->S, f->gcell};
+  const int nb = (int)(f->W / kCellBlock);
+  const PhaseArgs ph{s_in, s_out, fin, md->npart, nb, md->nbn};
+  const dim3 grid(nb + (phase_gates(phase) ? 0 : 1)), block(kCellBlock);
+#define MM_CELLS(M, O, P)                                                                     \
+  hipLaunchKernelGGL((md_cells_kernel<M, O, P>), grid, block, 0, s, c, md->pos, ph, fout)
+#define MM_CELLS_PHASE(M)                                                   \
+  switch (phase) {                                                          \
+    case kPhNveEnd: MM_CELLS(M, kOutGradient, kPhNveEnd); break;            \
+    case kPhLtFirst: MM_CELLS(M, kOutGradient, kPhLtFirst); break;          \
+    case kPhLtNext: MM_CELLS(M, kOutGradient, kPhLtNext); break;            \
+    case kPhBaroEndPostPre: MM_CELLS(M, kOutGradient, kPhBaroEndPostPre); break; \
+    case kPhMainEndNpt: MM_CELLS(M, kOutVirial, kPhMainEndNpt); break;      \
+    default: return hipErrorInvalidValue;                                   \
+  }
+  if (f->model == 0) {
+    MM_CELLS_PHASE(0)
+  } else {
+    MM_CELLS_PHASE(1)
+  }
+#undef MM_CELLS_PHASE
+#undef MM_CELLS
+  return hipGetLastError();
+}
+
+// The barostat's main force evaluation and the cell pass of its post call, from the positions
+// and velocities of gather_drift_merged on: the scalar block is in S2.
+hipError_t row_main(mm_md* md, bool last, hipStream_t s) {
+  const bool lt = md->thermo == MM_THERMO_LANGEVIN;
+  ForceArgs a = force_args(md);
+  a.rvecs = md->S2 + MM_S_RVECS;
+  MM_TRY(launch_cells(a, s));
+  MM_TRY(gather_kick(md, true, lt, s, false, last ? kGatherStore : kGatherKeep, false, md->S2,
+                     Carry{md->S}));
+  if (last) return hipSuccess;
+  return md_cells(md, kPhMainEndNpt, md->S, md->S2, md->field->partials, md->fpart2, s);
+}
+
+// The first step of a row of merged steps, without its closing phase.
+hipError_t row_open(mm_md* md, hipStream_t s) {
+  const bool lt = md->thermo == MM_THERMO_LANGEVIN;
+  if (md->baro) {
+    MM_TRY(scalar(md, kPhBaroPre, 1, s));
+    ForceArgs a = force_args(md);
+    a.xmat = md->S + MM_S_XMAT;
+    a.xmat2 = md->S + MM_S_XMAT2;
+    a.xmat2_on = md->S + MM_S_XMAT2_ON;
+    MM_TRY(launch_cells(a, s));
+    MM_TRY(gather_drift_merged(md, lt, s));
+    return row_main(md, false, s);
+  }
+  if (md->thermo == MM_THERMO_NHC) {
+    MM_TRY(scalar(md, kPhNvtPre, 1, s));
+    MM_TRY(kick_drift(md, false, s));
+    return force(md, true, false, s);
+  }
+  MM_TRY(kick_drift(md, lt, s));
+  return force(md, true, lt, s, false, kGatherKeep, nullptr, true);
+}
+
+// A further step, from the closing phase of the one before it on; first: that one opened the row;
+// last: this one ends it (with its closing phase).
+hipError_t row_next(mm_md* md, bool first, bool last, hipStream_t s) {
+  const bool lt = md->thermo == MM_THERMO_LANGEVIN;
+  double* f0 = md->field->partials;
+  const int nf = 10 * (int)(md->field->W / kCellBlock);
+  if (md->baro) {
+    MM_TRY(md_cells(md, kPhBaroEndPostPre, md->S2, md->S, md->fpart2, f0, s));
+    MM_TRY(gather_drift_merged(md, lt, s));
+    MM_TRY(row_main(md, last, s));
+    if (!last) return hipSuccess;
+    MM_TRY(scalar(md, kPhMainEndNpt, 1, s));
+    return baro_call(md, kPhBaroEndPost, s, true);
+  }
+  if (md->thermo == MM_THERMO_NHC) {
+    MM_TRY(kick_drift_merged(md, s));
+    MM_TRY(launch_cells(force_args(md), s));
+    MM_TRY(gather_kick(md, true, false, s, false, kGatherStore, false, md->S2, Carry{md->S}));
+    return last ? scalar(md, kPhNvtEnd, 1, s) : hipSuccess;
+  }
+  MM_TRY(md_cells(md, !lt ? kPhNveEnd : first ? kPhLtFirst : kPhLtNext, md->S, md->S, f0,
+                  md->fpart2, s));
+  MM_TRY(gather_kick(md, true, lt, s, false, last ? kGatherStore : kGatherKeep, !last, md->S,
+                     Carry{nullptr, md->fpart2, f0, nf}));
+  return last ? scalar(md, lt ? kPhLtLast : kPhNveEnd, 1, s) : hipSuccess;
+}
+
 // Whether the one-workgroup kernel steps this system.
 bool small_system(const mm_md* md) {
   return md->nsys == 1 && md->N > 0 && md->N <= kSmall && md->field->W > 0 &&
@@ -1901,12 +2206,12 @@ int end(mm_md* md, void* stream) {
 
 namespace {
 
-// Capture one step into an executable graph (replayed once per step).
-hipError_t capture_step(mm_md* md, bool lean, bool pre, hipGraph_t* graph,
-                        hipGraphExec_t* exec) {
+// Capture what enqueue puts on the engine's stream into an executable graph.
+template <typename Enqueue>
+hipError_t capture(mm_md* md, hipGraph_t* graph, hipGraphExec_t* exec, Enqueue enqueue) {
   hipError_t e = hipStreamBeginCapture(md->stream, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return e;
-  const hipError_t e2 = enqueue_step(md, md->stream, lean, pre);
+  const hipError_t e2 = enqueue();
   e = hipStreamEndCapture(md->stream, graph);
   if (e2 != hipSuccess) e = e2;
   if (e == hipSuccess) e = hipGraphInstantiate(exec, *graph, nullptr, nullptr, 0);
@@ -1977,7 +2282,12 @@ int mm_md_create_batch(mm_md** out, mm_field* field, int32_t nsys, const int64_t
     most = std::max(most, cptr[s + 1] - cptr[s]);
     most = std::max(most, sys_nblk[s + 1] - sys_nblk[s]);
   }
-  md->slices = std::min(kScalarSlices, std::max(1, (most + 255) / 256));
+  md->slices = most <= kMergeMaxBlocks ? 1 : std::min(kScalarSlices, (most + 255) / 256);
+  md->merge = nsys == 1 && md->slices == 1 && field->W > 0 && field->N > 0 && !small_system(md);
+  if (e == hipSuccess && md->merge)
+    e = hipMalloc((void**)&md->S2, sizeof(double) * MM_S_COUNT);
+  if (e == hipSuccess && md->merge)
+    e = hipMalloc((void**)&md->fpart2, sizeof(double) * 10 * (field->W / kCellBlock));
   if (e == hipSuccess) e = hipMalloc((void**)&md->npart, sizeof(double) * kNodePartial * md->nbn);
   if (e == hipSuccess) e = hipMemset(md->npart, 0, sizeof(double) * kNodePartial * md->nbn);
   if (e == hipSuccess)
@@ -2050,26 +2360,41 @@ int mm_md_step(mm_md* md, int32_t nsteps, int use_graph, void* stream) {
     if (md->graph_split != md->field->split) drop_graph(md);
     md->graph_split = md->field->split;
     // every step but the last is followed by another before the call returns
-    const bool lean = nsteps > 1;
-    if (!lean && !md->exec) e = capture_step(md, false, true, &md->graph, &md->exec);
-    if (lean && !md->exec_lean) e = capture_step(md, true, false, &md->graph_lean, &md->exec_lean);
-    if (lean && e == hipSuccess && !md->exec_last)
-      e = capture_step(md, false, false, &md->graph_last, &md->exec_last);
+    hipStream_t q = md->stream;
+    const bool row = nsteps > 1;
+    if (!row && !md->exec)
+      e = capture(md, &md->graph, &md->exec, [&] { return enqueue_step(md, q); });
+    if (row && !md->exec_lean)
+      e = capture(md, &md->graph_lean, &md->exec_lean, [&] {
+        return md->merge ? row_next(md, false, false, q) : enqueue_step(md, q, true, false);
+      });
+    if (row && e == hipSuccess && !md->exec_last)
+      e = capture(md, &md->graph_last, &md->exec_last, [&] {
+        return md->merge ? row_next(md, false, true, q) : enqueue_step(md, q, false, false);
+      });
     if (e != hipSuccess) return hip_error(e, "capturing the MD step");
-    if (lean) {
+    if (row) {
+      // the first step, or its opening phase, is like no other, and with the Langevin thermostat
+      // the second merged one
       int i = 0;
-      if (md->baro || md->thermo == MM_THERMO_NHC) {
-        e = scalar(md, md->baro ? kPhBaroPre : kPhNvtPre, 1, md->stream);
+      const bool lt = md->thermo == MM_THERMO_LANGEVIN && !md->baro;
+      if (md->merge) {
+        e = row_open(md, q);
+        i = 1;
+        if (e == hipSuccess && lt) {
+          e = row_next(md, true, nsteps == 2, q);
+          i = 2;
+        }
+      } else if (md->baro || md->thermo == MM_THERMO_NHC) {
+        e = scalar(md, md->baro ? kPhBaroPre : kPhNvtPre, 1, q);
       } else {
-        // the first step is like no other
-        e = enqueue_step(md, md->stream, true, true);
-        ++i;
+        e = enqueue_step(md, q, true, true);
+        i = 1;
       }
-      for (; i + 1 < nsteps && e == hipSuccess; ++i)
-        e = hipGraphLaunch(md->exec_lean, md->stream);
-      if (e == hipSuccess) e = hipGraphLaunch(md->exec_last, md->stream);
+      for (; i + 1 < nsteps && e == hipSuccess; ++i) e = hipGraphLaunch(md->exec_lean, q);
+      if (i < nsteps && e == hipSuccess) e = hipGraphLaunch(md->exec_last, q);
     } else {
-      e = hipGraphLaunch(md->exec, md->stream);
+      e = hipGraphLaunch(md->exec, q);
     }
   } else {
     const bool lean = nsteps > 1;
@@ -2125,6 +2450,8 @@ void mm_md_destroy(mm_md* md) {
   if (md->npart) (void)hipFree(md->npart);
   if (md->slice_buf) (void)hipFree(md->slice_buf);
   if (md->counters) (void)hipFree(md->counters);
+  if (md->S2) (void)hipFree(md->S2);
+  if (md->fpart2) (void)hipFree(md->fpart2);
   if (md->node_blk_sys) (void)hipFree(md->node_blk_sys);
   if (md->sys_nblk) (void)hipFree(md->sys_nblk);
   delete md;

@@ -1,6 +1,7 @@
-"""Systems of at most 512 work slots and nodes step in one launch (use_graph, the default): the same
-bits as the step's kernels one by one (use_graph=False), which is an identity of the arithmetic, so
-there is no tolerance."""
+"""Systems of at most 512 work slots and nodes step in one launch (use_graph, the default), those
+of at most 512 blocks run a step's scalar phases inside its other kernels: the same bits as the
+step's kernels one by one (use_graph=False), which is an identity of the arithmetic, so there
+is no tolerance."""
 
 import ctypes
 
@@ -21,10 +22,10 @@ FS = units.femtosecond
 
 # shape, probability of the two-state type, of a hole, periodic: one cell; one wave; one type and
 # two types in one and two blocks with holes and open faces; the most nodes (512); one node layer
-# and one slot block more than fit, which step by graph replays
+# and one slot block more than fit one workgroup; some fifty blocks
 SYSTEMS = [((1, 1, 1), 0.0, 0.0, False), ((3, 3, 3), 0.5, 0.0, True), ((4, 3, 5), 0.3, 0.2, False),
            ((2, 3, 20), 1.0, 0.1, True), ((7, 7, 7), 0.5, 0.0, False), ((8, 8, 8), 0.0, 0.0, True),
-           ((8, 8, 9), 0.0, 0.1, True), ((9, 9, 9), 0.5, 0.0, False)]
+           ((8, 8, 9), 0.0, 0.1, True), ((9, 9, 9), 0.5, 0.0, False), ((24, 19, 27), 0.3, 0.1, True)]
 
 
 def integrator(shape, p_b, p_hole, pbc, ensemble, model, graph):
@@ -64,6 +65,16 @@ def test_one_launch_steps_have_the_bits_of_the_kernels(ensemble, model):
         a = integrator(shape, p_b, p_hole, pbc, ensemble, model, True)
         b = integrator(shape, p_b, p_hole, pbc, ensemble, model, False)
         assert_same_bits(a, b, (1, 2, 9, 20))
+
+
+@pytest.mark.parametrize("ensemble", ["nve", "nvt", "langevin", "npt"])
+@pytest.mark.parametrize("shape", [(50, 51, 50), (54, 54, 52)])
+def test_merged_phases_up_to_512_blocks(shape, ensemble):
+    """Just below and above the most blocks whose phases are merged into other kernels."""
+    print("merged", shape, ensemble, flush=True)
+    a, b = (integrator(shape, 0.3, 0.0, True, ensemble, "corner8", graph)
+            for graph in (True, False))
+    assert_same_bits(a, b, (2, 7))
 
 
 def test_long_call_is_cut_into_launches():
