@@ -20,16 +20,21 @@
 //   [30]     dE/dw, w = det(h0)/8 (eight-corner model) or det(h0) (averaged model)
 //   [31]     dE/d(free energy) = p_s, the state's Boltzmann weight
 // followed by one entry per row, dE/d(kT). The caller maps (Cv, P, w, kT) to (Cv, h0, T_eff).
+// They are bilinear in the corners' strains, so the kernel works in the metric of the edges as
+// the force kernels do (mm_device.h): with x the six Gram entries of a corner less the state's
+// rest metric and p_s the state's weight it sums p_s x_I x_J (21), p_s x_I (6) and p_s, and
+// metric_entries_kernel turns the sums of a (row, state) into its 32 entries.
 //
-// Lanes: one per (cell, corner), 8 cells per wave, 32 cells per block; lane 8c + b owns the
-// corner at offset (b & 1, b >> 1 & 1, b >> 2) of cell c. Blocks lie inside one 256-slot segment
-// of the work order, so the type row and the system are uniform per block.
+// Lanes: one per cell, one wave per block. Blocks lie inside one 256-slot segment of the work
+// order, so the type row and the system are uniform per block.
 //
 // HBM layout of the outputs:
-//   part   [2 * kSysQ][W / 32]     per block: energy, virial (9), domain-vector gradient (9);
+//   part   [2 * kSysQ][W / 64]     per block: energy, virial (9), domain-vector gradient (9);
 //                                  rows kSysQ.. hold the tangents
-//   ppart  [2 * npar][W / 32]      per block: row 2i value, 2i + 1 tangent of parameter entry i
-//   gcell, gcell2 [8][3][W]        vertex gradients and their tangents (gathered into gpos)
+//   ppart  [2 * npar][W / 64]      per block: row 2i value, 2i + 1 tangent of metric sum i of a
+//                                  state's 32 (0..20 x x, 21..26 x, 27 p), or of dE/d(kT)
+//   gcell, gcell2 [4][3][S]        vertex gradients and their tangents, as the cell pass's
+//                                  face-class records (mm_force.hip), gathered into gpos
 // All sums run in a fixed order; there are no floating-point atomics.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -37,6 +42,7 @@
 #include <vector>
 
 #include "../../include/micmec_amd.h"
+#include "mm_cell.h"
 #include "mm_device.h"
 #include "mm_internal.h"
 #include "mm_kernels.h"
@@ -79,409 +85,445 @@ template <> __device__ __forceinline__ Dual make<Dual>(double v, double d) { ret
 template <typename T> struct IsDual { static constexpr bool value = false; };
 template <> struct IsDual<Dual> { static constexpr bool value = true; };
 
-// Lane exchanges inside groups of eight lanes, as DPP moves (VALU, no LDS round trip): lane l
-// receives the value of lane l ^ mask. Masks 1 and 2 are quad permutations ([1,0,3,2] and
-// [2,3,0,1]); mask 4 swaps the two 4-lane banks of each half row, as a row shift left by 4
-// written to banks 0 and 2 and a row shift right by 4 written to banks 1 and 3 (dpp_f64: a
-// double moves as its two 32-bit halves).
-template <int kMask>
-__device__ __forceinline__ double xs8(double v) {
-  static_assert(kMask == 1 || kMask == 2 || kMask == 4, "exchanges inside 8 lanes");
-  if (kMask == 1) return dpp_f64<0xB1, 0xF>(v, v);
-  if (kMask == 2) return dpp_f64<0x4E, 0xF>(v, v);
-  const double t = dpp_f64<0x104, 0x5>(v, v);
-  return dpp_f64<0x114, 0xA>(t, v);
+// a b + c, fused in every component.
+__device__ __forceinline__ double mad(double a, double b, double c) {
+  return __builtin_fma(a, b, c);
 }
-__device__ __forceinline__ double xs(double v, int mask) {
-  return mask == 1 ? xs8<1>(v) : mask == 2 ? xs8<2>(v) : xs8<4>(v);
+__device__ __forceinline__ Dual mad(Dual a, Dual b, Dual c) {
+  return {__builtin_fma(a.v, b.v, c.v), __builtin_fma(a.v, b.d, __builtin_fma(a.d, b.v, c.d))};
 }
-__device__ __forceinline__ Dual xs(Dual v, int mask) { return {xs(v.v, mask), xs(v.d, mask)}; }
-__device__ __forceinline__ double bc(double v, int src) { return __shfl(v, src, 64); }
-__device__ __forceinline__ Dual bc(Dual v, int src) {
-  return {__shfl(v.v, src, 64), __shfl(v.d, src, 64)};
+__device__ __forceinline__ Dual mad(double a, Dual b, Dual c) {
+  return {__builtin_fma(a, b.v, c.v), __builtin_fma(a, b.d, c.d)};
 }
-// Sum over the 8 lanes of a cell (xor butterfly: every lane gets the same bits).
-template <typename T>
-__device__ __forceinline__ T sum8(T v) {
-  v = v + xs(v, 1);
-  v = v + xs(v, 2);
-  v = v + xs(v, 4);
-  return v;
-}
-
-// Sums over the 8 lanes of a cell of eight values c[0..7] at once: lane b returns the sum of
-// c[b]. Each level keeps half of the lane's values and adds the partner's copy of them, over
-// the same pairs, quads and halves as sum8, so every sum equals sum8 of that value bit for bit
-// (addition commutes), with 7 exchanges instead of 24.
-template <typename T>
-__device__ __forceinline__ T rs8(const T (&c)[8], int b) {
-  const bool b0 = (b & 1) != 0, b1 = (b & 2) != 0, b2 = (b & 4) != 0;
-  T a[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const T keep = b0 ? c[2 * k + 1] : c[2 * k];
-    const T send = b0 ? c[2 * k] : c[2 * k + 1];
-    a[k] = keep + xs(send, 1);  // value 2k + b0
-  }
-  T a2[2];
-#pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    const T keep = b1 ? a[2 * m + 1] : a[2 * m];
-    const T send = b1 ? a[2 * m] : a[2 * m + 1];
-    a2[m] = keep + xs(send, 2);  // value 4m + 2 b1 + b0
-  }
-  const T keep = b2 ? a2[1] : a2[0];
-  const T send = b2 ? a2[0] : a2[1];
-  return keep + xs(send, 4);
-}
+// Keeps the work on either side of it apart.
+__device__ __forceinline__ void fence(double& a) { asm("" : "+v"(a)); }
+__device__ __forceinline__ void fence(Dual& a) { asm("" : "+v"(a.v), "+v"(a.d)); }
 
 // Upper triangle of the 6x6 Voigt matrix, row by row: entry q is (kUpperI[q], kUpperJ[q]).
 __device__ constexpr int kUpperI[21] = {0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 1, 2, 2, 2, 2, 3, 3, 3, 4, 4, 5};
 __device__ constexpr int kUpperJ[21] = {0, 1, 2, 3, 4, 5, 1, 2, 3, 4, 5, 2, 3, 4, 5, 3, 4, 5, 4, 5, 5};
 
-constexpr int kAdjCells = 32;  // cells per block
+constexpr int kAdjCells = 64;  // cells per block
 constexpr int kAdjPerSeg = kCellBlock / kAdjCells;  // adjoint blocks per cell-pass block
 static_assert(kCellBlock % kAdjCells == 0, "cell-pass blocks hold whole adjoint blocks");
 constexpr int kNps = 32;       // parameter entries per (row, state)
 constexpr int kSysQ = 19;      // energy, virial (9), domain-vector gradient (9)
-// corner (x + 2y + 4z) -> corner index of the reference order (000,100,010,001,110,101,011,111)
-__device__ constexpr int kRefCorner[8] = {0, 1, 2, 4, 3, 5, 6, 7};
 
-// The lead lane of each cell stores the value (and tangent) of one per-cell quantity in the
-// cell's staging row; padding cells store zero.
-template <typename T>
-__device__ __forceinline__ void stage(double* row, int q, T x, bool lead, bool valid) {
-  if (lead) {
-    row[q] = valid ? val(x) : 0.0;
-    if (IsDual<T>::value) row[32 + q] = valid ? tan_(x) : 0.0;
-  }
-}
-
-// Sum the staged rows of the block's 32 cells: value entry q goes to row vbase + vstep * q of
-// out, tangent entry q to row tbase + tstep * q (rows of length stride). Thread t sums cells
-// 8p..8p+7 of one (entry, half), p = t mod 4, and the four parts are added by two shuffles
-// (a fixed order). Entry `extra` (< 0: none), if staged, goes to row xbase / xbase + 1.
-template <typename T>
-__device__ __forceinline__ void flush(const double* vsh, int nq, double* out, int64_t vbase,
-                                      int64_t vstep, int64_t tbase, int64_t tstep,
-                                      int64_t stride, int extra = -1, int64_t xbase = 0) {
-  __syncthreads();
-  const int part = threadIdx.x & 3;
-  const int col = threadIdx.x >> 2;        // 0..63: half * 32 + q
-  const int q = col & 31, half = col >> 5;
-  double s = 0.0;
-  // without dual numbers the tangent rows are written as zeros
-  if ((q < nq || q == extra) && (half == 0 || IsDual<T>::value)) {
+// Sums over the wave of NQ quantities q(0), q(1), ... (dual numbers: values and tangents) by the
+// reduce-scatter butterfly; put(i, half, sum) is called on one lane per quantity and half.
+// Without dual numbers the tangents are zero.
+template <int NQ, typename T, typename Quantity, typename Put>
+__device__ __forceinline__ void wave_sums(Quantity q, Put put) {
+  const int lane = threadIdx.x & 63, at = scatter_index(lane);
+  constexpr int n0 = NQ < 16 ? NQ : 16, n1 = NQ - n0;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) s += vsh[(part * 8 + c) * 64 + col];
+  for (int h = 0; h < 2; ++h) {
+    auto part = [&](int i) { return h == 0 ? val(q(i)) : tan_(q(i)); };
+    double t = 0.0, u = 0.0;
+    if (h == 0 || IsDual<T>::value) {
+      double c[n0];
+#pragma unroll
+      for (int i = 0; i < n0; ++i) c[i] = part(i);
+      t = wave_reduce_scatter<n0>(c, lane);
+      if constexpr (n1 > 0) {
+        double d[n1];
+#pragma unroll
+        for (int i = 0; i < n1; ++i) d[i] = part(16 + i);
+        u = wave_reduce_scatter<n1>(d, lane);
+      }
+    }
+    if ((lane & 3) == 0) {
+      if (at < n0) put(at, h, t);
+      if (n1 > 0 && at < n1) put(16 + at, h, u);
+    }
   }
-  s += xs8<1>(s);
-  s += xs8<2>(s);
-  if (part == 0 && (q < nq || q == extra)) {
-    int64_t r;
-    if (q == extra) r = xbase + half;
-    else r = half == 0 ? vbase + vstep * q : tbase + tstep * q;
-    out[r * stride + blockIdx.x] = s;
-  }
-  __syncthreads();
 }
 
+// Strain x of the i-th corner in the metric of the edges (Gram entries less the rest metric R,
+// halved on the diagonal) from the edges E and their squares s, its stress K x: the diagonal
+// entries added to their edges' D, the others in O; returns x . K x.
 template <typename T, int kModel>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+__device__ __forceinline__ T adjoint_corner(const const_f64 ts, int i,
+                                            const T (&E)[Frame<kModel>::NE][3],
+                                            const T (&s)[Frame<kModel>::NE], T (&x)[6],
+                                            T (&D)[Frame<kModel>::NE], T (&O)[3]) {
+  using F = Frame<kModel>;
+  const const_f64 K = ts + kMetricOffset, R = ts + kRestOffset;
+  const int a = F::corner(i);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) x[d] = mad(0.5, s[F::edge(a, d)], make<T>(-R[d], 0.0));
+#pragma unroll
+  for (int o = 0; o < 3; ++o) {
+    const T(&A)[3] = E[F::edge(a, F::axis0(o))];
+    const T(&B)[3] = E[F::edge(a, F::axis1(o))];
+    x[3 + o] = mad(A[2], B[2], mad(A[1], B[1], mad(A[0], B[0], make<T>(-R[3 + o], 0.0))));
+  }
+  T u = make<T>(0.0, 0.0);
+#pragma unroll
+  for (int I = 0; I < 6; ++I) {
+    T t = K[6 * I] * x[0];
+#pragma unroll
+    for (int J = 1; J < 6; ++J) t = mad(K[6 * I + J], x[J], t);
+    u = mad(x[I], t, u);
+    if (I < 3) {
+      const int e = F::edge(a, I);
+      D[e] = F::first(e) < i ? D[e] + t : t;
+    } else {
+      O[I < 3 ? 0 : I - 3] = t;
+    }
+  }
+  return u;
+}
+
+// Column q of a lane's LDS (64 lanes side by side; a dual number takes two).
+template <typename T>
+__device__ __forceinline__ T get_column(const double* col, int q) {
+  return IsDual<T>::value ? make<T>(col[128 * q], col[128 * q + 64]) : make<T>(col[64 * q], 0.0);
+}
+template <typename T>
+__device__ __forceinline__ void put_column(double* col, int q, T v) {
+  col[(IsDual<T>::value ? 128 : 64) * q] = val(v);
+  if (IsDual<T>::value) col[128 * q + 64] = tan_(v);
+}
+
+// Energy of a cell, dE/dkT, the stresses weighted by the states' p_s in the lane's columns (edge
+// e's diagonal in e, the others of the i-th corner behind them, then the states' energies), and
+// the metric sums of every state over the wave (put_sum(state, quantity, half, sum)).
+template <typename T, int kModel, bool kMulti, typename PutSum>
+__device__ __forceinline__ void adjoint_states(const const_f64 tab, int ns, double kt,
+                                               const T (&E)[Frame<kModel>::NE][3],
+                                               const T (&sq)[Frame<kModel>::NE], bool valid,
+                                               double* col, T& ecell, T& dkt, PutSum put_sum) {
+  using F = Frame<kModel>;
+  constexpr int NE = F::NE, NC = F::NC, NS = NE + 3 * NC;
+  T zsum = make<T>(1.0, 0.0);
+  double emin = 0.0;
+  if (kMulti) {
+    // pass 1: E_s = sum_a w u_a + f_s (mmff.py:380-384) and Z = sum_s exp(-(E_s - E_min)/kT), which
+    // the weights of pass 2 need first; E = E_min - kT ln Z (mmff.py:386-395)
+    for (int s = 0; s < ns; ++s) {
+      const const_f64 ts = tab + s * kTabStride;
+      T D[NE], u = make<T>(0.0, 0.0);
+#pragma unroll
+      for (int i = 0; i < NC; ++i) {
+        T x[6], O[3];
+        u = u + adjoint_corner<T, kModel>(ts, i, E, sq, x, D, O);
+        fence(u);
+      }
+      const T es = 0.5 * u + ts[10];
+      put_column(col, NS + s, es);
+      emin = (s == 0 || val(es) < emin) ? val(es) : emin;
+    }
+    zsum = make<T>(0.0, 0.0);
+    for (int s = 0; s < ns; ++s) zsum = zsum + dexp(-(get_column<T>(col, NS + s) - emin) / kt);
+    const T lnz = dlog(zsum);
+    ecell = emin - kt * lnz;
+    // dE/dkT = -ln Z - sum_s p_s (E_s - E_min) / kT
+    dkt = -lnz;
+  }
+  if (kMulti) {
+#pragma unroll
+    for (int q = 0; q < NS; ++q) put_column(col, q, make<T>(0.0, 0.0));
+  }
+  // pass 2: stresses weighted by p_s (mmff.py:396-398) and the metric sums
+  for (int s = 0; s < ns; ++s) {
+    const const_f64 ts = tab + s * kTabStride;
+    T D[NE], u = make<T>(0.0, 0.0), ps = make<T>(1.0, 0.0);
+    if (kMulti) {
+      const T d = get_column<T>(col, NS + s) - emin;
+      ps = dexp(-d / kt) / zsum;
+      dkt = dkt - (ps * d) / kt;
+    }
+    auto add = [&](int q, T v) {
+      if (kMulti) v = mad(ps, v, get_column<T>(col, q));
+      put_column(col, q, v);
+    };
+    T X2[21], X1[6];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      T x[6], O[3];
+      u = u + adjoint_corner<T, kModel>(ts, i, E, sq, x, D, O);
+#pragma unroll
+      for (int q = 0; q < 21; ++q)
+        X2[q] = i == 0 ? x[kUpperI[q]] * x[kUpperJ[q]] : mad(x[kUpperI[q]], x[kUpperJ[q]], X2[q]);
+#pragma unroll
+      for (int I = 0; I < 6; ++I) X1[I] = i == 0 ? x[I] : X1[I] + x[I];
+#pragma unroll
+      for (int o = 0; o < 3; ++o) add(NE + 3 * i + o, O[o]);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const int e = F::edge(F::corner(i), d);
+        if (F::last(e) == i) add(e, D[e]);
+      }
+      fence(u);
+#pragma unroll
+      for (int q = 0; q < 21; ++q) fence(X2[q]);
+    }
+    if (!kMulti) ecell = 0.5 * u + ts[10];
+    if (kMulti) {
+#pragma unroll
+      for (int q = 0; q < 21; ++q) X2[q] = ps * X2[q];
+#pragma unroll
+      for (int I = 0; I < 6; ++I) X1[I] = ps * X1[I];
+    }
+    wave_sums<28, T>(
+        [&](int q) -> T {
+          const T v = q < 21 ? X2[q] : q < 27 ? X1[q - 21] : ps;
+          return valid ? v : make<T>(0.0, 0.0);
+        },
+        [&](int q, int half, double t) { put_sum(s, q, half, t); });
+  }
+}
+
+// One lane a cell, one wave a block: the eight corners of a cell follow each other on the lane, so
+// that its sums over the corners need no exchange between lanes and an edge's square and gradient
+// are formed once; the 56 sums of a state over the wave are one butterfly for 64 cells. The edges
+// (36 dual numbers) stay in registers, in part in accumulation registers, one wave a SIMD; the
+// stresses, weighted over the states, go through LDS (36 KB a wave, four waves a CU). The waves' own
+// instructions bound it (5000 for one state, 9500 for two, six in ten of them FP64): 64
+// configurations of 16^3 cells, eight-corner model with tangents, 206 us with one lane a corner and
+// products with P per corner, 154 us with one lane a corner in the metric of the edges, 103 us so;
+// 5 of 7^3 cells with the averaged model 18.7, 13.1 and 15.5 us (five waves: one wave's time).
+template <typename T, int kModel>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1)))
 adjoint_kernel(const double* __restrict__ pos, const double* __restrict__ dpos,
                const double* __restrict__ rvecs, const double* __restrict__ drvecs,
                const int32_t* __restrict__ blk_sys, const int32_t* __restrict__ cnode,
                const int32_t* __restrict__ cwrap, const int32_t* __restrict__ blk_row,
                const double* __restrict__ tab_g, const double* __restrict__ kt_g,
                const int32_t* __restrict__ nstates_g, int32_t max_states, int64_t W,
-               double* __restrict__ gcell, double* __restrict__ gcell2,
-               double* __restrict__ part, double* __restrict__ ppart) {
-  __shared__ double es_sh[kMaxStates * kAdjCells * 2];
-  __shared__ double vsh[kAdjCells * 64];
+               const int32_t* __restrict__ cbase, int64_t S, double* __restrict__ gcell,
+               double* __restrict__ gcell2, double* __restrict__ part,
+               double* __restrict__ ppart) {
+  using F = Frame<kModel>;
+  constexpr int NE = F::NE, NC = F::NC;
+  extern __shared__ double st_sh[];  // columns: the stresses, then the states' energies
   const int64_t nblk = gridDim.x;
   const int seg = blockIdx.x / kAdjPerSeg;
   const int trow = blk_row[seg];
   const int sys = blk_sys[seg];
   const int ns = nstates_g[trow];
   const double kt = kt_g[trow];
-  const double* tab = tab_g + (int64_t)trow * max_states * kTabStride;
-  const int b = threadIdx.x & 7;
-  const int kref = kRefCorner[b];
-  const int lane = threadIdx.x & 63;
-  const int lead_lane = lane & ~7;
-  const bool lead = b == 0;
-  const int cl = threadIdx.x >> 3;
-  double* vrow = vsh + cl * 64;
-  const int64_t w = (int64_t)blockIdx.x * kAdjCells + cl;
-  const int n = cnode[w * 8 + kref];
-  const bool valid = cnode[w * 8] >= 0;
+  const const_f64 tab = (const_f64)tab_g + (int64_t)trow * max_states * kTabStride;
+  const int lane = threadIdx.x;
+  const int64_t w = (int64_t)blockIdx.x * kAdjCells + lane;
+  int n[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) n[k] = cnode[w * 8 + k];
+  const bool valid = n[0] >= 0;
   const int wrap = valid ? cwrap[w] : 0;
-  const double* rv = rvecs + 9 * (int64_t)sys;
-  const double* drv = drvecs ? drvecs + 9 * (int64_t)sys : nullptr;
+  auto stress = [&](int q) -> T { return get_column<T>(st_sh + lane, q); };
 
-  // vertex of this lane: r_0 = p_0, r_k = p_0 + ((p_k - p_0) + shift_k) (mmff.py:347-371).
-  // Every load is issued unconditionally (a padding slot reads node 0 and discards it) and the
-  // shifts use factors 0 or 1 (exact products), so that no load sits behind a branch.
-  const int64_t nn = valid ? n : 0;
-  double pv[3], dv[3] = {0.0, 0.0, 0.0}, rvv[9], drvv[9];
-#pragma unroll
-  for (int j = 0; j < 3; ++j) pv[j] = pos[3 * nn + j];
-  if (dpos) {
-#pragma unroll
-    for (int j = 0; j < 3; ++j) dv[j] = dpos[3 * nn + j];
-  }
-#pragma unroll
-  for (int q = 0; q < 9; ++q) {
-    rvv[q] = rv[q];
-    drvv[q] = drv ? drv[q] : 0.0;
-  }
-  T p[3];
-#pragma unroll
-  for (int j = 0; j < 3; ++j) p[j] = make<T>(valid ? pv[j] : 0.0, valid ? dv[j] : 0.0);
-  T r[3], r0[3];
+  // edges (mmff.py:347-371): differences of the corners' positions plus the domain vector of the
+  // edge's axis when the cell wraps along it (a factor 0 or 1; a padding slot reads node 0)
+  T E[NE][3], sq[NE];
   {
-    const int moved = b & wrap;
-    const double fx = (double)(moved & 1), fy = (double)((moved >> 1) & 1),
-                 fz = (double)((moved >> 2) & 1);
+    T p[8][3], t[12][3];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      r0[j] = bc(p[j], lead_lane);
-      const T s0 = make<T>(fx * rvv[0 + j], fx * drvv[0 + j]);
-      const T s1 = make<T>(fy * rvv[3 + j], fy * drvv[3 + j]);
-      const T s2 = make<T>(fz * rvv[6 + j], fz * drvv[6 + j]);
-      const T dvec = (p[j] - r0[j]) + ((s0 + s1) + s2);
-      r[j] = b ? r0[j] + dvec : p[j];
+    for (int k = 0; k < 8; ++k) {
+      const int64_t i = 3 * (int64_t)(valid ? n[k] : 0);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) p[k][j] = make<T>(pos[i + j], dpos ? dpos[i + j] : 0.0);
     }
-  }
-  // X: the lane's corner matrix (rows = +x, +y, +z edges through the corner), or for the
-  // averaged model H = (1/8) sum of the eight corner matrices, identical on the cell's lanes
-  T X[9];
 #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const int bit = (b >> d) & 1;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const T other = xs(r[j], 1 << d);
-      X[3 * d + j] = bit ? r[j] - other : other - r[j];
-    }
-  }
-  if (kModel == 1) {
-#pragma unroll
-    for (int i = 0; i < 9; ++i) X[i] = 0.125 * sum8(X[i]);
-  }
-
-  // pass 1 (multistate rows): E_s = w * sum_a u_a + f_s for every state (mmff.py:380-384),
-  // which the weights of pass 2 need first; a single-state cell's energy comes out of pass 2
-  double emin = 0.0;
-  for (int s = 0; s < (ns > 1 ? ns : 0); ++s) {
-    const double* ts = tab + s * kTabStride;
-    const double* P = ts;
-    const double* Cv = ts + kCvOffset;
-    T B[9];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-        B[3 * i + j] = (P[3 * i + 0] * X[0 + j] + P[3 * i + 1] * X[3 + j]) + P[3 * i + 2] * X[6 + j];
-    T e[6];
-    e[0] = 0.5 * (((B[0] * B[0] + B[1] * B[1]) + B[2] * B[2]) - 1.0);
-    e[1] = 0.5 * (((B[3] * B[3] + B[4] * B[4]) + B[5] * B[5]) - 1.0);
-    e[2] = 0.5 * (((B[6] * B[6] + B[7] * B[7]) + B[8] * B[8]) - 1.0);
-    e[3] = (B[3] * B[6] + B[4] * B[7]) + B[5] * B[8];
-    e[4] = (B[0] * B[6] + B[1] * B[7]) + B[2] * B[8];
-    e[5] = (B[0] * B[3] + B[1] * B[4]) + B[2] * B[5];
-    T u = make<T>(0.0, 0.0);
-#pragma unroll
-    for (int I = 0; I < 6; ++I) {
-      const T sI = ((((Cv[6 * I + 0] * e[0] + Cv[6 * I + 1] * e[1]) + Cv[6 * I + 2] * e[2]) +
-                     Cv[6 * I + 3] * e[3]) + Cv[6 * I + 4] * e[4]) + Cv[6 * I + 5] * e[5];
-      u = u + e[I] * sI;
-    }
-    u = 0.5 * u;
-    const T usum = kModel == 0 ? sum8(u) : u;
-    const T es = ts[9] * usum + ts[10];
-    if (lead) {
-      es_sh[(s * kAdjCells + cl) * 2 + 0] = val(es);
-      es_sh[(s * kAdjCells + cl) * 2 + 1] = tan_(es);
-    }
-    emin = (s == 0 || val(es) < emin) ? val(es) : emin;
-  }
-  if (ns > 1) __syncthreads();  // uniform over the block (one row per block)
-  // E = E_min - kT ln Z, Z = sum_s exp(-(E_s - E_min)/kT) (mmff.py:386-395); one state: E = E_0
-  T ecell = make<T>(0.0, 0.0), zsum = make<T>(1.0, 0.0), dkt = make<T>(0.0, 0.0);
-  if (ns > 1) {
-    zsum = make<T>(0.0, 0.0);
-    for (int s = 0; s < ns; ++s) {
-      const T es = make<T>(es_sh[(s * kAdjCells + cl) * 2], es_sh[(s * kAdjCells + cl) * 2 + 1]);
-      zsum = zsum + dexp(-(es - emin) / kt);
-    }
-    const T lnz = dlog(zsum);
-    ecell = emin - kt * lnz;
-    // dE/dkT = -ln Z - sum_s p_s (E_s - E_min) / kT
-    dkt = -lnz;
-  }
-
-  // pass 2: gradients, weighted by p_s (mmff.py:396-398)
-  T gacc[9];
-#pragma unroll
-  for (int i = 0; i < 9; ++i) gacc[i] = make<T>(0.0, 0.0);
-  for (int s = 0; s < ns; ++s) {
-    const double* ts = tab + s * kTabStride;
-    const double* P = ts;
-    const double wt = ts[9];
-    const double* Cv = ts + kCvOffset;
-    T ps = make<T>(1.0, 0.0);
-    if (ns > 1) {
-      const T es = make<T>(es_sh[(s * kAdjCells + cl) * 2], es_sh[(s * kAdjCells + cl) * 2 + 1]);
-      const T x = es - emin;
-      ps = dexp(-x / kt) / zsum;
-      dkt = dkt - (ps * x) / kt;
-    }
-    T B[9];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-        B[3 * i + j] = (P[3 * i + 0] * X[0 + j] + P[3 * i + 1] * X[3 + j]) + P[3 * i + 2] * X[6 + j];
-    T e[6];
-    e[0] = 0.5 * (((B[0] * B[0] + B[1] * B[1]) + B[2] * B[2]) - 1.0);
-    e[1] = 0.5 * (((B[3] * B[3] + B[4] * B[4]) + B[5] * B[5]) - 1.0);
-    e[2] = 0.5 * (((B[6] * B[6] + B[7] * B[7]) + B[8] * B[8]) - 1.0);
-    e[3] = (B[3] * B[6] + B[4] * B[7]) + B[5] * B[8];
-    e[4] = (B[0] * B[6] + B[1] * B[7]) + B[2] * B[8];
-    e[5] = (B[0] * B[3] + B[1] * B[4]) + B[2] * B[5];
-    T sv[6];
-    T u = make<T>(0.0, 0.0);
-#pragma unroll
-    for (int I = 0; I < 6; ++I) {
-      sv[I] = ((((Cv[6 * I + 0] * e[0] + Cv[6 * I + 1] * e[1]) + Cv[6 * I + 2] * e[2]) +
-                Cv[6 * I + 3] * e[3]) + Cv[6 * I + 4] * e[4]) + Cv[6 * I + 5] * e[5];
-      u = u + e[I] * sv[I];
-    }
-    u = 0.5 * u;
-    if (ns == 1) ecell = wt * (kModel == 0 ? sum8(u) : u) + ts[10];
-    // dU/dB = S B with S the symmetric stress of the Voigt vector Cv e; dU/dX = P^T (S B)
-    const T S[9] = {sv[0], sv[5], sv[4], sv[5], sv[1], sv[3], sv[4], sv[3], sv[2]};
-    T Tm[9];
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-        Tm[3 * i + j] = (S[3 * i + 0] * B[0 + j] + S[3 * i + 1] * B[3 + j]) + S[3 * i + 2] * B[6 + j];
-    const T sw = wt * ps;
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
+    for (int e = 0; e < 12; ++e) {
+      const int d = e / 4;
+      const double f = (double)((wrap >> d) & 1);
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
-        const T G = (P[0 + i] * Tm[0 + j] + P[3 + i] * Tm[3 + j]) + P[6 + i] * Tm[6 + j];
-        gacc[3 * i + j] = gacc[3 * i + j] + sw * G;
+        const int q = 9 * sys + 3 * d + j;
+        t[e][j] = mad(f, make<T>(rvecs[q], drvecs ? drvecs[q] : 0.0),
+                      p[kEdgeHi[e]][j] - p[kEdgeLo[e]][j]);
       }
-    // parameter entries of this state, summed over the cell's corners: entry q < 21 is
-    // 1/2 e_I e_J (upper triangle), 21 <= q < 30 is (dU/dB X^T)_ik = (dU/dP)_ik, 30 is u
-    auto entry = [&](int q) -> T {
-      if (q < 21) return 0.5 * (e[kUpperI[q]] * e[kUpperJ[q]]);
-      if (q < 30) {
-        const int i = (q - 21) / 3, k = (q - 21) % 3;
-        return (Tm[3 * i + 0] * X[3 * k + 0] + Tm[3 * i + 1] * X[3 * k + 1]) +
-               Tm[3 * i + 2] * X[3 * k + 2];
-      }
-      return q == 30 ? u : make<T>(0.0, 0.0);
-    };
-    if (kModel == 0) {
-      // eight entries at a time, summed over the cell's lanes by a reduce-scatter: lane b ends
-      // with entry 8g + b and stages it (entry 31, the weight p_s, is not a sum)
-#pragma unroll
-      for (int g = 0; g < kNps / 8; ++g) {
-        T c[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) c[i] = entry(8 * g + i);
-        const T sum = rs8(c, b);
-        const int q = 8 * g + b;
-        const T v = q == 31 ? ps : (q == 30 ? ps : sw) * sum;
-        vrow[q] = valid ? val(v) : 0.0;
-        if (IsDual<T>::value) vrow[32 + q] = valid ? tan_(v) : 0.0;
-      }
-    } else {
-      // the averaged model's entries are the same on all eight lanes of a cell
-#pragma unroll
-      for (int q = 0; q < 30; ++q) stage(vrow, q, sw * entry(q), lead, valid);
-      stage(vrow, 30, ps * u, lead, valid);
-      stage(vrow, 31, ps, lead, valid);
     }
-    flush<T>(vsh, kNps, ppart, (int64_t)2 * s * kNps, 2, (int64_t)2 * s * kNps + 1, 2, nblk);
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        E[e][j] = kModel == 0 ? t[e][j]
+                              : 0.25 * ((t[4 * e % 12][j] + t[(4 * e + 1) % 12][j]) +
+                                        (t[(4 * e + 2) % 12][j] + t[(4 * e + 3) % 12][j]));
+      sq[e] = mad(E[e][2], E[e][2], mad(E[e][1], E[e][1], E[e][0] * E[e][0]));
+    }
   }
 
-  // vertex gradient: corner b is the upper end of the d edges of corners b and b ^ (1 << d)
-  // when bit d of b is set, the lower end otherwise (averaged model: a quarter of the row)
-  T g[3];
-#pragma unroll
-  for (int j = 0; j < 3; ++j) g[j] = make<T>(0.0, 0.0);
-#pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const int bit = (b >> d) & 1;
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const T row = kModel == 0 ? gacc[3 * d + j] + xs(gacc[3 * d + j], 1 << d)
-                                : 0.25 * gacc[3 * d + j];
-      g[j] = bit ? g[j] + row : g[j] - row;
-    }
-  }
-  if (valid) {
-#pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      __builtin_nontemporal_store(val(g[j]), &gcell[(int64_t)(3 * kref + j) * W + w]);
-      if (IsDual<T>::value)
-        __builtin_nontemporal_store(tan_(g[j]), &gcell2[(int64_t)(3 * kref + j) * W + w]);
-    }
-  }
-  // energy, virial sum_v g_v (x) (r_v - r_0) and the domain-vector gradient: corner b moves
-  // with domain vector d when the cell wraps along d and the corner lies at +d
-  // (entries 1..18 summed over the cell's lanes eight at a time, as the parameter entries;
-  // the energy and dE/dkT, the same on every lane of the cell, ride along as entries 0 and
-  // kSysQ, the latter into its parameter rows)
-  auto sys_entry = [&](int q) -> T {
-    if (q >= 1 && q <= 9) return g[(q - 1) / 3] * (r[(q - 1) % 3] - r0[(q - 1) % 3]);
-    if (q >= 10 && q <= 18) {
-      const int d = (q - 10) / 3;
-      const double moves = (double)(((b & wrap) >> d) & 1);
-      return moves * g[(q - 10) % 3];
-    }
-    return make<T>(0.0, 0.0);
+  T ecell = make<T>(0.0, 0.0), dkt = make<T>(0.0, 0.0);
+  auto put_sum = [&](int s, int q, int half, double t) {
+    ppart[((int64_t)2 * (s * kNps + q) + half) * nblk + blockIdx.x] = t;
   };
+  if (ns > 1)
+    adjoint_states<T, kModel, true>(tab, ns, kt, E, sq, valid, st_sh + lane, ecell, dkt, put_sum);
+  else
+    adjoint_states<T, kModel, false>(tab, 1, kt, E, sq, valid, st_sh + lane, ecell, dkt, put_sum);
+
+  // dE/d(edge) = D_e E_e + the rows of S M off the diagonal (edge_gradient): an edge closes at its
+  // second corner and pulls at its upper vertex, pushes at its lower one (averaged model: a
+  // quarter of the mean edge's at every vertex), adds gE (x) E to the virial and, when the cell
+  // wraps along its axis, gE to that domain vector's gradient
+  T gE[NE][3], g[8][3], vir[6], gdom[3][3];
 #pragma unroll
-  for (int gq = 0; gq < 3; ++gq) {
-    T c[8];
+  for (int v = 0; v < 8; ++v)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) c[i] = sys_entry(8 * gq + i);
-    const T sum = rs8(c, b);
-    const int q = 8 * gq + b;
-    const T v = q == 0 ? ecell : q == kSysQ ? dkt : sum;
-    if (q <= kSysQ) {
-      vrow[q] = valid ? val(v) : 0.0;
-      if (IsDual<T>::value) vrow[32 + q] = valid ? tan_(v) : 0.0;
+    for (int j = 0; j < 3; ++j) g[v][j] = make<T>(-0.0, -0.0);
+#pragma unroll
+  for (int v = 0; v < 6; ++v) vir[v] = make<T>(0.0, 0.0);
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) gdom[d][j] = make<T>(0.0, 0.0);
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int a = F::corner(i);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const int e = F::edge(a, d);
+      if (F::first(e) == i) {
+        const T De = stress(e);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) gE[e][j] = De * E[e][j];
+      }
+    }
+#pragma unroll
+    for (int o = 0; o < 3; ++o) {
+      const int e0 = F::edge(a, F::axis0(o)), e1 = F::edge(a, F::axis1(o));
+      const T Oo = stress(NE + 3 * i + o);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        gE[e0][j] = mad(Oo, E[e1][j], gE[e0][j]);
+        gE[e1][j] = mad(Oo, E[e0][j], gE[e1][j]);
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const int e = F::edge(a, d);
+      if (F::last(e) != i) continue;
+      constexpr int kK[6] = {0, 1, 2, 1, 0, 0}, kL[6] = {0, 1, 2, 2, 2, 1};
+#pragma unroll
+      for (int v = 0; v < 6; ++v) vir[v] = mad(gE[e][kK[v]], E[e][kL[v]], vir[v]);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        gdom[d][j] = gdom[d][j] + gE[e][j];
+        if (kModel == 0) {
+          g[kEdgeHi[e]][j] = g[kEdgeHi[e]][j] + gE[e][j];
+          g[kEdgeLo[e]][j] = g[kEdgeLo[e]][j] - gE[e][j];
+        } else {
+          const T t = 0.25 * gE[e][j];
+#pragma unroll
+          for (int v = 0; v < 8; ++v) g[v][j] = kOff[v][d] ? g[v][j] + t : g[v][j] - t;
+        }
+      }
     }
   }
-  __syncthreads();
-  {
-    // the system rows go to `part`, the kT entry to `ppart`: two writers of one staged block
-    const int pq = threadIdx.x & 3;
-    const int col = threadIdx.x >> 2;
-    const int q = col & 31, half = col >> 5;
-    double sum = 0.0;
-    if (q <= kSysQ && (half == 0 || IsDual<T>::value)) {
+  wave_sums<17, T>(
+      [&](int q) -> T {
+        T t = q == 0 ? ecell : q < 7 ? vir[(q - 1) % 6] : q < 16 ? gdom[(q - 7) / 3 % 3][(q - 7) % 3] : dkt;
+        if (q >= 7 && q < 16) t = (double)((wrap >> ((q - 7) / 3)) & 1) * t;
+        return valid ? t : make<T>(0.0, 0.0);
+      },
+      [&](int q, int half, double t) {
+        if (q == 16) {
+          ppart[((int64_t)2 * max_states * kNps + half) * nblk + blockIdx.x] = t;
+          return;
+        }
+        // rows of the energy, of the full 3x3 virial (both copies of an off-diagonal entry) and of
+        // the domain-vector gradient, as nibbles
+        const int row = q < 7 ? (int)(0x2369510ull >> (4 * q)) & 0xf : q + 3;
+        double* out = part + (int64_t)(half * kSysQ) * nblk + blockIdx.x;
+        out[(int64_t)row * nblk] = t;
+        if (q >= 4 && q < 7) out[(int64_t)((int)(0x478ull >> (4 * (q - 4))) & 0xf) * nblk] = t;
+      });
+  double gv[8][3];
 #pragma unroll
-      for (int c = 0; c < 8; ++c) sum += vsh[(pq * 8 + c) * 64 + col];
-    }
-    sum += xs8<1>(sum);
-    sum += xs8<2>(sum);
-    if (pq == 0 && q < kSysQ)
-      part[(int64_t)(half == 0 ? q : kSysQ + q) * nblk + blockIdx.x] = sum;
-    if (pq == 0 && q == kSysQ)
-      ppart[((int64_t)2 * max_states * kNps + half) * nblk + blockIdx.x] = sum;
+  for (int v = 0; v < 8; ++v)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) gv[v][j] = valid ? val(g[v][j]) : -0.0;
+  store_cell<true>(w, wrap, valid, cbase, W, S, gcell, gv);
+  if (IsDual<T>::value) {
+#pragma unroll
+    for (int v = 0; v < 8; ++v)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) gv[v][j] = valid ? tan_(g[v][j]) : -0.0;
+    store_cell<true>(w, wrap, valid, cbase, W, S, gcell2, gv);
   }
 }
 
-// Row sums of per-block partials over lists of segments (8 blocks each): one block per
+// The 32 parameter entries of every (row, state) from its metric sums, in place in params
+// [nrows][npar][2]: with T the map of x to the engineering strain e = T x (metric_entry),
+// X2 = sum p x x^T and X1 = sum p x, S = Cv T x the stress and G = 2 x + R the Gram matrix,
+//   dE/dCv = w T X2 T^T / 2,  dE/dP_ik = w sum_mn P_mn (sum p S_im G_nk),
+//   dE/dw = tr(Cv^T T X2 T^T) / 2,
+// all linear in the sums, so values and tangents alike. One wave per (row, state); lane 32 h + i
+// works on half h.
+__global__ void __launch_bounds__(64)
+metric_entries_kernel(const double* __restrict__ tab, const int32_t* __restrict__ nstates,
+                      int max_states, int64_t npar, double* __restrict__ params) {
+  const int row = blockIdx.x / max_states, s = blockIdx.x % max_states;
+  if (s >= nstates[row]) return;
+  const double* ts = tab + (int64_t)blockIdx.x * kTabStride;
+  const double* C = ts + kCvOffset;
+  const double* R = ts + kRestOffset;
+  const double w = ts[9];
+  double* out = params + 2 * (row * npar + (int64_t)s * kNps);
+  __shared__ double T[36], P[9], X2[2][36], X1[2][6], A[2][36], E[2][36], Q[2][36], B[2][6], p[2];
+  const int h = threadIdx.x >> 5, i = threadIdx.x & 31;
+  if (threadIdx.x < 9) P[threadIdx.x] = ts[threadIdx.x];
+  if (i < 28) {
+    const double v = out[2 * i + h];
+    if (i < 21)
+      X2[h][6 * kUpperI[i] + kUpperJ[i]] = X2[h][6 * kUpperJ[i] + kUpperI[i]] = v;
+    else if (i < 27)
+      X1[h][i - 21] = v;
+    else
+      p[h] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x < 36) T[threadIdx.x] = strain_map(P, threadIdx.x / 6, threadIdx.x % 6);
+  __syncthreads();
+  for (int q = i; q < 36; q += 32) {
+    double t = 0.0;
+    for (int k = 0; k < 6; ++k) t += T[6 * (q / 6) + k] * X2[h][6 * k + q % 6];
+    A[h][q] = t;
+  }
+  __syncthreads();
+  for (int q = i; q < 36; q += 32) {
+    double t = 0.0, c = 0.0;
+    for (int k = 0; k < 6; ++k) {
+      t += A[h][6 * (q / 6) + k] * T[6 * (q % 6) + k];
+      c += C[6 * (q / 6) + k] * A[h][6 * k + q % 6];
+    }
+    E[h][q] = t;
+    Q[h][q] = c;
+  }
+  if (i < 6) {
+    double t = 0.0;
+    for (int k = 0; k < 6; ++k)
+      for (int l = 0; l < 6; ++l) t += (C[6 * i + k] * T[6 * k + l]) * X1[h][l];
+    B[h][i] = t;
+  }
+  __syncthreads();
+  double v = 0.0;
+  if (i < 21) {
+    v = 0.5 * (w * E[h][6 * kUpperI[i] + kUpperJ[i]]);
+  } else if (i < 30) {
+    constexpr int kVoigt[9] = {0, 5, 4, 5, 1, 3, 4, 3, 2};
+    const int a = (i - 21) / 3, k = (i - 21) % 3;
+    for (int m = 0; m < 3; ++m)
+      for (int n = 0; n < 3; ++n) {
+        const int sm = kVoigt[3 * a + m], gn = kVoigt[3 * n + k];
+        const double sg = B[h][sm] * R[gn] + Q[h][6 * sm + gn];
+        v += P[3 * m + n] * (n == k ? 2.0 * sg : sg);
+      }
+    v *= w;
+  } else if (i == 30) {
+    for (int q = 0; q < 36; ++q) v += C[q] * E[h][q];
+    v *= 0.5;
+  } else {
+    v = p[h];
+  }
+  out[2 * i + h] = v;
+}
+
+// Row sums of per-block partials over lists of segments (4 blocks each): one block per
 // (list, row of the partial array). Rows q with q % weight_every == 0 are scaled per segment by
 // weight[system of the segment] when weight is given.
 __global__ void __launch_bounds__(256)
@@ -628,10 +670,10 @@ param_grads_kernel(const double* __restrict__ entries, int64_t stride, int add_n
 struct mm_adjoint {
   mm_field* field = nullptr;
   int64_t npar = 0;            // parameter entries per row: max_states * 32 + 1
-  int64_t nblk = 0;            // W / 32
+  int64_t nblk = 0;            // W / 64
   double* part = nullptr;      // [2 kSysQ][nblk]
   double* ppart = nullptr;     // [2 npar][nblk]
-  double* gcell2 = nullptr;    // [8][3][W]
+  double* gcell2 = nullptr;    // [4][3][S]
   int32_t* row_ptr = nullptr;  // [nrows + 1] CSR of the segments of every table row
   int32_t* row_idx = nullptr;  // [W / kCellBlock]
   double* vjp = nullptr;       // [3][N][3] + [nsys][9]: dpos, gpos, dgpos, drvecs of mm_adjoint_vjp
@@ -668,7 +710,7 @@ int mm_adjoint_create(mm_adjoint** out, mm_field* field, int64_t* npar) {
   e = hipMalloc((void**)&a->part, sizeof(double) * 2 * kSysQ * nb);
   if (e == hipSuccess) e = hipMalloc((void**)&a->ppart, sizeof(double) * 2 * a->npar * nb);
   if (e == hipSuccess)
-    e = hipMalloc((void**)&a->gcell2, sizeof(double) * 24 * (field->W > 0 ? field->W : 1));
+    e = hipMalloc((void**)&a->gcell2, sizeof(double) * 12 * (field->S > 0 ? field->S : 1));
   if (e == hipSuccess)
     e = hipMalloc((void**)&a->vjp, sizeof(double) * (9 * (size_t)field->N + 9 * field->nsys));
   if (e == hipSuccess) e = hipMalloc((void**)&a->row_ptr, sizeof(int32_t) * row_ptr.size());
@@ -710,11 +752,13 @@ int mm_adjoint_compute(mm_adjoint* a, const double* pos, const double* dpos, con
   const int64_t nblk = a->nblk;
   hipError_t e = hipSuccess;
   if (nblk > 0) {
+    const size_t lds = sizeof(double) * 64 * (dual ? 2 : 1) *
+                       ((f->model == 0 ? 36 : 6) + (f->max_states > 1 ? f->max_states : 0));
 #define MM_ADJ(T, MODEL)                                                                        \
-  hipLaunchKernelGGL((adjoint_kernel<T, MODEL>), dim3((unsigned)nblk), dim3(256), 0, s, pos,    \
+  hipLaunchKernelGGL((adjoint_kernel<T, MODEL>), dim3((unsigned)nblk), dim3(64), lds, s, pos,   \
                      dpos, rvecs, drvecs, f->blk_sys, f->cnode, f->cwrap, f->blk_row, f->tab,  \
-                     f->kt, f->nstates, f->max_states, f->W, f->gcell, a->gcell2, a->part,     \
-                     a->ppart)
+                     f->kt, f->nstates, f->max_states, f->W, f->cbase, f->S, f->gcell,         \
+                     a->gcell2, a->part, a->ppart)
     if (dual) {
       if (f->model == 0) MM_ADJ(Dual, 0); else MM_ADJ(Dual, 1);
     } else {
@@ -736,12 +780,16 @@ int mm_adjoint_compute(mm_adjoint* a, const double* pos, const double* dpos, con
                          f->blk_sys, energy_weight, 2, params);
       e = hipGetLastError();
     }
+    if (e == hipSuccess && f->nrows > 0) {
+      hipLaunchKernelGGL(metric_entries_kernel, dim3((unsigned)(f->nrows * f->max_states)),
+                         dim3(64), 0, s, f->tab, f->nstates, f->max_states, a->npar, params);
+      e = hipGetLastError();
+    }
     if (e == hipSuccess && f->N > 0 && gpos) {
       ForceArgs g{};
-      g.ncell = f->ncell;
+      g.ncell = f->nrec;
       g.gcell = f->gcell;
-      g.rstride = f->W;
-      g.rshift = 3;
+      g.rstride = f->S;
       g.N = f->N;
       g.W = f->W;
       g.gpos = gpos;

@@ -142,7 +142,6 @@ void free_field(mm_field* f) {
   (void)hipFree(f->cnode);
   (void)hipFree(f->cwrap);
   (void)hipFree(f->blk_row);
-  (void)hipFree(f->ncell);
   (void)hipFree(f->nrec);
   (void)hipFree(f->cbase);
   (void)hipFree(f->nstates);
@@ -192,7 +191,6 @@ void field_args(const mm_field* f, ForceArgs& a) {
   a.ncell = f->nrec;
   a.gcell = f->gcell;
   a.rstride = f->S;
-  a.rshift = 2;
   a.cbase = f->cbase;
   a.partials = f->partials;
   a.model = f->model;
@@ -333,13 +331,6 @@ int create_field(mm_field** out, int device, int model, int32_t nsys, int64_t nc
     sys_ptr[sy + 1] = sys_ptr[sy] + (int32_t)sys_blocks[sy].size();
     sys_idx.insert(sys_idx.end(), sys_blocks[sy].begin(), sys_blocks[sy].end());
   }
-  std::vector<int32_t> ncell((size_t)8 * nnodes, -1);
-  for (int64_t n = 0; n < nnodes; ++n) {
-    for (int k = 0; k < 8; ++k) {
-      const int64_t c = surrounding_cells[n * 8 + k];
-      if (c >= 0) ncell[(size_t)k * nnodes + n] = (int32_t)(slot[c] * 8 + k);
-    }
-  }
   // Shared faces along z, the axis along which the reference numbers consecutive cells: when
   // slot w + 1 of the same wave holds the +z neighbour of slot w (corner 3 of w is corner 0 of
   // w + 1), the cell pass adds w's upper-face vertex gradients (corners 3, 5, 6, 7) to w + 1's
@@ -398,10 +389,10 @@ int create_field(mm_field** out, int device, int model, int32_t nsys, int64_t nc
   f->slot_of_cell = std::move(slot);
   const int64_t nb = W / kCellBlock;
   if ((rc = dmalloc(&f->cnode, (size_t)8 * W)) || (rc = dmalloc(&f->cwrap, W)) ||
-      (rc = dmalloc(&f->blk_row, nb)) || (rc = dmalloc(&f->ncell, (size_t)8 * nnodes)) ||
+      (rc = dmalloc(&f->blk_row, nb)) ||
       (rc = dmalloc(&f->nrec, (size_t)8 * nnodes)) || (rc = dmalloc(&f->cbase, W / 64)) ||
       (rc = dmalloc(&f->nstates, nrows)) || (rc = dmalloc(&f->tab, tab.size())) ||
-      (rc = dmalloc(&f->kt, kt.size())) || (rc = dmalloc(&f->gcell, (size_t)24 * W)) ||
+      (rc = dmalloc(&f->kt, kt.size())) || (rc = dmalloc(&f->gcell, (size_t)12 * f->S)) ||
       (rc = dmalloc(&f->partials, (size_t)kPartialStride * (nb > 0 ? nb : 1))) ||
       (rc = dmalloc(&f->cgpart, (size_t)8 * (nnodes > 0 ? (nnodes + 255) / 256 : 1))) ||
       (rc = dmalloc(&f->nanflag, 1)) || (rc = dmalloc(&f->blk_sys, nb)) ||
@@ -412,7 +403,6 @@ int create_field(mm_field** out, int device, int model, int32_t nsys, int64_t nc
   }
   if ((rc = h2d(f->cnode, cnode.data(), cnode.size())) || (rc = h2d(f->cwrap, cwrap.data(), W)) ||
       (rc = h2d(f->blk_row, blk_row.data(), blk_row.size())) ||
-      (rc = h2d(f->ncell, ncell.data(), ncell.size())) ||
       (rc = h2d(f->nrec, nrec.data(), nrec.size())) ||
       (rc = h2d(f->cbase, cbase.data(), cbase.size())) ||
       (rc = h2d(f->nstates, nstates, (size_t)nrows)) ||

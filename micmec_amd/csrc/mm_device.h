@@ -54,25 +54,28 @@ __host__ __device__ inline double inverse3_cof(const double* h, double* inv) {
   return det;
 }
 
-// K and R of one table entry from h0, P = h0^-1, w and Cv. T maps the Gram entries e6 to the
-// engineering strain: eps_ij = sum_ab P_ia P_jb e_ab, i.e. with (i,j) and (a,b) the pairs of
-// rows I and columns J, T_IJ = P_ia P_ja (a = b) or (P_ia P_jb + P_ib P_ja) / 2 (a != b, where
-// e6 holds 2 e_ab), doubled for the shear rows I >= 3. Shared by the host and the device table
+// Entry IJ of the map T of the Gram entries e6 to the engineering strain: eps_ij = sum_ab P_ia P_jb
+// e_ab, i.e. with (i,j) and (a,b) the pairs of rows I and columns J, T_IJ = P_ia P_ja (a = b) or
+// (P_ia P_jb + P_ib P_ja) / 2 (a != b, where e6 holds 2 e_ab), doubled for the shear rows I >= 3.
+__host__ __device__ inline double strain_map(const double* P, int I, int J) {
+#pragma clang fp contract(off)
+  const int pi[6] = {0, 1, 2, 1, 0, 0}, pj[6] = {0, 1, 2, 2, 2, 1};
+  const double* a = P + 3 * pi[I];
+  const double* b = P + 3 * pj[I];
+  const double cross = a[pi[J]] * b[pj[J]] + a[pj[J]] * b[pi[J]];
+  return (I < 3) == (J < 3) ? (I < 3 ? a[pi[J]] * b[pi[J]] : cross)
+                            : (I < 3 ? 0.5 * cross : cross);
+}
+
+// K and R of one table entry from h0, P = h0^-1, w and Cv. Shared by the host and the device table
 // builders, without contraction, so both round the same way.
 __host__ __device__ inline void metric_entry(const double* h0, const double* P, double w,
                                              const double* Cv, double* K, double* R) {
 #pragma clang fp contract(off)
   const int pi[6] = {0, 1, 2, 1, 0, 0}, pj[6] = {0, 1, 2, 2, 2, 1};
   double T[36], CT[36];
-  for (int I = 0; I < 6; ++I) {
-    const double* a = P + 3 * pi[I];
-    const double* b = P + 3 * pj[I];
-    for (int J = 0; J < 6; ++J) {
-      const double cross = a[pi[J]] * b[pj[J]] + a[pj[J]] * b[pi[J]];
-      T[6 * I + J] = (I < 3) == (J < 3) ? (I < 3 ? a[pi[J]] * b[pi[J]] : cross)
-                                        : (I < 3 ? 0.5 * cross : cross);
-    }
-  }
+  for (int I = 0; I < 6; ++I)
+    for (int J = 0; J < 6; ++J) T[6 * I + J] = strain_map(P, I, J);
   for (int I = 0; I < 6; ++I)
     for (int J = 0; J < 6; ++J) {
       double t = 0.0;
@@ -375,8 +378,8 @@ __device__ __forceinline__ void vecmat(const double v[3], const double* M, doubl
 }
 
 // g = the sum of node n's records in k order (mmff.py:303-318): record e = ncell[k * N + n]
-// (none when e < 0) holds the three components gcell[(3 * (e & (2^rshift - 1)) + j) * RS +
-// (e >> rshift)]; g starts at +0.0 and takes the records present in k order.
+// (none when e < 0) holds the three components gcell[(3 * (e & 3) + j) * RS + (e >> 2)];
+// g starts at +0.0 and takes the records present in k order.
 // kAllLoads: the eight indices are loaded first and then all 24 components, a none reading those
 // of record 0 (always allocated) and left out of the sum, so that every load of the lane is in
 // flight at once (two memory round trips instead of up to sixteen), at the cost of about 50
@@ -387,7 +390,7 @@ __device__ __forceinline__ void vecmat(const double v[3], const double* M, doubl
 template <bool kAllLoads, bool kStream = true>
 __device__ __forceinline__ void sum_node_records(const int32_t* __restrict__ ncell,
                                                  const double* gcell, int64_t N, int64_t RS,
-                                                 int rshift, int64_t n, double g[3]) {
+                                                 int64_t n, double g[3]) {
   auto load = [](const auto* p) { return kStream ? __builtin_nontemporal_load(p) : *p; };
 #pragma unroll
   for (int j = 0; j < 3; ++j) g[j] = 0.0;
@@ -396,8 +399,8 @@ __device__ __forceinline__ void sum_node_records(const int32_t* __restrict__ nce
     for (int k = 0; k < 8; ++k) {
       const int32_t e = load(&ncell[k * N + n]);
       if (e >= 0) {
-        const int64_t w = e >> rshift;
-        const int p = e & ((1 << rshift) - 1);
+        const int64_t w = e >> 2;
+        const int p = e & 3;
 #pragma unroll
         for (int j = 0; j < 3; ++j)
           g[j] += load(&gcell[(int64_t)(3 * p + j) * RS + w]);
@@ -412,8 +415,8 @@ __device__ __forceinline__ void sum_node_records(const int32_t* __restrict__ nce
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const int32_t c = e[k] >= 0 ? e[k] : 0;
-    const int64_t w = c >> rshift;
-    const int p = c & ((1 << rshift) - 1);
+    const int64_t w = c >> 2;
+    const int p = c & 3;
 #pragma unroll
     for (int j = 0; j < 3; ++j)
       r[k][j] = load(&gcell[(int64_t)(3 * p + j) * RS + w]);

@@ -166,7 +166,7 @@ __device__ __forceinline__ void block_sum_max_store(double (&v)[NS + NM], double
 template <bool DOT, bool kAllLoads>
 __global__ void __launch_bounds__(256)
 gather_kernel(const int32_t* __restrict__ ncell, const double* __restrict__ gcell, int64_t N,
-              int64_t RS, int rshift, double* __restrict__ gpos, int accumulate, int* __restrict__ nanflag,
+              int64_t RS, double* __restrict__ gpos, int accumulate, int* __restrict__ nanflag,
               const double* __restrict__ dir, const double* __restrict__ gold,
               double* __restrict__ dpart) {
   __shared__ double sg[768];
@@ -189,7 +189,7 @@ gather_kernel(const int32_t* __restrict__ ncell, const double* __restrict__ gcel
     }
   }
   double g[3] = {0.0, 0.0, 0.0};
-  if (n < N) sum_node_records<kAllLoads>(ncell, gcell, N, RS, rshift, n, g);
+  if (n < N) sum_node_records<kAllLoads>(ncell, gcell, N, RS, n, g);
   __syncthreads();
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
   if (n < N) {
@@ -337,11 +337,11 @@ hipError_t launch_gather(const ForceArgs& a, hipStream_t stream) {
   const int gb = (int)((a.N + 255) / 256);
   if (gb <= kGatherAllLoadsMaxBlocks)
     hipLaunchKernelGGL((gather_kernel<false, true>), dim3(gb), dim3(256), 0, stream, a.ncell,
-                       a.gcell, a.N, a.rstride, a.rshift, a.gpos, a.accumulate, a.nanflag,
+                       a.gcell, a.N, a.rstride, a.gpos, a.accumulate, a.nanflag,
                        nullptr, nullptr, nullptr);
   else
     hipLaunchKernelGGL((gather_kernel<false, false>), dim3(gb), dim3(256), 0, stream, a.ncell,
-                       a.gcell, a.N, a.rstride, a.rshift, a.gpos, a.accumulate, a.nanflag,
+                       a.gcell, a.N, a.rstride, a.gpos, a.accumulate, a.nanflag,
                        nullptr, nullptr, nullptr);
   return hipGetLastError();
 }
@@ -352,11 +352,11 @@ hipError_t launch_gather_dot(const ForceArgs& a, const double* dir, const double
   const int gb = (int)((a.N + 255) / 256);
   if (gb <= kGatherAllLoadsMaxBlocks)
     hipLaunchKernelGGL((gather_kernel<true, true>), dim3(gb), dim3(256), 0, stream, a.ncell,
-                       a.gcell, a.N, a.rstride, a.rshift, a.gpos, a.accumulate, a.nanflag, dir,
+                       a.gcell, a.N, a.rstride, a.gpos, a.accumulate, a.nanflag, dir,
                        gold, dpart);
   else
     hipLaunchKernelGGL((gather_kernel<true, false>), dim3(gb), dim3(256), 0, stream, a.ncell,
-                       a.gcell, a.N, a.rstride, a.rshift, a.gpos, a.accumulate, a.nanflag, dir,
+                       a.gcell, a.N, a.rstride, a.gpos, a.accumulate, a.nanflag, dir,
                        gold, dpart);
   return hipGetLastError();
 }

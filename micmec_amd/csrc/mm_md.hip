@@ -1343,7 +1343,7 @@ gather_kick_kernel(const int32_t* __restrict__ ncell, const double* __restrict__
   if (own) {
     if (kAllLoads) load_node();
     if (gmode != kGatherNone) {
-      sum_node_records<kAllLoads>(ncell, gcell, N, RS, 2, n, g);
+      sum_node_records<kAllLoads>(ncell, gcell, N, RS, n, g);
 #pragma unroll
       for (int j = 0; j < 3; ++j) {
         if (gmode == kGatherStore) gpos[3 * n + j] = g[j];
@@ -1842,7 +1842,6 @@ ForceArgs force_args(mm_md* md) {
   a.ncell = f->nrec;
   a.gcell = f->gcell;
   a.rstride = f->S;
-  a.rshift = 2;
   a.cbase = f->cbase;
   a.partials = f->partials;
   a.energy = nullptr;
