@@ -114,12 +114,13 @@ __device__ __forceinline__ void cell_eval(const_f64 tab, int ns, double kt, bool
     if constexpr (kModel == 0 && !kMulti) {
       ecell = tab[10] + sweep_cell<kOut>(tab, p, f, rv, vir, gacc);
     } else {
-      double E[F::NE][3], s2[F::NE], D[F::NE], O[F::NC][3];
+      double E[F::NE][3], q[F::NE], D[F::NE], O[F::NC][3];
       form_edges<kModel>(p, f, rv, E);
 #pragma unroll
-      for (int e = 0; e < F::NE; ++e) s2[e] = edge_square(E[e]);
+      for (int e = 0; e < F::NE; ++e)
+        q[e] = edge_strain(E[e], F::along(e), tab[kRestOffset + F::along(e)]);
       if (!kMulti) {
-        ecell = tab[10] + state_stress<kModel>(tab, E, s2, D, O);
+        ecell = tab[10] + state_stress<kModel>(tab, tab + kRestOffset, E, q, D, O);
       } else {
         // one pass over the states (mmff.py:386-398): E = E_min - kT ln Z with Z = sum_s c_s,
         // c_s = exp(-(E_s - E_min)/kT), and the stresses sum_s c_s S_s accumulated in LDS, both
@@ -127,7 +128,7 @@ __device__ __forceinline__ void cell_eval(const_f64 tab, int ns, double kt, bool
         double emin = 0.0, zsum = 0.0;
         for (int s = 0; s < ns; ++s) {
           const const_f64 ts = tab + s * kTabStride;
-          const double es = ts[10] + state_stress<kModel>(ts, E, s2, D, O);
+          const double es = ts[10] + state_stress<kModel>(ts, tab + kRestOffset, E, q, D, O);
           double keep = 0.0, c = 1.0;  // factors of the sums so far and of this state
           if (s == 0) {
             emin = es;

@@ -178,19 +178,25 @@ __device__ __forceinline__ double edge_dot(const double (&A)[3], const double (&
 #pragma clang fp contract(off)
   return __builtin_fma(A[2], B[2], __builtin_fma(A[1], B[1], __builtin_fma(A[0], B[0], -g0)));
 }
-__device__ __forceinline__ double edge_square(const double (&A)[3]) {
+// Diagonal strain of an edge along d against half its rest metric g0: (A.A)/2 - g0, the sum begun
+// with the component along d less 2 g0. That product is exact inside the fused multiply-add, so
+// where the rest cell is near the axes the error is relative to the strain, not to the edge.
+__device__ __forceinline__ double edge_strain(const double (&A)[3], int d, double g0) {
 #pragma clang fp contract(off)
-  return __builtin_fma(A[2], A[2], __builtin_fma(A[1], A[1], A[0] * A[0]));
+  const int b = d == 0 ? 1 : 0, c = d == 2 ? 1 : 2;
+  return 0.5 * __builtin_fma(A[c], A[c],
+                             __builtin_fma(A[b], A[b], __builtin_fma(A[d], A[d], -2.0 * g0)));
 }
 
 // Energy (weighted, without the free-energy offset) and stress of one (type, state) at all
-// corners, from the edges E and their squared lengths s: D[e] = the diagonal stress along edge
-// e summed over its corners, O[a][q] the off-diagonal stresses of corner a. The sums are fused
+// corners, from the edges E and their strains q against the rest metric r0 of the type's first
+// state: D[e] = the diagonal stress along edge e summed over its corners, O[a][q] the
+// off-diagonal stresses of corner a. The sums are fused
 // multiply-adds in a fixed order, so every kernel that evaluates a state gets the same bits.
 template <int kModel>
-__device__ __forceinline__ double state_stress(const_f64 tab,
+__device__ __forceinline__ double state_stress(const_f64 tab, const_f64 r0,
                                                const double (&E)[Frame<kModel>::NE][3],
-                                               const double (&s)[Frame<kModel>::NE],
+                                               const double (&q)[Frame<kModel>::NE],
                                                double (&D)[Frame<kModel>::NE],
                                                double (&O)[Frame<kModel>::NC][3]) {
 #pragma clang fp contract(off)
@@ -202,7 +208,7 @@ __device__ __forceinline__ double state_stress(const_f64 tab,
     const int a = F::corner(i);
     double x[6];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) x[d] = __builtin_fma(0.5, s[F::edge(a, d)], -g0[d]);
+    for (int d = 0; d < 3; ++d) x[d] = q[F::edge(a, d)] + (r0[d] - g0[d]);
 #pragma unroll
     for (int o = 0; o < 3; ++o)
       x[3 + o] = edge_dot(E[F::edge(a, F::axis0(o))], E[F::edge(a, F::axis1(o))], g0[3 + o]);
@@ -317,7 +323,7 @@ __device__ __forceinline__ double sweep_cell(const_f64 tab,
       const int e = F::edge(a, d);
       if (F::first(e) == i) {
         form_edge(p, e, f[d], &rv[3 * d], E[e]);
-        q[e] = __builtin_fma(0.5, edge_square(E[e]), -g0[d]);
+        q[e] = edge_strain(E[e], d, g0[d]);
       }
       x[d] = q[e];
     }
