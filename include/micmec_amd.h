@@ -69,6 +69,12 @@ int mm_field_create(mm_field** out, int device, int model, int64_t ncells, int64
 int mm_field_compute(mm_field* f, const double* pos, const double* rvecs, double* energy,
                      double* gpos, double* vtens, int accumulate, void* stream);
 
+/* mm_field_compute of a single-system object on host arrays: pos [N][3] and rvecs [3][3] are read
+ * and *energy, gpos [N][3] and vtens [3][3] (the last two may be NULL) overwritten before the call
+ * returns; it waits for the stream. Calls on one field run one after the other. */
+int mm_field_compute_host(mm_field* f, const double* pos, const double* rvecs, double* energy,
+                          double* gpos, double* vtens, void* stream);
+
 /* mm_field_compute without any allocation, for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the
  * vertex-gradient records and block partials go to a static workspace of 64 MiB that every

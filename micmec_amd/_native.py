@@ -47,6 +47,7 @@ def _load():
     L.mm_field_create.argtypes = [ctypes.POINTER(P), ctypes.c_int, ctypes.c_int, i64, i64, P, P,
                                   P, P, i32, i32, P, P, P, P, P, f64]
     L.mm_field_compute.argtypes = [P, P, P, P, P, P, ctypes.c_int, P]
+    L.mm_field_compute_host.argtypes = [P, P, P, P, P, P, P]
     L.mm_field_check.argtypes = [P, P, ctypes.POINTER(i32)]
     L.mm_field_launch_cells.argtypes = [P, P, P, P]
     L.mm_cg_trial.argtypes = [P, P, P, P, f64, ctypes.c_int, f64, P, P, P, P, P, P]

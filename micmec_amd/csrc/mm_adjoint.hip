@@ -799,11 +799,11 @@ int mm_adjoint_compute(mm_adjoint* a, const double* pos, const double* dpos, con
       g.gpos = gpos;
       g.accumulate = 0;
       g.nanflag = f->nanflag;
-      e = launch_gather(g, s);
+      e = launch_gather(g, ReduceList{}, s);
       if (e == hipSuccess && dgpos) {
         g.gcell = a->gcell2;
         g.gpos = dgpos;
-        e = launch_gather(g, s);
+        e = launch_gather(g, ReduceList{}, s);
       }
     }
   } else {

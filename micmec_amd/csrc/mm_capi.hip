@@ -151,6 +151,8 @@ void free_field(mm_field* f) {
   (void)hipFree(f->partials);
   (void)hipFree(f->cgpart);
   if (f->cghost) (void)hipHostFree(f->cghost);
+  if (f->hostio) (void)hipHostFree(f->hostio);
+  (void)hipFree(f->hostin);
   (void)hipFree(f->nanflag);
   (void)hipFree(f->blk_sys);
   (void)hipFree(f->sys_cblk_ptr);
@@ -526,7 +528,7 @@ int mm_batch_compute(mm_field* f, const double* pos, const double* rvecs, double
   a.accumulate = 0;
   a.force_grad = 1;
   hipError_t e = launch_cells(a, (hipStream_t)stream);
-  if (e == hipSuccess && gpos) e = launch_gather(a, (hipStream_t)stream);
+  if (e == hipSuccess && gpos) e = launch_gather(a, ReduceList{}, (hipStream_t)stream);
   if (e == hipSuccess)
     e = launch_batch_finalize(f->partials, (int)(f->W / kCellBlock), f->sys_cblk_ptr,
                               f->sys_cblk_idx, f->nsys, energies, vtens, f->nanflag,
@@ -611,6 +613,53 @@ int mm_field_compute_static(mm_field* f, const double* pos, const double* rvecs,
   a.accumulate = accumulate;
   hipError_t e = launch_force(a, (hipStream_t)stream);
   if (e != hipSuccess) return hip_error(e, "force kernels");
+  return MM_OK;
+}
+
+// The kernels write the results straight into mapped pinned memory: no copy commands, and the
+// call waits once. A small field's kernel reads its inputs there too; a larger one's cells read
+// every position eight times, so a kernel takes the inputs to device memory first.
+int mm_field_compute_host(mm_field* f, const double* pos, const double* rvecs, double* energy,
+                          double* gpos, double* vtens, void* stream) {
+  if (!f) return set_error(MM_ERR_ARG, "field is NULL");
+  if (f->nsys != 1)
+    return set_error(MM_ERR_ARG, "mm_field_compute_host needs a single-system object");
+  if (!energy) return set_error(MM_ERR_ARG, "energy output is required");
+  if (f->N > 0 && !pos) return set_error(MM_ERR_ARG, "pos is NULL");
+  if (!rvecs) return set_error(MM_ERR_ARG, "rvecs is NULL");
+  DeviceGuard guard(f->device);
+  const std::lock_guard<std::mutex> lock(f->hostmu);
+  const hipStream_t s = (hipStream_t)stream;
+  const size_t np = 3 * (size_t)f->N, in = 9 + np;
+  const bool small = f->N <= kSmallForce && f->W <= kSmallForce;
+  hipError_t e = hipSuccess;
+  if (!f->hostio)
+    e = hipHostMalloc((void**)&f->hostio, (in + 10 + np) * sizeof(double), hipHostMallocDefault);
+  if (e == hipSuccess && !small && !f->hostin)
+    e = hipMalloc((void**)&f->hostin, in * sizeof(double));
+  if (e != hipSuccess) return hip_error(e, "staging of host arrays");
+  double* res = f->hostio + in;
+  std::memcpy(f->hostio, rvecs, 9 * sizeof(double));
+  if (np) std::memcpy(f->hostio + 9, pos, np * sizeof(double));
+  if (gpos && (f->W == 0 || f->N == 0)) std::memset(res + 10, 0, np * sizeof(double));
+  ForceArgs a;
+  const double* src = small ? f->hostio : f->hostin;
+  a.rvecs = src;
+  a.pos = src + 9;
+  field_args(f, a);
+  a.energy = res;
+  a.vtens = vtens ? res + 1 : nullptr;
+  a.gpos = gpos ? res + 10 : nullptr;
+  a.accumulate = 0;
+  if (!small) e = launch_stage(f->hostio, f->hostin, (int64_t)in, s);
+  if (e == hipSuccess) e = launch_force(a, s);
+  // also after an error: nothing queued may still use the staging when the next call fills it
+  const hipError_t done = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = done;
+  if (e != hipSuccess) return hip_error(e, "force kernels");
+  *energy = res[0];
+  if (vtens) std::memcpy(vtens, res + 1, 9 * sizeof(double));
+  if (gpos && np) std::memcpy(gpos, res + 10, np * sizeof(double));
   return MM_OK;
 }
 

@@ -42,9 +42,9 @@ namespace mm {
 // gradient too); the energies and virials of all three are the same bits. The latter two take the
 // node positions through the pending transforms xmat (and xmat2 first, when its flag is set) when
 // they are given: a barostat call whose position scaling is stored by a later node pass.
-// The single-state instance sweeps the corners (sweep_cell) in 166 VGPRs, three waves a SIMD (146
+// The single-state instance sweeps the corners (sweep_cell) in 168 VGPRs, three waves a SIMD (156
 // without the gradient); the multistate one keeps the stresses of all corners for the state sum
-// (219 VGPRs and 72 KB of LDS a block, two waves). The compiler's default scheduler is the one that
+// (239 VGPRs and 72 KB of LDS a block, two waves). The compiler's default scheduler is the one that
 // keeps both free of spills. HBM bounds the gradient pass: about 450 MB at 128^3 (20% two-state,
 // 5% empty) in 100 us, with 1000 / 1800 VALU instructions a wave (60 us of issue); the form
 // with B = P M per corner took 1735 / 4000 and 150 us, and 120 us for the pass without
@@ -157,23 +157,70 @@ __device__ __forceinline__ void block_sum_max_store(double (&v)[NS + NM], double
   }
 }
 
+// One block of 256 threads reduces an item's src[0..n) (sum in a fixed order, or a NaN-propagating
+// maximum) into dst[0] (added to it when acc). A NaN total sets the item's bit in nanflag.
+__device__ __forceinline__ void reduce_item(const ReduceItem it, int* __restrict__ nanflag) {
+  constexpr int kUnroll = 8;
+  __shared__ double red[4];
+  const bool is_max = it.op == kReduceMax;
+  const double zero = is_max ? -HUGE_VAL : 0.0;
+  double acc = zero;
+  for (int64_t base = threadIdx.x; base < it.n; base += 256 * kUnroll) {
+    double v[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int64_t i = base + (int64_t)u * 256;
+      v[u] = i < it.n ? it.src[i] : zero;
+    }
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) acc = is_max ? nan_max(acc, v[u]) : acc + v[u];
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const double o = __shfl_down(acc, off, 64);
+    acc = is_max ? nan_max(acc, o) : acc + o;
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 0) red[wave] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = red[0];
+    for (int w = 1; w < 4; ++w) t = is_max ? nan_max(t, red[w]) : t + red[w];
+    if (it.acc) t += it.dst[0];
+    it.dst[0] = t;
+    if (t != t && it.nanbit) atomicOr(nanflag, it.nanbit);
+  }
+}
+
+// One block per item.
+__global__ void __launch_bounds__(256)
+reduce_items_kernel(ReduceList list, int* __restrict__ nanflag) {
+  reduce_item(list.item[blockIdx.x], nanflag);
+}
+
 // gpos[n] (+)= sum_{k=0..7} gcell[k][:][w(n,k)] in fixed k order (mmff.py:303-318). A workgroup
 // owns 256 consecutive nodes; their 768 gpos values (and, with DOT, dir and gold values) move
 // between HBM and LDS in contiguous runs, and each thread takes its node's three from LDS. With
 // DOT (a line-search trial), also the workgroup partials of sum_n gpos_n . dir_n,
 // sum_n |gpos_n|^2, sum_n gpos_n . gold_n and max_n |gpos_n|^2 into dpart rows 0-3 (row stride =
-// workgroups).
+// workgroups). The launch's blocks from gb on reduce an item of the cell pass's partials each
+// (energy and virial), beside the gather: a launch less than a reduction behind it (72x80x96
+// 79.3 -> 75.0 us).
 template <bool DOT, bool kAllLoads>
 __global__ void __launch_bounds__(256)
 gather_kernel(const int32_t* __restrict__ ncell, const double* __restrict__ gcell, int64_t N,
               int64_t RS, double* __restrict__ gpos, int accumulate, int* __restrict__ nanflag,
               const double* __restrict__ dir, const double* __restrict__ gold,
-              double* __restrict__ dpart) {
+              double* __restrict__ dpart, int gb, ReduceList list) {
+  if (!DOT && (int)blockIdx.x >= gb) {
+    reduce_item(list.item[blockIdx.x - gb], nanflag);
+    return;
+  }
   __shared__ double sg[768];
   __shared__ double sd[DOT ? 768 : 1], so[DOT ? 768 : 1];
   const int t = threadIdx.x;
   // node blocks dealt to the XCDs in contiguous ranges: neighbouring blocks share record lines
-  const int blk = xcd_block((int)blockIdx.x, (int)gridDim.x);
+  const int blk = xcd_block((int)blockIdx.x, gb);
   const int64_t n0 = (int64_t)blk * 256, n = n0 + t;
   const int64_t e0 = 3 * n0;
   const int64_t ne = 3 * (N < n0 + 256 ? N - n0 : (int64_t)256);  // values of this workgroup
@@ -214,44 +261,7 @@ gather_kernel(const int32_t* __restrict__ ncell, const double* __restrict__ gcel
     const int li = r * 256 + t;
     if (li < ne) gpos[e0 + li] = sg[li];
   }
-  if (DOT) block_sum_max_store<3, 1>(acc, dpart + blk, gridDim.x);
-}
-
-// One block per item: item i reduces src[0..n) (sum in a fixed order, or a NaN-propagating
-// maximum) into dst[0] (added to it when acc). A NaN total sets the item's bit in nanflag.
-__global__ void __launch_bounds__(1024)
-reduce_items_kernel(ReduceList list, int* __restrict__ nanflag) {
-  constexpr int kUnroll = 8;
-  __shared__ double red[16];
-  const ReduceItem it = list.item[blockIdx.x];
-  const bool is_max = it.op == kReduceMax;
-  const double zero = is_max ? -HUGE_VAL : 0.0;
-  double acc = zero;
-  for (int64_t base = threadIdx.x; base < it.n; base += 1024 * kUnroll) {
-    double v[kUnroll];
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int64_t i = base + (int64_t)u * 1024;
-      v[u] = i < it.n ? it.src[i] : zero;
-    }
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) acc = is_max ? nan_max(acc, v[u]) : acc + v[u];
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const double o = __shfl_down(acc, off, 64);
-    acc = is_max ? nan_max(acc, o) : acc + o;
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) red[wave] = acc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double t = red[0];
-    for (int w = 1; w < 16; ++w) t = is_max ? nan_max(t, red[w]) : t + red[w];
-    if (it.acc) t += it.dst[0];
-    it.dst[0] = t;
-    if (t != t && it.nanbit) atomicOr(nanflag, it.nanbit);
-  }
+  if (DOT) block_sum_max_store<3, 1>(acc, dpart + blk, gb);
 }
 
 hipError_t launch_cells(const ForceArgs& a, hipStream_t stream) {
@@ -273,9 +283,12 @@ hipError_t launch_cells(const ForceArgs& a, hipStream_t stream) {
   // -> 47.8 / 109 -> 37.4 / 81.1 us (the last two with the gathers' all-loads form), at 48^3
   // (about 430 blocks) 59.2 / 138.7 -> 58.8 / 127.5 us, -> 53.8 / 117.5 us in one launch; at
   // 64^3 (about 1030 blocks) the fork is the faster (NVT 74.0 vs 76.4 us back to back), at
-  // 96^3 too (NPT 329 vs 343 us). The results are the same bits in every form.
+  // 96^3 too (NPT 329 vs 343 us). The averaged model's kernels are as short in either kind and
+  // the device holds twice as many: one launch whatever the size (61x64x67, 1022 blocks, whole
+  // evaluation 52.4 -> 29.1 us, with the totals in the gather's launch). The results are the same
+  // bits in every form.
   const bool fork = a.side != nullptr && a.ev_fork != nullptr && a.ev_join != nullptr &&
-                    mn > 0 && sn > 0 && nb > kForkMinBlocks;
+                    mn > 0 && sn > 0 && nb > kForkMinBlocks && a.model == 0;
   hipStream_t ms = fork ? a.side : stream;
   hipError_t e = hipSuccess;
   if (fork) {
@@ -298,7 +311,7 @@ hipError_t launch_cells(const ForceArgs& a, hipStream_t stream) {
   // place only as that drains (npt 128^3 step 0.580 -> 0.576 ms; equal at 72x80x96 with seven
   // of ten cells two-state).
   // a pass that the device holds at once, with blocks of both kinds: one launch
-  const bool both = mn > 0 && sn > 0 && nb <= kForkMinBlocks;
+  const bool both = mn > 0 && sn > 0 && (nb <= kForkMinBlocks || a.model != 0);
 #define MM_LAUNCH_BOTH(MODEL, OUT)                                                           \
   hipLaunchKernelGGL((cell_kernel_both<MODEL, OUT>), dim3(nb), dim3(kCellBlock), 0, stream,     \
                      a.pos, a.rvecs, a.rvecs_stride, a.blk_sys, a.cnode, a.cwrap,              \
@@ -332,39 +345,33 @@ hipError_t launch_cells(const ForceArgs& a, hipStream_t stream) {
   return e;
 }
 
-hipError_t launch_gather(const ForceArgs& a, hipStream_t stream) {
-  if (a.gpos == nullptr || a.N <= 0 || a.W <= 0) return hipSuccess;
+template <bool DOT>
+static hipError_t gather(const ForceArgs& a, const double* dir, const double* gold, double* dpart,
+                         const ReduceList& list, hipStream_t stream) {
+  if (a.gpos == nullptr || a.N <= 0 || a.W <= 0) return launch_reduce(list, a.nanflag, stream);
   const int gb = (int)((a.N + 255) / 256);
+  const dim3 grid(gb + list.count);
   if (gb <= kGatherAllLoadsMaxBlocks)
-    hipLaunchKernelGGL((gather_kernel<false, true>), dim3(gb), dim3(256), 0, stream, a.ncell,
-                       a.gcell, a.N, a.rstride, a.gpos, a.accumulate, a.nanflag,
-                       nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL((gather_kernel<DOT, true>), grid, dim3(256), 0, stream, a.ncell, a.gcell,
+                       a.N, a.rstride, a.gpos, a.accumulate, a.nanflag, dir, gold, dpart, gb, list);
   else
-    hipLaunchKernelGGL((gather_kernel<false, false>), dim3(gb), dim3(256), 0, stream, a.ncell,
-                       a.gcell, a.N, a.rstride, a.gpos, a.accumulate, a.nanflag,
-                       nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL((gather_kernel<DOT, false>), grid, dim3(256), 0, stream, a.ncell, a.gcell,
+                       a.N, a.rstride, a.gpos, a.accumulate, a.nanflag, dir, gold, dpart, gb, list);
   return hipGetLastError();
+}
+
+hipError_t launch_gather(const ForceArgs& a, const ReduceList& list, hipStream_t stream) {
+  return gather<false>(a, nullptr, nullptr, nullptr, list, stream);
 }
 
 hipError_t launch_gather_dot(const ForceArgs& a, const double* dir, const double* gold,
                              double* dpart, hipStream_t stream) {
-  if (a.gpos == nullptr || a.N <= 0 || a.W <= 0) return hipSuccess;
-  const int gb = (int)((a.N + 255) / 256);
-  if (gb <= kGatherAllLoadsMaxBlocks)
-    hipLaunchKernelGGL((gather_kernel<true, true>), dim3(gb), dim3(256), 0, stream, a.ncell,
-                       a.gcell, a.N, a.rstride, a.gpos, a.accumulate, a.nanflag, dir,
-                       gold, dpart);
-  else
-    hipLaunchKernelGGL((gather_kernel<true, false>), dim3(gb), dim3(256), 0, stream, a.ncell,
-                       a.gcell, a.N, a.rstride, a.gpos, a.accumulate, a.nanflag, dir,
-                       gold, dpart);
-  return hipGetLastError();
+  return gather<true>(a, dir, gold, dpart, ReduceList{}, stream);
 }
 
 hipError_t launch_reduce(const ReduceList& list, int* nanflag, hipStream_t stream) {
   if (list.count <= 0) return hipSuccess;
-  hipLaunchKernelGGL(reduce_items_kernel, dim3(list.count), dim3(1024), 0, stream, list,
-                     nanflag);
+  hipLaunchKernelGGL(reduce_items_kernel, dim3(list.count), dim3(256), 0, stream, list, nanflag);
   return hipGetLastError();
 }
 
@@ -375,15 +382,161 @@ void add_force_totals(ReduceList& list, const ForceArgs& a, int nb) {
       list.add(a.partials + (int64_t)(1 + q) * nb, nb, kReduceSum, a.vtens + q, a.accumulate, 4);
 }
 
+// One force evaluation in one launch by one workgroup, for a field of at most kSmallForce work
+// slots and nodes: three launches (cells, gather, totals) and the trips to memory between them take
+// longer than its arithmetic. Thread t owns slot t and node t; positions, stresses or vertex
+// records and the wave sums stay in LDS (a slot's column holds its multistate sums, then its
+// records: lower faces in rows 0..11, upper in 12..23). pos, rvecs and the outputs may be host
+// memory that the device maps: every word of it is read and written once, side by side. Same
+// arithmetic and order of sums as the separate kernels, so the same bits. The limit is what LDS
+// holds: 36 columns of 512 sums are 144 of its 160 KB. 5^3 cells from host arrays, whole plugin
+// call: 111 us with three launches and five waiting copies, 44 us so (some 20 us of it Python).
+struct ForceSmallArgs {
+  const double *pos, *rvecs;
+  const int32_t *cnode, *cwrap, *blk_row, *nstates, *nrec, *cbase;
+  const double *tab, *kt;
+  int32_t max_states;
+  int W, N;
+  double *energy, *gpos, *vtens;
+  int accumulate;
+  int* nanflag;
+};
+
+template <int kModel, int kOut>
+__global__ void __launch_bounds__(kSmallForce, 2) force_small_kernel(ForceSmallArgs a) {
+  using F = Frame<kModel>;
+  constexpr int NS = F::NE + 3 * F::NC;
+  constexpr int NR = NS > 24 ? NS : 24;
+  constexpr int kWaves = kSmallForce / 64;
+  __shared__ double col[NR * kSmallForce];
+  __shared__ double xs[3 * kSmallForce];
+  __shared__ double rvs[9];
+  __shared__ double red[7 * kWaves];  // zero where no wave writes
+  unsigned short* top_slot = reinterpret_cast<unsigned short*>(col);  // before the cells only
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  for (int i = t; i < 3 * a.N; i += blockDim.x) xs[i] = a.pos[i];
+  if (t < 9) rvs[t] = a.rvecs[t];
+  if (t < 7 * kWaves) red[t] = 0.0;
+  const bool has_slot = 64 * wave < a.W;  // W is a multiple of the block size
+  int n[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) n[k] = has_slot ? a.cnode[8 * t + k] : -1;
+  const bool valid = n[0] >= 0;
+  const int wrap = valid ? a.cwrap[t] : 0;
+  const int trow = has_slot ? ((const_i32)a.blk_row)[wave >> 2] : 0;
+  const int ns = ((const_i32)a.nstates)[trow];
+  const double kt = ((const_f64)a.kt)[trow];
+  const const_f64 tab = (const_f64)a.tab + (int64_t)trow * a.max_states * kTabStride;
+  {
+    const bool open_top = valid && !(wrap & 16);
+    const uint64_t tops = __ballot(open_top);
+    if (open_top) top_slot[((const_i32)a.cbase)[wave] + __popcll(tops & ((1ull << lane) - 1ull))] = t;
+  }
+  __syncthreads();
+  // the node's records as places in col, -1 for none
+  const bool own = kOut == kOutGradient && t < a.N;
+  int place[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int e = own ? a.nrec[k * a.N + t] : -1;
+    const int slot = e >> 2, row = 3 * (e & 3);
+    place[k] = e < 0 ? -1
+                     : slot < a.W ? row * kSmallForce + slot
+                                  : (12 + row) * kSmallForce + top_slot[slot - a.W];
+  }
+  __syncthreads();
+  if (has_slot) {
+    double rv[9];
+#pragma unroll
+    for (int q = 0; q < 9; ++q) rv[q] = rvs[q];
+    double ecell, vir[6], gacc[8][3];
+    auto corners = [&](double (&p)[8][3]) {
+      load_corners(xs, n, p, false, nullptr, false, nullptr);
+    };
+    if (ns > 1)
+      cell_eval<kModel, kOut, true, kSmallForce>(tab, ns, kt, valid, corners, wrap, rv, col + t,
+                                                 ecell, vir, gacc);
+    else
+      cell_eval<kModel, kOut, false, kSmallForce>(tab, ns, kt, valid, corners, wrap, rv, col + t,
+                                                  ecell, vir, gacc);
+    if (kOut == kOutGradient) {
+      fold_cell(wrap, gacc);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          col[(3 * q + j) * kSmallForce + t] = gacc[kLowerCorner[q]][j];
+          col[(12 + 3 * q + j) * kSmallForce + t] = gacc[kUpperCorner[q]][j];
+        }
+    }
+    cell_wave_totals(ecell, vir, red + 7 * wave);
+  }
+  __syncthreads();
+  if (t < 10) {
+    // the totals of the slots' blocks, in block order
+    double s = cell_block_total(red, t);
+    for (int b = 1; b < a.W / kCellBlock; ++b)
+      s += cell_block_total(red + 7 * b * (kCellBlock / 64), t);
+    double* dst = t == 0 ? a.energy : a.vtens ? a.vtens + (t - 1) : nullptr;
+    if (dst) {
+      if (a.accumulate) s += *dst;
+      *dst = s;
+      if (s != s) atomicOr(a.nanflag, t == 0 ? 1 : 4);
+    }
+  }
+  if (own) {
+    double g[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int j = 0; j < 3; ++j)
+        if (place[k] >= 0) g[j] += col[place[k] + j * kSmallForce];
+    if (g[0] != g[0] || g[1] != g[1] || g[2] != g[2]) atomicOr(a.nanflag, 2);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      double* dst = a.gpos + 3 * t + j;
+      *dst = a.accumulate ? *dst + g[j] : g[j];
+    }
+  }
+}
+
+static hipError_t launch_force_small(const ForceArgs& a, hipStream_t stream) {
+  const ForceSmallArgs s{a.pos, a.rvecs, a.cnode, a.cwrap, a.blk_row, a.nstates, a.ncell,
+                         a.cbase, a.tab, a.kt, a.max_states, (int)a.W, (int)a.N, a.energy,
+                         a.gpos, a.vtens, a.accumulate, a.nanflag};
+  const dim3 block(a.W > kSmallForce / 2 || a.N > kSmallForce / 2 ? kSmallForce : kSmallForce / 2);
+#define MM_SMALL(M, O) hipLaunchKernelGGL((force_small_kernel<M, O>), dim3(1), block, 0, stream, s)
+  if (a.model == 0) {
+    if (a.gpos) MM_SMALL(0, kOutGradient); else MM_SMALL(0, kOutVirial);
+  } else {
+    if (a.gpos) MM_SMALL(1, kOutGradient); else MM_SMALL(1, kOutVirial);
+  }
+#undef MM_SMALL
+  return hipGetLastError();
+}
+
 hipError_t launch_force(const ForceArgs& a, hipStream_t stream) {
-  const int nb = (int)(a.W / kCellBlock);
+  if (a.energy && a.N > 0 && a.N <= kSmallForce && a.W > 0 && a.W <= kSmallForce)
+    return launch_force_small(a, stream);
   hipError_t err = launch_cells(a, stream);
   if (err != hipSuccess) return err;
-  err = launch_gather(a, stream);
-  if (err != hipSuccess) return err;
   ReduceList list;
-  add_force_totals(list, a, nb);
-  return launch_reduce(list, a.nanflag, stream);
+  add_force_totals(list, a, (int)(a.W / kCellBlock));
+  return launch_gather(a, list, stream);
+}
+
+// Inputs of a host call from mapped host memory into device buffers.
+__global__ void __launch_bounds__(256)
+stage_kernel(const double* __restrict__ src, double* __restrict__ dst, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) dst[i] = src[i];
+}
+
+hipError_t launch_stage(const double* src, double* dst, int64_t n, hipStream_t stream) {
+  if (n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(stage_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, src,
+                     dst, n);
+  return hipGetLastError();
 }
 
 // Trial point of a line search over 256 nodes a workgroup: optionally d <- beta d - g first,

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <vector>
 
 namespace mm {
@@ -38,6 +39,11 @@ struct mm_field {
   double* partials = nullptr;
   double* cgpart = nullptr;           // [8][(N + 255) / 256] node-block partials (mm_cg_*)
   double* cghost = nullptr;           // [8] pinned host staging of mm_cg_* results
+  // mm_field_compute_host, made on its first call: pinned staging [9 + 3 N] in, [10 + 3 N] out, and
+  // the inputs on the device (larger fields only); one call at a time
+  double* hostio = nullptr;
+  double* hostin = nullptr;
+  std::mutex hostmu;
   int* nanflag = nullptr;
   int32_t nsys = 1;                   // independent systems sharing the object
   int32_t* blk_sys = nullptr;         // [W/256] system of every cell block

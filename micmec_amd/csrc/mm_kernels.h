@@ -7,7 +7,8 @@
 namespace mm {
 
 constexpr int kCellBlock = 256;
-// Cell passes of more blocks than this run their two instances concurrently; smaller ones run
+// Cell passes of the eight-corner model of more blocks than this run their two instances
+// concurrently; smaller ones, and all of the averaged model, run
 // both kinds of block in one launch (cell_kernel_both).
 constexpr int kForkMinBlocks = 512;
 // Node gathers over at most this many 256-node blocks (at most four waves a SIMD) load all of
@@ -17,6 +18,9 @@ constexpr int kForkMinBlocks = 512;
 // extra registers cost more than the loads in flight gain (80^3 NPT 223 -> 234 us, 128^3
 // 650 -> 666 us). The same bits either way.
 constexpr int kGatherAllLoadsMaxBlocks = 1024;
+// Single-system fields of at most this many work slots and nodes are evaluated in one launch by
+// one workgroup (force_small_kernel).
+constexpr int kSmallForce = 512;
 constexpr int kPartialStride = 16;
 constexpr int kMaxStates = 8;  // metastable states per cell type
 
@@ -110,8 +114,11 @@ hipError_t launch_cg_stats(const double* x, const double* xo, const double* g, c
 hipError_t launch_batch_finalize(const double* partials, int nb, const int32_t* sys_ptr,
                                  const int32_t* sys_idx, int nsys, double* energies,
                                  double* vtens, int* nanflag, hipStream_t stream);
-// Node gather of gcell into gpos (overwrite or accumulate, as a.accumulate).
-hipError_t launch_gather(const ForceArgs& a, hipStream_t stream);
+// Node gather of gcell into gpos (overwrite or accumulate, as a.accumulate), with the reductions of
+// list (of what earlier launches wrote) in the same launch.
+hipError_t launch_gather(const ForceArgs& a, const ReduceList& list, hipStream_t stream);
+// dst[0..n) = src[0..n), src mapped host memory.
+hipError_t launch_stage(const double* src, double* dst, int64_t n, hipStream_t stream);
 // Cell kernel only: per-cell gradients into gcell, energy/virial block partials.
 hipError_t launch_cells(const ForceArgs& a, hipStream_t stream);
 

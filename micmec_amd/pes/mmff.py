@@ -28,6 +28,10 @@ from ..topology import Grid, periodic_wrap_bits
 __all__ = ["ForcePart", "MicMecForceField", "ForcePartMechanical", "ForcePartPressure",
            "parse_type_params"]
 
+# Host arrays of at most this many nodes go through the library's own pinned staging (48 bytes a
+# node, kept with the field); larger ones through tensors, where the transfers dominate.
+HOST_MAX_NODES = 32768
+
 
 def _is_torch(x):
     return isinstance(x, torch.Tensor)
@@ -260,6 +264,18 @@ class DeviceField(object):
                                         _native.stream_ptr(stream))
         _native.check(rc, "mm_field_compute")
 
+    def compute_host(self, pos, rvecs, gpos=None, vtens=None):
+        """Energy at host arrays ``pos`` [N, 3] and ``rvecs`` [3, 3], on the current stream; ``gpos``
+        [N, 3] and ``vtens`` [3, 3] are overwritten. C-contiguous float64 arrays throughout."""
+        energy = ctypes.c_double(0.0)
+        at = lambda a: None if a is None else a.ctypes.data
+        stream = torch.cuda.current_stream(self.device)
+        rc = self._lib.mm_field_compute_host(self._handle, at(pos), at(rvecs),
+                                             ctypes.byref(energy), at(gpos), at(vtens),
+                                             _native.stream_ptr(stream))
+        _native.check(rc, "mm_field_compute_host")
+        return energy.value
+
     def cg_trial(self, x, g, d, beta, set_dir, alpha, rvecs, xa, ga, out, host_out=None,
                  stream=None):
         """One line-search trial: with ``set_dir`` first d <- beta d - g, then xa <- x + alpha d,
@@ -353,6 +369,7 @@ class ForcePartMechanical(ForcePart):
         self._vtens_d = torch.zeros((3, 3), **kw)
         self._energy_d = torch.zeros(1, **kw)
         self._rvecs_d = torch.zeros((3, 3), **kw)
+        self._rvecs_last = np.zeros((3, 3))  # what it holds
 
     @staticmethod
     def get_pbc(rvecs):
@@ -363,16 +380,32 @@ class ForcePartMechanical(ForcePart):
                              "systems, not %iD periodic systems." % nper)
         return pbc
 
-    def rvecs_device(self, rvecs=None):
+    def _rvecs_host(self, rvecs=None):
         rv = np.zeros((3, 3))
         r = np.asarray(self.system.domain.rvecs if rvecs is None else rvecs, dtype=np.float64)
         if r.size:
             rv[: len(r)] = r
+        return rv
+
+    def rvecs_device(self, rvecs=None):
+        rv = self._rvecs_host(rvecs)
         self._rvecs_d.copy_(torch.from_numpy(rv))
+        self._rvecs_last = rv
         return self._rvecs_d
 
     def _internal_compute(self, gpos, vtens):
         pos = self.system.pos
+        plain = lambda a, shape: isinstance(a, np.ndarray) and a.dtype == np.float64 and \
+            a.flags.c_contiguous and a.shape == shape
+        N = len(self._pos_d)
+        if N <= HOST_MAX_NODES and plain(pos, (N, 3)) and \
+                (gpos is None or plain(gpos, (N, 3)) and gpos.flags.writeable) and \
+                (vtens is None or plain(vtens, (3, 3)) and vtens.flags.writeable):
+            # one library call with one wait; copies through tensors wait five times
+            rv = self._rvecs_host()
+            if not np.array_equal(rv, self._rvecs_last):
+                self.rvecs_device()  # whoever holds the device copy sees the current domain
+            return self.field.compute_host(pos, rv, gpos, vtens)
         if _is_torch(pos):
             pos_d = pos.to(device=self.device, dtype=torch.float64).contiguous()
         else:
