@@ -173,7 +173,7 @@ int mm_field_set_params_device(mm_field* f, const int32_t* nstates, const double
  * with the automatic derivatives of micmec/pes/mmff_jax.py:249-250.
  *
  * mm_adjoint_create allocates the work buffers of an object (about (2 * npar + 38) / 32 + 24
- * doubles per work slot, and 9 per node) and returns npar = max_states * 32 + 1, the parameter
+ * doubles per work slot, and 3 per node) and returns npar = max_states * 32 + 1, the parameter
  * entries per row.
  *
  * mm_adjoint_compute evaluates, at positions pos [nnodes][3] and domain vectors rvecs [nsys][9]:
@@ -204,8 +204,8 @@ int mm_adjoint_compute(mm_adjoint* a, const double* pos, const double* dpos, con
  * and params as for mm_adjoint_compute (the position-independent rest of the product is
  * small: dL/drvecs = gE dE/drvecs + d(dE/drvecs) + (dE/drvecs) gV and dL/dtheta = the sum of
  * the value and tangent rows of params). node_sys [nnodes] int32 gives each node's system.
- * Uses work buffers of the object (9 nnodes + 9 nsys doubles, made by mm_adjoint_create). No
- * reference counterpart (differentiation form). */
+ * Uses work buffers of the object (made by mm_adjoint_create). No reference counterpart
+ * (differentiation form). */
 int mm_adjoint_vjp(mm_adjoint* a, const double* pos, const double* rvecs,
                    const int32_t* node_sys, const double* gE, const double* gG, const double* gV,
                    double* sys_out, double* g_pos, double* params, void* stream);
@@ -222,6 +222,31 @@ int mm_adjoint_vjp(mm_adjoint* a, const double* pos, const double* rvecs,
 int mm_adjoint_param_grads(mm_adjoint* a, const double* entries, int64_t stride, int add_next,
                            const double* h0, double boltzmann, double* g_cv, double* g_h0,
                            double* g_free, double* g_teff, void* stream);
+
+/* The product above in full: mm_adjoint_vjp with the small rest formed on the device too. Outputs,
+ * each overwritten: g_pos [nnodes][3] and g_rv [nsys][9] (either may be NULL: not formed), and,
+ * all or none, g_cv, g_h0, g_free and g_teff as mm_adjoint_param_grads gives them for the sum of
+ * values and tangents. No reference counterpart (differentiation form). */
+int mm_adjoint_backward(mm_adjoint* a, const double* pos, const double* rvecs,
+                        const int32_t* node_sys, const double* gE, const double* gG,
+                        const double* gV, const double* h0, double boltzmann, double* g_pos,
+                        double* g_rv, double* g_cv, double* g_h0, double* g_free, double* g_teff,
+                        void* stream);
+
+/* Force-and-stress matching loss
+ *   *loss = mean((g - g_target)^2) / f_scale + mean((v inv_volume - v_target)^2) / s_scale
+ * over node gradients g [nnodes][3] and virials v [nsys][9] with inv_volume [nsys], and the
+ * backward pass of mm_adjoint_backward for its cotangents scaled by *gl (gE: zeros [nsys]). Device
+ * pointers. No reference counterpart (differentiation form). */
+int mm_fit_loss(mm_adjoint* a, const double* g, const double* g_target, const double* v,
+                const double* v_target, const double* inv_volume, double f_scale, double s_scale,
+                double* loss, void* stream);
+int mm_fit_backward(mm_adjoint* a, const double* pos, const double* rvecs,
+                    const int32_t* node_sys, const double* gE, const double* g,
+                    const double* g_target, const double* v, const double* v_target,
+                    const double* inv_volume, double f_scale, double s_scale, const double* gl,
+                    const double* h0, double boltzmann, double* g_pos, double* g_rv, double* g_cv,
+                    double* g_h0, double* g_free, double* g_teff, void* stream);
 void mm_adjoint_destroy(mm_adjoint* a);
 
 /* ------------------------------------------------------------------------------------------

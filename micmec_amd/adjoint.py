@@ -18,10 +18,10 @@ outputs back-propagates to ``pos``, ``rvecs`` and the parameter tensors
 The energy model is the reference's (micmec/pes/nanocell.py:40-132, nanocell_original.py:46-132,
 micmec/pes/mmff.py:380-398); the reference itself differentiates only with respect to positions
 (mmff.py:384-398) and, in mmff_jax.py:249-250, a deformation of the domain. The forward pass is
-the plain force path (``mm_batch_compute``); the backward pass is one ``mm_adjoint_vjp`` call:
-the tangent direction below, one launch of the hand-written adjoint kernel in dual numbers
-(``mm_adjoint_compute``), which recomputes everything from the positions (no per-corner
-intermediate is stored between the passes), and the position cotangent.
+the plain force path (``mm_batch_compute``); the backward pass is one ``mm_adjoint_backward`` call:
+the tangent direction below, one launch of the hand-written adjoint kernel in dual numbers, which
+recomputes everything from the positions (no per-corner intermediate is stored between the
+passes), and the cotangents of the inputs that need one.
 
 Backward, for cotangents (gE, gG, gV) of (E, gpos, vtens): with the tangent direction
 u = (dpos, drvecs) = (gG + pos gV^T, rvecs gV^T) the kernel returns the values (gpos, dE/drvecs,
@@ -34,7 +34,7 @@ dE/dtheta) and their derivatives along u; then
 (the last terms of the first two lines come from vtens = sum_v g_v (x) r_v, whose derivative
 along a deformation D is the derivative of E along (pos D, rvecs D)). The parameter entries of
 the kernel (derivatives with respect to Cv, P = h0^-1, the weight w = det(h0)/8 or det(h0), the
-free energies and kT) are mapped here to (cv, h0, free, teff).
+free energies and kT) are mapped to (cv, h0, free, teff) on the device.
 """
 
 import ctypes
@@ -62,6 +62,10 @@ _native.register_signature("mm_adjoint_compute", [_P, _P, _P, _P, _P, _P, _P, _P
 _native.register_signature("mm_adjoint_vjp", [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P])
 _native.register_signature("mm_adjoint_param_grads",
                            [_P, _P, _i64, ctypes.c_int, _P, _f64, _P, _P, _P, _P, _P])
+_native.register_signature("mm_adjoint_backward", [_P] * 8 + [_f64] + [_P] * 7)
+_native.register_signature("mm_fit_loss", [_P] * 6 + [_f64, _f64, _P, _P])
+_native.register_signature("mm_fit_backward",
+                           [_P] * 10 + [_f64, _f64, _P, _P, _f64] + [_P] * 7)
 
 NPS = 32       # parameter entries per (type, state) of the adjoint kernel
 SYSQ = 19      # energy, virial (9), domain-vector gradient (9)
@@ -175,6 +179,7 @@ class DiffField(object):
         self.node_sys = torch.tensor(np.repeat(np.arange(self.nsys), counts), dtype=torch.long,
                                      device=self.device)
         self._node_sys32 = self.node_sys.to(torch.int32)
+        self._no_weight = torch.zeros(self.nsys, dtype=torch.float64, device=self.device)
 
     # ------------------------------------------------------------------ inputs
     def positions(self):
@@ -313,9 +318,7 @@ class DiffField(object):
                 ent.numel() != T * self.npar * (2 if add_next else 1):
             raise ValueError("entries must be float64 [%d, %d%s] on %s"
                              % (T, self.npar, ", 2" if add_next else "", self.device))
-        h0 = params.h0.detach().to(**kw).contiguous()
-        if h0.shape != (T, S, 3, 3):
-            raise ValueError("h0 must be [%d, %d, 3, 3]" % (T, S))
+        h0 = self._rest_cells(params)
         g_cv = torch.empty((T, S, 6, 6), **kw)
         g_h0 = torch.empty((T, S, 3, 3), **kw)
         g_free = torch.empty((T, S), **kw)
@@ -326,6 +329,25 @@ class DiffField(object):
             _native.ptr(g_free), _native.ptr(g_teff), _native.stream_ptr())
         _native.check(rc, "mm_adjoint_param_grads")
         return g_cv, g_h0, g_free, g_teff
+
+    def _rest_cells(self, params):
+        h0 = params.h0.detach().to(dtype=torch.float64, device=self.device).contiguous()
+        if h0.shape != (self.nrows, self.max_states, 3, 3):
+            raise ValueError("h0 must be [%d, %d, 3, 3]" % (self.nrows, self.max_states))
+        return h0
+
+    def _backward(self, needs, params, call):
+        """Cotangents (pos, rvecs, cv, h0, free, teff) of which ``needs`` says what is wanted (None
+        for the others): ``call(h0, outputs)`` is the library call, with raw pointers."""
+        self.set_params(params)
+        T, S = self.nrows, self.max_states
+        kw = dict(dtype=torch.float64, device=self.device)
+        want = list(needs[:2]) + [any(needs[2:])] * 4
+        shapes = [(self.N, 3), (self.nsys, 3, 3), (T, S, 6, 6), (T, S, 3, 3), (T, S), (T,)]
+        out = [torch.empty(s, **kw) if w else None for s, w in zip(shapes, want)]
+        h0 = self._rest_cells(params) if want[2] else None
+        call(_native.ptr(h0), [_native.ptr(t) for t in out])
+        return out
 
     def __del__(self):
         lib = getattr(self, "lib", None)
@@ -354,29 +376,74 @@ class _MicMecEnergy(torch.autograd.Function):
         ctx.field = field
         ctx.params = params
         ctx.rv_shape = rvecs.shape
+        ctx.set_materialize_grads(False)  # an output without a cotangent: none, not zeros
         ctx.save_for_backward(pos_c, rv_c)
         return e, g, v
 
     @staticmethod
     @once_differentiable
     def backward(ctx, gE, gG, gV):
-        field, params = ctx.field, ctx.params
+        field = ctx.field
         pos, rv = ctx.saved_tensors
-        kw = dict(dtype=torch.float64, device=pos.device)
-        gE = torch.zeros(field.nsys, **kw) if gE is None else gE.contiguous()
+        # contiguous float64 on the field's device, as autograd hands them on
+        gE = field._no_weight if gE is None else gE.contiguous()
+        gG = None if gG is None else gG.contiguous()
+        gV = None if gV is None else gV.contiguous()
+        P = _native.ptr
+
+        def call(h0, out):
+            rc = field.lib.mm_adjoint_backward(field._adj, P(pos), P(rv), P(field._node_sys32),
+                                               P(gE), P(gG), P(gV), h0, float(units.boltzmann),
+                                               *out, _native.stream_ptr())
+            _native.check(rc, "mm_adjoint_backward")
+        out = field._backward(ctx.needs_input_grad[2:], ctx.params, call)
+        if out[1] is not None:
+            out[1] = out[1].reshape(ctx.rv_shape)
+        return (None, None, *out)
+
+
+class _FitLoss(torch.autograd.Function):
+    """The loss of a ``FitProblem``: the force pass and the loss in two more kernels; backward, the
+    loss' cotangents are formed by the kernel that uses them."""
+
+    @staticmethod
+    def forward(ctx, problem, params, pos, rvecs, cv, h0, free, teff):
+        field = problem.field
         field.set_params(params)
-        # one library call: direction (gG + pos gV^T, rvecs gV^T), the dual-number adjoint along
-        # it with energy weights gE, and the position cotangent gE gpos + d(gpos) + gpos gV
-        out = field.vjp(pos, rv, gE, None if gG is None else gG.contiguous(),
-                        None if gV is None else gV.contiguous().reshape(-1, 3, 3))
-        g_pos = out["g_pos"]
-        grv = out["grvecs"]
-        g_rv = gE[:, None, None] * grv + out["dgrvecs"]
-        if gV is not None:
-            gV = gV.contiguous().reshape(-1, 3, 3)
-            g_rv = g_rv + (grv.unsqueeze(3) * gV.unsqueeze(1)).sum(2)
-        g_cv, g_h0, g_free, g_teff = field.param_grads(out["raw_params"], params, add_next=True)
-        return (None, None, g_pos, g_rv.reshape(ctx.rv_shape), g_cv, g_h0, g_free, g_teff)
+        pos_c = pos.detach().contiguous()
+        rv_c = rvecs.detach().reshape(field.nsys, 3, 3).contiguous()
+        _, g, v = field.compute(pos_c, rv_c)
+        loss = torch.empty((), dtype=torch.float64, device=field.device)
+        targets = (problem._g_target, problem._vv_target, problem._inv_volume)
+        scales = (float(problem.f_scale), float(problem.s_scale))
+        P = _native.ptr
+        gt, vt, inv = targets
+        rc = field.lib.mm_fit_loss(field._adj, P(g), P(gt), P(v), P(vt), P(inv), *scales, P(loss),
+                                   _native.stream_ptr())
+        _native.check(rc, "mm_fit_loss")
+        ctx.field, ctx.params, ctx.scales = field, params, scales
+        ctx.rv_shape = rvecs.shape
+        ctx.save_for_backward(pos_c, rv_c, g, v, *targets)
+        return loss
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, gl):
+        field = ctx.field
+        pos, rv, g, v, gt, vt, inv = ctx.saved_tensors
+        gl = gl.contiguous()
+        P = _native.ptr
+
+        def call(h0, out):
+            rc = field.lib.mm_fit_backward(field._adj, P(pos), P(rv), P(field._node_sys32),
+                                           P(field._no_weight), P(g), P(gt), P(v), P(vt), P(inv),
+                                           *ctx.scales, P(gl), h0, float(units.boltzmann), *out,
+                                           _native.stream_ptr())
+            _native.check(rc, "mm_fit_backward")
+        out = field._backward(ctx.needs_input_grad[2:], ctx.params, call)
+        if out[1] is not None:
+            out[1] = out[1].reshape(ctx.rv_shape)
+        return (None, None, *out)
 
 
 def micmec_energy(field, pos, rvecs, params):
@@ -404,16 +471,13 @@ class FitProblem(object):
         self.f_scale = float((self.f_target ** 2).mean())
         self.s_scale = float((self.s_target ** 2).mean())
         # the same squared errors with the signs folded into the targets: mean((g - gt)^2)
-        # and mean((v / V - vt / V)^2), each one fused kernel forward and backward
+        # and mean((v / V - vt / V)^2)
         self._g_target = g.contiguous()
         self._vv_target = (v / self.volume[:, None, None]).contiguous()
         self._inv_volume = (1.0 / self.volume)[:, None, None].contiguous()
 
     def loss(self, params):
-        e, g, v = micmec_energy(self.field, self.pos, self.rvecs, params)
-        lf = torch.nn.functional.mse_loss(g, self._g_target) / self.f_scale
-        ls = torch.nn.functional.mse_loss(v * self._inv_volume, self._vv_target) / self.s_scale
-        return lf + ls
+        return _FitLoss.apply(self, params, self.pos, self.rvecs, *params.tensors())
 
 
 def fit_workload(count=64, n=16, seed=3, c_noise=0.10, device=None, model="corner8"):

@@ -39,6 +39,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "../../include/micmec_amd.h"
@@ -436,6 +437,7 @@ adjoint_kernel(const double* __restrict__ pos, const double* __restrict__ dpos,
         out[(int64_t)row * nblk] = t;
         if (q >= 4 && q < 7) out[(int64_t)((int)(0x478ull >> (4 * (q - 4))) & 0xf) * nblk] = t;
       });
+  if (!gcell) return;  // no position gradient wanted
   double gv[8][3];
 #pragma unroll
   for (int v = 0; v < 8; ++v)
@@ -451,18 +453,68 @@ adjoint_kernel(const double* __restrict__ pos, const double* __restrict__ dpos,
   }
 }
 
+// Where the gradients of the parameter tensors go (mm_adjoint_param_grads; cv null: not wanted).
+struct GradOut {
+  const double* h0;
+  int corner8;
+  double boltzmann;
+  double *cv, *h, *free, *teff;
+};
+
+// Gradients of (Cv, h0, free energy) of (row, state) t from its 32 entries ent (LDS), by one wave:
+// the 21 upper-triangle entries give the symmetric Voigt gradient, P^T = cof / det with the rows
+// r1 x r2, r2 x r0, r0 x r1 of cof, dE/dh0 = -P^T (dE/dP) P^T + (dE/dw) w P^T with w = det / 8
+// (corner8) or det, an entry a lane; zeros for a state that the row does not have (!on).
+__device__ __forceinline__ void state_gradients(const double* ent, bool on, int64_t t,
+                                                const GradOut& o) {
+  const int lane = threadIdx.x;
+  if (lane < 36) {
+    const int I = lane / 6, J = lane % 6, a = I < J ? I : J, b = I < J ? J : I;
+    o.cv[t * 36 + lane] = on ? ent[6 * a - a * (a - 1) / 2 + b - a] : 0.0;
+  }
+  if (lane < 9) {
+    const double* h = o.h0 + t * 9;
+    const int i = lane / 3, j = lane % 3;
+    double pt[9], m1[3];
+    for (int a = 0; a < 3; ++a) {
+      const double* u = h + 3 * ((a + 1) % 3);
+      const double* v = h + 3 * ((a + 2) % 3);
+      pt[3 * a + 0] = u[1] * v[2] - u[2] * v[1];
+      pt[3 * a + 1] = u[2] * v[0] - u[0] * v[2];
+      pt[3 * a + 2] = u[0] * v[1] - u[1] * v[0];
+    }
+    const double det = (h[0] * pt[0] + h[1] * pt[1]) + h[2] * pt[2];
+    for (int k = 0; k < 9; ++k) pt[k] = pt[k] / det;
+    const double p0 = pt[3 * i], p1 = pt[3 * i + 1], p2 = pt[3 * i + 2];
+    for (int k = 0; k < 3; ++k) m1[k] = (p0 * ent[21 + k] + p1 * ent[24 + k]) + p2 * ent[27 + k];
+    const double m2 = (m1[0] * pt[j] + m1[1] * pt[3 + j]) + m1[2] * pt[6 + j];
+    const double w = o.corner8 ? det / 8.0 : det;
+    o.h[t * 9 + lane] = on ? -m2 + ent[30] * w * pt[3 * i + j] : 0.0;
+  }
+  if (lane == 0) o.free[t] = on ? ent[31] : 0.0;
+}
+
 // The 32 parameter entries of every (row, state) from its metric sums, in place in params
 // [nrows][npar][2]: with T the map of x to the engineering strain e = T x (metric_entry),
 // X2 = sum p x x^T and X1 = sum p x, S = Cv T x the stress and G = 2 x + R the Gram matrix,
 //   dE/dCv = w T X2 T^T / 2,  dE/dP_ik = w sum_mn P_mn (sum p S_im G_nk),
 //   dE/dw = tr(Cv^T T X2 T^T) / 2,
 // all linear in the sums, so values and tangents alike. One wave per (row, state); lane 32 h + i
-// works on half h.
+// works on half h. With grads.cv the gradients of the parameter tensors, from values plus
+// tangents, are formed too.
 __global__ void __launch_bounds__(64)
 metric_entries_kernel(const double* __restrict__ tab, const int32_t* __restrict__ nstates,
-                      int max_states, int64_t npar, double* __restrict__ params) {
+                      int max_states, int64_t npar, double* __restrict__ params, GradOut grads) {
   const int row = blockIdx.x / max_states, s = blockIdx.x % max_states;
-  if (s >= nstates[row]) return;
+  __shared__ double ent[32];
+  if (grads.cv && s == 0 && threadIdx.x == 0) {
+    const double* e = params + 2 * (row * npar + (int64_t)max_states * kNps);
+    grads.teff[row] = (e[0] + e[1]) * grads.boltzmann;
+  }
+  if (s >= nstates[row]) {
+    if (grads.cv) state_gradients(ent, false, blockIdx.x, grads);
+    return;
+  }
   const double* ts = tab + (int64_t)blockIdx.x * kTabStride;
   const double* C = ts + kCvOffset;
   const double* R = ts + kRestOffset;
@@ -525,51 +577,84 @@ metric_entries_kernel(const double* __restrict__ tab, const int32_t* __restrict_
     v = p[h];
   }
   out[2 * i + h] = v;
+  if (!grads.cv) return;
+  const double d = __shfl_down(v, 32, 64);
+  if (h == 0) ent[i] = v + d;
+  __syncthreads();
+  state_gradients(ent, true, blockIdx.x, grads);
 }
 
-// Row sums of per-block partials over lists of segments (4 blocks each): one block per
-// (list, row of the partial array). Rows q with q % weight_every == 0 are scaled per segment by
-// weight[system of the segment] when weight is given.
+// Row sums of per-block partials over lists of segments (kAdjPerSeg blocks each). Rows q with
+// q % weight_every == 0 are scaled per segment by weight[system of the segment] when weight is given.
+struct SegmentSums {
+  const double* part;
+  int lists, nrows_part;  // outputs [list][row of part]
+  const int32_t *list_ptr, *list_idx;
+  const double* weight;
+  int weight_every;
+  double* out;
+};
+
+// One block per (list, row): first those of x, then those of y.
 __global__ void __launch_bounds__(256)
-segment_sum_kernel(const double* __restrict__ part, int64_t nblk, int nrows_part,
-                   const int32_t* __restrict__ list_ptr, const int32_t* __restrict__ list_idx,
-                   const int32_t* __restrict__ blk_sys, const double* __restrict__ weight,
-                   int weight_every, double* __restrict__ out) {
+segment_sum_kernel(SegmentSums x, SegmentSums y, int64_t nblk, const int32_t* __restrict__ blk_sys) {
   __shared__ double red[4];
-  const int li = blockIdx.x / nrows_part;
-  const int q = blockIdx.x % nrows_part;
-  const bool weighted = weight != nullptr && (q % weight_every) == 0;
-  const int i0 = list_ptr[li], i1 = list_ptr[li + 1];
+  const int nx = x.lists * x.nrows_part;
+  const bool first = (int)blockIdx.x < nx;
+  const SegmentSums a = first ? x : y;
+  const int at = first ? blockIdx.x : blockIdx.x - nx;
+  const int li = at / a.nrows_part;
+  const int q = at % a.nrows_part;
+  const bool weighted = a.weight != nullptr && (q % a.weight_every) == 0;
+  const int i0 = a.list_ptr[li], i1 = a.list_ptr[li + 1];
   double acc = 0.0;
   for (int i = i0 + threadIdx.x; i < i1; i += 256) {
-    const int seg = list_idx[i];
+    const int seg = a.list_idx[i];
     double s = 0.0;
 #pragma unroll
-    for (int k = 0; k < kAdjPerSeg; ++k) s += part[(int64_t)q * nblk + (int64_t)seg * kAdjPerSeg + k];
-    acc += weighted ? weight[blk_sys[seg]] * s : s;
+    for (int k = 0; k < kAdjPerSeg; ++k)
+      s += a.part[(int64_t)q * nblk + (int64_t)seg * kAdjPerSeg + k];
+    acc += weighted ? a.weight[blk_sys[seg]] * s : s;
   }
   for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
   __syncthreads();
-  if (threadIdx.x == 0) out[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
+  if (threadIdx.x == 0) a.out[at] = ((red[0] + red[1]) + red[2]) + red[3];
 }
+
+// A force-and-stress loss (mm_fit_loss) whose cotangents are formed where they are used:
+//   gG = gl 2 (g - gt) / (3 N f_scale),  gV = gl 2 (v inv - vt) inv / (9 nsys s_scale).
+struct FitTerms {
+  const double *g, *gt, *v, *vt, *inv;  // [N][3], [N][3], [nsys][9], [nsys][9], [nsys]
+  const double* gl;                     // the loss' own cotangent
+  double cf, cs;                        // 2 / (3 N f_scale), 2 / (9 nsys s_scale)
+  double* gV;                           // [nsys][9], for the kernels after the direction
+  __device__ double stress(int64_t sy, int q) const {
+    return *gl * cs * (v[9 * sy + q] * inv[sy] - vt[9 * sy + q]) * inv[sy];
+  }
+};
 
 // Tangent direction of a vector-Jacobian product from the cotangents (gE, gG, gV) of
 // (E, gpos, vtens): dpos_n = gG_n + pos_n gV_s^T (s = node_sys[n]), and for the threads past the
-// nodes drvecs_s = rvecs_s gV_s^T. gG or gV may be null (zero).
+// nodes drvecs_s = rvecs_s gV_s^T. gG or gV may be null (zero); kFit: those of the loss.
+template <bool kFit>
 __global__ void __launch_bounds__(256)
 vjp_direction_kernel(const double* __restrict__ pos, const double* __restrict__ rvecs,
                      const int32_t* __restrict__ node_sys, const double* __restrict__ gG,
-                     const double* __restrict__ gV, int64_t N, int nsys,
+                     const double* __restrict__ gV, FitTerms fit, int64_t N, int nsys,
                      double* __restrict__ dpos, double* __restrict__ drv) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  auto stress = [&](int64_t sy, int q) { return kFit ? fit.stress(sy, q) : gV[9 * sy + q]; };
   if (t < N) {
-    const double* V = gV ? gV + 9 * (int64_t)node_sys[t] : nullptr;
+    const bool on = kFit || gV;
+    const int64_t sy = on ? node_sys[t] : 0;
+    const double cf = kFit ? *fit.gl * fit.cf : 0.0;
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
-      double d = gG ? gG[3 * t + l] : 0.0;
-      if (V)
-        d += (pos[3 * t] * V[3 * l] + pos[3 * t + 1] * V[3 * l + 1]) + pos[3 * t + 2] * V[3 * l + 2];
+      double d = kFit ? cf * (fit.g[3 * t + l] - fit.gt[3 * t + l]) : gG ? gG[3 * t + l] : 0.0;
+      if (on)
+        d += (pos[3 * t] * stress(sy, 3 * l) + pos[3 * t + 1] * stress(sy, 3 * l + 1)) +
+             pos[3 * t + 2] * stress(sy, 3 * l + 2);
       dpos[3 * t + l] = d;
     }
   } else if (t < N + 9 * (int64_t)nsys) {
@@ -578,97 +663,119 @@ vjp_direction_kernel(const double* __restrict__ pos, const double* __restrict__ 
     const int dd = (int)(q % 9) / 3, l = (int)(q % 3);
     const double* R = rvecs + 9 * sy;
     double d = 0.0;
-    if (gV) {
-      const double* V = gV + 9 * sy;
-      d = (R[3 * dd] * V[3 * l] + R[3 * dd + 1] * V[3 * l + 1]) + R[3 * dd + 2] * V[3 * l + 2];
-    }
+    if (kFit || gV)
+      d = (R[3 * dd] * stress(sy, 3 * l) + R[3 * dd + 1] * stress(sy, 3 * l + 1)) +
+          R[3 * dd + 2] * stress(sy, 3 * l + 2);
     drv[q] = d;
+    if (kFit) fit.gV[q] = stress(sy, (int)(q % 9));
   }
 }
 
-// Position cotangent of the product: g_n = gE_s gpos_n + dgpos_n + gpos_n gV_s (gV may be null:
-// zero).
+// The product's position cotangent, g_n = gE_s gpos_n + dgpos_n + gpos_n gV_s, from the vertex
+// gradients' and their tangents' records (nb blocks, none when g_pos is null), and beyond them the
+// domain vectors' (g_rv, null: none), dL/drvecs = gE dE/drvecs + d(dE/drvecs) + (dE/drvecs) gV,
+// from sys_out. gV may be null: zero. One pass in place of two gathers and a pass over their
+// results.
+template <bool kAllLoads>
 __global__ void __launch_bounds__(256)
-vjp_position_kernel(const double* __restrict__ gpos, const double* __restrict__ dgpos,
-                    const int32_t* __restrict__ node_sys, const double* __restrict__ gE,
-                    const double* __restrict__ gV, int64_t N, double* __restrict__ out) {
-  const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
+vjp_output_kernel(const int32_t* __restrict__ ncell, const double* __restrict__ gcell,
+                  const double* __restrict__ gcell2, int64_t N, int64_t RS,
+                  const int32_t* __restrict__ node_sys, const double* __restrict__ gE,
+                  const double* __restrict__ gV, const double* __restrict__ sys_out, int nsys,
+                  int nb, double* __restrict__ g_pos, double* __restrict__ g_rv,
+                  int* __restrict__ nanflag) {
+  if ((int)blockIdx.x >= nb) {
+    const int q = ((int)blockIdx.x - nb) * 256 + threadIdx.x;
+    if (q >= 9 * nsys) return;
+    const int sy = q / 9, i = q % 9;
+    const double* r = sys_out + (int64_t)sy * 2 * kSysQ + 10;
+    double v = gE[sy] * r[i] + r[kSysQ + i];
+    if (gV) {
+      const double *a = r + 3 * (i / 3), *V = gV + 9 * (int64_t)sy + i % 3;
+      v += (a[0] * V[0] + a[1] * V[3]) + a[2] * V[6];
+    }
+    g_rv[q] = v;
+    return;
+  }
+  const int64_t n = (int64_t)xcd_block((int)blockIdx.x, nb) * 256 + threadIdx.x;
   if (n >= N) return;
+  double g[3], d[3];
+  sum_node_records<kAllLoads>(ncell, gcell, N, RS, n, g);
+  sum_node_records<kAllLoads>(ncell, gcell2, N, RS, n, d);
+  bool bad = false;
+#pragma unroll
+  for (int l = 0; l < 3; ++l) bad |= g[l] != g[l] || d[l] != d[l];
+  if (bad) atomicOr(nanflag, 2);
   const int sy = node_sys[n];
   const double e = gE[sy];
   const double* V = gV ? gV + 9 * (int64_t)sy : nullptr;
-  const double g0 = gpos[3 * n], g1 = gpos[3 * n + 1], g2 = gpos[3 * n + 2];
 #pragma unroll
   for (int l = 0; l < 3; ++l) {
-    double v = e * gpos[3 * n + l] + dgpos[3 * n + l];
-    if (V) v += (g0 * V[l] + g1 * V[3 + l]) + g2 * V[6 + l];
-    out[3 * n + l] = v;
+    double v = e * g[l] + d[l];
+    if (V) v += (g[0] * V[l] + g[1] * V[3 + l]) + g[2] * V[6 + l];
+    g_pos[3 * n + l] = v;
   }
+}
+
+// Sums of squares for the force-and-stress loss. Per block of the node terms (g - gt)^2:
+constexpr int kLossBlocks = 1024;
+__global__ void __launch_bounds__(256)
+fit_loss_partial_kernel(const double* __restrict__ g, const double* __restrict__ gt, int64_t n,
+                        double* __restrict__ part) {
+  __shared__ double red[4];
+  double acc[1] = {0.0};
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const double d = g[i] - gt[i];
+    acc[0] += d * d;
+  }
+  wave_reduce<1>(acc);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc[0];
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
+}
+
+// loss = mean (g - gt)^2 / f_scale + mean (v inv - vt)^2 / s_scale over n and m values; one block.
+__global__ void __launch_bounds__(256)
+fit_loss_kernel(const double* __restrict__ part, int nb, int64_t n, const double* __restrict__ v,
+                const double* __restrict__ vt, const double* __restrict__ inv, int m,
+                double f_scale, double s_scale, double* __restrict__ loss) {
+  __shared__ double red[8];
+  double acc[2] = {0.0, 0.0};
+  for (int i = threadIdx.x; i < nb; i += 256) acc[0] += part[i];
+  for (int i = threadIdx.x; i < m; i += 256) {
+    const double d = v[i] * inv[i / 9] - vt[i];
+    acc[1] += d * d;
+  }
+  wave_reduce<2>(acc);
+  if ((threadIdx.x & 63) == 0) {
+    red[threadIdx.x >> 6] = acc[0];
+    red[4 + (threadIdx.x >> 6)] = acc[1];
+  }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    *loss = (((red[0] + red[1]) + red[2]) + red[3]) / (double)n / f_scale +
+            (((red[4] + red[5]) + red[6]) + red[7]) / (double)m / s_scale;
 }
 
 }  // namespace mm
 
 using namespace mm;
 
-// Gradients of (Cv, h0, free energy, T_eff) from the parameter entries of one (row, state) per
-// thread: the 21 upper-triangle entries give the symmetric Voigt gradient, the inverse P = h0^-1
-// by cofactors (rows r1 x r2, r2 x r0, r0 x r1 of cof; P^T = cof / det), dE/dh0 =
-// -P^T (dE/dP) P^T + (dE/dw) w P^T with w = det / 8 (corner8) or det; states beyond the row's
-// count get zeros; thread (row, 0) also writes boltzmann dE/d(kT).
-__global__ void __launch_bounds__(256)
-param_grads_kernel(const double* __restrict__ entries, int64_t stride, int add_next,
-                   int64_t npar, int nrows, int max_states, const int32_t* __restrict__ nstates,
-                   const double* __restrict__ h0, int corner8, double boltzmann,
-                   double* __restrict__ g_cv, double* __restrict__ g_h0,
-                   double* __restrict__ g_free, double* __restrict__ g_teff) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nrows * max_states) return;
-  const int row = t / max_states, s = t % max_states;
+// Gradients of (Cv, h0, free energy, T_eff) from parameter entries, one wave per (row, state).
+__global__ void __launch_bounds__(64)
+param_grads_kernel(const double* __restrict__ entries, int64_t stride, int add_next, int64_t npar,
+                   int max_states, const int32_t* __restrict__ nstates, GradOut grads) {
+  const int row = blockIdx.x / max_states, s = blockIdx.x % max_states;
   const double* er = entries + (int64_t)row * npar * stride;
-  auto ent = [&](int64_t q) {
+  auto get = [&](int64_t q) {
     return add_next ? er[q * stride] + er[q * stride + 1] : er[q * stride];
   };
-  const bool on = s < nstates[row];
-  const int64_t q0 = (int64_t)s * kNps;
-  double* gc = g_cv + (int64_t)t * 36;
-  int q = 0;
-  for (int I = 0; I < 6; ++I) {
-    for (int J = I; J < 6; ++J, ++q) {
-      const double v = on ? ent(q0 + q) : 0.0;
-      gc[6 * I + J] = v;
-      gc[6 * J + I] = v;
-    }
-  }
-  const double* h = h0 + (int64_t)t * 9;
-  double cof[9];
-  // cof row 0 = r1 x r2, row 1 = r2 x r0, row 2 = r0 x r1
-  for (int a = 0; a < 3; ++a) {
-    const double* u = h + 3 * ((a + 1) % 3);
-    const double* v = h + 3 * ((a + 2) % 3);
-    cof[3 * a + 0] = u[1] * v[2] - u[2] * v[1];
-    cof[3 * a + 1] = u[2] * v[0] - u[0] * v[2];
-    cof[3 * a + 2] = u[0] * v[1] - u[1] * v[0];
-  }
-  const double det = (h[0] * cof[0] + h[1] * cof[1]) + h[2] * cof[2];
-  double pt[9], gp[9], m1[9];
-  for (int k = 0; k < 9; ++k) {
-    pt[k] = cof[k] / det;
-    gp[k] = ent(q0 + 21 + k);
-  }
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j)
-      m1[3 * i + j] = (pt[3 * i] * gp[j] + pt[3 * i + 1] * gp[3 + j]) + pt[3 * i + 2] * gp[6 + j];
-  const double w = corner8 ? det / 8.0 : det;
-  const double gww = ent(q0 + 30) * w;
-  double* gh = g_h0 + (int64_t)t * 9;
-  for (int i = 0; i < 3; ++i)
-    for (int j = 0; j < 3; ++j) {
-      const double m2 =
-          (m1[3 * i] * pt[j] + m1[3 * i + 1] * pt[3 + j]) + m1[3 * i + 2] * pt[6 + j];
-      gh[3 * i + j] = on ? -m2 + gww * pt[3 * i + j] : 0.0;
-    }
-  g_free[t] = on ? ent(q0 + 31) : 0.0;
-  if (s == 0) g_teff[row] = ent((int64_t)max_states * kNps) * boltzmann;
+  __shared__ double ent[32];
+  if (threadIdx.x < 32) ent[threadIdx.x] = get((int64_t)s * kNps + threadIdx.x);
+  if (s == 0 && threadIdx.x == 0)
+    grads.teff[row] = get((int64_t)max_states * kNps) * grads.boltzmann;
+  __syncthreads();
+  state_gradients(ent, s < nstates[row], blockIdx.x, grads);
 }
 
 struct mm_adjoint {
@@ -680,7 +787,10 @@ struct mm_adjoint {
   double* gcell2 = nullptr;    // [4][3][S]
   int32_t* row_ptr = nullptr;  // [nrows + 1] CSR of the segments of every table row
   int32_t* row_idx = nullptr;  // [W / kCellBlock]
-  double* vjp = nullptr;       // [3][N][3] + [nsys][9]: dpos, gpos, dgpos, drvecs of mm_adjoint_vjp
+  // of the products: direction [N][3] and [nsys][9], sys_out [nsys][2 kSysQ], params
+  // [nrows][npar][2], stress cotangents [nsys][9], loss partials [kLossBlocks]
+  double *vjp = nullptr, *drv = nullptr, *sys_out = nullptr, *params = nullptr, *gV = nullptr,
+         *lpart = nullptr;
 };
 
 extern "C" {
@@ -716,7 +826,16 @@ int mm_adjoint_create(mm_adjoint** out, mm_field* field, int64_t* npar) {
   if (e == hipSuccess)
     e = hipMalloc((void**)&a->gcell2, sizeof(double) * 12 * (field->S > 0 ? field->S : 1));
   if (e == hipSuccess)
-    e = hipMalloc((void**)&a->vjp, sizeof(double) * (9 * (size_t)field->N + 9 * field->nsys));
+    e = hipMalloc((void**)&a->vjp,
+                  sizeof(double) * (3 * (size_t)field->N + (18 + 2 * kSysQ) * (size_t)field->nsys +
+                                    2 * (size_t)a->npar * field->nrows + kLossBlocks));
+  if (e == hipSuccess) {
+    a->drv = a->vjp + 3 * field->N;
+    a->sys_out = a->drv + 9 * (int64_t)field->nsys;
+    a->gV = a->sys_out + 2 * kSysQ * (int64_t)field->nsys;
+    a->params = a->gV + 9 * (int64_t)field->nsys;
+    a->lpart = a->params + 2 * a->npar * field->nrows;
+  }
   if (e == hipSuccess) e = hipMalloc((void**)&a->row_ptr, sizeof(int32_t) * row_ptr.size());
   if (e == hipSuccess)
     e = hipMalloc((void**)&a->row_idx, sizeof(int32_t) * (row_idx.empty() ? 1 : row_idx.size()));
@@ -738,6 +857,128 @@ int mm_adjoint_create(mm_adjoint** out, mm_field* field, int64_t* npar) {
   return MM_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+// The adjoint kernel and its sums on the current device: sys_out, params (and grads from them),
+// and with records the vertex gradients' and tangents' records.
+hipError_t adjoint_passes(mm_adjoint* a, const double* pos, const double* dpos,
+                          const double* rvecs, const double* drvecs, const double* energy_weight,
+                          double* sys_out, double* params, bool records, const GradOut& grads,
+                          hipStream_t s) {
+  mm_field* f = a->field;
+  const bool dual = dpos != nullptr;
+  const int64_t nblk = a->nblk;
+  if (nblk == 0) {
+    hipError_t e = hipMemsetAsync(sys_out, 0, sizeof(double) * 2 * kSysQ * f->nsys, s);
+    if (e == hipSuccess)
+      e = hipMemsetAsync(params, 0, sizeof(double) * 2 * a->npar * f->nrows, s);
+    return e;
+  }
+  const size_t lds = sizeof(double) * 64 * (dual ? 2 : 1) *
+                     ((f->model == 0 ? 36 : 6) + (f->max_states > 1 ? f->max_states : 0));
+#define MM_ADJ(T, MODEL)                                                                        \
+  hipLaunchKernelGGL((adjoint_kernel<T, MODEL>), dim3((unsigned)nblk), dim3(64), lds, s, pos,   \
+                     dpos, rvecs, drvecs, f->blk_sys, f->cnode, f->cwrap, f->blk_row, f->tab,  \
+                     f->kt, f->nstates, f->max_states, f->W, f->cbase, f->S,                   \
+                     records ? f->gcell : nullptr, a->gcell2, a->part, a->ppart)
+  if (dual) {
+    if (f->model == 0) MM_ADJ(Dual, 0); else MM_ADJ(Dual, 1);
+  } else {
+    if (f->model == 0) MM_ADJ(double, 0); else MM_ADJ(double, 1);
+  }
+#undef MM_ADJ
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  // per system: energy, virial, domain-vector gradient (value rows, then tangent rows); per
+  // table row: parameter entries (value rows scaled by the system's energy weight)
+  const SegmentSums x{a->part, f->nsys, 2 * kSysQ, f->sys_cblk_ptr, f->sys_cblk_idx, nullptr, 1,
+                      sys_out};
+  const SegmentSums y{a->ppart, f->nrows, (int)(2 * a->npar), a->row_ptr, a->row_idx,
+                      energy_weight, 2, params};
+  hipLaunchKernelGGL(segment_sum_kernel,
+                     dim3((unsigned)(x.lists * x.nrows_part + y.lists * y.nrows_part)), dim3(256),
+                     0, s, x, y, nblk, f->blk_sys);
+  e = hipGetLastError();
+  if (e != hipSuccess || f->nrows == 0) return e;
+  hipLaunchKernelGGL(metric_entries_kernel, dim3((unsigned)(f->nrows * f->max_states)), dim3(64),
+                     0, s, f->tab, f->nstates, f->max_states, a->npar, params, grads);
+  return hipGetLastError();
+}
+
+hipError_t launch_param_grads(mm_adjoint* a, const double* entries, int64_t stride, int add_next,
+                              const GradOut& grads, hipStream_t s) {
+  const mm_field* f = a->field;
+  const int n = f->nrows * f->max_states;
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(param_grads_kernel, dim3((unsigned)n), dim3(64), 0, s, entries, stride,
+                     add_next, a->npar, f->max_states, f->nstates, grads);
+  return hipGetLastError();
+}
+
+// A vector-Jacobian product on the current device (fit: of the loss; then gG and gV are not read).
+// g_pos, g_rv and grads.cv may be null. Five launches: direction, adjoint kernel, sums, entries with
+// the parameter gradients, outputs. The host's work per launch and tensor bounds both uses: nine
+// launches and some fifteen torch kernels for loss, cotangents and domain gradients took 500 us a
+// fit step (64 configurations of 16^3 cells; its parameters alone need a gradient, so no records
+// are stored nor gathered) and 430 us for all gradients of 5 of 7^3 cells, now 349 and 351 us.
+hipError_t vjp_passes(mm_adjoint* a, const double* pos, const double* rvecs,
+                      const int32_t* node_sys, const double* gE, const double* gG,
+                      const double* gV, const FitTerms* fit, double* sys_out, double* params,
+                      double* g_pos, double* g_rv, const GradOut& grads, hipStream_t s) {
+  mm_field* f = a->field;
+  const int64_t nt = f->N + 9 * (int64_t)f->nsys;
+  const dim3 grid((unsigned)((nt + 255) / 256));
+  if (fit) {
+    hipLaunchKernelGGL(vjp_direction_kernel<true>, grid, dim3(256), 0, s, pos, rvecs, node_sys, gG,
+                       gV, *fit, f->N, f->nsys, a->vjp, a->drv);
+    gV = a->gV;
+  } else {
+    hipLaunchKernelGGL(vjp_direction_kernel<false>, grid, dim3(256), 0, s, pos, rvecs, node_sys,
+                       gG, gV, FitTerms{}, f->N, f->nsys, a->vjp, a->drv);
+  }
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess)
+    e = adjoint_passes(a, pos, a->vjp, rvecs, a->drv, gE, sys_out, params, g_pos != nullptr,
+                       grads, s);
+  if (e == hipSuccess && a->nblk == 0 && grads.cv)
+    e = launch_param_grads(a, params, 2, 1, grads, s);
+  if (e != hipSuccess) return e;
+  const int nb = g_pos ? (int)((f->N + 255) / 256) : 0;
+  const int nr = g_rv ? (9 * f->nsys + 255) / 256 : 0;
+  if (nb + nr == 0) return hipSuccess;
+#define MM_OUT(A)                                                                               \
+  hipLaunchKernelGGL(vjp_output_kernel<A>, dim3(nb + nr), dim3(256), 0, s, f->nrec, f->gcell,     \
+                     a->gcell2, f->N, f->S, node_sys, gE, gV, sys_out, f->nsys, nb, g_pos, g_rv, \
+                     f->nanflag)
+  if (nb <= kGatherAllLoadsMaxBlocks) MM_OUT(true); else MM_OUT(false);
+#undef MM_OUT
+  return hipGetLastError();
+}
+
+struct CurrentDevice {
+  int cur = 0;
+  explicit CurrentDevice(int device) {
+    (void)hipGetDevice(&cur);
+    (void)hipSetDevice(device);
+  }
+  ~CurrentDevice() { (void)hipSetDevice(cur); }
+};
+
+int grad_out(const mm_adjoint* a, const double* h0, double boltzmann, double* g_cv, double* g_h0,
+             double* g_free, double* g_teff, GradOut& out) {
+  if ((g_cv || g_h0 || g_free || g_teff) && !(h0 && g_cv && g_h0 && g_free && g_teff))
+    return set_error(MM_ERR_ARG, "h0, g_cv, g_h0, g_free and g_teff go together");
+  out = GradOut{h0, a->field->model == MM_MODEL_CORNER8 ? 1 : 0, boltzmann, g_cv, g_h0, g_free,
+                g_teff};
+  return MM_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
 int mm_adjoint_compute(mm_adjoint* a, const double* pos, const double* dpos, const double* rvecs,
                        const double* drvecs, const double* energy_weight, double* sys_out,
                        double* gpos, double* dgpos, double* params, void* stream) {
@@ -748,70 +989,27 @@ int mm_adjoint_compute(mm_adjoint* a, const double* pos, const double* dpos, con
   if ((dpos == nullptr) != (drvecs == nullptr))
     return set_error(MM_ERR_ARG, "dpos and drvecs go together");
   if (dgpos && !dpos) return set_error(MM_ERR_ARG, "dgpos needs a tangent direction");
-  const bool dual = dpos != nullptr;
-  int cur = 0;
-  (void)hipGetDevice(&cur);
-  (void)hipSetDevice(f->device);
+  const CurrentDevice device(f->device);
   hipStream_t s = (hipStream_t)stream;
-  const int64_t nblk = a->nblk;
-  hipError_t e = hipSuccess;
-  if (nblk > 0) {
-    const size_t lds = sizeof(double) * 64 * (dual ? 2 : 1) *
-                       ((f->model == 0 ? 36 : 6) + (f->max_states > 1 ? f->max_states : 0));
-#define MM_ADJ(T, MODEL)                                                                        \
-  hipLaunchKernelGGL((adjoint_kernel<T, MODEL>), dim3((unsigned)nblk), dim3(64), lds, s, pos,   \
-                     dpos, rvecs, drvecs, f->blk_sys, f->cnode, f->cwrap, f->blk_row, f->tab,  \
-                     f->kt, f->nstates, f->max_states, f->W, f->cbase, f->S, f->gcell,         \
-                     a->gcell2, a->part, a->ppart)
-    if (dual) {
-      if (f->model == 0) MM_ADJ(Dual, 0); else MM_ADJ(Dual, 1);
-    } else {
-      if (f->model == 0) MM_ADJ(double, 0); else MM_ADJ(double, 1);
-    }
-#undef MM_ADJ
-    e = hipGetLastError();
-    // per system: energy, virial, domain-vector gradient (value rows, then tangent rows)
-    if (e == hipSuccess) {
-      hipLaunchKernelGGL(segment_sum_kernel, dim3((unsigned)(f->nsys * 2 * kSysQ)), dim3(256), 0,
-                         s, a->part, nblk, 2 * kSysQ, f->sys_cblk_ptr, f->sys_cblk_idx,
-                         f->blk_sys, (const double*)nullptr, 1, sys_out);
-      e = hipGetLastError();
-    }
-    // per table row: parameter entries (value rows scaled by the system's energy weight)
-    if (e == hipSuccess) {
-      hipLaunchKernelGGL(segment_sum_kernel, dim3((unsigned)(f->nrows * 2 * a->npar)), dim3(256),
-                         0, s, a->ppart, nblk, (int)(2 * a->npar), a->row_ptr, a->row_idx,
-                         f->blk_sys, energy_weight, 2, params);
-      e = hipGetLastError();
-    }
-    if (e == hipSuccess && f->nrows > 0) {
-      hipLaunchKernelGGL(metric_entries_kernel, dim3((unsigned)(f->nrows * f->max_states)),
-                         dim3(64), 0, s, f->tab, f->nstates, f->max_states, a->npar, params);
-      e = hipGetLastError();
-    }
-    if (e == hipSuccess && f->N > 0 && gpos) {
-      ForceArgs g{};
-      g.ncell = f->nrec;
-      g.gcell = f->gcell;
-      g.rstride = f->S;
-      g.N = f->N;
-      g.W = f->W;
-      g.gpos = gpos;
-      g.accumulate = 0;
-      g.nanflag = f->nanflag;
+  hipError_t e = adjoint_passes(a, pos, dpos, rvecs, drvecs, energy_weight, sys_out, params,
+                                gpos != nullptr, GradOut{}, s);
+  if (e == hipSuccess && a->nblk > 0 && f->N > 0 && gpos) {
+    ForceArgs g{};
+    g.ncell = f->nrec;
+    g.gcell = f->gcell;
+    g.rstride = f->S;
+    g.N = f->N;
+    g.W = f->W;
+    g.gpos = gpos;
+    g.accumulate = 0;
+    g.nanflag = f->nanflag;
+    e = launch_gather(g, ReduceList{}, s);
+    if (e == hipSuccess && dgpos) {
+      g.gcell = a->gcell2;
+      g.gpos = dgpos;
       e = launch_gather(g, ReduceList{}, s);
-      if (e == hipSuccess && dgpos) {
-        g.gcell = a->gcell2;
-        g.gpos = dgpos;
-        e = launch_gather(g, ReduceList{}, s);
-      }
     }
-  } else {
-    e = hipMemsetAsync(sys_out, 0, sizeof(double) * 2 * kSysQ * f->nsys, s);
-    if (e == hipSuccess)
-      e = hipMemsetAsync(params, 0, sizeof(double) * 2 * a->npar * f->nrows, s);
   }
-  (void)hipSetDevice(cur);
   if (e != hipSuccess) return hip_error(e, "adjoint kernels");
   return MM_OK;
 }
@@ -823,31 +1021,74 @@ int mm_adjoint_vjp(mm_adjoint* a, const double* pos, const double* rvecs,
   mm_field* f = a->field;
   if ((f->N > 0 && (!pos || !node_sys || !g_pos)) || !rvecs || !gE || !sys_out || !params)
     return set_error(MM_ERR_ARG, "missing argument (gE is required: zeros for none)");
-  double* dpos = a->vjp;
-  double* gtmp = dpos + 3 * f->N;
-  double* dgtmp = gtmp + 3 * f->N;
-  double* drv = dgtmp + 3 * f->N;
-  int cur = 0;
-  (void)hipGetDevice(&cur);
-  (void)hipSetDevice(f->device);
-  hipStream_t s = (hipStream_t)stream;
-  const int64_t nt = f->N + 9 * (int64_t)f->nsys;
-  hipLaunchKernelGGL(vjp_direction_kernel, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s,
-                     pos, rvecs, node_sys, gG, gV, f->N, f->nsys, dpos, drv);
-  hipError_t e = hipGetLastError();
-  (void)hipSetDevice(cur);
-  if (e != hipSuccess) return hip_error(e, "vector-Jacobian direction kernel");
-  const int rc =
-      mm_adjoint_compute(a, pos, dpos, rvecs, drv, gE, sys_out, gtmp, dgtmp, params, stream);
+  const CurrentDevice device(f->device);
+  const hipError_t e = vjp_passes(a, pos, rvecs, node_sys, gE, gG, gV, nullptr, sys_out, params,
+                                  g_pos, nullptr, GradOut{}, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_error(e, "vector-Jacobian product kernels");
+  return MM_OK;
+}
+
+int mm_adjoint_backward(mm_adjoint* a, const double* pos, const double* rvecs,
+                        const int32_t* node_sys, const double* gE, const double* gG,
+                        const double* gV, const double* h0, double boltzmann, double* g_pos,
+                        double* g_rv, double* g_cv, double* g_h0, double* g_free, double* g_teff,
+                        void* stream) {
+  if (!a) return set_error(MM_ERR_ARG, "adjoint is NULL");
+  mm_field* f = a->field;
+  if ((f->N > 0 && (!pos || !node_sys)) || !rvecs || !gE)
+    return set_error(MM_ERR_ARG, "missing argument (gE is required: zeros for none)");
+  GradOut grads;
+  const int rc = grad_out(a, h0, boltzmann, g_cv, g_h0, g_free, g_teff, grads);
   if (rc != MM_OK) return rc;
-  if (f->N > 0) {
-    (void)hipSetDevice(f->device);
-    hipLaunchKernelGGL(vjp_position_kernel, dim3((unsigned)((f->N + 255) / 256)), dim3(256), 0, s,
-                       gtmp, dgtmp, node_sys, gE, gV, f->N, g_pos);
-    e = hipGetLastError();
-    (void)hipSetDevice(cur);
-    if (e != hipSuccess) return hip_error(e, "vector-Jacobian position kernel");
-  }
+  const CurrentDevice device(f->device);
+  const hipError_t e = vjp_passes(a, pos, rvecs, node_sys, gE, gG, gV, nullptr, a->sys_out,
+                                  a->params, g_pos, g_rv, grads, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_error(e, "backward kernels");
+  return MM_OK;
+}
+
+int mm_fit_loss(mm_adjoint* a, const double* g, const double* g_target, const double* v,
+                const double* v_target, const double* inv_volume, double f_scale, double s_scale,
+                double* loss, void* stream) {
+  if (!a) return set_error(MM_ERR_ARG, "adjoint is NULL");
+  mm_field* f = a->field;
+  if ((f->N > 0 && (!g || !g_target)) || !v || !v_target || !inv_volume || !loss)
+    return set_error(MM_ERR_ARG, "missing argument");
+  const CurrentDevice device(f->device);
+  const hipStream_t s = (hipStream_t)stream;
+  const int64_t n = 3 * f->N;
+  const int nb = (int)std::min<int64_t>((n + 1023) / 1024, kLossBlocks);
+  if (nb > 0)
+    hipLaunchKernelGGL(fit_loss_partial_kernel, dim3(nb), dim3(256), 0, s, g, g_target, n,
+                       a->lpart);
+  hipLaunchKernelGGL(fit_loss_kernel, dim3(1), dim3(256), 0, s, a->lpart, nb, n, v, v_target,
+                     inv_volume, 9 * f->nsys, f_scale, s_scale, loss);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return hip_error(e, "loss kernels");
+  return MM_OK;
+}
+
+int mm_fit_backward(mm_adjoint* a, const double* pos, const double* rvecs,
+                    const int32_t* node_sys, const double* gE, const double* g,
+                    const double* g_target, const double* v, const double* v_target,
+                    const double* inv_volume, double f_scale, double s_scale, const double* gl,
+                    const double* h0, double boltzmann, double* g_pos, double* g_rv, double* g_cv,
+                    double* g_h0, double* g_free, double* g_teff, void* stream) {
+  if (!a) return set_error(MM_ERR_ARG, "adjoint is NULL");
+  mm_field* f = a->field;
+  if ((f->N > 0 && (!pos || !node_sys || !g || !g_target)) || !rvecs || !gE || !v || !v_target ||
+      !inv_volume || !gl)
+    return set_error(MM_ERR_ARG, "missing argument (gE is required: zeros)");
+  GradOut grads;
+  const int rc = grad_out(a, h0, boltzmann, g_cv, g_h0, g_free, g_teff, grads);
+  if (rc != MM_OK) return rc;
+  const CurrentDevice device(f->device);
+  const FitTerms fit{g, g_target, v, v_target, inv_volume, gl,
+                     2.0 / (3.0 * (double)f->N * f_scale), 2.0 / (9.0 * f->nsys * s_scale),
+                     a->gV};
+  const hipError_t e = vjp_passes(a, pos, rvecs, node_sys, gE, nullptr, nullptr, &fit, a->sys_out,
+                                  a->params, g_pos, g_rv, grads, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_error(e, "backward kernels of the loss");
   return MM_OK;
 }
 
@@ -859,18 +1100,12 @@ int mm_adjoint_param_grads(mm_adjoint* a, const double* entries, int64_t stride,
     return set_error(MM_ERR_ARG, "missing argument");
   if (stride < 1 || (add_next && stride < 2))
     return set_error(MM_ERR_ARG, "stride %lld with add_next %d", (long long)stride, add_next);
-  mm_field* f = a->field;
-  const int n = f->nrows * f->max_states;
-  if (n == 0) return MM_OK;
-  int cur = 0;
-  (void)hipGetDevice(&cur);
-  (void)hipSetDevice(f->device);
-  hipLaunchKernelGGL(param_grads_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                     (hipStream_t)stream, entries, stride, add_next, a->npar, f->nrows,
-                     f->max_states, f->nstates, h0, f->model == MM_MODEL_CORNER8 ? 1 : 0,
-                     boltzmann, g_cv, g_h0, g_free, g_teff);
-  const hipError_t e = hipGetLastError();
-  (void)hipSetDevice(cur);
+  GradOut grads;
+  const int rc = grad_out(a, h0, boltzmann, g_cv, g_h0, g_free, g_teff, grads);
+  if (rc != MM_OK) return rc;
+  const CurrentDevice device(a->field->device);
+  const hipError_t e = launch_param_grads(a, entries, stride, add_next, grads,
+                                          (hipStream_t)stream);
   if (e != hipSuccess) return hip_error(e, "parameter gradient kernel");
   return MM_OK;
 }

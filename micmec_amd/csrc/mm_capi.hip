@@ -528,11 +528,10 @@ int mm_batch_compute(mm_field* f, const double* pos, const double* rvecs, double
   a.accumulate = 0;
   a.force_grad = 1;
   hipError_t e = launch_cells(a, (hipStream_t)stream);
-  if (e == hipSuccess && gpos) e = launch_gather(a, ReduceList{}, (hipStream_t)stream);
   if (e == hipSuccess)
-    e = launch_batch_finalize(f->partials, (int)(f->W / kCellBlock), f->sys_cblk_ptr,
-                              f->sys_cblk_idx, f->nsys, energies, vtens, f->nanflag,
-                              (hipStream_t)stream);
+    e = launch_gather_batch(a, BatchTotals{f->partials, (int)(f->W / kCellBlock), f->nsys,
+                                           f->sys_cblk_ptr, f->sys_cblk_idx, energies, vtens},
+                            (hipStream_t)stream);
   if (e != hipSuccess) return hip_error(e, "batched force kernels");
   return MM_OK;
 }

@@ -67,33 +67,38 @@ __host__ __device__ inline double strain_map(const double* P, int I, int J) {
                             : (I < 3 ? 0.5 * cross : cross);
 }
 
-// K and R of one table entry from h0, P = h0^-1, w and Cv. Shared by the host and the device table
-// builders, without contraction, so both round the same way.
-__host__ __device__ inline void metric_entry(const double* h0, const double* P, double w,
-                                             const double* Cv, double* K, double* R) {
+// Entries IJ of CT = (w Cv) T and of K = T^T CT, and entry I of the rest metric (metric_entry).
+__host__ __device__ inline double stiffness_half(double w, const double* Cv, const double* T, int I,
+                                                 int J) {
+#pragma clang fp contract(off)
+  double t = 0.0;
+  for (int L = 0; L < 6; ++L) t += (w * Cv[6 * I + L]) * T[6 * L + J];
+  return t;
+}
+__host__ __device__ inline double stiffness_entry(const double* T, const double* CT, int I, int J) {
+#pragma clang fp contract(off)
+  double t = 0.0;
+  for (int L = 0; L < 6; ++L) t += T[6 * L + I] * CT[6 * L + J];
+  return t;
+}
+__host__ __device__ inline double rest_entry(const double* h0, int I) {
 #pragma clang fp contract(off)
   const int pi[6] = {0, 1, 2, 1, 0, 0}, pj[6] = {0, 1, 2, 2, 2, 1};
+  const double* a = h0 + 3 * pi[I];
+  const double* b = h0 + 3 * pj[I];
+  const double r = (a[0] * b[0] + a[1] * b[1]) + a[2] * b[2];
+  return I < 3 ? 0.5 * r : r;
+}
+
+// K and R of one table entry from h0, P = h0^-1, w and Cv. Shared by the host and the device table
+// builders, without contraction, so both round the same way.
+inline void metric_entry(const double* h0, const double* P, double w, const double* Cv, double* K,
+                         double* R) {
   double T[36], CT[36];
-  for (int I = 0; I < 6; ++I)
-    for (int J = 0; J < 6; ++J) T[6 * I + J] = strain_map(P, I, J);
-  for (int I = 0; I < 6; ++I)
-    for (int J = 0; J < 6; ++J) {
-      double t = 0.0;
-      for (int L = 0; L < 6; ++L) t += (w * Cv[6 * I + L]) * T[6 * L + J];
-      CT[6 * I + J] = t;
-    }
-  for (int I = 0; I < 6; ++I)
-    for (int J = 0; J < 6; ++J) {
-      double t = 0.0;
-      for (int L = 0; L < 6; ++L) t += T[6 * L + I] * CT[6 * L + J];
-      K[6 * I + J] = t;
-    }
-  for (int I = 0; I < 6; ++I) {
-    const double* a = h0 + 3 * pi[I];
-    const double* b = h0 + 3 * pj[I];
-    const double r = (a[0] * b[0] + a[1] * b[1]) + a[2] * b[2];
-    R[I] = I < 3 ? 0.5 * r : r;
-  }
+  for (int q = 0; q < 36; ++q) T[q] = strain_map(P, q / 6, q % 6);
+  for (int q = 0; q < 36; ++q) CT[q] = stiffness_half(w, Cv, T, q / 6, q % 6);
+  for (int q = 0; q < 36; ++q) K[q] = stiffness_entry(T, CT, q / 6, q % 6);
+  for (int I = 0; I < 6; ++I) R[I] = rest_entry(h0, I);
 }
 
 // Edge endpoints: corner a, axis d -> lower / upper corner of the edge along d through a.

@@ -198,6 +198,47 @@ reduce_items_kernel(ReduceList list, int* __restrict__ nanflag) {
   reduce_item(list.item[blockIdx.x], nanflag);
 }
 
+// Per-system totals of a batch: one block per system sums its own cell blocks in list order.
+__device__ __forceinline__ void batch_totals(const BatchTotals& a, int s,
+                                             int* __restrict__ nanflag) {
+  __shared__ double red[10 * 4];
+  const double* partials = a.partials;
+  const int32_t *sys_ptr = a.sys_ptr, *sys_idx = a.sys_idx;
+  double *energies = a.energies, *vtens = a.vtens;
+  const int nb = a.nb;
+  const int b0 = sys_ptr[s], b1 = sys_ptr[s + 1];
+  double acc[10];
+#pragma unroll
+  for (int q = 0; q < 10; ++q) acc[q] = 0.0;
+  for (int i = b0 + threadIdx.x; i < b1; i += 256) {
+    const int b = sys_idx[i];
+#pragma unroll
+    for (int q = 0; q < 10; ++q) acc[q] += partials[(int64_t)q * nb + b];
+  }
+  wave_reduce<10>(acc);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 0) {
+#pragma unroll
+    for (int q = 0; q < 10; ++q) red[wave * 10 + q] = acc[q];
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int bad = 0;
+    for (int q = 0; q < 10; ++q) {
+      const double t = ((red[q] + red[10 + q]) + red[20 + q]) + red[30 + q];
+      if (t != t) bad |= q == 0 ? 1 : 4;
+      if (q == 0 && energies) energies[s] = t;
+      if (q > 0 && vtens) vtens[9 * (int64_t)s + q - 1] = t;
+    }
+    if (bad) atomicOr(nanflag, bad);
+  }
+}
+
+__global__ void __launch_bounds__(256)
+batch_totals_kernel(BatchTotals a, int* __restrict__ nanflag) {
+  batch_totals(a, blockIdx.x, nanflag);
+}
+
 // gpos[n] (+)= sum_{k=0..7} gcell[k][:][w(n,k)] in fixed k order (mmff.py:303-318). A workgroup
 // owns 256 consecutive nodes; their 768 gpos values (and, with DOT, dir and gold values) move
 // between HBM and LDS in contiguous runs, and each thread takes its node's three from LDS. With
@@ -211,9 +252,13 @@ __global__ void __launch_bounds__(256)
 gather_kernel(const int32_t* __restrict__ ncell, const double* __restrict__ gcell, int64_t N,
               int64_t RS, double* __restrict__ gpos, int accumulate, int* __restrict__ nanflag,
               const double* __restrict__ dir, const double* __restrict__ gold,
-              double* __restrict__ dpart, int gb, ReduceList list) {
+              double* __restrict__ dpart, int gb, ReduceList list, BatchTotals batch) {
   if (!DOT && (int)blockIdx.x >= gb) {
-    reduce_item(list.item[blockIdx.x - gb], nanflag);
+    const int i = (int)blockIdx.x - gb;
+    if (i < list.count)
+      reduce_item(list.item[i], nanflag);
+    else
+      batch_totals(batch, i - list.count, nanflag);
     return;
   }
   __shared__ double sg[768];
@@ -347,26 +392,40 @@ hipError_t launch_cells(const ForceArgs& a, hipStream_t stream) {
 
 template <bool DOT>
 static hipError_t gather(const ForceArgs& a, const double* dir, const double* gold, double* dpart,
-                         const ReduceList& list, hipStream_t stream) {
-  if (a.gpos == nullptr || a.N <= 0 || a.W <= 0) return launch_reduce(list, a.nanflag, stream);
+                         const ReduceList& list, const BatchTotals& batch, hipStream_t stream) {
   const int gb = (int)((a.N + 255) / 256);
-  const dim3 grid(gb + list.count);
+  const dim3 grid(gb + list.count + batch.nsys);
   if (gb <= kGatherAllLoadsMaxBlocks)
     hipLaunchKernelGGL((gather_kernel<DOT, true>), grid, dim3(256), 0, stream, a.ncell, a.gcell,
-                       a.N, a.rstride, a.gpos, a.accumulate, a.nanflag, dir, gold, dpart, gb, list);
+                       a.N, a.rstride, a.gpos, a.accumulate, a.nanflag, dir, gold, dpart, gb, list,
+                       batch);
   else
     hipLaunchKernelGGL((gather_kernel<DOT, false>), grid, dim3(256), 0, stream, a.ncell, a.gcell,
-                       a.N, a.rstride, a.gpos, a.accumulate, a.nanflag, dir, gold, dpart, gb, list);
+                       a.N, a.rstride, a.gpos, a.accumulate, a.nanflag, dir, gold, dpart, gb, list,
+                       batch);
   return hipGetLastError();
 }
 
+static bool no_gather(const ForceArgs& a) { return a.gpos == nullptr || a.N <= 0 || a.W <= 0; }
+
 hipError_t launch_gather(const ForceArgs& a, const ReduceList& list, hipStream_t stream) {
-  return gather<false>(a, nullptr, nullptr, nullptr, list, stream);
+  if (no_gather(a)) return launch_reduce(list, a.nanflag, stream);
+  return gather<false>(a, nullptr, nullptr, nullptr, list, BatchTotals{}, stream);
+}
+
+hipError_t launch_gather_batch(const ForceArgs& a, const BatchTotals& batch, hipStream_t stream) {
+  if (!no_gather(a))
+    return gather<false>(a, nullptr, nullptr, nullptr, ReduceList{}, batch, stream);
+  if (batch.nsys <= 0) return hipSuccess;
+  hipLaunchKernelGGL(batch_totals_kernel, dim3(batch.nsys), dim3(256), 0, stream, batch,
+                     a.nanflag);
+  return hipGetLastError();
 }
 
 hipError_t launch_gather_dot(const ForceArgs& a, const double* dir, const double* gold,
                              double* dpart, hipStream_t stream) {
-  return gather<true>(a, dir, gold, dpart, ReduceList{}, stream);
+  if (no_gather(a)) return hipSuccess;
+  return gather<true>(a, dir, gold, dpart, ReduceList{}, BatchTotals{}, stream);
 }
 
 hipError_t launch_reduce(const ReduceList& list, int* nanflag, hipStream_t stream) {
@@ -625,38 +684,49 @@ hipError_t launch_cg_stats(const double* x, const double* xo, const double* g, c
   return launch_reduce(list, nanflag, stream);
 }
 
-// Parameter table entries (row t, state s) from device arrays, one thread per entry, with the
-// arithmetic of the host builder (Voigt input), so both give the same bits; entries of states
-// beyond nstates[t] are zero. kt[t] = boltzmann * temp_eff[t].
+// Parameter table entries (row t, state s) from device arrays, one wave per entry and one lane per
+// matrix element, with the arithmetic of the host builder (Voigt input, metric_entry), so both give
+// the same bits; entries of states beyond nstates[t] are zero. kt[t] = boltzmann * temp_eff[t]. One
+// thread per entry took 6.5 us, a serial chain of 432 products.
 __global__ void __launch_bounds__(64)
-build_table_kernel(int corner8, int nrows, int max_states, const int32_t* __restrict__ nstates,
+build_table_kernel(int corner8, int max_states, const int32_t* __restrict__ nstates,
                    const double* __restrict__ h0, const double* __restrict__ cv,
                    const double* __restrict__ free_energy, const double* __restrict__ temp_eff,
                    double boltzmann, double* __restrict__ tab, double* __restrict__ kt) {
 #pragma clang fp contract(off)
-  const int ts = (int)blockIdx.x * 64 + threadIdx.x;
-  if (ts >= nrows * max_states) return;
+  __shared__ double P[9], T[36], CT[36], C[36], H[9], W;
+  const int ts = blockIdx.x, q = threadIdx.x;
   const int t = ts / max_states, s = ts % max_states;
   double* e = tab + (int64_t)ts * kTabStride;
-  if (s == 0) kt[t] = boltzmann * temp_eff[t];
+  if (s == 0 && q == 0) kt[t] = boltzmann * temp_eff[t];
   if (s >= nstates[t]) {
-    for (int q = 0; q < kTabStride; ++q) e[q] = 0.0;
+    for (int i = q; i < kTabStride; i += 64) e[i] = 0.0;
     return;
   }
-  double inv[9];
-  const double det = inverse3_cof(h0 + (int64_t)ts * 9, inv);
-#pragma unroll
-  for (int q = 0; q < 9; ++q) e[q] = inv[q];
-  const double w = corner8 ? 0.125 * det : det;
-  e[9] = w;
-  e[10] = free_energy[ts];
-  e[11] = 0.0;
-#pragma unroll
-  for (int q = 0; q < 36; ++q) e[kCvOffset + q] = cv[(int64_t)ts * 36 + q];
-  metric_entry(h0 + (int64_t)ts * 9, inv, w, cv + (int64_t)ts * 36, e + kMetricOffset,
-               e + kRestOffset);
-  e[kRestOffset + 6] = 0.0;
-  e[kRestOffset + 7] = 0.0;
+  if (q < 36) C[q] = cv[(int64_t)ts * 36 + q];
+  if (q < 9) H[q] = h0[(int64_t)ts * 9 + q];
+  __syncthreads();
+  if (q == 0) {
+    double inv[9];
+    const double det = inverse3_cof(H, inv);
+    W = corner8 ? 0.125 * det : det;
+    for (int i = 0; i < 9; ++i) P[i] = inv[i];
+  }
+  __syncthreads();
+  if (q < 36) {
+    T[q] = strain_map(P, q / 6, q % 6);
+    e[kCvOffset + q] = C[q];
+  }
+  if (q < 9) e[q] = P[q];
+  if (q == 9) e[9] = W;
+  if (q == 10) e[10] = free_energy[ts];
+  if (q == 11) e[11] = 0.0;
+  if (q < 6) e[kRestOffset + q] = rest_entry(H, q);
+  if (q == 6 || q == 7) e[kRestOffset + q] = 0.0;
+  __syncthreads();
+  if (q < 36) CT[q] = stiffness_half(W, C, T, q / 6, q % 6);
+  __syncthreads();
+  if (q < 36) e[kMetricOffset + q] = stiffness_entry(T, CT, q / 6, q % 6);
 }
 
 hipError_t launch_build_table(int corner8, int nrows, int max_states, const int32_t* nstates,
@@ -665,54 +735,8 @@ hipError_t launch_build_table(int corner8, int nrows, int max_states, const int3
                               hipStream_t stream) {
   const int n = nrows * max_states;
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(build_table_kernel, dim3((n + 63) / 64), dim3(64), 0, stream, corner8,
-                     nrows, max_states, nstates, h0, cv, free_energy, temp_eff, boltzmann, tab,
-                     kt);
-  return hipGetLastError();
-}
-
-// Per-system totals of a batch: one block per system sums its own cell blocks in list order.
-__global__ void __launch_bounds__(256)
-batch_finalize_kernel(const double* __restrict__ partials, int nb,
-                      const int32_t* __restrict__ sys_ptr, const int32_t* __restrict__ sys_idx,
-                      double* __restrict__ energies, double* __restrict__ vtens,
-                      int* __restrict__ nanflag) {
-  __shared__ double red[10 * 4];
-  const int s = blockIdx.x;
-  const int b0 = sys_ptr[s], b1 = sys_ptr[s + 1];
-  double acc[10];
-#pragma unroll
-  for (int q = 0; q < 10; ++q) acc[q] = 0.0;
-  for (int i = b0 + threadIdx.x; i < b1; i += 256) {
-    const int b = sys_idx[i];
-#pragma unroll
-    for (int q = 0; q < 10; ++q) acc[q] += partials[(int64_t)q * nb + b];
-  }
-  wave_reduce<10>(acc);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-#pragma unroll
-    for (int q = 0; q < 10; ++q) red[wave * 10 + q] = acc[q];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int bad = 0;
-    for (int q = 0; q < 10; ++q) {
-      const double t = ((red[q] + red[10 + q]) + red[20 + q]) + red[30 + q];
-      if (t != t) bad |= q == 0 ? 1 : 4;
-      if (q == 0 && energies) energies[s] = t;
-      if (q > 0 && vtens) vtens[9 * (int64_t)s + q - 1] = t;
-    }
-    if (bad) atomicOr(nanflag, bad);
-  }
-}
-
-hipError_t launch_batch_finalize(const double* partials, int nb, const int32_t* sys_ptr,
-                                 const int32_t* sys_idx, int nsys, double* energies,
-                                 double* vtens, int* nanflag, hipStream_t stream) {
-  if (nsys <= 0) return hipSuccess;
-  hipLaunchKernelGGL(batch_finalize_kernel, dim3(nsys), dim3(256), 0, stream, partials, nb,
-                     sys_ptr, sys_idx, energies, vtens, nanflag);
+  hipLaunchKernelGGL(build_table_kernel, dim3(n), dim3(64), 0, stream, corner8, max_states,
+                     nstates, h0, cv, free_energy, temp_eff, boltzmann, tab, kt);
   return hipGetLastError();
 }
 

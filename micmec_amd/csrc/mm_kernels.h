@@ -8,8 +8,8 @@ namespace mm {
 
 constexpr int kCellBlock = 256;
 // Cell passes of the eight-corner model of more blocks than this run their two instances
-// concurrently; smaller ones, and all of the averaged model, run
-// both kinds of block in one launch (cell_kernel_both).
+// concurrently; smaller ones, and all of the averaged model, run both kinds of block in one launch
+// (cell_kernel_both).
 constexpr int kForkMinBlocks = 512;
 // Node gathers over at most this many 256-node blocks (at most four waves a SIMD) load all of
 // a node's records at once (sum_node_records<true>): latency bounds such a pass. NVT-NHC / NPT
@@ -89,6 +89,14 @@ struct ReduceList {
     item[count++] = ReduceItem{src, n, dst, op, acc, nanbit};
   }
 };
+// Per-system energy and virial of a batch, energies[s] and vtens[9 s] (either may be null), from the
+// partials [10][nb] of its cell blocks.
+struct BatchTotals {
+  const double* partials = nullptr;
+  int nb = 0, nsys = 0;
+  const int32_t *sys_ptr = nullptr, *sys_idx = nullptr;  // CSR of the blocks of every system
+  double *energies = nullptr, *vtens = nullptr;
+};
 hipError_t launch_reduce(const ReduceList& list, int* nanflag, hipStream_t stream);
 
 hipError_t launch_force(const ForceArgs& a, hipStream_t stream);
@@ -110,13 +118,10 @@ hipError_t launch_cg_trial(const double* x, const double* g, double* d, double b
 hipError_t launch_cg_stats(const double* x, const double* xo, const double* g, const double* go,
                            int64_t N, double* part, double* out, int* nanflag,
                            hipStream_t stream);
-// Per-system energy and virial of a batch: energies[s], vtens[9 s] (either may be null).
-hipError_t launch_batch_finalize(const double* partials, int nb, const int32_t* sys_ptr,
-                                 const int32_t* sys_idx, int nsys, double* energies,
-                                 double* vtens, int* nanflag, hipStream_t stream);
 // Node gather of gcell into gpos (overwrite or accumulate, as a.accumulate), with the reductions of
 // list (of what earlier launches wrote) in the same launch.
 hipError_t launch_gather(const ForceArgs& a, const ReduceList& list, hipStream_t stream);
+hipError_t launch_gather_batch(const ForceArgs& a, const BatchTotals& batch, hipStream_t stream);
 // dst[0..n) = src[0..n), src mapped host memory.
 hipError_t launch_stage(const double* src, double* dst, int64_t n, hipStream_t stream);
 // Cell kernel only: per-cell gradients into gcell, energy/virial block partials.
