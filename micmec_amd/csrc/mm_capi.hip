@@ -699,11 +699,10 @@ int mm_field_launch_cells(mm_field* f, const double* pos, const double* rvecs, v
   return MM_OK;
 }
 
-// Copy n results from the device to host_out through the object's pinned staging, after the
-// work queued on the stream (a synchronising read).
-static int read_results(mm_field* f, const double* out, double* host_out, int n, hipStream_t s) {
-  hipError_t e = hipMemcpyAsync(f->cghost, out, sizeof(double) * n, hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
+// The n results that the reduction wrote to the object's pinned staging as well: wait for the stream
+// and hand them on (no copy command, 5 us of a trial).
+static int read_results(mm_field* f, double* host_out, int n, hipStream_t s) {
+  const hipError_t e = hipStreamSynchronize(s);
   if (e != hipSuccess) return hip_error(e, "reading line-search results");
   std::memcpy(host_out, f->cghost, sizeof(double) * n);
   return MM_OK;
@@ -737,16 +736,20 @@ int mm_cg_trial(mm_field* f, const double* x, const double* g, double* d, double
   if (e == hipSuccess) e = launch_gather_dot(a, d, g, gpart, s);
   if (e == hipSuccess) {
     ReduceList list;
+    double* h = host_out ? f->cghost : nullptr;
+    auto host = [&](int q) { return h ? h + q : nullptr; };
     add_force_totals(list, a, (int)(f->W / kCellBlock));
+    list.item[0].host = host(0);
     const int maxop = nbn > 0 ? kReduceMax : kReduceSum;  // an empty maximum is 0
     for (int q = 0; q < 4; ++q)
-      list.add(gpart + q * nbn, nbn, q < 3 ? kReduceSum : maxop, out + 1 + q, 0, MM_NAN_GPOS);
-    list.add(tpart, nbn, kReduceSum, out + 5, 0, 0);
-    list.add(tpart + nbn, nbn, maxop, out + 6, 0, 0);
+      list.add(gpart + q * nbn, nbn, q < 3 ? kReduceSum : maxop, out + 1 + q, 0, MM_NAN_GPOS,
+               host(1 + q));
+    list.add(tpart, nbn, kReduceSum, out + 5, 0, 0, host(5));
+    list.add(tpart + nbn, nbn, maxop, out + 6, 0, 0, host(6));
     e = launch_reduce(list, f->nanflag, s);
   }
   if (e != hipSuccess) return hip_error(e, "line-search trial kernels");
-  return host_out ? read_results(f, out, host_out, 7, s) : MM_OK;
+  return host_out ? read_results(f, host_out, 7, s) : MM_OK;
 }
 
 int mm_cg_stats(mm_field* f, const double* x, const double* x_old, const double* g,
@@ -759,14 +762,16 @@ int mm_cg_stats(mm_field* f, const double* x, const double* x_old, const double*
   hipStream_t s = (hipStream_t)stream;
   hipError_t e;
   if (f->N > 0) {
-    e = launch_cg_stats(x, x_old, g, g_old, f->N, f->cgpart, out, f->nanflag, s);
+    e = launch_cg_stats(x, x_old, g, g_old, f->N, f->cgpart, out, host_out ? f->cghost : nullptr,
+                        f->nanflag, s);
   } else {
     ReduceList list;  // empty sums: five zeros
-    for (int q = 0; q < 5; ++q) list.add(f->cgpart, 0, kReduceSum, out + q, 0, 0);
+    for (int q = 0; q < 5; ++q)
+      list.add(f->cgpart, 0, kReduceSum, out + q, 0, 0, host_out ? f->cghost + q : nullptr);
     e = launch_reduce(list, f->nanflag, s);
   }
   if (e != hipSuccess) return hip_error(e, "line-search statistics kernels");
-  return host_out ? read_results(f, out, host_out, 5, s) : MM_OK;
+  return host_out ? read_results(f, host_out, 5, s) : MM_OK;
 }
 
 int mm_field_info(const mm_field* f, int64_t* ncells, int64_t* nnodes, int64_t* nslots) {

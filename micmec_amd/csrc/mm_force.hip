@@ -188,6 +188,7 @@ __device__ __forceinline__ void reduce_item(const ReduceItem it, int* __restrict
     for (int w = 1; w < 4; ++w) t = is_max ? nan_max(t, red[w]) : t + red[w];
     if (it.acc) t += it.dst[0];
     it.dst[0] = t;
+    if (it.host) *it.host = t;
     if (t != t && it.nanbit) atomicOr(nanflag, it.nanbit);
   }
 }
@@ -671,7 +672,7 @@ cg_stats_kernel(const double* __restrict__ x, const double* __restrict__ xo,
 }
 
 hipError_t launch_cg_stats(const double* x, const double* xo, const double* g, const double* go,
-                           int64_t N, double* part, double* out, int* nanflag,
+                           int64_t N, double* part, double* out, double* host, int* nanflag,
                            hipStream_t stream) {
   if (N <= 0) return hipSuccess;
   const int nb = (int)((N + 255) / 256);
@@ -680,7 +681,8 @@ hipError_t launch_cg_stats(const double* x, const double* xo, const double* g, c
   if (e != hipSuccess) return e;
   ReduceList list;
   for (int q = 0; q < 5; ++q)
-    list.add(part + (int64_t)q * nb, nb, q < 3 ? kReduceSum : kReduceMax, out + q, 0, 0);
+    list.add(part + (int64_t)q * nb, nb, q < 3 ? kReduceSum : kReduceMax, out + q, 0, 0,
+             host ? host + q : nullptr);
   return launch_reduce(list, nanflag, stream);
 }
 

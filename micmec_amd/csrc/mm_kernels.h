@@ -81,12 +81,14 @@ struct ReduceItem {
   int op;      // kReduceSum (fixed order) or kReduceMax (NaN-propagating)
   int acc;     // add the total to dst[0] instead of overwriting it
   int nanbit;  // bit set in the NaN flag when the total is NaN (0: none)
+  double* host;  // mapped host memory that takes the result too (null: none)
 };
 struct ReduceList {
   ReduceItem item[kReduceItems];
   int count = 0;
-  void add(const double* src, int64_t n, int op, double* dst, int acc, int nanbit) {
-    item[count++] = ReduceItem{src, n, dst, op, acc, nanbit};
+  void add(const double* src, int64_t n, int op, double* dst, int acc, int nanbit,
+           double* host = nullptr) {
+    item[count++] = ReduceItem{src, n, dst, op, acc, nanbit, host};
   }
 };
 // Per-system energy and virial of a batch, energies[s] and vtens[9 s] (either may be null), from the
@@ -114,9 +116,10 @@ hipError_t launch_cg_trial(const double* x, const double* g, double* d, double b
                            double alpha, double* xa, int64_t N, double* part,
                            hipStream_t stream);
 // out[0..5) = sum_n |g_n|^2, sum_n g_n . go_n, sum_n |x_n - xo_n|^2, max_n |g_n|^2,
-// max_n |x_n - xo_n|^2 over N nodes of 3 values; part holds 5 (N + 255) / 256 doubles.
+// max_n |x_n - xo_n|^2 over N nodes of 3 values; part holds 5 (N + 255) / 256 doubles; host (mapped
+// host memory or null) takes the results too.
 hipError_t launch_cg_stats(const double* x, const double* xo, const double* g, const double* go,
-                           int64_t N, double* part, double* out, int* nanflag,
+                           int64_t N, double* part, double* out, double* host, int* nanflag,
                            hipStream_t stream);
 // Node gather of gcell into gpos (overwrite or accumulate, as a.accumulate), with the reductions of
 // list (of what earlier launches wrote) in the same launch.

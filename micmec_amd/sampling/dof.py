@@ -242,21 +242,32 @@ class CartesianDOF(DOF):
         self.th_gpos_rms = gpos_rms
         self.th_dpos_rms = dpos_rms
         self.select = select
-        DOF.__init__(self, mmf)
-        self._last_pos = None
-        self._last_pos_dev = None
-        self._cg_engine = None
         try:
             self._device = _DeviceEnergy(mmf)
         except NotImplementedError:
             self._device = None
+        DOF.__init__(self, mmf)
+        self._last_pos = None
+        self._last_pos_dev = None
+        self._cg_engine = None
 
     def _init_initial(self):
         pos = np.asarray(self.mmf.system.pos)
-        self.x0 = (pos.ravel() if self.select is None else pos[self.select].ravel()).copy()
-        self._pos = pos.copy()
+        if self._device is not None and self.select is None and pos.dtype == np.float64:
+            # Pinned arrays: a copy from or to the device is one DMA transfer, and torch's host
+            # allocator hands their pages out again, where fresh pages of 24 B a node are faulted
+            # in one by one (48^3 nodes: some 0.2 ms an array).
+            self._pos_pin = torch.empty(pos.shape, dtype=torch.float64, pin_memory=True)
+            self._gpos_pin = torch.zeros(pos.shape, dtype=torch.float64, pin_memory=True)
+            self._pos, self._gpos = self._pos_pin.numpy(), self._gpos_pin.numpy()
+            self._pos[...] = pos
+            self.x0 = torch.empty(pos.size, dtype=torch.float64, pin_memory=True).numpy()
+            self.x0[...] = pos.ravel()
+        else:
+            self.x0 = (pos.ravel() if self.select is None else pos[self.select].ravel()).copy()
+            self._pos = pos.copy()
+            self._gpos = np.zeros(pos.shape, float)
         self._dpos = np.zeros(pos.shape, float)
-        self._gpos = np.zeros(pos.shape, float)
 
     @property
     def device(self):
@@ -279,7 +290,6 @@ class CartesianDOF(DOF):
                 not (isinstance(x0, torch.Tensor) and x0.is_cuda):
             return None
         self._cg_engine = _DeviceCGEngine(self, x0)
-        self._pin_host_arrays()  # made before the run: page-locking 2 x 24 B per node is slow
         return self._cg_engine
 
     def fun(self, x, do_gradient=False):
@@ -323,15 +333,6 @@ class CartesianDOF(DOF):
                 self._gpos[:] = np.asarray(g).reshape(-1, 3)
             else:
                 self._gpos[self.select] = np.asarray(g).reshape(-1, 3)
-
-    def _pin_host_arrays(self):
-        """Back the host position and gradient arrays with pinned memory, so that a copy from
-        the device is one DMA transfer straight into them."""
-        if getattr(self, "_pos_pin", None) is None:
-            self._pos_pin = torch.from_numpy(self._pos).pin_memory()
-            self._gpos_pin = torch.from_numpy(self._gpos).pin_memory()
-            self._pos = self._pos_pin.numpy()
-            self._gpos = self._gpos_pin.numpy()
 
     def sync_from_device(self):
         """Copy the last device positions and gradient into the host arrays and the system."""

@@ -10,6 +10,7 @@ one launch of the HIP force kernels; only scalars return to the host.
 """
 
 import time
+import weakref
 from math import isfinite
 
 import numpy as np
@@ -255,7 +256,11 @@ class CGOptimizer(BaseOptimizer):
                                  device=dof.device)
             make = getattr(dof, "cg_engine", None)
             engine = make(x0) if make is not None else None
-        self.minimizer = ConjugateGradientSearch(x0, self.fun, engine=engine)
+        # The search holds its optimiser weakly: without a cycle the arrays of a finished run are
+        # free at once, and the next run finds their (pinned) pages in the allocators.
+        this = weakref.ref(self)
+        self.minimizer = ConjugateGradientSearch(
+            x0, lambda x, do_gradient=False: (this() or dof).fun(x, do_gradient), engine=engine)
         BaseOptimizer.__init__(self, dof, state, hooks, counter0)
 
     def initialize(self):
