@@ -140,12 +140,12 @@ __device__ __forceinline__ void wave_sums(Quantity q, Put put) {
   }
 }
 
-// Strain x of the i-th corner in the metric of the edges (Gram entries less the rest metric R,
-// halved on the diagonal) from the edges E and their strains q against the rest metric R0 of the
-// type's first state, its stress K x: the diagonal entries added to their edges' D, the others
+// Strain x of the i-th corner in the metric of the edges (Gram entries less the rest metric,
+// halved on the diagonal) from the edges E and their strains q against that of the type's first
+// state, its stress K x: the diagonal entries added to their edges' D, the others
 // in O; returns x . K x.
 template <typename T, int kModel>
-__device__ __forceinline__ T adjoint_corner(const const_f64 ts, const const_f64 R0, int i,
+__device__ __forceinline__ T adjoint_corner(const const_f64 ts, int i,
                                             const T (&E)[Frame<kModel>::NE][3],
                                             const T (&q)[Frame<kModel>::NE], T (&x)[6],
                                             T (&D)[Frame<kModel>::NE], T (&O)[3]) {
@@ -153,7 +153,7 @@ __device__ __forceinline__ T adjoint_corner(const const_f64 ts, const const_f64 
   const const_f64 K = ts + kMetricOffset, R = ts + kRestOffset;
   const int a = F::corner(i);
 #pragma unroll
-  for (int d = 0; d < 3; ++d) x[d] = q[F::edge(a, d)] + (R0[d] - R[d]);
+  for (int d = 0; d < 3; ++d) x[d] = q[F::edge(a, d)] + ts[kShiftOffset + d];
 #pragma unroll
   for (int o = 0; o < 3; ++o) {
     const T(&A)[3] = E[F::edge(a, F::axis0(o))];
@@ -209,7 +209,7 @@ __device__ __forceinline__ void adjoint_states(const const_f64 tab, int ns, doub
 #pragma unroll
       for (int i = 0; i < NC; ++i) {
         T x[6], O[3];
-        u = u + adjoint_corner<T, kModel>(ts, tab + kRestOffset, i, E, sq, x, D, O);
+        u = u + adjoint_corner<T, kModel>(ts, i, E, sq, x, D, O);
         fence(u);
       }
       const T es = 0.5 * u + ts[10];
@@ -244,7 +244,7 @@ __device__ __forceinline__ void adjoint_states(const const_f64 tab, int ns, doub
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
       T x[6], O[3];
-      u = u + adjoint_corner<T, kModel>(ts, tab + kRestOffset, i, E, sq, x, D, O);
+      u = u + adjoint_corner<T, kModel>(ts, i, E, sq, x, D, O);
 #pragma unroll
       for (int q = 0; q < 21; ++q)
         X2[q] = i == 0 ? x[kUpperI[q]] * x[kUpperJ[q]] : mad(x[kUpperI[q]], x[kUpperJ[q]], X2[q]);
@@ -347,8 +347,9 @@ adjoint_kernel(const double* __restrict__ pos, const double* __restrict__ dpos,
                                         (t[(4 * e + 2) % 12][j] + t[(4 * e + 3) % 12][j]));
       // the strain (E.E)/2 - R, the sum begun as in edge_strain
       const int d = F::along(e), b = d == 0 ? 1 : 0, c = d == 2 ? 1 : 2;
-      const T r = make<T>(-2.0 * tab[kRestOffset + d], 0.0);
-      sq[e] = 0.5 * mad(E[e][c], E[e][c], mad(E[e][b], E[e][b], mad(E[e][d], E[e][d], r)));
+      const T r = make<T>(-tab[kRestOffset + d], 0.0);
+      sq[e] = mad(0.5, mad(E[e][c], E[e][c], mad(E[e][b], E[e][b], mad(E[e][d], E[e][d], r))),
+                  make<T>(-tab[kRestLowOffset + d], 0.0));
     }
   }
 
@@ -566,8 +567,8 @@ metric_entries_kernel(const double* __restrict__ tab, const int32_t* __restrict_
     for (int m = 0; m < 3; ++m)
       for (int n = 0; n < 3; ++n) {
         const int sm = kVoigt[3 * a + m], gn = kVoigt[3 * n + k];
-        const double sg = B[h][sm] * R[gn] + Q[h][6 * sm + gn];
-        v += P[3 * m + n] * (n == k ? 2.0 * sg : sg);
+        const double q = Q[h][6 * sm + gn];
+        v += P[3 * m + n] * (B[h][sm] * R[gn] + (n == k ? 2.0 * q : q));
       }
     v *= w;
   } else if (i == 30) {

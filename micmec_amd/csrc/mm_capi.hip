@@ -89,7 +89,9 @@ int build_param_table(int model, int32_t nrows, int32_t max_states, const int32_
       } else {
         voigt_average(c0 + ts * 81, e + kCvOffset);
       }
-      metric_entry(h0 + ts * 9, e, e[9], e + kCvOffset, e + kMetricOffset, e + kRestOffset);
+      const size_t t0 = (size_t)t * max_states;  // the type's first state, built before
+      metric_entry(h0 + ts * 9, e, e[9], e + kCvOffset, h0 + t0 * 9, &tab[t0 * kTabStride],
+                   e + kMetricOffset, e + kRestOffset);
     }
   }
   return MM_OK;

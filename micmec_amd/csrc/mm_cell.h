@@ -118,9 +118,10 @@ __device__ __forceinline__ void cell_eval(const_f64 tab, int ns, double kt, bool
       form_edges<kModel>(p, f, rv, E);
 #pragma unroll
       for (int e = 0; e < F::NE; ++e)
-        q[e] = edge_strain(E[e], F::along(e), tab[kRestOffset + F::along(e)]);
+        q[e] = edge_strain(E[e], F::along(e), tab[kRestOffset + F::along(e)],
+                           tab[kRestLowOffset + F::along(e)]);
       if (!kMulti) {
-        ecell = tab[10] + state_stress<kModel>(tab, tab + kRestOffset, E, q, D, O);
+        ecell = tab[10] + state_stress<kModel>(tab, E, q, D, O);
       } else {
         // one pass over the states (mmff.py:386-398): E = E_min - kT ln Z with Z = sum_s c_s,
         // c_s = exp(-(E_s - E_min)/kT), and the stresses sum_s c_s S_s accumulated in LDS, both
@@ -128,7 +129,7 @@ __device__ __forceinline__ void cell_eval(const_f64 tab, int ns, double kt, bool
         double emin = 0.0, zsum = 0.0;
         for (int s = 0; s < ns; ++s) {
           const const_f64 ts = tab + s * kTabStride;
-          const double es = ts[10] + state_stress<kModel>(ts, tab + kRestOffset, E, q, D, O);
+          const double es = ts[10] + state_stress<kModel>(ts, E, q, D, O);
           double keep = 0.0, c = 1.0;  // factors of the sums so far and of this state
           if (s == 0) {
             emin = es;

@@ -22,12 +22,15 @@ namespace mm {
 //   [11]     unused
 //   [12..47] Voigt matrix Cv[6][6] (row-major), averaged over index orderings
 //   [48..83] K = T^T (w Cv) T, the weighted matrix of the force kernels (metric_entry)
-//   [84..89] rest metric R = h0 h0^T: R00/2, R11/2, R22/2, R12, R02, R01
-//   [90..91] unused
-constexpr int kTabStride = 92;
+//   [84..89] rest metric R (rest_entry): R00, R11, R22, R12, R02, R01
+//   [90..92] half of what the first three lack to R00, R11, R22
+//   [93..95] the diagonal of R/2 of the type's first state less this state's
+constexpr int kTabStride = 96;
 constexpr int kCvOffset = 12;
 constexpr int kMetricOffset = 48;
 constexpr int kRestOffset = 84;
+constexpr int kRestLowOffset = 90;
+constexpr int kShiftOffset = 93;
 
 // Tables that no kernel of a launch writes: read with scalar loads wherever the index is uniform,
 // also where other memory changes during the launch.
@@ -67,7 +70,7 @@ __host__ __device__ inline double strain_map(const double* P, int I, int J) {
                             : (I < 3 ? 0.5 * cross : cross);
 }
 
-// Entries IJ of CT = (w Cv) T and of K = T^T CT, and entry I of the rest metric (metric_entry).
+// Entries IJ of CT = (w Cv) T and of K = T^T CT.
 __host__ __device__ inline double stiffness_half(double w, const double* Cv, const double* T, int I,
                                                  int J) {
 #pragma clang fp contract(off)
@@ -81,24 +84,67 @@ __host__ __device__ inline double stiffness_entry(const double* T, const double*
   for (int L = 0; L < 6; ++L) t += T[6 * L + I] * CT[6 * L + J];
   return t;
 }
-__host__ __device__ inline double rest_entry(const double* h0, int I) {
+// start + sum_k a[k sa] b[k sb] as the sum of the result and lo, from exact products and sums.
+__host__ __device__ inline double dot3_exact(const double* a, int sa, const double* b, int sb,
+                                             double start, double& lo) {
+#pragma clang fp contract(off)
+  double s = start, c = 0.0;
+  for (int k = 0; k < 3; ++k) {
+    const double p = a[k * sa] * b[k * sb], e = __builtin_fma(a[k * sa], b[k * sb], -p);
+    const double t = s + p, z = t - s;
+    c += ((s - (t - z)) + (p - z)) + e;
+    s = t;
+  }
+  lo = c;
+  return s;
+}
+// R is the metric that P, rounded as it is, takes to the identity, R = P^-1 P^-T: with the rounding
+// of h0 h0^T in its place every cell would carry the same strain of 1e-17, which a virial of
+// small strains of either sign does not average out. P h0 = I + E, so to first order in E (1e-16)
+// R = h0 h0^T - h0 (E + E^T) h0^T. Returns the entry rounded, half of the rest in lo.
+__host__ __device__ inline double rest_entry(const double* h0, const double* P, int I, double& lo) {
 #pragma clang fp contract(off)
   const int pi[6] = {0, 1, 2, 1, 0, 0}, pj[6] = {0, 1, 2, 2, 2, 1};
+  double E[9], l;
+  for (int q = 0; q < 9; ++q) {
+    E[q] = dot3_exact(P + 3 * (q / 3), 1, h0 + q % 3, 3, q % 4 == 0 ? -1.0 : 0.0, l);
+    E[q] += l;
+  }
   const double* a = h0 + 3 * pi[I];
   const double* b = h0 + 3 * pj[I];
-  const double r = (a[0] * b[0] + a[1] * b[1]) + a[2] * b[2];
-  return I < 3 ? 0.5 * r : r;
+  double c = 0.0;
+  for (int m = 0; m < 3; ++m)
+    for (int n = 0; n < 3; ++n) c += a[m] * (E[3 * m + n] + E[3 * n + m]) * b[n];
+  const double r = dot3_exact(a, 1, b, 1, 0.0, l);
+  l -= c;
+  const double hi = r + l;
+  lo = 0.5 * ((r - hi) + l);
+  return hi;
+}
+// Entry d of the shift: R/2 of the first state (h00, P00) less R/2 of this one.
+__host__ __device__ inline double shift_entry(const double* h00, const double* P00,
+                                              const double* h0, const double* P, int d) {
+#pragma clang fp contract(off)
+  double l0, l1;
+  const double r0 = rest_entry(h00, P00, d, l0), r1 = rest_entry(h0, P, d, l1);
+  return 0.5 * (r0 - r1) + (l0 - l1);
 }
 
-// K and R of one table entry from h0, P = h0^-1, w and Cv. Shared by the host and the device table
-// builders, without contraction, so both round the same way.
-inline void metric_entry(const double* h0, const double* P, double w, const double* Cv, double* K,
-                         double* R) {
+// K (36) and the rest entries (12, from kRestOffset) of a table entry from h0, P = h0^-1, w and Cv, and
+// those of the type's first state. Shared by the host and the device table builders, without
+// contraction, so both round the same way.
+inline void metric_entry(const double* h0, const double* P, double w, const double* Cv,
+                         const double* h00, const double* P00, double* K, double* R) {
   double T[36], CT[36];
   for (int q = 0; q < 36; ++q) T[q] = strain_map(P, q / 6, q % 6);
   for (int q = 0; q < 36; ++q) CT[q] = stiffness_half(w, Cv, T, q / 6, q % 6);
   for (int q = 0; q < 36; ++q) K[q] = stiffness_entry(T, CT, q / 6, q % 6);
-  for (int I = 0; I < 6; ++I) R[I] = rest_entry(h0, I);
+  double lo;
+  for (int I = 0; I < 6; ++I) R[I] = rest_entry(h0, P, I, lo);
+  for (int d = 0; d < 3; ++d) {
+    (void)rest_entry(h0, P, d, R[kRestLowOffset - kRestOffset + d]);
+    R[kShiftOffset - kRestOffset + d] = shift_entry(h00, P00, h0, P, d);
+  }
 }
 
 // Edge endpoints: corner a, axis d -> lower / upper corner of the edge along d through a.
@@ -183,23 +229,24 @@ __device__ __forceinline__ double edge_dot(const double (&A)[3], const double (&
 #pragma clang fp contract(off)
   return __builtin_fma(A[2], B[2], __builtin_fma(A[1], B[1], __builtin_fma(A[0], B[0], -g0)));
 }
-// Diagonal strain of an edge along d against half its rest metric g0: (A.A)/2 - g0, the sum begun
-// with the component along d less 2 g0. That product is exact inside the fused multiply-add, so
-// where the rest cell is near the axes the error is relative to the strain, not to the edge.
-__device__ __forceinline__ double edge_strain(const double (&A)[3], int d, double g0) {
+// Diagonal strain of an edge along d against its rest metric g0 + 2 lo: (A.A - g0)/2 - lo, the sum
+// begun with the component along d less g0. That product is exact inside the fused multiply-add,
+// so where the rest cell is near the axes the error is relative to the strain, not to the edge.
+__device__ __forceinline__ double edge_strain(const double (&A)[3], int d, double g0, double lo) {
 #pragma clang fp contract(off)
   const int b = d == 0 ? 1 : 0, c = d == 2 ? 1 : 2;
-  return 0.5 * __builtin_fma(A[c], A[c],
-                             __builtin_fma(A[b], A[b], __builtin_fma(A[d], A[d], -2.0 * g0)));
+  const double t = __builtin_fma(A[c], A[c],
+                                 __builtin_fma(A[b], A[b], __builtin_fma(A[d], A[d], -g0)));
+  return __builtin_fma(0.5, t, -lo);
 }
 
 // Energy (weighted, without the free-energy offset) and stress of one (type, state) at all
-// corners, from the edges E and their strains q against the rest metric r0 of the type's first
+// corners, from the edges E and their strains q against the rest metric of the type's first
 // state: D[e] = the diagonal stress along edge e summed over its corners, O[a][q] the
 // off-diagonal stresses of corner a. The sums are fused
 // multiply-adds in a fixed order, so every kernel that evaluates a state gets the same bits.
 template <int kModel>
-__device__ __forceinline__ double state_stress(const_f64 tab, const_f64 r0,
+__device__ __forceinline__ double state_stress(const_f64 tab,
                                                const double (&E)[Frame<kModel>::NE][3],
                                                const double (&q)[Frame<kModel>::NE],
                                                double (&D)[Frame<kModel>::NE],
@@ -213,7 +260,7 @@ __device__ __forceinline__ double state_stress(const_f64 tab, const_f64 r0,
     const int a = F::corner(i);
     double x[6];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) x[d] = q[F::edge(a, d)] + (r0[d] - g0[d]);
+    for (int d = 0; d < 3; ++d) x[d] = q[F::edge(a, d)] + tab[kShiftOffset + d];
 #pragma unroll
     for (int o = 0; o < 3; ++o)
       x[3 + o] = edge_dot(E[F::edge(a, F::axis0(o))], E[F::edge(a, F::axis1(o))], g0[3 + o]);
@@ -328,7 +375,7 @@ __device__ __forceinline__ double sweep_cell(const_f64 tab,
       const int e = F::edge(a, d);
       if (F::first(e) == i) {
         form_edge(p, e, f[d], &rv[3 * d], E[e]);
-        q[e] = edge_strain(E[e], d, g0[d]);
+        q[e] = edge_strain(E[e], d, g0[d], tab[kRestLowOffset + d]);
       }
       x[d] = q[e];
     }

@@ -42,9 +42,9 @@ namespace mm {
 // gradient too); the energies and virials of all three are the same bits. The latter two take the
 // node positions through the pending transforms xmat (and xmat2 first, when its flag is set) when
 // they are given: a barostat call whose position scaling is stored by a later node pass.
-// The single-state instance sweeps the corners (sweep_cell) in 168 VGPRs, three waves a SIMD (156
+// The single-state instance sweeps the corners (sweep_cell) in 165 VGPRs, three waves a SIMD (148
 // without the gradient); the multistate one keeps the stresses of all corners for the state sum
-// (239 VGPRs and 72 KB of LDS a block, two waves). The compiler's default scheduler is the one that
+// (219 VGPRs and 72 KB of LDS a block, two waves). The compiler's default scheduler is the one that
 // keeps both free of spills. HBM bounds the gradient pass: about 450 MB at 128^3 (20% two-state,
 // 5% empty) in 100 us, with 1000 / 1800 VALU instructions a wave (60 us of issue); the form
 // with B = P M per corner took 1735 / 4000 and 150 us, and 120 us for the pass without
@@ -696,7 +696,7 @@ build_table_kernel(int corner8, int max_states, const int32_t* __restrict__ nsta
                    const double* __restrict__ free_energy, const double* __restrict__ temp_eff,
                    double boltzmann, double* __restrict__ tab, double* __restrict__ kt) {
 #pragma clang fp contract(off)
-  __shared__ double P[9], T[36], CT[36], C[36], H[9], W;
+  __shared__ double P[9], T[36], CT[36], C[36], H[9], H0[9], P0[9], W;
   const int ts = blockIdx.x, q = threadIdx.x;
   const int t = ts / max_states, s = ts % max_states;
   double* e = tab + (int64_t)ts * kTabStride;
@@ -706,13 +706,16 @@ build_table_kernel(int corner8, int max_states, const int32_t* __restrict__ nsta
     return;
   }
   if (q < 36) C[q] = cv[(int64_t)ts * 36 + q];
-  if (q < 9) H[q] = h0[(int64_t)ts * 9 + q];
+  if (q < 9) {
+    H[q] = h0[(int64_t)ts * 9 + q];
+    H0[q] = h0[(int64_t)t * max_states * 9 + q];
+  }
   __syncthreads();
-  if (q == 0) {
+  if (q < 2) {  // this state's inverse and the first one's
     double inv[9];
-    const double det = inverse3_cof(H, inv);
-    W = corner8 ? 0.125 * det : det;
-    for (int i = 0; i < 9; ++i) P[i] = inv[i];
+    const double det = inverse3_cof(q == 0 ? H : H0, inv);
+    if (q == 0) W = corner8 ? 0.125 * det : det;
+    for (int i = 0; i < 9; ++i) (q == 0 ? P : P0)[i] = inv[i];
   }
   __syncthreads();
   if (q < 36) {
@@ -723,8 +726,14 @@ build_table_kernel(int corner8, int max_states, const int32_t* __restrict__ nsta
   if (q == 9) e[9] = W;
   if (q == 10) e[10] = free_energy[ts];
   if (q == 11) e[11] = 0.0;
-  if (q < 6) e[kRestOffset + q] = rest_entry(H, q);
-  if (q == 6 || q == 7) e[kRestOffset + q] = 0.0;
+  if (q < 6) {
+    double lo;
+    e[kRestOffset + q] = rest_entry(H, P, q, lo);
+    if (q < 3) {
+      e[kRestLowOffset + q] = lo;
+      e[kShiftOffset + q] = shift_entry(H0, P0, H, P, q);
+    }
+  }
   __syncthreads();
   if (q < 36) CT[q] = stiffness_half(W, C, T, q / 6, q % 6);
   __syncthreads();
