@@ -102,17 +102,18 @@ __host__ __device__ inline double dot3_exact(const double* a, int sa, const doub
 // of h0 h0^T in its place every cell would carry the same strain of 1e-17, which a virial of
 // small strains of either sign does not average out. P h0 = I + E, so to first order in E (1e-16)
 // R = h0 h0^T - h0 (E + E^T) h0^T. Returns the entry rounded, half of the rest in lo.
-__host__ __device__ inline double rest_entry(const double* h0, const double* P, int I, double& lo) {
+__host__ __device__ inline double inverse_residual(const double* P, const double* h0, int q) {
+#pragma clang fp contract(off)
+  double lo;  // entry q of E
+  const double hi = dot3_exact(P + 3 * (q / 3), 1, h0 + q % 3, 3, q % 4 == 0 ? -1.0 : 0.0, lo);
+  return hi + lo;
+}
+__host__ __device__ inline double rest_entry(const double* h0, const double* E, int I, double& lo) {
 #pragma clang fp contract(off)
   const int pi[6] = {0, 1, 2, 1, 0, 0}, pj[6] = {0, 1, 2, 2, 2, 1};
-  double E[9], l;
-  for (int q = 0; q < 9; ++q) {
-    E[q] = dot3_exact(P + 3 * (q / 3), 1, h0 + q % 3, 3, q % 4 == 0 ? -1.0 : 0.0, l);
-    E[q] += l;
-  }
   const double* a = h0 + 3 * pi[I];
   const double* b = h0 + 3 * pj[I];
-  double c = 0.0;
+  double c = 0.0, l;
   for (int m = 0; m < 3; ++m)
     for (int n = 0; n < 3; ++n) c += a[m] * (E[3 * m + n] + E[3 * n + m]) * b[n];
   const double r = dot3_exact(a, 1, b, 1, 0.0, l);
@@ -121,12 +122,9 @@ __host__ __device__ inline double rest_entry(const double* h0, const double* P, 
   lo = 0.5 * ((r - hi) + l);
   return hi;
 }
-// Entry d of the shift: R/2 of the first state (h00, P00) less R/2 of this one.
-__host__ __device__ inline double shift_entry(const double* h00, const double* P00,
-                                              const double* h0, const double* P, int d) {
+// Half of the first state's diagonal entry r0, l0 less this one's r1, l1.
+__host__ __device__ inline double rest_shift(double r0, double l0, double r1, double l1) {
 #pragma clang fp contract(off)
-  double l0, l1;
-  const double r0 = rest_entry(h00, P00, d, l0), r1 = rest_entry(h0, P, d, l1);
   return 0.5 * (r0 - r1) + (l0 - l1);
 }
 
@@ -139,11 +137,17 @@ inline void metric_entry(const double* h0, const double* P, double w, const doub
   for (int q = 0; q < 36; ++q) T[q] = strain_map(P, q / 6, q % 6);
   for (int q = 0; q < 36; ++q) CT[q] = stiffness_half(w, Cv, T, q / 6, q % 6);
   for (int q = 0; q < 36; ++q) K[q] = stiffness_entry(T, CT, q / 6, q % 6);
-  double lo;
-  for (int I = 0; I < 6; ++I) R[I] = rest_entry(h0, P, I, lo);
-  for (int d = 0; d < 3; ++d) {
-    (void)rest_entry(h0, P, d, R[kRestLowOffset - kRestOffset + d]);
-    R[kShiftOffset - kRestOffset + d] = shift_entry(h00, P00, h0, P, d);
+  double E[9], E0[9], lo, lo0;
+  for (int q = 0; q < 9; ++q) {
+    E[q] = inverse_residual(P, h0, q);
+    E0[q] = inverse_residual(P00, h00, q);
+  }
+  for (int I = 0; I < 6; ++I) {
+    R[I] = rest_entry(h0, E, I, lo);
+    if (I >= 3) continue;
+    const double r0 = rest_entry(h00, E0, I, lo0);
+    R[kRestLowOffset - kRestOffset + I] = lo;
+    R[kShiftOffset - kRestOffset + I] = rest_shift(r0, lo0, R[I], lo);
   }
 }
 

@@ -688,15 +688,18 @@ hipError_t launch_cg_stats(const double* x, const double* xo, const double* g, c
 
 // Parameter table entries (row t, state s) from device arrays, one wave per entry and one lane per
 // matrix element, with the arithmetic of the host builder (Voigt input, metric_entry), so both give
-// the same bits; entries of states beyond nstates[t] are zero. kt[t] = boltzmann * temp_eff[t]. One
-// thread per entry took 6.5 us, a serial chain of 432 products.
+// the same bits; entries of states beyond nstates[t] are zero. kt[t] = boltzmann * temp_eff[t]. A
+// serial chain bounds it, the inverse and its residual above all: 5.9 us; one thread per entry, without
+// the residual, took 6.5 us.
 __global__ void __launch_bounds__(64)
 build_table_kernel(int corner8, int max_states, const int32_t* __restrict__ nstates,
                    const double* __restrict__ h0, const double* __restrict__ cv,
                    const double* __restrict__ free_energy, const double* __restrict__ temp_eff,
                    double boltzmann, double* __restrict__ tab, double* __restrict__ kt) {
 #pragma clang fp contract(off)
-  __shared__ double P[9], T[36], CT[36], C[36], H[9], H0[9], P0[9], W;
+  // of this state and of the type's first one: rest cell, inverse, its residual, rest metric
+  __shared__ double H[2][9], P[2][9], E[2][9], R[2][6], low[2][6];
+  __shared__ double T[36], CT[36], C[36], W;
   const int ts = blockIdx.x, q = threadIdx.x;
   const int t = ts / max_states, s = ts % max_states;
   double* e = tab + (int64_t)ts * kTabStride;
@@ -706,33 +709,31 @@ build_table_kernel(int corner8, int max_states, const int32_t* __restrict__ nsta
     return;
   }
   if (q < 36) C[q] = cv[(int64_t)ts * 36 + q];
-  if (q < 9) {
-    H[q] = h0[(int64_t)ts * 9 + q];
-    H0[q] = h0[(int64_t)t * max_states * 9 + q];
-  }
+  if (q < 18) H[q / 9][q % 9] = h0[(int64_t)(q < 9 ? ts : t * max_states) * 9 + q % 9];
   __syncthreads();
-  if (q < 2) {  // this state's inverse and the first one's
+  if (q < 2) {
     double inv[9];
-    const double det = inverse3_cof(q == 0 ? H : H0, inv);
+    const double det = inverse3_cof(H[q], inv);
     if (q == 0) W = corner8 ? 0.125 * det : det;
-    for (int i = 0; i < 9; ++i) (q == 0 ? P : P0)[i] = inv[i];
+    for (int i = 0; i < 9; ++i) P[q][i] = inv[i];
   }
   __syncthreads();
   if (q < 36) {
-    T[q] = strain_map(P, q / 6, q % 6);
+    T[q] = strain_map(P[0], q / 6, q % 6);
     e[kCvOffset + q] = C[q];
   }
-  if (q < 9) e[q] = P[q];
+  if (q < 18) E[q / 9][q % 9] = inverse_residual(P[q / 9], H[q / 9], q % 9);
+  if (q < 9) e[q] = P[0][q];
   if (q == 9) e[9] = W;
   if (q == 10) e[10] = free_energy[ts];
   if (q == 11) e[11] = 0.0;
-  if (q < 6) {
-    double lo;
-    e[kRestOffset + q] = rest_entry(H, P, q, lo);
-    if (q < 3) {
-      e[kRestLowOffset + q] = lo;
-      e[kShiftOffset + q] = shift_entry(H0, P0, H, P, q);
-    }
+  __syncthreads();
+  if (q < 12) R[q / 6][q % 6] = rest_entry(H[q / 6], E[q / 6], q % 6, low[q / 6][q % 6]);
+  __syncthreads();
+  if (q < 6) e[kRestOffset + q] = R[0][q];
+  if (q < 3) {
+    e[kRestLowOffset + q] = low[0][q];
+    e[kShiftOffset + q] = rest_shift(R[1][q], low[1][q], R[0][q], low[0][q]);
   }
   __syncthreads();
   if (q < 36) CT[q] = stiffness_half(W, C, T, q / 6, q % 6);
