@@ -284,7 +284,8 @@ __device__ __forceinline__ void adjoint_states(const const_f64 tab, int ns, doub
 // stresses, weighted over the states, go through LDS (36 KB a wave, four waves a CU). The waves' own
 // instructions bound it (5000 for one state, 9500 for two, six in ten of them FP64): 64
 // configurations of 16^3 cells, eight-corner model with tangents, 206 us with one lane a corner and
-// products with P per corner, 154 us with one lane a corner in the metric of the edges, 103 us so;
+// products with P per corner, 154 us with one lane a corner in the metric of the edges, 103 us so
+// (94 us where positions need no gradient and no records are stored);
 // 5 of 7^3 cells with the averaged model 18.7, 13.1 and 15.5 us (five waves: one wave's time).
 template <typename T, int kModel>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1)))
