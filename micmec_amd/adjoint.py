@@ -330,6 +330,27 @@ class DiffField(object):
         _native.check(rc, "mm_adjoint_param_grads")
         return g_cv, g_h0, g_free, g_teff
 
+    def _require(self, what, tensors, shapes):
+        """Refuse tensors (None: absent) that a kernel could not read as contiguous float64 arrays
+        of ``shapes`` on the field's device."""
+        for t, shape in zip(tensors, shapes):
+            if t is None:
+                continue
+            if t.dtype != torch.float64 or t.device != self.device or not t.is_contiguous():
+                raise TypeError("%s must be contiguous float64 tensors on %s"
+                                % (what, self.device))
+            if t.shape != shape:
+                raise ValueError("%s: a tensor of shape %s where %s is needed"
+                                 % (what, tuple(t.shape), shape))
+
+    def _inputs(self, pos, rvecs):
+        """Contiguous positions [N, 3] and domain vectors [nsys, 3, 3] of a forward pass."""
+        pos = pos.detach().contiguous()
+        rvecs = rvecs.detach().reshape(self.nsys, 3, 3).contiguous()
+        self._require("positions and domain vectors", (pos, rvecs),
+                      ((self.N, 3), (self.nsys, 3, 3)))
+        return pos, rvecs
+
     def _rest_cells(self, params):
         h0 = params.h0.detach().to(dtype=torch.float64, device=self.device).contiguous()
         if h0.shape != (self.nrows, self.max_states, 3, 3):
@@ -369,9 +390,8 @@ _native.register_signature("mm_adjoint_destroy", [_P])
 class _MicMecEnergy(torch.autograd.Function):
     @staticmethod
     def forward(ctx, field, params, pos, rvecs, cv, h0, free, teff):
+        pos_c, rv_c = field._inputs(pos, rvecs)
         field.set_params(params)
-        pos_c = pos.detach().contiguous()
-        rv_c = rvecs.detach().reshape(field.nsys, 3, 3).contiguous()
         e, g, v = field.compute(pos_c, rv_c)
         ctx.field = field
         ctx.params = params
@@ -384,11 +404,13 @@ class _MicMecEnergy(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, gE, gG, gV):
         field = ctx.field
-        pos, rv = ctx.saved_tensors
-        # contiguous float64 on the field's device, as autograd hands them on
+        pos, rv = ctx.saved_tensors  # a saved-tensor hook may have changed them
         gE = field._no_weight if gE is None else gE.contiguous()
         gG = None if gG is None else gG.contiguous()
         gV = None if gV is None else gV.contiguous()
+        n, s = (field.N, 3), (field.nsys, 3, 3)
+        field._require("saved tensors and cotangents", (pos, rv, gE, gG, gV),
+                       (n, s, (field.nsys,), n, s))
         P = _native.ptr
 
         def call(h0, out):
@@ -407,14 +429,19 @@ class _FitLoss(torch.autograd.Function):
     loss' cotangents are formed by the kernel that uses them."""
 
     @staticmethod
+    def shapes(field):
+        """Of node arrays, system matrices, inverse volumes and the loss."""
+        return (field.N, 3), (field.nsys, 3, 3), (field.nsys, 1, 1), ()
+
+    @staticmethod
     def forward(ctx, problem, params, pos, rvecs, cv, h0, free, teff):
         field = problem.field
+        pos_c, rv_c = field._inputs(pos, rvecs)
+        targets = (problem._g_target, problem._vv_target, problem._inv_volume)
+        field._require("targets", targets, _FitLoss.shapes(field)[:3])
         field.set_params(params)
-        pos_c = pos.detach().contiguous()
-        rv_c = rvecs.detach().reshape(field.nsys, 3, 3).contiguous()
         _, g, v = field.compute(pos_c, rv_c)
         loss = torch.empty((), dtype=torch.float64, device=field.device)
-        targets = (problem._g_target, problem._vv_target, problem._inv_volume)
         scales = (float(problem.f_scale), float(problem.s_scale))
         P = _native.ptr
         gt, vt, inv = targets
@@ -430,8 +457,11 @@ class _FitLoss(torch.autograd.Function):
     @once_differentiable
     def backward(ctx, gl):
         field = ctx.field
-        pos, rv, g, v, gt, vt, inv = ctx.saved_tensors
+        pos, rv, g, v, gt, vt, inv = ctx.saved_tensors  # a saved-tensor hook may have changed them
         gl = gl.contiguous()
+        n, s, inverse, one = _FitLoss.shapes(field)
+        field._require("saved tensors and cotangent", (pos, rv, g, v, gt, vt, inv, gl),
+                       (n, s, n, s, n, s, inverse, one))
         P = _native.ptr
 
         def call(h0, out):

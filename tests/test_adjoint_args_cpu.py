@@ -1,0 +1,116 @@
+"""The differentiable energy and the fit loss hand raw pointers to the library: inputs that are not
+float64 on the field's device, or of another shape, are refused before any library call, and so are
+saved tensors that a hook gives back changed."""
+
+import numpy as np
+import pytest
+import torch
+
+from micmec_amd import _native
+from micmec_amd.adjoint import CellParams, DiffField, FitProblem, micmec_energy
+
+N, NSYS = 6, 2
+
+
+class Library(object):
+    """Records the names of the calls, which do nothing; ``allowed`` False: none may come."""
+
+    def __init__(self, allowed):
+        self.allowed, self.calls = allowed, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            assert self.allowed, "%s was called" % name
+            self.calls.append(name)
+            return 0
+        return call
+
+
+def field_of(allowed, monkeypatch):
+    monkeypatch.setattr(_native, "stream_ptr", lambda stream=None: None)
+    f = object.__new__(DiffField)
+    f.device, f.N, f.nsys, f.nrows, f.max_states = torch.device("cpu"), N, NSYS, 1, 1
+    f.lib, f._field, f._adj = Library(allowed), None, None
+    f._node_sys32 = torch.zeros(N, dtype=torch.int32)
+    f._no_weight = torch.zeros(NSYS, dtype=torch.float64)
+    return f
+
+
+def params():
+    z = lambda *s: torch.zeros(s, dtype=torch.float64, requires_grad=True)
+    return CellParams(z(1, 1, 6, 6), z(1, 1, 3, 3), z(1, 1), z(1), [1])
+
+
+def inputs():
+    return (torch.zeros((N, 3), dtype=torch.float64),
+            torch.eye(3, dtype=torch.float64).repeat(NSYS, 1, 1))
+
+
+def problem_of(field):
+    p = object.__new__(FitProblem)
+    p.field, (p.pos, p.rvecs) = field, inputs()
+    p.f_scale = p.s_scale = 1.0
+    p._g_target = torch.zeros((N, 3), dtype=torch.float64)
+    p._vv_target = torch.zeros((NSYS, 3, 3), dtype=torch.float64)
+    p._inv_volume = torch.ones((NSYS, 1, 1), dtype=torch.float64)
+    return p
+
+
+BAD = [("pos", lambda t: t.float(), TypeError), ("pos", lambda t: t.to("meta"), TypeError),
+       ("pos", lambda t: t[:-1], ValueError), ("pos", lambda t: t.reshape(-1), ValueError),
+       ("rvecs", lambda t: t.float(), TypeError), ("rvecs", lambda t: t.to("meta"), TypeError)]
+
+
+@pytest.mark.parametrize("name,change,error", BAD)
+def test_energy_refuses(name, change, error, monkeypatch):
+    field = field_of(False, monkeypatch)
+    t = dict(zip(("pos", "rvecs"), inputs()))
+    t[name] = change(t[name])
+    with pytest.raises(error):
+        micmec_energy(field, t["pos"], t["rvecs"], params())
+
+
+@pytest.mark.parametrize("name,change,error", BAD + [
+    ("_g_target", lambda t: t[:-1], ValueError), ("_vv_target", lambda t: t.float(), TypeError),
+    ("_inv_volume", lambda t: t[:1], ValueError)])
+def test_loss_refuses(name, change, error, monkeypatch):
+    problem = problem_of(field_of(False, monkeypatch))
+    setattr(problem, name, change(getattr(problem, name)))
+    with pytest.raises(error):
+        problem.loss(params())
+
+
+@pytest.mark.parametrize("unpack", [lambda t: t.float(), lambda t: t.to("meta"),
+                                    lambda t: t.clone().t().contiguous().t()
+                                    if t.dim() == 2 else t])
+@pytest.mark.parametrize("loss", [False, True])
+def test_backward_refuses_changed_saved_tensors(loss, unpack, monkeypatch):
+    field = field_of(True, monkeypatch)
+    p = params()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        if loss:
+            out = problem_of(field).loss(p)
+        else:
+            pos, rv = inputs()
+            out = micmec_energy(field, pos.requires_grad_(True), rv, p)[0].sum()
+        field.lib.allowed = False
+        with pytest.raises(TypeError):
+            torch.autograd.grad(out, p.tensors())
+
+
+@pytest.mark.parametrize("loss", [False, True])
+def test_accepted(loss, monkeypatch):
+    """Strided positions and domain vectors of another shape with nine entries a system."""
+    field = field_of(True, monkeypatch)
+    p = params()
+    pos = torch.zeros((3, N), dtype=torch.float64).t().requires_grad_(True)
+    rv = torch.zeros((3 * NSYS, 3), dtype=torch.float64)
+    if loss:
+        problem = problem_of(field)
+        problem.pos, problem.rvecs = pos, rv
+        out = problem.loss(p)
+    else:
+        out = micmec_energy(field, pos, rv, p)[0].sum()
+    grads = torch.autograd.grad(out, (pos,) + p.tensors())
+    assert grads[0].shape == pos.shape
+    assert field.lib.calls[-1] == ("mm_fit_backward" if loss else "mm_adjoint_backward")
