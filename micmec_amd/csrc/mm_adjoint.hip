@@ -501,8 +501,8 @@ __device__ __forceinline__ void state_gradients(const double* ent, bool on, int6
 // X2 = sum p x x^T and X1 = sum p x, S = Cv T x the stress and G = 2 x + R the Gram matrix,
 //   dE/dCv = w T X2 T^T / 2,  dE/dP_ik = w sum_mn P_mn (sum p S_im G_nk),
 //   dE/dw = tr(Cv^T T X2 T^T) / 2,
-// all linear in the sums, so values and tangents alike. One wave per (row, state); lane 32 h + i
-// works on half h. With grads.cv the gradients of the parameter tensors, from values plus
+// all linear in the sums, so values and tangents alike; zeros for a state that the row does not
+// have. One wave per (row, state); lane 32 h + i works on half h. With grads.cv the gradients of the parameter tensors, from values plus
 // tangents, are formed too.
 __global__ void __launch_bounds__(64)
 metric_entries_kernel(const double* __restrict__ tab, const int32_t* __restrict__ nstates,
@@ -513,7 +513,10 @@ metric_entries_kernel(const double* __restrict__ tab, const int32_t* __restrict_
     const double* e = params + 2 * (row * npar + (int64_t)max_states * kNps);
     grads.teff[row] = (e[0] + e[1]) * grads.boltzmann;
   }
+  double* out = params + 2 * (row * npar + (int64_t)s * kNps);
   if (s >= nstates[row]) {
+    // the sums of a state that the row no longer has are those of an earlier evaluation
+    out[threadIdx.x] = 0.0;
     if (grads.cv) state_gradients(ent, false, blockIdx.x, grads);
     return;
   }
@@ -521,7 +524,6 @@ metric_entries_kernel(const double* __restrict__ tab, const int32_t* __restrict_
   const double* C = ts + kCvOffset;
   const double* R = ts + kRestOffset;
   const double w = ts[9];
-  double* out = params + 2 * (row * npar + (int64_t)s * kNps);
   __shared__ double T[36], P[9], X2[2][36], X1[2][6], A[2][36], E[2][36], Q[2][36], B[2][6], p[2];
   const int h = threadIdx.x >> 5, i = threadIdx.x & 31;
   if (threadIdx.x < 9) P[threadIdx.x] = ts[threadIdx.x];
@@ -847,7 +849,7 @@ int mm_adjoint_create(mm_adjoint** out, mm_field* field, int64_t* npar) {
   if (e == hipSuccess && !row_idx.empty())
     e = hipMemcpy(a->row_idx, row_idx.data(), sizeof(int32_t) * row_idx.size(),
                   hipMemcpyHostToDevice);
-  // rows of states that a type does not have are never written: they stay zero
+  // rows of states that a type does not have are summed too (metric_entries_kernel drops the sums)
   if (e == hipSuccess) e = hipMemset(a->ppart, 0, sizeof(double) * 2 * a->npar * nb);
   (void)hipSetDevice(cur);
   if (e != hipSuccess) {
