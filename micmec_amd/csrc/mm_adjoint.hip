@@ -158,7 +158,8 @@ __device__ __forceinline__ T adjoint_corner(const const_f64 ts, int i,
   for (int o = 0; o < 3; ++o) {
     const T(&A)[3] = E[F::edge(a, F::axis0(o))];
     const T(&B)[3] = E[F::edge(a, F::axis1(o))];
-    x[3 + o] = mad(A[2], B[2], mad(A[1], B[1], mad(A[0], B[0], make<T>(-R[3 + o], 0.0))));
+    x[3 + o] = mad(A[2], B[2], mad(A[1], B[1], mad(A[0], B[0], make<T>(-R[3 + o], 0.0)))) -
+               ts[kRestLowOffset + 3 + o];
   }
   T u = make<T>(0.0, 0.0);
 #pragma unroll

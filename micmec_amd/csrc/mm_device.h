@@ -23,14 +23,15 @@ namespace mm {
 //   [12..47] Voigt matrix Cv[6][6] (row-major), averaged over index orderings
 //   [48..83] K = T^T (w Cv) T, the weighted matrix of the force kernels (metric_entry)
 //   [84..89] rest metric R (rest_entry): R00, R11, R22, R12, R02, R01
-//   [90..92] half of what the first three lack to R00, R11, R22
-//   [93..95] the diagonal of R/2 of the type's first state less this state's
-constexpr int kTabStride = 96;
+//   [90..95] what they lack: half of it for R00, R11, R22, all of it for the others
+//   [96..98] the diagonal of R/2 of the type's first state less this state's
+//   [99..103] unused (entries begin at cache lines)
+constexpr int kTabStride = 104;
 constexpr int kCvOffset = 12;
 constexpr int kMetricOffset = 48;
 constexpr int kRestOffset = 84;
 constexpr int kRestLowOffset = 90;
-constexpr int kShiftOffset = 93;
+constexpr int kShiftOffset = 96;
 
 // Tables that no kernel of a launch writes: read with scalar loads wherever the index is uniform,
 // also where other memory changes during the launch.
@@ -101,7 +102,8 @@ __host__ __device__ inline double dot3_exact(const double* a, int sa, const doub
 // R is the metric that P, rounded as it is, takes to the identity, R = P^-1 P^-T: with the rounding
 // of h0 h0^T in its place every cell would carry the same strain of 1e-17, which a virial of
 // small strains of either sign does not average out. P h0 = I + E, so to first order in E (1e-16)
-// R = h0 h0^T - h0 (E + E^T) h0^T. Returns the entry rounded, half of the rest in lo.
+// R = h0 h0^T - h0 (E + E^T) h0^T. Returns the entry rounded, the rest (half of it on the diagonal,
+// as the strains take it) in lo.
 __host__ __device__ inline double inverse_residual(const double* P, const double* h0, int q) {
 #pragma clang fp contract(off)
   double lo;  // entry q of E
@@ -119,7 +121,8 @@ __host__ __device__ inline double rest_entry(const double* h0, const double* E, 
   const double r = dot3_exact(a, 1, b, 1, 0.0, l);
   l -= c;
   const double hi = r + l;
-  lo = 0.5 * ((r - hi) + l);
+  lo = (r - hi) + l;
+  if (I < 3) lo *= 0.5;
   return hi;
 }
 // Half of the first state's diagonal entry r0, l0 less this one's r1, l1.
@@ -128,7 +131,7 @@ __host__ __device__ inline double rest_shift(double r0, double l0, double r1, do
   return 0.5 * (r0 - r1) + (l0 - l1);
 }
 
-// K (36) and the rest entries (12, from kRestOffset) of a table entry from h0, P = h0^-1, w and Cv, and
+// K (36) and the rest entries (15, from kRestOffset) of a table entry from h0, P = h0^-1, w and Cv, and
 // those of the type's first state. Shared by the host and the device table builders, without
 // contraction, so both round the same way.
 inline void metric_entry(const double* h0, const double* P, double w, const double* Cv,
@@ -144,9 +147,9 @@ inline void metric_entry(const double* h0, const double* P, double w, const doub
   }
   for (int I = 0; I < 6; ++I) {
     R[I] = rest_entry(h0, E, I, lo);
+    R[kRestLowOffset - kRestOffset + I] = lo;
     if (I >= 3) continue;
     const double r0 = rest_entry(h00, E0, I, lo0);
-    R[kRestLowOffset - kRestOffset + I] = lo;
     R[kShiftOffset - kRestOffset + I] = rest_shift(r0, lo0, R[I], lo);
   }
 }
@@ -228,10 +231,11 @@ __device__ __forceinline__ void corner_stress(const_f64 K, int i,
   for (int o = 0; o < 3; ++o) u = __builtin_fma(x[3 + o], O[o], u);
 }
 
-// Off-diagonal strain o of the corner with edges E: their dot product less the rest metric's.
-__device__ __forceinline__ double edge_dot(const double (&A)[3], const double (&B)[3], double g0) {
+// Off-diagonal strain of a corner's edges A and B: their dot product less the rest metric's g0 + lo.
+__device__ __forceinline__ double edge_dot(const double (&A)[3], const double (&B)[3], double g0,
+                                           double lo) {
 #pragma clang fp contract(off)
-  return __builtin_fma(A[2], B[2], __builtin_fma(A[1], B[1], __builtin_fma(A[0], B[0], -g0)));
+  return __builtin_fma(A[2], B[2], __builtin_fma(A[1], B[1], __builtin_fma(A[0], B[0], -g0))) - lo;
 }
 // Diagonal strain of an edge along d against its rest metric g0 + 2 lo: (A.A - g0)/2 - lo, the sum
 // begun with the component along d less g0. That product is exact inside the fused multiply-add,
@@ -267,7 +271,8 @@ __device__ __forceinline__ double state_stress(const_f64 tab,
     for (int d = 0; d < 3; ++d) x[d] = q[F::edge(a, d)] + tab[kShiftOffset + d];
 #pragma unroll
     for (int o = 0; o < 3; ++o)
-      x[3 + o] = edge_dot(E[F::edge(a, F::axis0(o))], E[F::edge(a, F::axis1(o))], g0[3 + o]);
+      x[3 + o] = edge_dot(E[F::edge(a, F::axis0(o))], E[F::edge(a, F::axis1(o))], g0[3 + o],
+                          tab[kRestLowOffset + 3 + o]);
     corner_stress<kModel>(tab + kMetricOffset, i, x, D, O[a], u);
 #pragma unroll
     for (int d = 0; d < 3; ++d)
@@ -385,7 +390,8 @@ __device__ __forceinline__ double sweep_cell(const_f64 tab,
     }
 #pragma unroll
     for (int o = 0; o < 3; ++o)
-      x[3 + o] = edge_dot(E[F::edge(a, F::axis0(o))], E[F::edge(a, F::axis1(o))], g0[3 + o]);
+      x[3 + o] = edge_dot(E[F::edge(a, F::axis0(o))], E[F::edge(a, F::axis1(o))], g0[3 + o],
+                          tab[kRestLowOffset + 3 + o]);
     corner_stress<0>(tab + kMetricOffset, i, x, D, O, u);
     if (kOut != 0) {
       bool open[3];

@@ -730,11 +730,12 @@ build_table_kernel(int corner8, int max_states, const int32_t* __restrict__ nsta
   __syncthreads();
   if (q < 12) R[q / 6][q % 6] = rest_entry(H[q / 6], E[q / 6], q % 6, low[q / 6][q % 6]);
   __syncthreads();
-  if (q < 6) e[kRestOffset + q] = R[0][q];
-  if (q < 3) {
+  if (q < 6) {
+    e[kRestOffset + q] = R[0][q];
     e[kRestLowOffset + q] = low[0][q];
-    e[kShiftOffset + q] = rest_shift(R[1][q], low[1][q], R[0][q], low[0][q]);
   }
+  if (q < 8)
+    e[kShiftOffset + q] = q < 3 ? rest_shift(R[1][q], low[1][q], R[0][q], low[0][q]) : 0.0;
   __syncthreads();
   if (q < 36) CT[q] = stiffness_half(W, C, T, q / 6, q % 6);
   __syncthreads();
