@@ -244,6 +244,26 @@ class ConjugateGradientSearch(object):
         return True
 
 
+class _SearchFunction(object):
+    """The energy function of an optimiser's search. It holds the optimiser weakly: without a cycle
+    the arrays of a finished run are free at once, and the next run finds their (pinned) pages in
+    the allocators. Copied or pickled with its optimiser, it belongs to the copy."""
+
+    def __init__(self, optimizer, dof):
+        self.__setstate__((optimizer, dof))
+
+    def __call__(self, x, do_gradient=False):
+        optimizer = self._optimizer()
+        return (self._dof if optimizer is None else optimizer).fun(x, do_gradient)
+
+    def __getstate__(self):
+        return self._optimizer(), self._dof
+
+    def __setstate__(self, state):
+        optimizer, self._dof = state
+        self._optimizer = (lambda: None) if optimizer is None else weakref.ref(optimizer)
+
+
 class CGOptimizer(BaseOptimizer):
     """Conjugate-gradient optimiser (opt.py:147-180)."""
     log_name = "CGOPT"
@@ -256,11 +276,7 @@ class CGOptimizer(BaseOptimizer):
                                  device=dof.device)
             make = getattr(dof, "cg_engine", None)
             engine = make(x0) if make is not None else None
-        # The search holds its optimiser weakly: without a cycle the arrays of a finished run are
-        # free at once, and the next run finds their (pinned) pages in the allocators.
-        this = weakref.ref(self)
-        self.minimizer = ConjugateGradientSearch(
-            x0, lambda x, do_gradient=False: (this() or dof).fun(x, do_gradient), engine=engine)
+        self.minimizer = ConjugateGradientSearch(x0, _SearchFunction(self, dof), engine=engine)
         BaseOptimizer.__init__(self, dof, state, hooks, counter0)
 
     def initialize(self):
