@@ -453,19 +453,18 @@ __device__ __forceinline__ void vecmat(const double v[3], const double* M, doubl
 // flight at once (two memory round trips instead of up to sixteen), at the cost of about 50
 // more VGPRs; the same bits as skipping the nones. Without it each record is loaded behind
 // the test of its index, which keeps the registers few: the form for passes with enough
-// waves to hide the latency.
-// kBatch (without kAllLoads): 1 so, 2 to 4 with the indices loaded first and then that many records
-// at a time, a none as above; for the force gather, which holds little else: 72x80x96 cells, whole
-// evaluation 73.2 us with 1, 71.0 us with 2 and 4; in the MD gathers 128^3 NPT 561 -> 573 us a step.
+// waves to hide the latency. (Two or four records at a time there, nones read too, whole evaluation:
+// 72x80x96 cells 76.6 -> 74.1 us, but 80^3 66.4 -> 69.7, 96^3 99.8 -> 102, 128^3 202 -> 211 and 160^3
+// 401 -> 431 us.)
 // kStream: the loads carry the non-temporal hint.
-template <bool kAllLoads, int kBatch = 1, bool kStream = true>
+template <bool kAllLoads, bool kStream = true>
 __device__ __forceinline__ void sum_node_records(const int32_t* __restrict__ ncell,
                                                  const double* gcell, int64_t N, int64_t RS,
                                                  int64_t n, double g[3]) {
   auto load = [](const auto* p) { return kStream ? __builtin_nontemporal_load(p) : *p; };
 #pragma unroll
   for (int j = 0; j < 3; ++j) g[j] = 0.0;
-  if (!kAllLoads && kBatch == 1) {
+  if (!kAllLoads) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const int32_t e = load(&ncell[k * N + n]);
@@ -479,27 +478,23 @@ __device__ __forceinline__ void sum_node_records(const int32_t* __restrict__ nce
     }
     return;
   }
-  constexpr int kRows = kAllLoads ? 8 : kBatch;
   int32_t e[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) e[k] = load(&ncell[k * N + n]);
+  double r[8][3];
 #pragma unroll
-  for (int b = 0; b < 8; b += kRows) {
-    if (b) __builtin_amdgcn_sched_barrier(0);
-    double r[kRows][3];
+  for (int k = 0; k < 8; ++k) {
+    const int32_t c = e[k] >= 0 ? e[k] : 0;
+    const int64_t w = c >> 2;
+    const int p = c & 3;
 #pragma unroll
-    for (int k = 0; k < kRows; ++k) {
-      const int32_t c = e[b + k] >= 0 ? e[b + k] : 0;
-      const int64_t w = c >> 2;
-      const int p = c & 3;
-#pragma unroll
-      for (int j = 0; j < 3; ++j) r[k][j] = load(&gcell[(int64_t)(3 * p + j) * RS + w]);
-    }
-#pragma unroll
-    for (int k = 0; k < kRows; ++k)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) g[j] = e[b + k] >= 0 ? g[j] + r[k][j] : g[j];
+    for (int j = 0; j < 3; ++j)
+      r[k][j] = load(&gcell[(int64_t)(3 * p + j) * RS + w]);
   }
+#pragma unroll
+  for (int k = 0; k < 8; ++k)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) g[j] = e[k] >= 0 ? g[j] + r[k][j] : g[j];
 }
 
 // Workgroups are dealt to the 8 XCDs of the device in turn (block b runs on XCD b mod 8), and

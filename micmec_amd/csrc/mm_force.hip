@@ -282,7 +282,7 @@ gather_kernel(const int32_t* __restrict__ ncell, const double* __restrict__ gcel
     }
   }
   double g[3] = {0.0, 0.0, 0.0};
-  if (n < N) sum_node_records<kAllLoads, 4>(ncell, gcell, N, RS, n, g);
+  if (n < N) sum_node_records<kAllLoads>(ncell, gcell, N, RS, n, g);
   __syncthreads();
   double acc[4] = {0.0, 0.0, 0.0, 0.0};
   if (n < N) {
