@@ -329,12 +329,17 @@ hipError_t launch_cells(const ForceArgs& a, hipStream_t stream) {
   // -> 47.8 / 109 -> 37.4 / 81.1 us (the last two with the gathers' all-loads form), at 48^3
   // (about 430 blocks) 59.2 / 138.7 -> 58.8 / 127.5 us, -> 53.8 / 117.5 us in one launch; at
   // 64^3 (about 1030 blocks) the fork is the faster (NVT 74.0 vs 76.4 us back to back), at
-  // 96^3 too (NPT 329 vs 343 us). The averaged model's kernels are as short in either kind and
-  // the device holds twice as many: one launch whatever the size (61x64x67, 1022 blocks, whole
-  // evaluation 52.4 -> 29.1 us, with the totals in the gather's launch). The results are the same
-  // bits in every form.
+  // 96^3 too (NPT 329 vs 343 us). The averaged model's kernels are short in either kind and the
+  // device holds twice as many, so that the fork pays later: one launch against two, a fifth of
+  // the cells two-state, whole evaluation of 61x64x67 (1022 blocks) 27 / 50 us, 96^3 88 / 94,
+  // 104^3 108 / 115, 112^3 136 / 136, 128^3 197 / 197, 160^3 419 / 396 (with seven of ten cells
+  // two-state 85 / 98, 101 / 112, 130 / 139, 188 / 199, 416 / 412); NVT-NHC step, where a graph's
+  // fork costs less, 64^3 64 / 68, 96^3 137 / 132, 104^3 168 / 164, 112^3 199 / 188, 128^3 285 / 277;
+  // NPT 123 / 147, 265 / 263, 328 / 320, 385 / 365, 549 / 522. The results are the same bits in
+  // every form.
+  const int one = a.model == 0 ? kForkMinBlocks : kForkMinBlocksAveraged;
   const bool fork = a.side != nullptr && a.ev_fork != nullptr && a.ev_join != nullptr &&
-                    mn > 0 && sn > 0 && nb > kForkMinBlocks && a.model == 0;
+                    mn > 0 && sn > 0 && nb > one;
   hipStream_t ms = fork ? a.side : stream;
   hipError_t e = hipSuccess;
   if (fork) {
@@ -357,7 +362,7 @@ hipError_t launch_cells(const ForceArgs& a, hipStream_t stream) {
   // place only as that drains (npt 128^3 step 0.580 -> 0.576 ms; equal at 72x80x96 with seven
   // of ten cells two-state).
   // a pass that the device holds at once, with blocks of both kinds: one launch
-  const bool both = mn > 0 && sn > 0 && (nb <= kForkMinBlocks || a.model != 0);
+  const bool both = mn > 0 && sn > 0 && nb <= one;
 #define MM_LAUNCH_BOTH(MODEL, OUT)                                                           \
   hipLaunchKernelGGL((cell_kernel_both<MODEL, OUT>), dim3(nb), dim3(kCellBlock), 0, stream,     \
                      a.pos, a.rvecs, a.rvecs_stride, a.blk_sys, a.cnode, a.cwrap,              \

@@ -7,10 +7,9 @@
 namespace mm {
 
 constexpr int kCellBlock = 256;
-// Cell passes of the eight-corner model of more blocks than this run their two instances
-// concurrently; smaller ones, and all of the averaged model, run both kinds of block in one launch
-// (cell_kernel_both).
-constexpr int kForkMinBlocks = 512;
+// Cell passes of more blocks than this (eight-corner model, averaged model) run their two instances
+// concurrently; smaller ones run both kinds of block in one launch (cell_kernel_both).
+constexpr int kForkMinBlocks = 512, kForkMinBlocksAveraged = 4608;
 // Node gathers over at most this many 256-node blocks (at most four waves a SIMD) load all of
 // a node's records at once (sum_node_records<true>): latency bounds such a pass. NVT-NHC / NPT
 // step, records one at a time -> all at once: 32^3 46.3 / 105.9 -> 43.9 / 103.4 us, 48^3
