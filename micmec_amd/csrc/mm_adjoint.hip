@@ -446,13 +446,13 @@ adjoint_kernel(const double* __restrict__ pos, const double* __restrict__ dpos,
   for (int v = 0; v < 8; ++v)
 #pragma unroll
     for (int j = 0; j < 3; ++j) gv[v][j] = valid ? val(g[v][j]) : -0.0;
-  store_cell<true>(w, wrap, valid, cbase, W, S, gcell, gv);
+  store_cell(w, wrap, valid, cbase, W, S, gcell, gv);
   if (IsDual<T>::value) {
 #pragma unroll
     for (int v = 0; v < 8; ++v)
 #pragma unroll
       for (int j = 0; j < 3; ++j) gv[v][j] = valid ? tan_(g[v][j]) : -0.0;
-    store_cell<true>(w, wrap, valid, cbase, W, S, gcell2, gv);
+    store_cell(w, wrap, valid, cbase, W, S, gcell2, gv);
   }
 }
 

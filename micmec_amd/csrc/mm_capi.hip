@@ -390,7 +390,6 @@ int create_field(mm_field** out, int device, int model, int32_t nsys, int64_t nc
   f->nrows = nrows;
   f->max_states = max_states;
   f->nsys = nsys;
-  f->slot_of_cell = std::move(slot);
   const int64_t nb = W / kCellBlock;
   if ((rc = dmalloc(&f->cnode, (size_t)8 * W)) || (rc = dmalloc(&f->cwrap, W)) ||
       (rc = dmalloc(&f->blk_row, nb)) ||

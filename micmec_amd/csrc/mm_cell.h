@@ -76,14 +76,10 @@ __device__ constexpr int kLowerCorner[4] = {0, 1, 2, 4};
 __device__ constexpr int kUpperCorner[4] = {3, 5, 6, 7};
 
 // Entry i of a gradient plane (S < 2^29, so that the byte offset fits 32 bits beside the plane's
-// uniform base); kStream: with the non-temporal hint.
-template <bool kStream>
+// uniform base), with the non-temporal hint.
 __device__ __forceinline__ void store_record(double* plane, uint32_t i, double v) {
   double* t = reinterpret_cast<double*>(reinterpret_cast<char*>(plane) + (size_t)(i * 8u));
-  if (kStream)
-    __builtin_nontemporal_store(v, t);
-  else
-    *t = v;
+  __builtin_nontemporal_store(v, t);
 }
 
 // Energies of all states of a cell, combined by the log-sum-exp of mmff.py:386-398, with virial
@@ -198,7 +194,6 @@ __device__ __forceinline__ void fold_cell(int wrap, double (&gacc)[8][3]) {
 }
 
 // The vertex gradient of the cell in slot w as records (every lane of the wave calls this).
-template <bool kStream>
 __device__ __forceinline__ void store_cell(int64_t w, int wrap, bool valid,
                                            const int32_t* __restrict__ cbase, int64_t W,
                                            int64_t S, double* gcell, double (&gacc)[8][3]) {
@@ -210,7 +205,7 @@ __device__ __forceinline__ void store_cell(int64_t w, int wrap, bool valid,
     for (int q = 0; q < 4; ++q)
 #pragma unroll
       for (int j = 0; j < 3; ++j)
-        store_record<kStream>(gcell + (int64_t)(3 * q + j) * S, (uint32_t)w, gacc[kLowerCorner[q]][j]);
+        store_record(gcell + (int64_t)(3 * q + j) * S, (uint32_t)w, gacc[kLowerCorner[q]][j]);
   }
   const bool open_top = valid && !(wrap & 16);
   const uint64_t tops = __ballot(open_top);
@@ -222,7 +217,7 @@ __device__ __forceinline__ void store_cell(int64_t w, int wrap, bool valid,
     for (int q = 0; q < 4; ++q)
 #pragma unroll
       for (int j = 0; j < 3; ++j)
-        store_record<kStream>(gcell + (int64_t)(3 * q + j) * S, ci, gacc[kUpperCorner[q]][j]);
+        store_record(gcell + (int64_t)(3 * q + j) * S, ci, gacc[kUpperCorner[q]][j]);
   }
 }
 

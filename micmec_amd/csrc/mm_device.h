@@ -456,12 +456,12 @@ __device__ __forceinline__ void vecmat(const double v[3], const double* M, doubl
 // waves to hide the latency. (Two or four records at a time there, nones read too, whole evaluation:
 // 72x80x96 cells 76.6 -> 74.1 us, but 80^3 66.4 -> 69.7, 96^3 99.8 -> 102, 128^3 202 -> 211 and 160^3
 // 401 -> 431 us.)
-// kStream: the loads carry the non-temporal hint.
-template <bool kAllLoads, bool kStream = true>
+// The loads carry the non-temporal hint.
+template <bool kAllLoads>
 __device__ __forceinline__ void sum_node_records(const int32_t* __restrict__ ncell,
                                                  const double* gcell, int64_t N, int64_t RS,
                                                  int64_t n, double g[3]) {
-  auto load = [](const auto* p) { return kStream ? __builtin_nontemporal_load(p) : *p; };
+  auto load = [](const auto* p) { return __builtin_nontemporal_load(p); };
 #pragma unroll
   for (int j = 0; j < 3; ++j) g[j] = 0.0;
   if (!kAllLoads) {
@@ -593,38 +593,6 @@ __device__ __forceinline__ double wave_reduce_scatter(const double (&v)[NV], int
 
 __device__ __forceinline__ int scatter_index(int lane) {
   return ((lane >> 5) & 1) * 8 + ((lane >> 4) & 1) * 4 + ((lane >> 3) & 1) * 2 + ((lane >> 2) & 1);
-}
-
-// Sum SoA block partials part[q * nb + b] over b in a fixed order; one block of 1024 threads,
-// every thread receives the totals.
-template <int NV>
-__device__ __forceinline__ void reduce_soa(const double* __restrict__ part, int nb,
-                                           double (&out)[NV]) {
-  __shared__ double red[NV * 16];
-  __shared__ double tot[NV];
-  double acc[NV];
-#pragma unroll
-  for (int q = 0; q < NV; ++q) acc[q] = 0.0;
-  for (int bb = threadIdx.x; bb < nb; bb += 1024) {
-#pragma unroll
-    for (int q = 0; q < NV; ++q) acc[q] += part[(int64_t)q * nb + bb];
-  }
-  wave_reduce<NV>(acc);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-#pragma unroll
-    for (int q = 0; q < NV; ++q) red[wave * NV + q] = acc[q];
-  }
-  __syncthreads();
-  if (threadIdx.x < NV) {
-    double s = red[threadIdx.x];
-    for (int w = 1; w < 16; ++w) s += red[w * NV + threadIdx.x];
-    tot[threadIdx.x] = s;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < NV; ++q) out[q] = tot[q];
-  __syncthreads();
 }
 
 }  // namespace mm

@@ -96,7 +96,7 @@ __device__ __forceinline__ void cell_body(int bid, MM_CELL_PARAMS) {
       tab, ns, kt, valid,
       [&](double (&p)[8][3]) { load_corners(pos, n, p, on, xmat + soff, on2, xmat2 + soff); },
       wrap, rv, st_sh + threadIdx.x, ecell, vir, gacc);
-  if (kOut == kOutGradient) store_cell<true>(w, wrap, valid, cbase, W, S, gcell, gacc);
+  if (kOut == kOutGradient) store_cell(w, wrap, valid, cbase, W, S, gcell, gacc);
   cell_wave_totals(ecell, vir, red + 7 * (threadIdx.x >> 6));
   __syncthreads();
   if (threadIdx.x < 10)

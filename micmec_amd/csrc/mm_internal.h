@@ -49,7 +49,6 @@ struct mm_field {
   int32_t* blk_sys = nullptr;         // [W/256] system of every cell block
   int32_t* sys_cblk_ptr = nullptr;    // [nsys + 1] CSR of the cell blocks of every system
   int32_t* sys_cblk_idx = nullptr;    // [W/256]
-  std::vector<int64_t> slot_of_cell;  // reference cell index -> work slot
   std::vector<int32_t> blk_row_host;  // [W/256] copy of blk_row
   std::vector<int32_t> nstates_host;  // [nrows] copy of nstates
   int split = -1;                     // see ForceArgs::split

@@ -80,18 +80,10 @@ enum Phase {
 // Block totals of a node pass (one wave per block), written SoA: out[q * gridDim.x + blockIdx.x].
 template <int NV>
 __device__ __forceinline__ void block_sum_store(double (&v)[NV], double* part) {
-  if (NV >= 4) {
-    const int lane = threadIdx.x & 63;
-    const double t = wave_reduce_scatter<NV>(v, lane);
-    const int q = scatter_index(lane);
-    if ((lane & 3) == 0 && q < NV) part[(int64_t)q * gridDim.x + blockIdx.x] = t;
-    return;
-  }
-  wave_reduce<NV>(v);
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < NV; ++q) part[(int64_t)q * gridDim.x + blockIdx.x] = v[q];
-  }
+  const int lane = threadIdx.x & 63;
+  const double t = wave_reduce_scatter<NV>(v, lane);
+  const int q = scatter_index(lane);
+  if ((lane & 3) == 0 && q < NV) part[(int64_t)q * gridDim.x + blockIdx.x] = t;
 }
 
 // The same for blocks of kNodeBlock threads (waves summed in order through LDS), into the
@@ -1485,7 +1477,7 @@ md_cells_kernel(CellPass c, const double* __restrict__ x, PhaseArgs ph,
   else
     cell_eval<kModel, kOut, false, kCellBlock>(tab, ns, kt, valid, corners, wrap, rv, st_sh + t,
                                                ecell, vir, gacc);
-  if (kOut == kOutGradient) store_cell<true>(w, wrap, valid, c.cbase, c.W, c.S, c.gcell, gacc);
+  if (kOut == kOutGradient) store_cell(w, wrap, valid, c.cbase, c.W, c.S, c.gcell, gacc);
   cell_wave_totals(ecell, vir, cred + 7 * (t >> 6));
   __syncthreads();
   if (t < 10) partials[(int64_t)t * nblocks + bid] = cell_block_total(cred, t);
