@@ -172,8 +172,8 @@ int mm_field_set_params_device(mm_field* f, const int32_t* nstates, const double
  * and deformation derivatives agree with ForcePartMechanical (micmec/pes/mmff.py:288-323) and
  * with the automatic derivatives of micmec/pes/mmff_jax.py:249-250.
  *
- * mm_adjoint_create allocates the work buffers of an object (about (2 * npar + 38) / 32 + 24
- * doubles per work slot, and 3 per node) and returns npar = max_states * 32 + 1, the parameter
+ * mm_adjoint_create allocates the work buffers of an object (about (2 * npar + 38) / 64 + 12 to 24
+ * doubles per work slot, 3 per node, and a few per system and table row) and returns npar = max_states * 32 + 1, the parameter
  * entries per row.
  *
  * mm_adjoint_compute evaluates, at positions pos [nnodes][3] and domain vectors rvecs [nsys][9]:

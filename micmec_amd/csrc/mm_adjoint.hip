@@ -287,7 +287,10 @@ __device__ __forceinline__ void adjoint_states(const const_f64 tab, int ns, doub
 // configurations of 16^3 cells, eight-corner model with tangents, 206 us with one lane a corner and
 // products with P per corner, 154 us with one lane a corner in the metric of the edges, 103 us so
 // (94 us where positions need no gradient and no records are stored);
-// 5 of 7^3 cells with the averaged model 18.7, 13.1 and 15.5 us (five waves: one wave's time).
+// 5 of 7^3 cells with the averaged model 18.7, 13.1 and 15.5 us. A field of a few waves takes one
+// wave's time, which the cells' lanes make longer: eight-corner model, 2 of 5^3 cells 14.9 us with
+// one lane a corner, 24.6 us so, 8 of 12^3 19.9 and 26.7 us (a product of either, DiffField.vjp, 43.5
+// and 46 us, the launches being fewer).
 template <typename T, int kModel>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1)))
 adjoint_kernel(const double* __restrict__ pos, const double* __restrict__ dpos,
@@ -503,8 +506,8 @@ __device__ __forceinline__ void state_gradients(const double* ent, bool on, int6
 //   dE/dCv = w T X2 T^T / 2,  dE/dP_ik = w sum_mn P_mn (sum p S_im G_nk),
 //   dE/dw = tr(Cv^T T X2 T^T) / 2,
 // all linear in the sums, so values and tangents alike; zeros for a state that the row does not
-// have. One wave per (row, state); lane 32 h + i works on half h. With grads.cv the gradients of the parameter tensors, from values plus
-// tangents, are formed too.
+// have. One wave per (row, state); lane 32 h + i works on half h. With grads.cv the gradients of the
+// parameter tensors, from values plus tangents, are formed too.
 __global__ void __launch_bounds__(64)
 metric_entries_kernel(const double* __restrict__ tab, const int32_t* __restrict__ nstates,
                       int max_states, int64_t npar, double* __restrict__ params, GradOut grads) {

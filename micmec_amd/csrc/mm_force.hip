@@ -42,13 +42,13 @@ namespace mm {
 // gradient too); the energies and virials of all three are the same bits. The latter two take the
 // node positions through the pending transforms xmat (and xmat2 first, when its flag is set) when
 // they are given: a barostat call whose position scaling is stored by a later node pass.
-// The single-state instance sweeps the corners (sweep_cell) in 165 VGPRs, three waves a SIMD (148
+// The single-state instance sweeps the corners (sweep_cell) in 163 VGPRs, three waves a SIMD (168
 // without the gradient); the multistate one keeps the stresses of all corners for the state sum
-// (219 VGPRs and 72 KB of LDS a block, two waves). The compiler's default scheduler is the one that
-// keeps both free of spills. HBM bounds the gradient pass: about 450 MB at 128^3 (20% two-state,
-// 5% empty) in 100 us, with 1000 / 1800 VALU instructions a wave (60 us of issue); the form
+// (223 VGPRs and 72 KB of LDS a block, two waves). The compiler's default scheduler is the one that
+// keeps both free of vector spills. HBM bounds the gradient pass: 469 MB at 128^3 (20% two-state,
+// 5% empty) in 100 to 115 us, with 1185 / 1910 VALU instructions a wave (67 us of issue); the form
 // with B = P M per corner took 1735 / 4000 and 150 us, and 120 us for the pass without
-// gradient that now takes 84 us.
+// gradient that now takes 83 us.
 #define MM_CELL_PARAMS                                                                        \
   const double *__restrict__ pos, const double *__restrict__ rvecs, int64_t rvecs_stride,     \
       const int32_t *__restrict__ blk_sys, const int32_t *__restrict__ cnode,                 \
@@ -324,12 +324,14 @@ hipError_t launch_cells(const ForceArgs& a, hipStream_t stream) {
   // The second instance runs on the side stream, concurrently with the first, when the pass
   // has more cell blocks than the device holds at once (256 CUs x 2 blocks of 256 lanes at two
   // waves a SIMD). A smaller pass takes the time of one block per instance, less than the fork
-  // and join cost: it runs both kinds of block in one launch (cell_kernel_both). NVT-NHC / NPT
-  // step at 32^3 (129 blocks), fork -> back to back on one stream -> one launch: 51.0 / 120.7
-  // -> 47.8 / 109 -> 37.4 / 81.1 us (the last two with the gathers' all-loads form), at 48^3
-  // (about 430 blocks) 59.2 / 138.7 -> 58.8 / 127.5 us, -> 53.8 / 117.5 us in one launch; at
-  // 64^3 (about 1030 blocks) the fork is the faster (NVT 74.0 vs 76.4 us back to back), at
-  // 96^3 too (NPT 329 vs 343 us). The averaged model's kernels are short in either kind and the
+  // and join cost: it runs both kinds of block in one launch (cell_kernel_both). NVT-NHC step, NPT
+  // step and evaluation, one launch / fork, a fifth of the cells two-state: 32^3 (122 blocks) 34 / 43,
+  // 67 / 79 and 16 / 45 us, 48^3 (410) 48 / 53, 92 / 100 and 21 / 46 us; above the line 56^3 (652)
+  // 64 / 64, 130 / 140 and 29 / 46 us, 64^3 (974) 73 / 74, 155 / 162 and 38 / 48 us, 72^3 (1385)
+  // 88 / 83, 188 / 187 and 52 / 57 us, 80^3 (1900) 104 / 98, 219 / 206 and 65 / 67 us, 96^3 154 / 140,
+  // 330 / 293 and 104 / 101 us, 128^3 310 / 279, 675 / 564 and 224 / 202 us: between 512 and some
+  // 1000 blocks one launch would still be the faster in NPT and single evaluations.
+  // The averaged model's kernels are short in either kind and the
   // device holds twice as many, so that the fork pays later: one launch against two, a fifth of
   // the cells two-state, whole evaluation of 61x64x67 (1022 blocks) 27 / 50 us, 96^3 88 / 94,
   // 104^3 108 / 115, 112^3 136 / 136, 128^3 197 / 197, 160^3 419 / 396 (with seven of ten cells
@@ -360,8 +362,7 @@ hipError_t launch_cells(const ForceArgs& a, hipStream_t stream) {
   // The multistate instance is launched first, on the caller's stream: its blocks hold twice the
   // time and 74 KB of LDS each, and started behind the single-state instance they find their
   // place only as that drains (npt 128^3 step 0.580 -> 0.576 ms; equal at 72x80x96 with seven
-  // of ten cells two-state).
-  // a pass that the device holds at once, with blocks of both kinds: one launch
+  // of ten cells two-state). Passes of few blocks of both kinds: one launch.
   const bool both = mn > 0 && sn > 0 && nb <= one;
 #define MM_LAUNCH_BOTH(MODEL, OUT)                                                           \
   hipLaunchKernelGGL((cell_kernel_both<MODEL, OUT>), dim3(nb), dim3(kCellBlock), 0, stream,     \
@@ -694,8 +695,8 @@ hipError_t launch_cg_stats(const double* x, const double* xo, const double* g, c
 // Parameter table entries (row t, state s) from device arrays, one wave per entry and one lane per
 // matrix element, with the arithmetic of the host builder (Voigt input, metric_entry), so both give
 // the same bits; entries of states beyond nstates[t] are zero. kt[t] = boltzmann * temp_eff[t]. A
-// serial chain bounds it, the inverse and its residual above all: 5.9 us; one thread per entry, without
-// the residual, took 6.5 us.
+// serial chain bounds it, the inverse and its residual above all: 5.9 to 6.7 us; one thread per entry,
+// without the residual, took 6.5 us.
 __global__ void __launch_bounds__(64)
 build_table_kernel(int corner8, int max_states, const int32_t* __restrict__ nstates,
                    const double* __restrict__ h0, const double* __restrict__ cv,

@@ -52,7 +52,7 @@ struct mm_field {
   std::vector<int32_t> blk_row_host;  // [W/256] copy of blk_row
   std::vector<int32_t> nstates_host;  // [nrows] copy of nstates
   int split = -1;                     // see ForceArgs::split
-  hipStream_t side = nullptr;         // multistate instance of the cell pass runs here
+  hipStream_t side = nullptr;         // the single-state instance of a large cell pass runs here
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
 };
 

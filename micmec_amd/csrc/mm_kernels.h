@@ -11,11 +11,12 @@ constexpr int kCellBlock = 256;
 // concurrently; smaller ones run both kinds of block in one launch (cell_kernel_both).
 constexpr int kForkMinBlocks = 512, kForkMinBlocksAveraged = 4608;
 // Node gathers over at most this many 256-node blocks (at most four waves a SIMD) load all of
-// a node's records at once (sum_node_records<true>): latency bounds such a pass. NVT-NHC / NPT
-// step, records one at a time -> all at once: 32^3 46.3 / 105.9 -> 43.9 / 103.4 us, 48^3
-// 57.5 / 126.5 -> 54.1 / 121.6 us, 64^3 74.4 / 170.4 -> 73.3 / 170.9 us; with more blocks the
-// extra registers cost more than the loads in flight gain (80^3 NPT 223 -> 234 us, 128^3
-// 650 -> 666 us). The same bits either way.
+// a node's records at once (sum_node_records<true>): latency bounds such a pass. NVT-NHC step, NPT
+// step and evaluation, records one at a time -> all at once: 32^3 37.0 / 70.7 / 17.9 -> 33.8 / 67.4 /
+// 15.9 us, 48^3 50.8 / 94.4 / 24.0 -> 48.3 / 92.3 / 21.0 us, 64^3 73.5 / 163.4 / 50.3 -> 74.5 /
+// 162.3 / 47.8 us; with more blocks the extra registers cost more than the loads in flight gain
+// (80^3 96.1 / 205.9 / 66.8 -> 100.9 / 216.1 / 70.6 us, 128^3 280 / 569 / 203 -> 287 / 584 / 211 us).
+// The same bits either way.
 constexpr int kGatherAllLoadsMaxBlocks = 1024;
 // Single-system fields of at most this many work slots and nodes are evaluated in one launch by
 // one workgroup (force_small_kernel).
@@ -58,7 +59,8 @@ struct ForceArgs {
   const double* xmat2 = nullptr;
   const double* xmat2_on = nullptr;
   int split = -1;           // multistate blocks are [0, split), single-state [split, nb); -1: mixed
-  hipStream_t side = nullptr;   // stream of the multistate instance (null: the caller's stream)
+  // stream of the single-state instance where the two run concurrently (null: the caller's stream)
+  hipStream_t side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
 };
 

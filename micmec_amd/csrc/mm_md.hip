@@ -361,7 +361,7 @@ __device__ __forceinline__ void fma_matmul(const double (&A)[9], const double (&
 // (its first omitted term r^7 / 7! is then below 1e-17; a barostat velocity times dt / 2 is of
 // order 1e-5 to 1e-3), as I + X + X^2 / 2 + X^3 (I / 6 + X / 24 + X^2 / 120 + X^3 / 720), and of
 // degree 14 otherwise (the remainder is at most e^r times the first omitted term against
-// ||exp(X)|| >= e^-r: below 3e-17 relative at r = 1/2); the result is squared s times.
+// ||exp(X)|| >= e^-r: below 7e-17 relative at r = 1/2); the result is squared s times.
 __device__ __forceinline__ void expm_sym_half(const double (&A)[9], double sign, double dt,
                                               double (&P)[9]) {
 #pragma clang fp contract(off)
@@ -1282,7 +1282,7 @@ kick_drift_kernel(double* __restrict__ x, double* __restrict__ v, const double* 
 // With kDrift instead, the first half kick and the drift of the step (verlet.py:141-146) with
 // the barostat's pre-call gradient, which nothing else reads: the pending velocity transforms
 // (and the Langevin thermostat's pre update, its ekin after the update in partial row 15),
-// then v += a dt / 2 and x += dt v, as the node pass kKickDrift does from a stored gpos, with
+// then v += a dt / 2 and x += dt v, as kick_drift_kernel does from a stored gpos, with
 // x first taken through the barostat call's pending position scaling (the previous post
 // call's when it still waits, then the pre call's), which its cell pass applied on the fly.
 // With kKick and kDrift, the second half kick of a step and the first half kick and drift of the next
