@@ -215,6 +215,10 @@ class DiffField(object):
         kw = dict(dtype=torch.float64, device=self.device)
         cv, h0, free, teff = [x.detach().to(**kw).contiguous() for x in ts]
         ns = np.ascontiguousarray(params.nstates, dtype=np.int32)
+        T, S = self.nrows, self.max_states
+        if ns.size < T or cv.numel() < 36 * T * S or h0.numel() < 9 * T * S or \
+                free.numel() < T * S or teff.numel() < T:
+            raise ValueError("parameters must cover %d types of %d states" % (T, S))
         rc = self.lib.mm_field_set_params_device(
             self._field, ns.ctypes.data_as(ctypes.c_void_p), _native.ptr(h0), _native.ptr(cv),
             _native.ptr(free), _native.ptr(teff), float(units.boltzmann), _native.stream_ptr())

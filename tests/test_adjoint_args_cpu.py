@@ -114,3 +114,19 @@ def test_accepted(loss, monkeypatch):
     grads = torch.autograd.grad(out, (pos,) + p.tensors())
     assert grads[0].shape == pos.shape
     assert field.lib.calls[-1] == ("mm_fit_backward" if loss else "mm_adjoint_backward")
+
+
+@pytest.mark.parametrize("which", range(5))
+def test_short_parameters_refused(which, monkeypatch):
+    """Parameter tensors (or state counts) of fewer entries than the field's table has."""
+    field = field_of(False, monkeypatch)
+    field.nrows, field.max_states = 2, 3
+    full = [torch.zeros(s, dtype=torch.float64)
+            for s in ((2, 3, 36), (2, 3, 9), (6,), (2,))] + [[3, 1]]
+    short = list(full)
+    short[which] = full[which][:-1]
+    with pytest.raises(ValueError):
+        field.set_params(CellParams(*short))
+    field.lib.allowed = True
+    field.set_params(CellParams(*full))
+    assert field.lib.calls == ["mm_field_set_params_device"]
